@@ -126,22 +126,24 @@ int32_t tqmoe_dedup_maps(const int32_t * ids, const int32_t * slot_of, int32_t c
  * src/formats/weight/q4.cpp:295-326, 495-530, 577-606, 802-836). Per 32 weights of a row (a sub-block):
  *   IQ4_XS  codes 16 B: byte j = weights j (low nibble) and j + 16 (high) of the sub-block (GGUF order);
  *           aux 8 B per 256 weights: GGUF's d (f16), scales_h, scales_l[4] repacked (the eight 6-bit scales minus 32 as
- *           signed 6-bit fields, d in the 16 bits between them). Rows are stored in tiles of 32: the 16 B
- *           of sub-block s of the 32 rows of a tile are contiguous (512 B), tiles of a row group follow each other by
- *           sub-block, and the 8 B records likewise (256 B per tile and super-block); rows must be a multiple of 32.
- *           The other formats are row-major (codes of a row contiguous, then its records).
+ *           signed 6-bit fields, d in the 16 bits between them); rows must be a multiple of 32.
+ *           IQ4_XS, Q4_K, Q6_K, IQ3_S and NVFP4G are tile-major: rows are stored in tiles of 32 (the last tile of a bank may
+ *           have fewer, except IQ4_XS), and the same piece of a tile's rows is contiguous (16 B of 32 rows are 512 B),
+ *           pieces of a tile following each other along the row; records likewise. The other formats are row-major
+ *           (codes of a row contiguous, then its records).
  *   Q4_K    codes 16 B in the same nibble order; aux 16 B per 256 weights: d, dmin (f16), scales[12] as in GGUF.
- *   IQ3_S   codes 12 B: 8 lattice index bytes then 4 sign bytes; aux 16 B per 256 weights: d (f16), qh[8],
- *           scales[4], 2 B padding.
+ *   IQ3_S   codes 96 B per 256 weights: four 16 B pieces (8 low lattice index bytes of each of two sub-blocks), then two
+ *           16 B pieces (a dword of sign bits for each of four sub-blocks), in the order of the matrix operand; aux 16 B per
+ *           256 weights: d (f16), scale bytes 0 and 1, a byte of ninth index bits per sub-block, scale bytes 2 and 3, 2 B padding.
  *   NVFP4G  codes 16 B in the same nibble order (weights j and j + 16 of the sub-block); aux: one E4M3 scale per
- *           16 weights, [rows_total][cols / 16] bytes, then at the next multiple of 16 bytes rows_total fp32 globals
+ *           16 weights in pieces of 8 B, then at the next multiple of 16 bytes rows_total fp32 globals
  *           (one per row; rows whose blocks disagree are rejected by the reference loader, q4.cpp:519-521, and by
  *           tqmoe_bank_load through *status).
  *   Q5_K    codes 16 B: the low four bits in the same nibble order; aux 48 B per 256 weights: d, dmin, scales[12] as in
  *           GGUF, then one 32-bit word per sub-block with the fifth bit of its weights (bit j = weight j).
- *   Q6_K    codes 24 B: 16 B of low nibbles in the same order, then 8 B with the upper two bits (byte k = weights
- *           4 k .. 4 k + 3); aux 32 B per 256 weights: the sixteen int8 scales in GGUF order (two per sub-block), d (f16),
- *           padding.
+ *   Q6_K    codes 192 B per 256 weights: eight 16 B pieces of low nibbles in the same order, then four 16 B pieces with the
+ *           upper two bits of two sub-blocks each, in the order of the matrix operand; aux 32 B per 256 weights: the
+ *           sixteen int8 scales in GGUF order (two per sub-block), d (f16), padding.
  *   IQ3_XXS codes 12 B: 8 lattice index bytes, then GGUF's word of four 7-bit sign fields and the 4-bit scale; aux 16 B per
  *           256 weights: d (f16), padding.
  *   IQ2_S   codes 12 B: 4 low index bytes, 4 sign bytes, the sub-block's qh byte, its scale byte, 2 B padding; aux as

@@ -1,0 +1,39 @@
+"""GPU parity of the decode products of the tile-major formats where their split can go wrong: a row cut over five, six and
+seven waves, ragged last tiles (the row-wise kernels take them), batches that stage their input rows and that walk several
+row tiles a wave, more input rows of one expert than a block serves. Against float64 on the decoded weights."""
+import numpy as np
+import pytest
+import torch
+
+import synth
+from gpu_util import dev
+
+pytestmark = pytest.mark.gpu
+
+FORMATS = {"iq4_xs": 23, "q4_k": 12, "q6_k": 14, "iq3_s": 21, "nvfp4": 323}
+SHAPES = [(64, 1280, 1, 3), (96, 1536, 2, 3), (32, 1792, 1, 2), (40, 512, 5, 3), (33, 768, 14, 3), (1024, 512, 40, 4), (160, 2304, 13, 1)]
+
+
+@pytest.mark.parametrize("fmt", sorted(FORMATS))
+@pytest.mark.parametrize("rows,cols,n,experts", SHAPES)
+def test_decode_products(oracle, fmt, rows, cols, n, experts):
+    import tqllm_amd as tq
+    wtype = FORMATS[fmt]
+    if fmt == "iq4_xs" and rows % 32:
+        pytest.skip("IQ4_XS experts have whole tiles")
+    rng = np.random.default_rng(rows + cols + n)
+    k = min(2, experts)
+    raw = oracle.quantize(wtype, (rng.standard_normal((experts * rows, cols)) * 0.02).astype(np.float32))
+    bank = tq.ExpertBank(wtype, raw, experts, rows, cols)
+    dec = oracle.dequantize(wtype, raw, experts * rows * cols).reshape(experts, rows, cols).astype(np.float64)
+    x = rng.standard_normal((n, cols)).astype(np.float32)
+    xe = rng.standard_normal((n * k, cols)).astype(np.float32)
+    ids = np.stack([rng.permutation(experts)[:k] for _ in range(n)]).astype(np.int32)
+    two = tq.expert_matvec2(bank, bank, tq.quant_act(dev(x)), dev(ids))
+    one = tq.expert_matvec(bank, tq.quant_act(dev(xe)), dev(ids), per_expert_input=True)
+    torch.cuda.synchronize()
+    assert torch.equal(two[0], two[1])
+    for got, rows_in in ((two[0], np.repeat(x, k, axis=0)), (one, xe)):
+        want = np.stack([dec[e] @ rows_in[a].astype(np.float64) for a, e in enumerate(ids.reshape(-1))])
+        mx, rel = synth.errors(got.cpu().numpy(), want)
+        assert rel < 2e-4 and mx < 1e-3, (mx, rel)

@@ -23,10 +23,16 @@ template <class F> __device__ __forceinline__ void pack_sub(uint8_t * dst, F cod
 __global__ __launch_bounds__(256) void load_k(uint32_t type, const uint8_t * __restrict__ src, int64_t rows_total, int cols,
                                               uint8_t * __restrict__ codes, uint8_t * __restrict__ aux, int * __restrict__ status) {
     const int S = cols / 32;
-    const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= rows_total * S) return;
-    const int64_t row = idx / S;
-    const int s = int(idx % S);
+    int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x, row = idx / S;
+    int s = int(idx % S);
+    if (is_tile_major(type)) {   // a block per tile and super-block: what it writes is one contiguous piece of the planes
+        const int nsb = (S + 7) / 8;
+        row = int64_t(blockIdx.x) / nsb * 32 + (threadIdx.x >> 3);
+        s = int(blockIdx.x % nsb) * 8 + (threadIdx.x & 7);
+        idx = row * S + s;
+    }
+    if (row >= rows_total || s >= S) return;
+    const int h = tile_rows(row, rows_total);
     uint8_t * cd = codes + idx * code_bytes_per_sub(type);
     switch (type) {
         case TQMOE_IQ4_XS: {  // 136 B per 256: d, scales_h, scales_l[4], qs[128]; nibble order already canonical; tile-major
@@ -44,9 +50,9 @@ __global__ __launch_bounds__(256) void load_k(uint32_t type, const uint8_t * __r
             const uint8_t * blk = src + (row * (S / 8) + s / 8) * 144;
             const int ib = s & 7;
             const uint8_t * q = blk + 16 + 32 * (ib >> 1);
-            pack_sub(cd, [&](int j) { return (ib & 1) ? q[j] >> 4 : q[j] & 15; });
+            pack_sub(codes + tiled(row, h, S, s, 16), [&](int j) { return (ib & 1) ? q[j] >> 4 : q[j] & 15; });
             if (ib == 0) {
-                uint8_t * a = aux + (row * (S / 8) + s / 8) * 16;
+                uint8_t * a = aux + tiled(row, h, S / 8, s / 8, 16);
                 *reinterpret_cast<uint4 *>(a) = make_uint4(rd_u32(blk), rd_u32(blk + 4), rd_u32(blk + 8), rd_u32(blk + 12));
             }
             break;
@@ -54,14 +60,29 @@ __global__ __launch_bounds__(256) void load_k(uint32_t type, const uint8_t * __r
         case TQMOE_IQ3_S: {  // 110 B per 256: d, qs[64], qh[8], signs[32], scales[4]
             const uint8_t * blk = src + (row * (S / 8) + s / 8) * 110;
             const int ib = s & 7;
-            uint32_t * o = reinterpret_cast<uint32_t *>(cd);
-            o[0] = rd_u32(blk + 2 + 8 * ib);
-            o[1] = rd_u32(blk + 2 + 8 * ib + 4);
-            o[2] = rd_u32(blk + 74 + 4 * ib);
+            const uint32_t sg = rd_u32(blk + 74 + 4 * ib);   // bit l: weight l
+            uint32_t signs = 0;
+#pragma unroll
+            for (int g = 0; g < 2; ++g) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int grp = operand_group(g, q);
+                    w |= uint32_t(blk[2 + 8 * ib + grp]) << (8 * q);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) signs |= ((sg >> (4 * grp + j)) & 1u) << (8 * j + 4 * g + q);
+                }
+                *reinterpret_cast<uint32_t *>(codes + iq3s_qs_offset(row, h, S, s, g)) = w;
+            }
+            *reinterpret_cast<uint32_t *>(codes + iq3s_sign_offset(row, h, S, s)) = signs;
+            uint8_t * a = aux + tiled(row, h, S / 8, s / 8, 16);
+            uint32_t qh = 0;   // the ninth index bits, in operand order
+#pragma unroll
+            for (int b = 0; b < 8; ++b) qh |= ((uint32_t(blk[66 + ib]) >> operand_group(b >> 2, b & 3)) & 1u) << b;
+            a[4 + ib] = uint8_t(qh);
             if (ib == 0) {
-                uint8_t * a = aux + (row * (S / 8) + s / 8) * 16;
-                *reinterpret_cast<uint4 *>(a) = make_uint4(rd_u16(blk) | rd_u16(blk + 66) << 16, rd_u32(blk + 68),
-                                                           rd_u16(blk + 72) | rd_u16(blk + 106) << 16, rd_u16(blk + 108));
+                *reinterpret_cast<uint32_t *>(a) = rd_u16(blk) | rd_u16(blk + 106) << 16;
+                *reinterpret_cast<uint32_t *>(a + 12) = rd_u16(blk + 108);
             }
             break;
         }
@@ -174,16 +195,18 @@ __global__ __launch_bounds__(256) void load_k(uint32_t type, const uint8_t * __r
             const uint8_t * blk = src + (row * (S / 8) + s / 8) * 210;
             const int ib = s & 7, n = ib >> 2, j = ib & 3;
             const uint8_t * ql = blk + 64 * n + 32 * (j & 1), * qh = blk + 128 + 32 * n;
-            __attribute__((aligned(16))) uint8_t low[16];   // 24-byte code records are 8-byte aligned: stored as three 8-byte pieces
-            pack_sub(low, [&](int l) { return (j & 2) ? ql[l] >> 4 : ql[l] & 15; });
-            reinterpret_cast<uint2 *>(cd)[0] = reinterpret_cast<const uint2 *>(low)[0];
-            reinterpret_cast<uint2 *>(cd)[1] = reinterpret_cast<const uint2 *>(low)[1];
-            uint32_t hi[2] = {0, 0};   // two bits per weight, byte k = weights 4 k .. 4 k + 3
+            pack_sub(codes + q6k_low_offset(row, h, S, s), [&](int l) { return (j & 2) ? ql[l] >> 4 : ql[l] & 15; });
 #pragma unroll
-            for (int l = 0; l < 32; ++l) hi[l >> 4] |= uint32_t((qh[l] >> (2 * j)) & 3) << (2 * (l & 15));
-            *reinterpret_cast<uint2 *>(cd + 16) = make_uint2(hi[0], hi[1]);
+            for (int g = 0; g < 2; ++g) {
+                uint32_t w = 0;
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) w |= (((uint32_t(qh[4 * operand_group(g, q) + b]) >> (2 * j)) & 3u) ^ 2u) << (8 * b + 2 * q);
+                *reinterpret_cast<uint32_t *>(codes + q6k_high_offset(row, h, S, s, g)) = w;
+            }
             if (ib == 0) {
-                uint8_t * a = aux + (row * (S / 8) + s / 8) * 32;
+                uint8_t * a = aux + tiled(row, h, S / 8, s / 8, 32);
                 *reinterpret_cast<uint4 *>(a) = make_uint4(rd_u32(blk + 192), rd_u32(blk + 196), rd_u32(blk + 200), rd_u32(blk + 204));
                 *reinterpret_cast<uint4 *>(a + 16) = make_uint4(rd_u16(blk + 208), 0, 0, 0);
             }
@@ -207,8 +230,8 @@ __global__ __launch_bounds__(256) void load_k(uint32_t type, const uint8_t * __r
             const uint8_t * blk = src + (row * (S / 4) + s / 4) * 76;
             const int q4 = s & 3;
             const uint8_t * q = blk + 12 + 16 * q4;  // two 16-groups
-            pack_sub(cd, [&](int j) { const uint8_t b = q[8 * (j >> 4) + ((j & 15) >> 1)]; return (j & 1) ? b >> 4 : b & 15; });
-            uint8_t * a = aux + row * (cols / 16) + 2 * s;
+            pack_sub(codes + tiled(row, h, S, s, 16), [&](int j) { const uint8_t b = q[8 * (j >> 4) + ((j & 15) >> 1)]; return (j & 1) ? b >> 4 : b & 15; });
+            uint8_t * a = aux + nvfp4_scale_offset(row, h, S, s);
             a[0] = blk[4 + 2 * q4];
             a[1] = blk[4 + 2 * q4 + 1];
             const uint32_t g = rd_u32(blk), g0 = rd_u32(src + row * (S / 4) * 76);
@@ -261,9 +284,9 @@ extern "C" int32_t tqmoe_bank_load(uint32_t type, const void * gguf_blocks, int6
     if (int32_t rc = tqmoe_bank_layout(type, rows_total, cols, nullptr, nullptr, err)) return rc;
     if (!gguf_blocks || !codes || !aux) return fail(err, TQMOE_E_ARG, "tqmoe_bank_load: null pointer");
     if (int32_t rc = need_device(err, "tqmoe_bank_load")) return rc;
-    const int64_t subs = rows_total * (cols / 32);
-    if ((subs + 255) / 256 > 0x7FFFFFFF) return fail(err, TQMOE_E_ARG, "tqmoe_bank_load: bank too large for one call");
-    load_k<<<unsigned((subs + 255) / 256), 256, 0, static_cast<hipStream_t>(stream)>>>(type, static_cast<const uint8_t *>(gguf_blocks), rows_total, cols,
+    const int64_t blocks = is_tile_major(type) ? (rows_total + 31) / 32 * ((cols + 255) / 256) : (rows_total * (cols / 32) + 255) / 256;
+    if (blocks > 0x7FFFFFFF) return fail(err, TQMOE_E_ARG, "tqmoe_bank_load: bank too large for one call");
+    load_k<<<unsigned(blocks), 256, 0, static_cast<hipStream_t>(stream)>>>(type, static_cast<const uint8_t *>(gguf_blocks), rows_total, cols,
                                                                                       static_cast<uint8_t *>(codes), static_cast<uint8_t *>(aux), status);
     return launched(err, "tqmoe_bank_load");
 }

@@ -16,6 +16,7 @@
 #pragma once
 #include "act_image.cuh"
 #include "decode_api.cuh"
+#include "decode_mfma_kernels.cuh"
 #include "formats.cuh"
 
 namespace tqmoe {
@@ -64,16 +65,19 @@ template <bool SPLIT, bool HALF_MINS = false> __device__ __forceinline__ float d
     }
 }
 
-// Uniform base pointers of one bank for the rows [row0, ...) of expert e: lanes add 32-bit offsets to them.
-struct Tile { const uint8_t * codes; const uint8_t * aux; const uint8_t * aux2; };
-template <uint32_t FMT> __device__ __forceinline__ Tile tile_of(const BankView & b, int e, int row0) {
-    const int64_t row = int64_t(e) * b.rows + row0;
+// Uniform base pointers of one bank for the rows [row0, ...) of expert e: lanes add 32-bit offsets to them. Tile-major
+// formats: the planes themselves, the stacked row and the bank's rows.
+struct Tile { const uint8_t * codes; const uint8_t * aux; const uint8_t * aux2; int64_t row, rows_total; };
+template <uint32_t FMT> __device__ __forceinline__ Tile tile_at(const BankView & b, int64_t row) {
     Tile t;
-    t.codes = b.codes + row * code_row_bytes(FMT, b.cols);
-    t.aux = b.aux + row * aux_row_bytes(FMT, b.cols);
-    t.aux2 = FMT == TQMOE_NVFP4G ? b.aux + nvfp4_global_offset(b.rows_total, b.cols) + row * 4 : nullptr;
+    t.codes = b.codes + (is_tile_major(FMT) ? 0 : row * code_row_bytes(FMT, b.cols));
+    t.aux = b.aux + (is_tile_major(FMT) ? 0 : row * aux_row_bytes(FMT, b.cols));
+    t.aux2 = FMT == TQMOE_NVFP4G ? b.aux + nvfp4_global_offset(b.rows_total, b.cols) : nullptr;
+    t.row = row;
+    t.rows_total = b.rows_total;
     return t;
 }
+template <uint32_t FMT> __device__ __forceinline__ Tile tile_of(const BankView & b, int e, int row0) { return tile_at<FMT>(b, int64_t(e) * b.rows + row0); }
 
 template <uint32_t FMT> struct Sub;
 
@@ -82,8 +86,10 @@ template <> struct Sub<TQMOE_Q4_K> {
     struct Raw { uint4 c; uint4 rec; };
     static __device__ __forceinline__ Raw load(const Tile & t, uint32_t r, uint32_t S, uint32_t s) {
         Raw v;
-        v.c = *reinterpret_cast<const uint4 *>(t.codes + (r * S + s) * 16u);
-        v.rec = *reinterpret_cast<const uint4 *>(t.aux + (r * (S >> 3) + (s >> 3)) * 16u);
+        const int64_t row = t.row + r;
+        const int h = tile_rows(row, t.rows_total);
+        v.c = *reinterpret_cast<const uint4 *>(t.codes + tiled(row, h, int(S), int(s), 16));
+        v.rec = *reinterpret_cast<const uint4 *>(t.aux + tiled(row, h, int(S >> 3), int(s >> 3), 16));
         return v;
     }
     static __device__ __forceinline__ void decode(const Raw & r, int s, const uint32_t *, Dec & d) {
@@ -323,26 +329,28 @@ template <> struct Sub<TQMOE_Q5_K> {
 
 template <> struct Sub<TQMOE_Q6_K> {
     static constexpr bool kSplit = true;   // one scale per 16 weights: the sub-block's halves
-    struct Raw { uint2 c[3]; uint32_t sc; uint32_t d; };
+    struct Raw { uint4 c; uint32_t h[2]; uint32_t sc; uint32_t d; };
     static __device__ __forceinline__ Raw load(const Tile & t, uint32_t r, uint32_t S, uint32_t s) {
         Raw v;
-        const uint2 * cp = reinterpret_cast<const uint2 *>(t.codes + (r * S + s) * 24u);
-        v.c[0] = cp[0]; v.c[1] = cp[1]; v.c[2] = cp[2];
-        const uint8_t * a = t.aux + (r * (S >> 3) + (s >> 3)) * 32u;
+        const int64_t row = t.row + r;
+        const int h = tile_rows(row, t.rows_total);
+        v.c = *reinterpret_cast<const uint4 *>(t.codes + q6k_low_offset(row, h, int(S), int(s)));
+        v.h[0] = *reinterpret_cast<const uint32_t *>(t.codes + q6k_high_offset(row, h, int(S), int(s), 0));
+        v.h[1] = *reinterpret_cast<const uint32_t *>(t.codes + q6k_high_offset(row, h, int(S), int(s), 1));
+        const uint8_t * a = t.aux + tiled(row, h, int(S >> 3), int(s >> 3), 32);
         v.sc = *reinterpret_cast<const uint16_t *>(a + 2u * (s & 7u));
         v.d = *reinterpret_cast<const uint16_t *>(a + 16u);
         return v;
     }
     static __device__ __forceinline__ void decode(const Raw & r, int, const uint32_t *, Dec & d) {
-        const uint32_t w[4] = {r.c[0].x, r.c[0].y, r.c[1].x, r.c[1].y};
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            uint32_t lo, hi;
-            nibbles(w[q], lo, hi);
-            d.w[q] = minus32(lo | spread2x4(r.c[2].x >> (8 * q)) << 4);
-            d.w[4 + q] = minus32(hi | spread2x4(r.c[2].y >> (8 * q)) << 4);
+        for (int g = 0; g < 2; ++g) {
+            uint32_t w[4];
+            q6k_times4(g ? make_uint2(r.c.z, r.c.w) : make_uint2(r.c.x, r.c.y), r.h[g], w);
+#pragma unroll
+            for (int q = 0; q < 4; ++q) d.w[operand_group(g, q)] = w[q];
         }
-        const float dd = half_bits_to_float(uint16_t(r.d));
+        const float dd = 0.25f * half_bits_to_float(uint16_t(r.d));
         d.s0 = dd * float(int8_t(r.sc & 0xFFu));
         d.s1 = dd * float(int8_t(r.sc >> 8));
         d.mn = 0.f;
@@ -390,9 +398,11 @@ template <> struct Sub<TQMOE_NVFP4G> {
     struct Raw { uint4 c; uint32_t sc; float g; };
     static __device__ __forceinline__ Raw load(const Tile & t, uint32_t r, uint32_t S, uint32_t s) {
         Raw v;
-        v.c = *reinterpret_cast<const uint4 *>(t.codes + (r * S + s) * 16u);
-        v.sc = *reinterpret_cast<const uint16_t *>(t.aux + (r * S + s) * 2u);
-        v.g = *reinterpret_cast<const float *>(t.aux2 + r * 4u);
+        const int64_t row = t.row + r;
+        const int h = tile_rows(row, t.rows_total);
+        v.c = *reinterpret_cast<const uint4 *>(t.codes + tiled(row, h, int(S), int(s), 16));
+        v.sc = *reinterpret_cast<const uint16_t *>(t.aux + nvfp4_scale_offset(row, h, int(S), int(s)));
+        v.g = *reinterpret_cast<const float *>(t.aux2 + row * 4);
         return v;
     }
     static __device__ __forceinline__ void decode(const Raw & r, int, const uint32_t *, Dec & d) {
@@ -408,29 +418,31 @@ template <> struct Sub<TQMOE_NVFP4G> {
 
 template <> struct Sub<TQMOE_IQ3_S> {
     static constexpr bool kSplit = false;
-    struct Raw { uint32_t c[3]; uint4 rec; };
+    struct Raw { uint32_t qs[2], sg; uint4 rec; };
     static __device__ __forceinline__ Raw load(const Tile & t, uint32_t r, uint32_t S, uint32_t s) {
         Raw v;
-        const uint32_t * cp = reinterpret_cast<const uint32_t *>(t.codes + (r * S + s) * 12u);
-        v.c[0] = cp[0]; v.c[1] = cp[1]; v.c[2] = cp[2];
-        v.rec = *reinterpret_cast<const uint4 *>(t.aux + (r * (S >> 3) + (s >> 3)) * 16u);
+        const int64_t row = t.row + r;
+        const int h = tile_rows(row, t.rows_total);
+        v.qs[0] = *reinterpret_cast<const uint32_t *>(t.codes + iq3s_qs_offset(row, h, int(S), int(s), 0));
+        v.qs[1] = *reinterpret_cast<const uint32_t *>(t.codes + iq3s_qs_offset(row, h, int(S), int(s), 1));
+        v.sg = *reinterpret_cast<const uint32_t *>(t.codes + iq3s_sign_offset(row, h, int(S), int(s)));
+        v.rec = *reinterpret_cast<const uint4 *>(t.aux + tiled(row, h, int(S >> 3), int(s >> 3), 16));
         return v;
     }
     // grid: the 512-entry lattice in LDS
     static __device__ __forceinline__ void decode(const Raw & r, int s, const uint32_t * grid, Dec & d) {
         const int ib = s & 7;
-        const uint4 rec = r.rec;
-        const uint32_t qh = ib < 2 ? (rec.x >> (16 + 8 * ib)) & 0xFFu : ib < 6 ? (rec.y >> (8 * (ib - 2))) & 0xFFu : (rec.z >> (8 * (ib - 6))) & 0xFFu;
-        const uint32_t scb = (ib >> 1) < 2 ? (rec.z >> (16 + 8 * (ib >> 1))) & 0xFFu : (rec.w >> (8 * ((ib >> 1) - 2))) & 0xFFu;
+        const uint32_t qh = iq3s_qh(r.rec, ib);
 #pragma unroll
-        for (int w = 0; w < 8; ++w) {
-            const uint32_t g = grid[((r.c[w >> 2] >> (8 * (w & 3))) & 0xFFu) | (((qh >> w) & 1u) << 8)];
-            // four sign bits -> byte masks 0xFF; negate the selected bytes: (g ^ m) + (m & 0x01010101), no carry leaves a byte
-            const uint32_t bits = (((r.c[2] >> (4 * w)) & 15u) * 0x00204081u) & 0x01010101u;
-            const uint32_t m = (bits << 8) - bits;
-            d.w[w] = (g ^ m) + bits;
-        }
-        d.s0 = d.s1 = half_bits_to_float(uint16_t(rec.x & 0xFFFFu)) * float(1 + 2 * int((scb >> (4 * (ib & 1))) & 15u));
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t m = grid[((r.qs[g] >> (8 * q)) & 0xFFu) | (((qh >> (4 * g + q)) & 1u) << 8)];
+                // byte masks 0xFF of the sign bits: negate the selected bytes, (m ^ mask) + bits, no carry leaves a byte
+                const uint32_t bits = (r.sg >> (4 * g + q)) & 0x01010101u, mask = (bits << 8) - bits;
+                d.w[operand_group(g, q)] = (m ^ mask) + bits;
+            }
+        d.s0 = d.s1 = half_bits_to_float(uint16_t(r.rec.x & 0xFFFFu)) * float(1 + 2 * iq3s_ls(r.rec, ib));
         d.mn = 0.f;
     }
 };
@@ -647,12 +659,20 @@ template <uint32_t FMT, int LPR, int M> void launch_one_gateup(const GateupArgs 
 
 }  // namespace
 
+// The tile-major formats run on the matrix pipe; the kernels here take their ragged shapes only (rows that are no whole tiles,
+// a shared expert or columns that are no whole super-blocks).
 template <uint32_t FMT> void DecodeLaunch<FMT>::matvec(Split sp, int nb, const MatvecArgs & k, hipStream_t s) {
+    if constexpr (is_tile_major(FMT))
+        if (mfma_takes(k.b0.rows, k.b0.cols, k.shared_cols))
+            return mfma_launch<FMT>(nb, k.b0, k.b1, k.image, k.y0, k.y1, k.ytype, k.ids, k.A, k.xdiv, k.mode, k.slots, k.topk, k.shared_cols, 0, false, Glu{0.f, 0}, s);
 #define X(L, MM) if (sp.lpr == L && sp.m == MM) return launch_one_matvec<FMT, L, MM>(nb, k, s);
     TQMOE_FOR_SPLITS(X)
 #undef X
 }
 template <uint32_t FMT> void DecodeLaunch<FMT>::gateup(Split sp, const GateupArgs & k, hipStream_t s) {
+    if constexpr (is_tile_major(FMT))
+        if (mfma_takes(k.bg.rows, k.bg.cols, 0))
+            return mfma_launch<FMT>(2, k.bg, k.bu, k.ximage, k.aimage, nullptr, TQMOE_F32, k.ids, k.A, k.slots, k.mode, k.slots, k.topk, k.shared_ff, 1, true, k.glu, s);
 #define X(L, MM) if (sp.lpr == L && sp.m == MM) return launch_one_gateup<FMT, L, MM>(k, s);
     TQMOE_FOR_SPLITS(X)
 #undef X

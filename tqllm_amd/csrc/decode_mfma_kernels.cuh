@@ -1,0 +1,553 @@
+// Decode-sized products of the tile-major bank formats (IQ4_XS, Q4_K, Q6_K, IQ3_S, NVFP4G) on the matrix pipe.
+//
+// A block owns one expert, up to kTP of the input rows routed to it, and `tpw` tiles of 32 weight rows. Each wave takes
+// one row tile and a share of the row's 256-weight super-blocks. Per 32-weight sub-block a lane (n = lane % 32,
+// g = lane / 32) turns its half of weight row n's codes into 16 int8 values (MfmaFormat<FMT>::decode); that is operand
+// B of v_mfma_i32_32x32x32_i8 (of two v_mfma_i32_32x32x16_i8 where the format has a scale per 16 weights). Operand A is
+// the activation image: MFMA row 2j is the hi plane and row 2j + 1 the lo
+// plane of input row j (rows past 2 kTP repeat others), read straight from the image because its plane order is the order B's
+// bytes come in. The MFMA does the 32-term sums for all rows and planes at once, so no lane exchange is needed; its
+// result registers 0..3 of lane half g are (hi, lo) of input rows 2g and 2g + 1, which one fp32 multiply-add each folds
+// into the lane's running sum with weight scale * activation scale. Waves that split a row's super-blocks add their
+// partial sums through LDS in wave order (deterministic).
+// The weight bytes are the only cold data: every wave loads its share (codes and scale records) into registers one
+// super-block ahead of the one it is multiplying, so the loads of the next super-block are in flight while this one is
+// decoded.
+//
+// Why not v_dot4 products with a lane per sub-block (what the row-major formats run): those multiply every decoded weight
+// with both planes of every input row in the vector pipe (16 instructions per 32 weights and row) and serve two rows a
+// block; here the vector pipe only decodes and applies four scales per sub-block, and a block serves four rows.
+#pragma once
+#include "act_image.cuh"
+#include "decode_chunks.cuh"
+#include "decode_api.cuh"
+#include "formats.cuh"
+
+namespace tqmoe {
+namespace {
+
+typedef int v4i __attribute__((ext_vector_type(4)));
+typedef int v16i __attribute__((ext_vector_type(16)));
+
+constexpr int kTP = kChunkRowsMax;   // input rows per block
+constexpr int kMaxWaves = 8;
+
+// Sixteen-entry tables of int8 values looked up with two v_perm_b32 and one exclusive or. v_perm_b32 with selector bytes
+// 0..7 picks from an eight-byte pool; selectors 8..11 give 0x00 or 0xFF by the sign of pool bytes 1, 3, 5 and 7, 12
+// gives 0x00 and 13..15 give 0xFF. So pool A under the code c and pool B under c ^ 8 each give one of their entries for one
+// half of the codes and a known constant for the other half: with the other pool's constant folded into the entries
+// (entry ^ constant) the exclusive or of the two picks is the value. The constants depend on the sign bits of odd entries of
+// the other pool; taken in the order below every entry depends on entries already known. Eleven instructions for eight
+// codes; picking from both halves of the table and then between the picks takes thirteen.
+struct Table16 { uint32_t a0, a1, b0, b1; };
+constexpr Table16 table16(const int (&t)[16]) {
+    uint32_t a[8] = {}, b[8] = {};
+    auto neg = [](uint32_t v) { return (v & 0x80u) ? 0xFFu : 0u; };
+    auto val = [&](int i) { return uint32_t(t[i]) & 0xFFu; };
+    a[5] = val(5) ^ 0xFFu; a[6] = val(6) ^ 0xFFu; a[7] = val(7) ^ 0xFFu; a[4] = val(4);   // c = 4: selector 12 of pool B, 5..7: 13..15
+    b[5] = val(13) ^ 0xFFu; b[6] = val(14) ^ 0xFFu; b[7] = val(15) ^ 0xFFu; b[4] = val(12);
+    b[3] = val(11) ^ neg(a[7]); b[2] = val(10) ^ neg(a[5]);                             // codes 8..11: selectors 8..11 of pool A
+    a[3] = val(3) ^ neg(b[7]); a[2] = val(2) ^ neg(b[5]); a[1] = val(1) ^ neg(b[3]);
+    b[1] = val(9) ^ neg(a[3]); b[0] = val(8) ^ neg(a[1]);
+    a[0] = val(0) ^ neg(b[1]);
+    auto word = [](const uint32_t * v) { return v[0] | v[1] << 8 | v[2] << 16 | v[3] << 24; };
+    return Table16{word(a), word(a + 4), word(b), word(b + 4)};
+}
+constexpr int kIq4Table[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
+constexpr int kFp4Table[16] = {0, 1, 2, 3, 4, 6, 8, 12, 0, -1, -2, -3, -4, -6, -8, -12};   // twice the E2M1 values
+__device__ __forceinline__ uint32_t pick(const Table16 & t, uint32_t c) {   // four codes, one per byte
+    return __builtin_amdgcn_perm(t.a1, t.a0, c) ^ __builtin_amdgcn_perm(t.b1, t.b0, c ^ 0x08080808u);
+}
+__device__ __forceinline__ v4i decode_table(const Table16 & t, uint2 c) {
+    const uint32_t m = 0x0F0F0F0Fu;
+    return v4i{int(pick(t, c.x & m)), int(pick(t, (c.x >> 4) & m)), int(pick(t, c.y & m)), int(pick(t, (c.y >> 4) & m))};
+}
+
+// What the kernel needs of a format. A lane's part of a super-block: Codes and Rec, loaded from the tile's code and record
+// blocks (kCodeBytes, kRecBytes per tile and super-block). decode: operand B of sub-block ib. Scales: kGroups integer
+// scales per sub-block (kFloat: fp32 ones) with the super-block's d behind them; kMin: a minimum per sub-block times the
+// activations' sum. row_factor: a factor of the whole weight row.
+template <uint32_t FMT> struct MfmaFormat;
+struct MfmaBase {
+    static constexpr int kGroups = 1;
+    static constexpr bool kFloat = false, kMin = false, kRowFactor = false;
+    static constexpr int kLattice = 1;
+    static __device__ __forceinline__ float row_factor(const BankView &, int64_t) { return 1.f; }
+};
+struct MfmaNibbles : MfmaBase {   // sixteen code bytes a sub-block in the canonical order
+    static constexpr int kCodeBytes = 4096;
+    struct Codes { uint2 c[8]; };
+    static __device__ __forceinline__ void codes(const uint8_t * p, int n, int g, Codes & c) {
+        const uint8_t * q = p + n * 16 + g * 8;
+#pragma unroll
+        for (int ib = 0; ib < 8; ++ib) c.c[ib] = *reinterpret_cast<const uint2 *>(q + ib * 512);
+    }
+};
+template <> struct MfmaFormat<TQMOE_IQ4_XS> : MfmaNibbles {
+    static constexpr int kRecBytes = 256;
+    typedef uint2 Rec;
+    static __device__ __forceinline__ Rec rec(const uint8_t * p, int n) { return *reinterpret_cast<const uint2 *>(p + n * 8); }
+    static __device__ __forceinline__ v4i decode(const Codes & c, const Rec &, int ib, int, const uint32_t *) {
+        constexpr Table16 t = table16(kIq4Table);
+        return decode_table(t, c.c[ib]);
+    }
+    static __device__ __forceinline__ int scale(const Rec & r, int ib, int) { return iq4xs_lsm32(r, ib); }
+    static __device__ __forceinline__ float d(const Rec & r) { return half_bits_to_float(iq4xs_d_bits(r)); }
+};
+template <> struct MfmaFormat<TQMOE_Q4_K> : MfmaNibbles {
+    static constexpr int kRecBytes = 512;
+    static constexpr bool kMin = true;
+    typedef uint4 Rec;
+    static __device__ __forceinline__ Rec rec(const uint8_t * p, int n) { return *reinterpret_cast<const uint4 *>(p + n * 16); }
+    static __device__ __forceinline__ v4i decode(const Codes & c, const Rec &, int ib, int, const uint32_t *) {
+        const uint32_t m = 0x0F0F0F0Fu;
+        return v4i{int(c.c[ib].x & m), int((c.c[ib].x >> 4) & m), int(c.c[ib].y & m), int((c.c[ib].y >> 4) & m)};
+    }
+    static __device__ __forceinline__ int scale(const Rec & r, int ib, int) {
+        const uint32_t q[3] = {r.y, r.z, r.w};
+        int sc, mn;
+        q4k_scale_min(q, ib, sc, mn);
+        return sc;
+    }
+    static __device__ __forceinline__ float minimum(const Rec & r, int ib) {
+        const uint32_t q[3] = {r.y, r.z, r.w};
+        int sc, mn;
+        q4k_scale_min(q, ib, sc, mn);
+        return float(mn);
+    }
+    static __device__ __forceinline__ float d(const Rec & r) { return half_bits_to_float(uint16_t(r.x & 0xFFFFu)); }
+    static __device__ __forceinline__ float dmin(const Rec & r) { return half_bits_to_float(uint16_t(r.x >> 16)); }
+};
+template <> struct MfmaFormat<TQMOE_NVFP4G> : MfmaNibbles {
+    static constexpr int kRecBytes = 512, kGroups = 2;
+    static constexpr bool kFloat = true, kRowFactor = true;
+    typedef uint4 Rec;   // the sixteen scale bytes
+    static __device__ __forceinline__ Rec rec(const uint8_t * p, int n) {
+        const uint2 a = *reinterpret_cast<const uint2 *>(p + n * 8), b = *reinterpret_cast<const uint2 *>(p + 256 + n * 8);
+        return make_uint4(a.x, a.y, b.x, b.y);
+    }
+    static __device__ __forceinline__ v4i decode(const Codes & c, const Rec &, int ib, int, const uint32_t *) {
+        constexpr Table16 t = table16(kFp4Table);
+        return decode_table(t, c.c[ib]);
+    }
+    static __device__ __forceinline__ float scale(const Rec & r, int ib, int grp) {
+        const uint32_t w = ib < 2 ? r.x : ib < 4 ? r.y : ib < 6 ? r.z : r.w;
+        switch (2 * (ib & 1) + grp) {
+            case 0: return __builtin_amdgcn_cvt_f32_fp8(int(w), 0);
+            case 1: return __builtin_amdgcn_cvt_f32_fp8(int(w), 1);
+            case 2: return __builtin_amdgcn_cvt_f32_fp8(int(w), 2);
+            default: return __builtin_amdgcn_cvt_f32_fp8(int(w), 3);
+        }
+    }
+    static __device__ __forceinline__ float d(const Rec &) { return 1.f; }
+    static __device__ __forceinline__ float row_factor(const BankView & b, int64_t row) {   // half the row's global: the table holds twice the values
+        return 0.5f * *reinterpret_cast<const float *>(b.aux + nvfp4_global_offset(b.rows_total, b.cols) + row * 4);
+    }
+};
+template <> struct MfmaFormat<TQMOE_IQ3_S> : MfmaBase {
+    static constexpr int kCodeBytes = 3072, kRecBytes = 512, kLattice = 512;
+    struct Codes { uint2 qs[4]; uint4 sg[2]; };
+    typedef uint4 Rec;
+    static __device__ __forceinline__ void codes(const uint8_t * p, int n, int g, Codes & c) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c.qs[i] = *reinterpret_cast<const uint2 *>(p + i * 512 + n * 16 + g * 8);
+#pragma unroll
+        for (int i = 0; i < 2; ++i) c.sg[i] = *reinterpret_cast<const uint4 *>(p + 2048 + i * 512 + n * 16);
+    }
+    static __device__ __forceinline__ Rec rec(const uint8_t * p, int n) { return *reinterpret_cast<const uint4 *>(p + n * 16); }
+    // The lattice in LDS holds eight times the odd magnitudes: 8 (2 k + 1) is the byte k << 4 | 8, and its negative the same
+    // byte with the upper four bits inverted, so that a sign is one exclusive or.
+    static __device__ __forceinline__ v4i decode(const Codes & c, const Rec & r, int ib, int g, const uint32_t * lat) {
+        const uint32_t qs = (ib & 1) ? c.qs[ib >> 1].y : c.qs[ib >> 1].x;
+        const uint4 s4 = c.sg[ib >> 2];
+        const uint32_t sg = ((ib & 3) == 0 ? s4.x : (ib & 3) == 1 ? s4.y : (ib & 3) == 2 ? s4.z : s4.w) >> (4 * g);
+        const uint32_t qh = ((ib < 4 ? r.y : r.z) >> (8 * (ib & 3))) >> (4 * g);
+        v4i w;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t idx = ((qs >> (8 * q)) & 0xFFu) | ((qh << (8 - q)) & 0x100u);
+            const uint32_t mask = __builtin_amdgcn_perm(0u, 0x0000F000u, (sg >> q) & 0x01010101u);   // 0xF0 where the sign bit is set
+            w[q] = int(lat[idx] ^ mask);
+        }
+        return w;
+    }
+    static __device__ __forceinline__ int scale(const Rec & r, int ib, int) { return 1 + 2 * iq3s_ls(r, ib); }
+    static __device__ __forceinline__ float d(const Rec & r) { return 0.125f * half_bits_to_float(uint16_t(r.x & 0xFFFFu)); }
+};
+template <> struct MfmaFormat<TQMOE_Q6_K> : MfmaBase {
+    static constexpr int kCodeBytes = 6144, kRecBytes = 1024, kGroups = 2;
+    struct Codes { uint2 lo[8]; uint2 hi[4]; };
+    struct Rec { uint4 sc; uint32_t d; };
+    static __device__ __forceinline__ void codes(const uint8_t * p, int n, int g, Codes & c) {
+        const uint8_t * q = p + n * 16 + g * 8;
+#pragma unroll
+        for (int ib = 0; ib < 8; ++ib) c.lo[ib] = *reinterpret_cast<const uint2 *>(q + ib * 512);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c.hi[i] = *reinterpret_cast<const uint2 *>(q + 4096 + i * 512);
+    }
+    static __device__ __forceinline__ Rec rec(const uint8_t * p, int n) {
+        return Rec{*reinterpret_cast<const uint4 *>(p + n * 32), *reinterpret_cast<const uint16_t *>(p + n * 32 + 16)};
+    }
+    static __device__ __forceinline__ v4i decode(const Codes & c, const Rec &, int ib, int, const uint32_t *) {
+        uint32_t w[4];
+        q6k_times4(c.lo[ib], (ib & 1) ? c.hi[ib >> 1].y : c.hi[ib >> 1].x, w);
+        return v4i{int(w[0]), int(w[1]), int(w[2]), int(w[3])};
+    }
+    static __device__ __forceinline__ int scale(const Rec & r, int ib, int grp) {
+        const uint32_t w = ib < 2 ? r.sc.x : ib < 4 ? r.sc.y : ib < 6 ? r.sc.z : r.sc.w;
+        return __builtin_amdgcn_sbfe(int(w), 8 * (2 * (ib & 1) + grp), 8);
+    }
+    static __device__ __forceinline__ float d(const Rec & r) { return 0.25f * half_bits_to_float(uint16_t(r.d)); }
+};
+
+// NB banks (gate and up, or one). gateup != 0: out0 is the activation image that receives silu(gate) * up; else out0 /
+// out1 receive the products as rows of `ytype`. wk waves share a row's super-blocks, tpw row tiles per block.
+// Dynamic LDS: the match list and the copy of the ids while the block finds its input rows, later the partial sums.
+// UNI: every sub-block of an input row has the row's one activation scale (the images tqmoe_quant_act and the top-k
+// kernel write). The 6-bit weight scales then multiply the integer results and the sums stay integers over a whole
+// super-block; otherwise (rows quantised block by block, as the fused gate / up epilogue leaves them) each sub-block's
+// result is scaled in fp32.
+// MODE 0: input rows read straight from the image; 1: staged in LDS; 2: staged, and a wave takes tl_count row tiles in turn
+// Three waves a SIMD (168 registers) where that does not spill; two for the two-bank kernels of the formats with more codes or
+// scales in registers.
+template <uint32_t FMT, int NB, bool UNI, int MODE>
+constexpr int kDecodeWaves = NB == 2 && (FMT == TQMOE_Q6_K || (MODE == 0 && (FMT == TQMOE_Q4_K || (!UNI && FMT != TQMOE_IQ4_XS)))) ? 2 : 3;
+template <uint32_t FMT, int NB, bool UNI, int MODE>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWaves<FMT, NB, UNI, MODE>))) void decode_mfma_k(BankView b0, BankView b1, const uint8_t * __restrict__ image, void * out0, void * out1, uint32_t ytype,
+                                                    const int * __restrict__ ids, int A, int xdiv, int mode, int slots, int topk, int shared_lim, int wk,
+                                                    int tpw, int gateup, int a_off, int tl_count, Glu glu) {
+    using F = MfmaFormat<FMT>;
+    constexpr bool STAGED = MODE >= 1, MULTI = MODE == 2;
+    extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
+    __shared__ int meta[2], s_tok[kTP];
+    __shared__ float s_x0[kTP];
+    __shared__ int ql[kMaxWaves * 2][32];
+    __shared__ uint32_t lat[F::kLattice];
+    if constexpr (FMT == TQMOE_IQ3_S)   // eight times the magnitudes (behind a barrier before the first use)
+        for (int i = threadIdx.x; i < 512; i += blockDim.x) lat[i] = d_iq3s_grid.v[i] << 3;
+    const int a = blockIdx.y, e = fetch_ids(ids, A, a, mode, reinterpret_cast<int *>(stage));
+    if (e < 0 || int64_t(e) * b0.rows >= b0.rows_total) return;   // skipped assignment, or an id outside the bank
+    int tok[kTP];
+    const int n_tok = chunk_up(A, a, e, mode, kTP, reinterpret_cast<int *>(stage), meta, tok);   // the lists live in the dynamic space
+    if (n_tok == 0) return;
+    if (threadIdx.x < kTP) s_tok[threadIdx.x] = tok[threadIdx.x];
+
+    const int S = b0.cols / 32, NSB = S / 8, rows = b0.rows, tiles = rows / 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
+    const int wk_i = wave % wk, rt_l = wave / wk, tile = blockIdx.x * tl_count * tpw + rt_l;   // the wave's first (or only) row tile
+    const bool shared_slot = (a % slots) >= topk;
+    // the shared expert may have fewer rows (gate / up) or read a narrower input row (down)
+    const int row_lim = gateup && shared_slot ? shared_lim : rows;
+    const int s_end = !gateup && shared_slot ? shared_lim / 32 : S;
+    const bool valid = tile < tiles && tile * 32 < row_lim;
+
+    // The weight bytes of a super-block: 8 bytes of codes per sub-block and the row's scale record, per lane, in
+    // registers. The next super-block's are loaded before this one is multiplied (into the other of two sets that swap
+    // roles, no copies), so that there are always loads in flight under the decode work. Past the wave's last
+    // super-block the same one is fetched again: a branch around the loads would make every wait a wait for all of them.
+    // The first super-block's loads go out before the input rows are staged: the two trips to memory overlap.
+    const int sb_end = s_end / 8;   // whole super-blocks only (the launcher checks)
+    const bool working = valid && wk_i < sb_end;
+    struct Cold { typename F::Codes code[NB]; typename F::Rec rec[NB]; };
+    // the lane's addresses in the wave's first row tile, worked out once; a fetch adds 32-bit offsets (dt row tiles further on)
+    const uint8_t * code_base[NB], * rec_base[NB];
+    {
+        const int64_t at = (int64_t(e) * tiles + tile) * NSB;
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            code_base[nb] = (nb ? b1 : b0).codes + at * F::kCodeBytes;
+            rec_base[nb] = (nb ? b1 : b0).aux + at * F::kRecBytes;
+        }
+    }
+    auto fetch_tile = [&](int dt, int sb, Cold & c) {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) {
+            F::codes(code_base[nb] + uint32_t(dt * NSB + sb) * uint32_t(F::kCodeBytes), n, g, c.code[nb]);
+            c.rec[nb] = F::rec(rec_base[nb] + uint32_t(dt * NSB + sb) * uint32_t(F::kRecBytes), n);
+        }
+    };
+    auto fetch = [&](int sb, Cold & c) { fetch_tile(0, sb, c); };
+    Cold c0, c1;
+    if (working) fetch(wk_i, c0);
+    // The planes and scales of the block's input rows go to LDS once: [sub-block][input row][64 bytes of planes], then
+    // [input row][sub-block] scales. The product loop then has no loads from memory but the weights', so that its waits
+    // count exactly those (a wait for an operand A load would also wait for every weight load issued before it).
+    uint8_t * a_lds = stage + a_off;
+    float * xs_lds = reinterpret_cast<float *>(a_lds + S * 256);
+    [[maybe_unused]] float * sum_lds = xs_lds + (UNI ? 0 : S * kTP);      // formats with minimums: the activations' sums
+    if constexpr (STAGED) {
+        const uint8_t * src_row[kTP];
+#pragma unroll
+        for (int j = 0; j < kTP; ++j) src_row[j] = image_row_ptr(image, (tok[j] >= 0 ? tok[j] : tok[0]) / xdiv, S);   // rows not served: the first row's
+        for (int i0 = threadIdx.x; i0 < S * 16; i0 += 4 * blockDim.x) {   // four pieces a thread per trip to memory
+            auto piece = [&](int q) {   // past the end: the last piece again, not stored
+                const int i = min(i0 + q * int(blockDim.x), S * 16 - 1), j = (i >> 2) & 3;
+                const uint8_t * row = j == 0 ? src_row[0] : j == 1 ? src_row[1] : j == 2 ? src_row[2] : src_row[3];
+                return *reinterpret_cast<const uint4 *>(row + (i >> 4) * 64 + (i & 3) * 16);
+            };
+            auto put = [&](int q, const uint4 & v) {
+                const int i = i0 + q * int(blockDim.x);
+                if (i < S * 16) *reinterpret_cast<uint4 *>(a_lds + i * 16) = v;
+            };
+            // (four named values, not an array: an array indexed in two loops has been placed in scratch memory by the compiler,
+            // one trip to memory per piece)
+            const uint4 v0 = piece(0), v1 = piece(1), v2 = piece(2), v3 = piece(3);
+            put(0, v0); put(1, v1); put(2, v2); put(3, v3);
+        }
+        if constexpr (UNI) {   // the rows' one scale each
+            if (threadIdx.x < kTP) {
+                const int j = threadIdx.x;
+                s_x0[j] = image_scales(j == 0 ? src_row[0] : j == 1 ? src_row[1] : j == 2 ? src_row[2] : src_row[3], S)[0];
+            }
+        }
+        if constexpr (!UNI || F::kMin)
+            for (int i = threadIdx.x; i < S * kTP; i += blockDim.x) {
+                const int j = i / S;
+                const uint8_t * row = j == 0 ? src_row[0] : j == 1 ? src_row[1] : j == 2 ? src_row[2] : src_row[3];
+                if constexpr (!UNI) xs_lds[i] = image_scales(row, S)[i - j * S];
+                if constexpr (F::kMin) sum_lds[i] = image_sums(row, S)[i - j * S];
+            }
+    }
+    __syncthreads();
+
+    float accf[NB][2], accm[NB][2];   // products; minimums times the activations' sums
+    auto clear = [&]() {
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) accf[nb][0] = accf[nb][1] = accm[nb][0] = accm[nb][1] = 0.f;
+    };
+    clear();
+
+    // A row tile's sums to their place. tile0: the block's first row tile of this pass.
+    auto finish = [&](int tile0, bool wave_valid) {
+        if constexpr (UNI) {
+            if (wave_valid) {   // the rows' own scales, once
+                const float x0 = STAGED ? s_x0[2 * g] : image_scales(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S)[0];
+                const float x1 = STAGED ? s_x0[2 * g + 1] : image_scales(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S)[0];
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) { accf[nb][0] *= x0; accf[nb][1] *= x1; }
+            }
+        }
+        if constexpr (F::kMin) {
+#pragma unroll
+            for (int nb = 0; nb < NB; ++nb) { accf[nb][0] -= accm[nb][0]; accf[nb][1] -= accm[nb][1]; }
+        }
+        if constexpr (F::kRowFactor) {
+            if (wave_valid) {
+                const int64_t row = int64_t(e) * rows + (tile0 + rt_l) * 32 + n;
+#pragma unroll
+                for (int nb = 0; nb < NB; ++nb) { const float f = F::row_factor(nb ? b1 : b0, row); accf[nb][0] *= f; accf[nb][1] *= f; }
+            }
+        }
+        __syncthreads();                                       // the id list (or the previous pass's sums) is done with: the space now holds the partial sums
+        float (*red)[NB][kTP][32] = reinterpret_cast<float (*)[NB][kTP][32]>(stage);
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb) { red[wave][nb][2 * g][n] = accf[nb][0]; red[wave][nb][2 * g + 1][n] = accf[nb][1]; }
+        __syncthreads();
+
+        // the waves of a row tile hold the partial sums of its super-block shares: added here in wave order
+        const int groups = tpw * kTP, per_pass = blockDim.x >> 5;
+        for (int g0 = 0; g0 < groups; g0 += per_pass) {   // every wave runs every pass: the image quantiser exchanges lanes
+            const int grp = g0 + (threadIdx.x >> 5), i = threadIdx.x & 31;
+            const int rt = grp / kTP, j = grp % kTP, t = tile0 + rt;
+            const bool live = grp < groups && j < n_tok && t < tiles && t * 32 < row_lim;
+            float v0 = 0.f, v1 = 0.f;
+            if (live)
+                for (int w = 0; w < wk; ++w) { v0 += red[rt * wk + w][0][j][i]; if (NB == 2) v1 += red[rt * wk + w][NB - 1][j][i]; }
+            const int aj = live ? s_tok[j] : 0;
+            if (gateup) {
+                glu_clamp_inputs(glu, v0, v1);
+                const float act = glu_clamp_silu(glu, v0 / (1.f + expf(-v0))) * v1;
+                quantise_block_lanes(act, i, live, ql[threadIdx.x >> 5], static_cast<uint8_t *>(out0) + int64_t(aj) * tiles * kImageSubBytes, tiles, t);
+            } else if (live) {
+                const int64_t o = int64_t(aj) * rows + t * 32 + i;
+                if (ytype == TQMOE_F32) { static_cast<float *>(out0)[o] = v0; if (NB == 2) static_cast<float *>(out1)[o] = v1; }
+                else { static_cast<uint16_t *>(out0)[o] = float_to_bf16_bits(v0); if (NB == 2) static_cast<uint16_t *>(out1)[o] = float_to_bf16_bits(v1); }
+            }
+        }
+    };
+
+    if (working) {
+        // this lane's part of operand A: plane row n of the MFMA = plane (n & 1) of input row n >> 1 (rows 8 and up repeat
+        // rows 0..7: their sums land in result rows that nobody reads)
+        // (not staged: straight from the image, a stride of 64 bytes per sub-block instead of the staged 256)
+        const int a_tok = max(s_tok[(n & 7) >> 1], s_tok[0]);
+        const uint8_t * a_lane = STAGED ? a_lds + ((n & 7) >> 1) * 64 + (n & 1) * 32 + g * 16 : image_row_ptr(image, a_tok / xdiv, S) + (n & 1) * 32 + g * 16;
+        constexpr int kStrideA = STAGED ? 256 : 64;
+        // the two input rows whose sums land in this lane half's result registers
+        const float * sc0 = STAGED ? xs_lds + (2 * g) * S : image_scales(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S);
+        const float * sc1 = STAGED ? xs_lds + (2 * g + 1) * S : image_scales(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S);
+        const float * sum0 = STAGED ? sum_lds + (2 * g) * S : image_sums(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S);
+        const float * sum1 = STAGED ? sum_lds + (2 * g + 1) * S : image_sums(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S);
+        auto multiply = [&](int sb, const Cold & cur) {
+            // Staged rows: operand A and the scales of four sub-blocks at a time, right before their first use (an LDS read is
+            // covered by the step in front of it; all eight at once are 16 to 32 registers more, which Q4_K and Q6_K spilled).
+            // From the image: everything at the start, in one trip.
+            constexpr int kPart = STAGED ? 4 : 8;
+            v4i areg[kPart];
+            float xs0[kPart], xs1[kPart], xm0[kPart], xm1[kPart];
+            auto part_a = [&](int ib0) {
+#pragma unroll
+                for (int i = 0; i < kPart; ++i) areg[i] = *reinterpret_cast<const v4i *>(a_lane + (sb * 8 + ib0 + i) * kStrideA);
+            };
+            auto part_x = [&](int ib0) {
+                auto get = [&](const float * p, float (&v)[kPart]) {
+#pragma unroll
+                    for (int i = 0; i < kPart; i += 4) {
+                        const float4 f = *reinterpret_cast<const float4 *>(p + sb * 8 + ib0 + i);
+                        v[i] = f.x; v[i + 1] = f.y; v[i + 2] = f.z; v[i + 3] = f.w;
+                    }
+                };
+                if constexpr (!UNI) { get(sc0, xs0); get(sc1, xs1); }       // activation scales of the sub-blocks
+                if constexpr (F::kMin) { get(sum0, xm0); get(sum1, xm1); }  // and their sums
+            };
+            // The products of step (sub-block, bank, scale group) + 1 are issued before the sums of this step are read: the
+            // matrix pipe's latency passes under the next step's lookups instead of in front of this step's multiply-adds.
+            const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+            constexpr int G = F::kGroups, kSteps = 8 * NB * G;
+            v4i w;
+            auto issue = [&](int step) {
+                const int ib = step / (NB * G), nb = step / G % NB, grp = step % G;
+                if (step % (kPart * NB * G) == 0) part_a(ib);
+                if (grp == 0) w = F::decode(cur.code[nb], cur.rec[nb], ib, g, lat);
+                if constexpr (G == 1) return __builtin_amdgcn_mfma_i32_32x32x32_i8(areg[ib % kPart], w, zero, 0, 0, 0);
+                else {   // operand dwords 0 and 2 are the sub-block's first sixteen weights, 1 and 3 the others
+                    const long a2 = long(uint64_t(uint32_t(areg[ib % kPart][grp])) | uint64_t(uint32_t(areg[ib % kPart][grp + 2])) << 32);
+                    const long w2 = long(uint64_t(uint32_t(w[grp])) | uint64_t(uint32_t(w[grp + 2])) << 32);
+                    return __builtin_amdgcn_mfma_i32_32x32x16_i8(a2, w2, zero, 0, 0, 0);
+                }
+            };
+            constexpr bool kAhead = UNI;   // the other kernels lose more to the registers of a second result than they gain
+            v16i acc = issue(0);
+            int si[NB][4];   // (hi, lo) plane sums of the two input rows, weighted by the sub-block scales
+            float sm[NB][2];
+#pragma unroll
+            for (int step = 0; step < kSteps; ++step) {
+                const int ib = step / (NB * G), nb = step / G % NB, grp = step % G, ip = ib % kPart;
+                if (step % (kPart * NB * G) == 0) part_x(ib);
+                v16i ahead = zero;
+                if constexpr (kAhead) {
+                    if (step + 1 < kSteps) ahead = issue(step + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                const typename F::Rec & rec = cur.rec[nb];
+                if constexpr (F::kFloat) {
+                    const float sc = F::scale(rec, ib, grp);
+                    accf[nb][0] = fmaf(float((acc[0] << 7) + acc[1]), UNI ? sc : sc * xs0[ip], accf[nb][0]);
+                    accf[nb][1] = fmaf(float((acc[2] << 7) + acc[3]), UNI ? sc : sc * xs1[ip], accf[nb][1]);
+                } else if constexpr (UNI) {
+                    // |acc| <= 32 * 128 * 128 = 2^19 and |scale| <= 2^7: 24-bit products, and with a scale per sixteen weights
+                    // half the |acc|: sixteen of them stay below 2^30
+                    const int ls = F::scale(rec, ib, grp);
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) si[nb][q] = (ib || grp ? si[nb][q] : 0) + __mul24(acc[q], ls);
+                    if (ib == 7 && grp == G - 1) {
+                        const float d = F::d(rec);
+                        accf[nb][0] += (float(si[nb][0]) * 128.f + float(si[nb][1])) * d;
+                        accf[nb][1] += (float(si[nb][2]) * 128.f + float(si[nb][3])) * d;
+                    }
+                } else {
+                    const float ws = F::d(rec) * float(F::scale(rec, ib, grp));
+                    accf[nb][0] += float((acc[0] << 7) + acc[1]) * (ws * xs0[ip]);
+                    accf[nb][1] += float((acc[2] << 7) + acc[3]) * (ws * xs1[ip]);
+                }
+                if constexpr (F::kMin) {
+                    const float mn = F::minimum(rec, ib);
+                    sm[nb][0] = ib ? fmaf(mn, xm0[ip], sm[nb][0]) : mn * xm0[ip];
+                    sm[nb][1] = ib ? fmaf(mn, xm1[ip], sm[nb][1]) : mn * xm1[ip];
+                    if (ib == 7) {
+                        const float dm = F::dmin(rec);
+                        accm[nb][0] = fmaf(dm, sm[nb][0], accm[nb][0]);
+                        accm[nb][1] = fmaf(dm, sm[nb][1], accm[nb][1]);
+                    }
+                }
+                // only four of the sixteen result registers are read; the others count as in use until here, or they are handed
+                // to the next lookups while the matrix pipe still writes them and every such write waits for the pipe
+                asm volatile("" : : "v"(acc));
+                if constexpr (kAhead) acc = ahead;
+                else if (step + 1 < kSteps) acc = issue(step + 1);
+            }
+        };
+        if constexpr (MULTI) {
+            // Several row tiles a wave, one after the other (the launcher has made sure that every wave of the block has the
+            // same steps: no ragged tiles, no shorter shared expert): the block finds its input rows and stages them once, and
+            // the weight loads run on across the tiles' ends, the next tile's first under this tile's sums.
+            const int nsteps = sb_end / wk, total = tl_count * nsteps;
+            auto fetch_step = [&](int gs, Cold & c) { fetch_tile(gs / nsteps * tpw, wk_i + gs % nsteps * wk, c); };
+            auto after = [&](int gs) {   // step gs is done: was it its tile's last?
+                if ((gs + 1) % nsteps) return;
+                finish((int(blockIdx.x) * tl_count + gs / nsteps) * tpw, true);
+                clear();
+            };
+            for (int gs = 0; gs < total; gs += 2) {
+                fetch_step(min(gs + 1, total - 1), c1);
+                multiply(wk_i + gs % nsteps * wk, c0);
+                after(gs);
+                if (gs + 1 >= total) break;
+                fetch_step(min(gs + 2, total - 1), c0);
+                multiply(wk_i + (gs + 1) % nsteps * wk, c1);
+                after(gs + 1);
+            }
+        } else if constexpr (STAGED) {
+            const int last = wk_i + (sb_end - 1 - wk_i) / wk * wk;   // the wave's last super-block
+            for (int sb = wk_i; sb <= last; sb += 2 * wk) {
+                fetch(min(sb + wk, last), c1);
+                multiply(sb, c0);
+                if (sb + wk > last) break;
+                fetch(min(sb + 2 * wk, last), c0);
+                multiply(sb + wk, c1);
+            }
+        } else {   // short batches: most waves have one super-block, and nothing is fetched that is not multiplied
+            for (int sb = wk_i; sb < sb_end; sb += wk) {
+                if (sb + wk < sb_end) fetch(sb + wk, c1);
+                multiply(sb, c0);
+                c0 = c1;
+            }
+        }
+    }
+
+    if constexpr (!MULTI) finish(blockIdx.x * tpw, valid);
+}
+
+template <uint32_t FMT>
+void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void * out0, void * out1, uint32_t ytype, const int * ids, int A, int xdiv, int mode,
+            int slots, int topk, int shared_lim, int gateup, bool uniform, Glu glu, hipStream_t s) {
+    const int NSB = b0.cols / 256, tiles = b0.rows / 32;
+    // Waves that share a row's super-blocks: as many as it takes to put a few thousand waves in flight (a short batch
+    // is bound by the latency of one wave's chain), fewer when the batch has the waves anyway (a longer chain per
+    // wave streams with its loads one super-block ahead and saves the cross-wave sums).
+    const int64_t units = int64_t(A) * tiles;
+    const int cap = units >= 8192 ? 1 : units >= 2048 ? 2 : units >= 512 ? 4 : kMaxWaves;
+    int wk = 1;
+    for (int w = 1; w <= kMaxWaves && w <= cap; ++w) if (NSB % w == 0) wk = w;
+    const int waves = wk > 4 ? wk : 4;                    // per block: small blocks, a compute unit holds several and their phases interleave
+    int tpw = waves / wk;                                                 // row tiles per block
+    if (tpw > tiles) tpw = tiles;
+    const unsigned threads = unsigned(wk * tpw * 64);
+    // dynamic LDS: the match list and the copy of the ids (2 * kMaxList ints), later the partial sums; behind them the input
+    // rows' planes (256 bytes per sub-block) and, for rows with a scale per sub-block, the scales
+    size_t lds = mode ? size_t(2) * kMaxList * sizeof(int) : 0;
+    if (lds < size_t(wk * tpw) * nb * kTP * 32 * sizeof(float)) lds = size_t(wk * tpw) * nb * kTP * 32 * sizeof(float);
+    // the input rows go through LDS from a dozen tokens on (measured: 5 % at 16 and 32 tokens; the waves then overlap each
+    // other's waits, and what counts is that a wave's own weight loads stay in flight under its products); a short batch is
+    // one chain of dependent steps per wave, and the extra stop at a barrier costs more than the exact waits return
+    const bool staged = A >= 12 * slots;
+    // ... and a wave then takes up to four row tiles one after the other, as long as the grid keeps two blocks per compute
+    // unit: the block's search for its input rows and their staging are paid once for all of them
+    int tl = 1;
+    if (staged && nb == 1 && shared_lim == (gateup ? b0.rows : b0.cols))
+        while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= 512) tl *= 2;
+    const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl)), unsigned(A));
+    const int a_off = int(lds);
+    if (staged) lds += size_t(b0.cols / 32) * (256 + ((uniform ? 0 : 1) + (MfmaFormat<FMT>::kMin ? 1 : 0)) * kTP * sizeof(float));
+    auto go = [&](auto kernel) { kernel<<<grid, threads, lds, s>>>(b0, b1, image, out0, out1, ytype, ids, A, xdiv, mode, slots, topk, shared_lim, wk, tpw, gateup, a_off, tl, glu); };
+    if (nb == 2 && uniform) staged ? go(decode_mfma_k<FMT, 2, true, 1>) : go(decode_mfma_k<FMT, 2, true, 0>);
+    else if (nb == 2) staged ? go(decode_mfma_k<FMT, 2, false, 1>) : go(decode_mfma_k<FMT, 2, false, 0>);
+    else if (tl > 1) go(decode_mfma_k<FMT, 1, false, 2>);
+    else staged ? go(decode_mfma_k<FMT, 1, false, 1>) : go(decode_mfma_k<FMT, 1, false, 0>);
+}
+
+// the shapes the kernel takes: whole tiles, whole super-blocks (a narrower shared expert included)
+inline bool mfma_takes(int rows, int cols, int shared_cols) { return rows % 32 == 0 && cols % 256 == 0 && shared_cols % 256 == 0; }
+
+}  // namespace
+}  // namespace tqmoe

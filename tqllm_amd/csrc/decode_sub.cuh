@@ -8,7 +8,7 @@ namespace tqmoe {
 
 __device__ __forceinline__ void decode_sub32(uint32_t type, const uint8_t * __restrict__ codes, const uint8_t * __restrict__ aux, int64_t rows_total, int cols,
                                              int64_t row, int s, float * __restrict__ y) {
-    const int S = cols / 32, ib = s & 7;
+    const int S = cols / 32, ib = s & 7, h = tile_rows(row, rows_total);
     const uint8_t * cd = codes + (row * S + s) * code_bytes_per_sub(type);
     switch (type) {
         case TQMOE_IQ4_XS: {
@@ -29,13 +29,13 @@ __device__ __forceinline__ void decode_sub32(uint32_t type, const uint8_t * __re
             break;
         }
         case TQMOE_Q4_K: {
-            const uint4 rec = *reinterpret_cast<const uint4 *>(aux + (row * (S / 8) + s / 8) * 16);
+            const uint4 rec = *reinterpret_cast<const uint4 *>(aux + tiled(row, h, S / 8, s / 8, 16));
             const uint32_t sc12[3] = {rec.y, rec.z, rec.w};
             int sc, mn;
             q4k_scale_min(sc12, ib, sc, mn);
             const float d1 = __fmul_rn(half_bits_to_float(uint16_t(rec.x & 0xFFFFu)), float(sc));
             const float m1 = __fmul_rn(half_bits_to_float(uint16_t(rec.x >> 16)), float(mn));
-            const uint4 c = *reinterpret_cast<const uint4 *>(cd);
+            const uint4 c = *reinterpret_cast<const uint4 *>(codes + tiled(row, h, S, s, 16));
             const uint32_t w[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
             for (int q = 0; q < 4; ++q)
@@ -48,21 +48,20 @@ __device__ __forceinline__ void decode_sub32(uint32_t type, const uint8_t * __re
             break;
         }
         case TQMOE_IQ3_S: {
-            const uint4 rec = *reinterpret_cast<const uint4 *>(aux + (row * (S / 8) + s / 8) * 16);
-            // rec: d | qh[0..1] << 16, qh[2..5], qh[6..7] | scales[0..1] << 16, scales[2..3]
-            const uint32_t qh = ib < 2 ? (rec.x >> (16 + 8 * ib)) & 0xFFu : ib < 6 ? (rec.y >> (8 * (ib - 2))) & 0xFFu : (rec.z >> (8 * (ib - 6))) & 0xFFu;
-            const uint32_t scb = (ib >> 1) < 2 ? (rec.z >> (16 + 8 * (ib >> 1))) & 0xFFu : (rec.w >> (8 * ((ib >> 1) - 2))) & 0xFFu;
-            const float db = __fmul_rn(half_bits_to_float(uint16_t(rec.x & 0xFFFFu)), float(1 + 2 * int((scb >> (4 * (ib & 1))) & 15u)));
-            const uint32_t * c = reinterpret_cast<const uint32_t *>(cd);
-            const uint32_t qs[2] = {c[0], c[1]}, sg = c[2];
+            const uint4 rec = *reinterpret_cast<const uint4 *>(aux + tiled(row, h, S / 8, s / 8, 16));
+            const float db = __fmul_rn(half_bits_to_float(uint16_t(rec.x & 0xFFFFu)), float(1 + 2 * iq3s_ls(rec, ib)));
+            const uint32_t qh = iq3s_qh(rec, ib), sg = *reinterpret_cast<const uint32_t *>(codes + iq3s_sign_offset(row, h, S, s));
 #pragma unroll
-            for (int w = 0; w < 8; ++w) {
-                const uint32_t g = d_iq3s_grid.v[((qs[w >> 2] >> (8 * (w & 3))) & 0xFFu) | (((qh >> w) & 1u) << 8)];
-                const uint32_t sn = sg >> (4 * w);
+            for (int g = 0; g < 2; ++g) {
+                const uint32_t qs = *reinterpret_cast<const uint32_t *>(codes + iq3s_qs_offset(row, h, S, s, g));
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    const float mag = __fmul_rn(db, float((g >> (8 * j)) & 0xFFu));
-                    y[4 * w + j] = ((sn >> j) & 1u) ? -mag : mag;
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t m = d_iq3s_grid.v[((qs >> (8 * q)) & 0xFFu) | (((qh >> (4 * g + q)) & 1u) << 8)];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const float mag = __fmul_rn(db, float((m >> (8 * j)) & 0xFFu));
+                        y[4 * operand_group(g, q) + j] = ((sg >> (8 * j + 4 * g + q)) & 1u) ? -mag : mag;
+                    }
                 }
             }
             break;
@@ -206,23 +205,19 @@ __device__ __forceinline__ void decode_sub32(uint32_t type, const uint8_t * __re
             break;
         }
         case TQMOE_Q6_K: {  // dequant.cpp:194-208: (d * sc) * (q - 32), one int8 scale per 16 weights
-            const uint8_t * a = aux + (row * (S / 8) + s / 8) * 32;
+            const uint8_t * a = aux + tiled(row, h, S / 8, s / 8, 32);
             const float d = half_bits_to_float(*reinterpret_cast<const uint16_t *>(a + 16));
             const float d0 = __fmul_rn(d, float(int8_t(a[2 * ib]))), d1 = __fmul_rn(d, float(int8_t(a[2 * ib + 1])));
-            const uint2 c0 = *reinterpret_cast<const uint2 *>(cd), c1 = *reinterpret_cast<const uint2 *>(cd + 8), hi = *reinterpret_cast<const uint2 *>(cd + 16);
-            const uint32_t w[4] = {c0.x, c0.y, c1.x, c1.y};
-            const uint32_t h2[2] = {hi.x, hi.y};
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
+            for (int g = 0; g < 2; ++g) {
+                const uint2 low = *reinterpret_cast<const uint2 *>(codes + q6k_low_offset(row, h, S, s) + 8 * g);
+                uint32_t w[4];
+                q6k_times4(low, *reinterpret_cast<const uint32_t *>(codes + q6k_high_offset(row, h, S, s, g)), w);
 #pragma unroll
-                for (int b = 0; b < 4; ++b) {
-                    const uint32_t byte = (w[q] >> (8 * b)) & 0xFFu;
-                    const int j = 4 * q + b;
-                    const int lo = int((byte & 15u) | (((h2[0] >> (2 * j)) & 3u) << 4)) - 32;
-                    const int up = int((byte >> 4) | (((h2[1] >> (2 * j)) & 3u) << 4)) - 32;
-                    y[j] = __fmul_rn(d0, float(lo));
-                    y[16 + j] = __fmul_rn(d1, float(up));
-                }
+                for (int q = 0; q < 4; ++q)
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) y[4 * operand_group(g, q) + b] = __fmul_rn(q & 1 ? d1 : d0, float(int8_t(w[q] >> (8 * b)) >> 2));
+            }
             break;
         }
         case TQMOE_IQ4_NL: {  // dequant.cpp:351-360: d * kv[q]
@@ -254,9 +249,9 @@ __device__ __forceinline__ void decode_sub32(uint32_t type, const uint8_t * __re
         }
         case TQMOE_NVFP4G: {
             const float g = *reinterpret_cast<const float *>(aux + nvfp4_global_offset(rows_total, cols) + row * 4);
-            const uint8_t * sc = aux + row * (cols / 16) + 2 * s;
+            const uint8_t * sc = aux + nvfp4_scale_offset(row, h, S, s);
             const float d0 = __fmul_rn(e4m3_to_float(sc[0]), g), d1 = __fmul_rn(e4m3_to_float(sc[1]), g);
-            const uint4 c = *reinterpret_cast<const uint4 *>(cd);
+            const uint4 c = *reinterpret_cast<const uint4 *>(codes + tiled(row, h, S, s, 16));
             const uint32_t w[4] = {c.x, c.y, c.z, c.w};
 #pragma unroll
             for (int q = 0; q < 4; ++q) {

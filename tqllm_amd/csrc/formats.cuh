@@ -28,11 +28,33 @@ __host__ __device__ constexpr int64_t aux_row_bytes(uint32_t type, int cols) {
 // NVFP4G: offset of the per-row fp32 globals inside the aux plane
 __host__ __device__ constexpr int64_t nvfp4_global_offset(int64_t rows_total, int cols) { return (rows_total * (cols / 16) + 15) / 16 * 16; }
 
-// IQ4_XS banks are stored tile-major: 32 consecutive rows form a tile, and inside a tile the codes of sub-block s of
-// all 32 rows are contiguous (512 B), as are the 32 records of a super-block (256 B). A wave then reads whole tiles with
-// fully coalesced loads whichever lane owns which row. rows of an expert must be a multiple of 32.
-__host__ __device__ constexpr int64_t iq4xs_code_offset(int64_t row, int S, int s) { return (((row >> 5) * S + s) * 32 + (row & 31)) * 16; }
-__host__ __device__ constexpr int64_t iq4xs_aux_offset(int64_t row, int S, int sb) { return (((row >> 5) * (S >> 3) + sb) * 32 + (row & 31)) * 8; }
+// IQ4_XS, Q4_K, Q6_K, IQ3_S and NVFP4G banks are stored tile-major: 32 consecutive rows form a tile, and inside a tile the
+// same piece of all its rows is contiguous (16 bytes of each row are 512), so that a wave whose lanes own the rows of a
+// tile reads it with fully coalesced loads. The last tile of a bank may have fewer rows (tile_rows; not for IQ4_XS, whose
+// experts' rows are multiples of 32): its pieces lie closer, nothing is padded.
+__host__ __device__ constexpr bool is_tile_major(uint32_t type) { return type == TQMOE_IQ4_XS || type == TQMOE_Q4_K || type == TQMOE_Q6_K || type == TQMOE_IQ3_S || type == TQMOE_NVFP4G; }
+__host__ __device__ constexpr int tile_rows(int64_t row, int64_t rows_total) { return int(rows_total - (row & ~int64_t(31)) < 32 ? rows_total - (row & ~int64_t(31)) : 32); }
+// a row's piece `i` of `per_row` pieces of `bytes` each (h: rows of its tile)
+__host__ __device__ constexpr int64_t tiled(int64_t row, int h, int per_row, int i, int bytes) { return ((row & ~int64_t(31)) * per_row + int64_t(i) * h + (row & 31)) * bytes; }
+__host__ __device__ constexpr int64_t iq4xs_code_offset(int64_t row, int S, int s) { return tiled(row, 32, S, s, 16); }
+__host__ __device__ constexpr int64_t iq4xs_aux_offset(int64_t row, int S, int sb) { return tiled(row, 32, S >> 3, sb, 8); }
+// Inside a sub-block the weights split over the two halves g = 0, 1 of a wave as the matrix instruction's operand has them:
+// operand dword q of half g holds the four weights 4 w .. 4 w + 3 with w = 2 g + q / 2 + 4 (q % 2).
+__host__ __device__ constexpr int operand_group(int g, int q) { return 2 * g + (q >> 1) + 4 * (q & 1); }
+// IQ3_S: 96 bytes of codes per row and super-block: four 16-byte pieces, each a pair of sub-blocks (half g's 8 bytes: the
+// lattice indices' low bytes of its four operand dwords, sub-block 2 p then 2 p + 1), then two 16-byte pieces with a dword
+// of signs for each of four sub-blocks (bit 8 j + 4 g + q: weight j of operand dword q of half g). Aux 16 bytes: d | the
+// scale bytes' first half << 16, the ninth index bits of sub-blocks 0..3 and 4..7 (a byte each, bit 4 g + q), the scale bytes' other half.
+__host__ __device__ constexpr int64_t iq3s_qs_offset(int64_t row, int h, int S, int s, int g) { return (row & ~int64_t(31)) * (S >> 3) * 96 + int64_t(s >> 3) * h * 96 + ((s & 7) >> 1) * h * 16 + (row & 31) * 16 + g * 8 + (s & 1) * 4; }
+__host__ __device__ constexpr int64_t iq3s_sign_offset(int64_t row, int h, int S, int s) { return (row & ~int64_t(31)) * (S >> 3) * 96 + int64_t(s >> 3) * h * 96 + h * 64 + ((s & 7) >> 2) * h * 16 + (row & 31) * 16 + (s & 3) * 4; }
+// Q6_K: 192 bytes of codes per row and super-block: eight 16-byte pieces of low nibbles (a sub-block each, the canonical
+// order), then four 16-byte pieces of upper bits, each a pair of sub-blocks (half g's 8 bytes: a dword per sub-block, byte j
+// bits 2 q and 2 q + 1: weight j of operand dword q, the upper of the two inverted, so that 4 * (q - 32) is the six bits at the
+// top of a byte read as int8).
+__host__ __device__ constexpr int64_t q6k_low_offset(int64_t row, int h, int S, int s) { return (row & ~int64_t(31)) * (S >> 3) * 192 + int64_t(s >> 3) * h * 192 + (s & 7) * h * 16 + (row & 31) * 16; }
+__host__ __device__ constexpr int64_t q6k_high_offset(int64_t row, int h, int S, int s, int g) { return (row & ~int64_t(31)) * (S >> 3) * 192 + int64_t(s >> 3) * h * 192 + h * 128 + ((s & 7) >> 1) * h * 16 + (row & 31) * 16 + g * 8 + (s & 1) * 4; }
+// NVFP4G scales: pieces of eight bytes (four sub-blocks)
+__host__ __device__ constexpr int64_t nvfp4_scale_offset(int64_t row, int h, int S, int s) { return tiled(row, h, S >> 2, s >> 2, 8) + 2 * (s & 3); }
 
 // IQ4_NL / IQ4_XS value table {-127,-104,-83,-65,-49,-35,-22,-10,1,13,25,38,53,69,89,113} as four little-endian dwords
 constexpr uint32_t kIq4T0 = 0xBFAD9881u, kIq4T1 = 0xF6EADDCFu, kIq4T2 = 0x26190D01u, kIq4T3 = 0x71594535u;
@@ -194,5 +216,16 @@ __device__ __forceinline__ int iq4xs_lsm32(uint2 rec, int ib) {
 }
 __device__ __forceinline__ int iq4xs_ls(uint2 rec, int ib) { return iq4xs_lsm32(rec, ib) + 32; }
 __device__ __forceinline__ uint16_t iq4xs_d_bits(uint2 rec) { return uint16_t(__builtin_amdgcn_alignbit(rec.y, rec.x, 30) & 0xFFFFu); }
+
+// IQ3_S: the 4-bit scale and the eight ninth index bits of sub-block ib (see iq3s_qs_offset)
+__device__ __forceinline__ int iq3s_ls(uint4 rec, int ib) { return int((ib < 4 ? rec.x >> (16 + 4 * ib) : rec.w >> (4 * (ib - 4))) & 15u); }
+__device__ __forceinline__ uint32_t iq3s_qh(uint4 rec, int ib) { return ((ib < 4 ? rec.y : rec.z) >> (8 * (ib & 3))) & 0xFFu; }
+// Q6_K: the low nibbles and upper bits of one half of a sub-block -> four operand dwords of int8 values 4 * (q - 32)
+__device__ __forceinline__ void q6k_times4(uint2 low, uint32_t high, uint32_t (&w)[4]) {
+    w[0] = ((low.x << 2) & 0x3C3C3C3Cu) | ((high << 6) & 0xC0C0C0C0u);
+    w[1] = ((low.x >> 2) & 0x3C3C3C3Cu) | ((high << 4) & 0xC0C0C0C0u);
+    w[2] = ((low.y << 2) & 0x3C3C3C3Cu) | ((high << 2) & 0xC0C0C0C0u);
+    w[3] = ((low.y >> 2) & 0x3C3C3C3Cu) | (high & 0xC0C0C0C0u);
+}
 
 }  // namespace tqmoe

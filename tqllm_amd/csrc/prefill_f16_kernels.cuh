@@ -70,10 +70,7 @@ __device__ __forceinline__ uint2 i8x4_to_h4(uint32_t w, float scale, float c) {
 template <uint32_t FMT> struct F16Sub {
     typedef typename Sub<FMT>::Raw Raw;
     static __device__ __forceinline__ Raw load(const BankView & b, int64_t row, int s) {
-        Tile t;
-        t.codes = b.codes + row * code_row_bytes(FMT, b.cols);
-        t.aux = b.aux + row * aux_row_bytes(FMT, b.cols);
-        t.aux2 = FMT == TQMOE_NVFP4G ? b.aux + nvfp4_global_offset(b.rows_total, b.cols) + row * 4 : nullptr;
+        const Tile t = tile_at<FMT>(b, row);
         return Sub<FMT>::load(t, 0u, uint32_t(b.cols / 32), uint32_t(s));
     }
     // valid false: all zeros (a row or a sub-block past the end), through a zero scale and constant

@@ -213,7 +213,7 @@ struct WIq4xsSub : WIq4xs {
     }
 };
 
-struct WQ4k {   // row-major: 16 code bytes per sub-block, a 16-byte record (d | dmin << 16, twelve bytes of 6-bit scales and minimums) per super-block
+struct WQ4k {   // tile-major: 16 code bytes per sub-block, a 16-byte record (d | dmin << 16, twelve bytes of 6-bit scales and minimums) per super-block
     static constexpr bool kFoldSub = false;     // one scale per 32 weights: every sub-block's product is folded on its own
     static constexpr bool kWideChunks = false;   // chunks of sixteen row tiles on eight waves (two row tiles a wave)
     static constexpr int kPlanes = 3, kTabBytes = 64 * 32, kLattice = 1;
@@ -221,18 +221,19 @@ struct WQ4k {   // row-major: 16 code bytes per sub-block, a 16-byte record (d |
     struct Code { uint2 c; };
     typedef uint4 Rec;
     typedef uint32_t DRec;
-    struct Src { const uint8_t * codes, * aux; };
+    struct Src { const uint8_t * codes, * aux; int step; };   // step: bytes of a piece of the tile
     static __device__ __forceinline__ void tables(uint8_t * tab, uint32_t *, int tid, int threads) {   // per 6-bit scale sc: sc * q for the 16 codes
         for (int i = tid; i < 64 * 16; i += threads) split_planes((i & 15) * (i >> 4), tab[(i >> 4) * 32 + (i & 15)], tab[(i >> 4) * 32 + 16 + (i & 15)]);
     }
     static __device__ __forceinline__ Src src(const BankView & b, int e, int wtile, int n, int g) {
         const int S = b.cols / 32;
         const int64_t row = int64_t(e) * b.rows + wtile * 32 + n;
-        return Src{b.codes + row * S * 16 + g * 8, b.aux + row * (S / 8) * 16};
+        const int h = tile_rows(row, b.rows_total);
+        return Src{b.codes + tiled(row, h, S, 0, 16) + g * 8, b.aux + tiled(row, h, S / 8, 0, 16), h * 16};
     }
-    static __device__ __forceinline__ Code code(const Src & s, int sub) { return Code{*reinterpret_cast<const uint2 *>(s.codes + int64_t(sub) * 16)}; }
-    static __device__ __forceinline__ Rec rec(const Src & s, int sb) { return *reinterpret_cast<const uint4 *>(s.aux + int64_t(sb) * 16); }
-    static __device__ __forceinline__ DRec drec(const Src & s, int sb) { return *reinterpret_cast<const uint32_t *>(s.aux + int64_t(sb) * 16); }
+    static __device__ __forceinline__ Code code(const Src & s, int sub) { return Code{*reinterpret_cast<const uint2 *>(s.codes + int64_t(sub) * s.step)}; }
+    static __device__ __forceinline__ Rec rec(const Src & s, int sb) { return *reinterpret_cast<const uint4 *>(s.aux + int64_t(sb) * s.step); }
+    static __device__ __forceinline__ DRec drec(const Src & s, int sb) { return *reinterpret_cast<const uint32_t *>(s.aux + int64_t(sb) * s.step); }
     static __device__ __forceinline__ void planes(const Code & c, const Rec & r, int ib, int, const uint8_t * tab, const uint32_t *, v4i * p) {
         int sc, mn;
         q4k_scale_min_flat(r.y, r.z, r.w, ib, sc, mn);
@@ -270,15 +271,15 @@ struct WQ4kSub : WQ4k {
     }
 };
 
-struct WIq3s {   // row-major: 12 code bytes per sub-block (8 lattice indices, 32 sign bits), a 16-byte record per super-block
+struct WIq3s {   // tile-major: per half of a sub-block four lattice index bytes, a dword of signs for both, a 16-byte record per super-block
     static constexpr bool kFoldSub = false;     // one scale per 32 weights: every sub-block's product is folded on its own
     static constexpr bool kWideChunks = false;   // chunks of sixteen row tiles on eight waves (two row tiles a wave)
     static constexpr int kPlanes = 2, kTabBytes = 16 * 32, kLattice = 512;
     static constexpr bool kFp8 = false, kMin = false, kRowMul = false;
-    struct Code { uint32_t qs0, qs1, sg; };
-    typedef uint4 Rec;       // d | qh[0..1] << 16, qh[2..5], qh[6..7] | scales[0..1] << 16, scales[2..3]
+    struct Code { uint32_t qs, sg; };
+    typedef uint4 Rec;       // see iq3s_qs_offset
     typedef uint32_t DRec;
-    struct Src { const uint8_t * codes, * aux; };
+    struct Src { const uint8_t * qs, * sg, * aux; int h; };
     // per 4-bit scale ls the 16 products (1 + 2 ls) * (+-(2 j + 1)): code = sign << 3 | magnitude index j
     static __device__ __forceinline__ void tables(uint8_t * tab, uint32_t * lat, int tid, int threads) {
         for (int i = tid; i < 16 * 16; i += threads) {
@@ -287,28 +288,28 @@ struct WIq3s {   // row-major: 12 code bytes per sub-block (8 lattice indices, 3
         }
         for (int i = tid; i < 512; i += threads) lat[i] = d_iq3s_grid.v[i];
     }
-    static __device__ __forceinline__ Src src(const BankView & b, int e, int wtile, int n, int) {
+    static __device__ __forceinline__ Src src(const BankView & b, int e, int wtile, int n, int g) {
         const int S = b.cols / 32;
         const int64_t row = int64_t(e) * b.rows + wtile * 32 + n;
-        return Src{b.codes + row * S * 12, b.aux + row * (S / 8) * 16};
+        const int h = tile_rows(row, b.rows_total);
+        return Src{b.codes + iq3s_qs_offset(row, h, S, 0, g), b.codes + iq3s_sign_offset(row, h, S, 0), b.aux + tiled(row, h, S / 8, 0, 16), h};
     }
     static __device__ __forceinline__ Code code(const Src & s, int sub) {
-        const uint32_t * c = reinterpret_cast<const uint32_t *>(s.codes + int64_t(sub) * 12);
-        return Code{c[0], c[1], c[2]};
+        const int sb = sub >> 3, ib = sub & 7;
+        return Code{*reinterpret_cast<const uint32_t *>(s.qs + int64_t(sb) * s.h * 96 + (ib >> 1) * s.h * 16 + (ib & 1) * 4),
+                    *reinterpret_cast<const uint32_t *>(s.sg + int64_t(sb) * s.h * 96 + (ib >> 2) * s.h * 16 + (ib & 3) * 4)};
     }
-    static __device__ __forceinline__ Rec rec(const Src & s, int sb) { return *reinterpret_cast<const uint4 *>(s.aux + int64_t(sb) * 16); }
-    static __device__ __forceinline__ DRec drec(const Src & s, int sb) { return *reinterpret_cast<const uint32_t *>(s.aux + int64_t(sb) * 16); }
+    static __device__ __forceinline__ Rec rec(const Src & s, int sb) { return *reinterpret_cast<const uint4 *>(s.aux + int64_t(sb) * s.h * 16); }
+    static __device__ __forceinline__ DRec drec(const Src & s, int sb) { return *reinterpret_cast<const uint32_t *>(s.aux + int64_t(sb) * s.h * 16); }
     static __device__ __forceinline__ void planes(const Code & c, const Rec & r, int ib, int g, const uint8_t * tab, const uint32_t * lat, v4i * p) {
-        const uint32_t qh = ib < 2 ? (r.x >> (16 + 8 * ib)) & 0xFFu : ib < 6 ? (r.y >> (8 * (ib - 2))) & 0xFFu : (r.z >> (8 * (ib - 6))) & 0xFFu;
-        const uint32_t scb = (ib >> 1) < 2 ? (r.z >> (16 + 8 * (ib >> 1))) & 0xFFu : (r.w >> (8 * ((ib >> 1) - 2))) & 0xFFu;
-        const uint4 * t = reinterpret_cast<const uint4 *>(tab + ((scb >> (4 * (ib & 1))) & 15u) * 32);
+        const uint32_t qh = iq3s_qh(r, ib) >> (4 * g), sg = c.sg >> (4 * g);
+        const uint4 * t = reinterpret_cast<const uint4 *>(tab + iq3s_ls(r, ib) * 32);
         const uint4 th = t[0], tl = t[1];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {   // operand dword q = the group of four weights 2 g + q / 2 (+ 4 for odd q)
-            const int w = 2 * g + (q >> 1) + 4 * (q & 1);
-            const uint32_t idx = (((w < 4 ? c.qs0 : c.qs1) >> (8 * (w & 3))) & 0xFFu) | (((qh >> w) & 1u) << 8);
+        for (int q = 0; q < 4; ++q) {   // operand dword q
+            const uint32_t idx = ((c.qs >> (8 * q)) & 0xFFu) | (((qh >> q) & 1u) << 8);
             const uint32_t mag = lat[idx];                                      // bytes 1, 3, .., 15
-            const uint32_t i3 = (mag >> 1) & 0x07070707u, sel = (spread4(c.sg >> (4 * w)) << 2) | 0x03020100u;
+            const uint32_t i3 = (mag >> 1) & 0x07070707u, sel = (((sg >> q) << 2) & 0x04040404u) | 0x03020100u;
             p[0][q] = pick16(th, i3, sel);
             p[1][q] = pick16(tl, i3, sel);
         }
@@ -624,7 +625,7 @@ struct WNvfp4 {   // row-major: 16 code bytes per sub-block, one E4M3 scale byte
     struct Code { uint2 c; };
     typedef uint4 Rec;       // the 16 scale bytes of the row's super-block
     typedef uint32_t DRec;   // unused: nothing is folded
-    struct Src { const uint8_t * codes, * aux; };
+    struct Src { const uint8_t * codes, * aux; int h; };
     // per scale byte the 16 products e2m1(code) * e4m3(scale) / 8, rounded to E4M3 (nearest even); the division keeps the
     // largest product (6 * 448) inside the format, and rowmul() gives the 8 back
     static __device__ __forceinline__ void tables(uint8_t * tab, uint32_t *, int tid, int threads) {
@@ -644,10 +645,14 @@ struct WNvfp4 {   // row-major: 16 code bytes per sub-block, one E4M3 scale byte
     static __device__ __forceinline__ Src src(const BankView & b, int e, int wtile, int n, int g) {
         const int S = b.cols / 32;
         const int64_t row = int64_t(e) * b.rows + wtile * 32 + n;
-        return Src{b.codes + row * S * 16 + g * 8, b.aux + row * (b.cols / 16)};
+        const int h = tile_rows(row, b.rows_total);
+        return Src{b.codes + tiled(row, h, S, 0, 16) + g * 8, b.aux + nvfp4_scale_offset(row, h, S, 0), h};
     }
-    static __device__ __forceinline__ Code code(const Src & s, int sub) { return Code{*reinterpret_cast<const uint2 *>(s.codes + int64_t(sub) * 16)}; }
-    static __device__ __forceinline__ Rec rec(const Src & s, int sb) { return *reinterpret_cast<const uint4 *>(s.aux + int64_t(sb) * 16); }
+    static __device__ __forceinline__ Code code(const Src & s, int sub) { return Code{*reinterpret_cast<const uint2 *>(s.codes + int64_t(sub) * s.h * 16)}; }
+    static __device__ __forceinline__ Rec rec(const Src & s, int sb) {   // two pieces of four sub-blocks' scales
+        const uint2 a = *reinterpret_cast<const uint2 *>(s.aux + int64_t(sb) * s.h * 16), b = *reinterpret_cast<const uint2 *>(s.aux + int64_t(sb) * s.h * 16 + s.h * 8);
+        return make_uint4(a.x, a.y, b.x, b.y);
+    }
     static __device__ __forceinline__ DRec drec(const Src &, int) { return 0; }
     static __device__ __forceinline__ void planes(const Code & c, const Rec & r, int ib, int, const uint8_t * tab, const uint32_t *, v4i * p) {
         const uint32_t pair = ((ib >> 1) == 0 ? r.x : (ib >> 1) == 1 ? r.y : (ib >> 1) == 2 ? r.z : r.w) >> (16 * (ib & 1));
