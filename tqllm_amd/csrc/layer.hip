@@ -2,8 +2,13 @@
 #include <algorithm>
 
 #include "formats.cuh"
+#include "grouped_f16_api.cuh"
 
 namespace tqmoe {
+void enqueue_prepare_rows(const void * x, uint32_t xtype, int64_t rows, int cols, uint16_t * out, float * xs, hipStream_t s);
+void enqueue_grouped_plan(const int * counts, const int * offsets, int experts, int4 * plan, hipStream_t s);
+void enqueue_grouped_f16(const tqmoe_bank & b0, const tqmoe_bank * b1, const uint16_t * x, const float * xs, const int * perm, const int4 * plan, int64_t assignments,
+                         int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s);
 int32_t check_bank(const tqmoe_bank * b, const char * what, tqmoe_error * err);
 int32_t enqueue_topk(const float * logits, int32_t * ids, float * weights, float * shared_weights, int32_t * ext_ids, int32_t extra, const void * x,
                      uint32_t xtype, int32_t cols, void * image, int32_t experts, int32_t topk, int32_t n, float scale, int32_t gating,
@@ -26,6 +31,9 @@ int32_t gemm_f16_common(const tqmoe_bank * b0, const tqmoe_bank * b1, const void
 
 namespace {
 
+// From here on the down product of Q4_K banks leaves its rows as halves, as its int8 products always have: the sum over a
+// token's experts reads half the bytes (4096 tokens: 45 us of the layer). Smaller batches and other formats keep fp32 rows.
+constexpr int kQ4kHalfRows = 2048;
 // Where the descriptor asks for the int8 grouped products (act_blocks nonzero), IQ4_XS banks take them from kGroupedMin tokens.
 constexpr int kGroupedMin = 64;
 // Left to the library (act_blocks zero), IQ4_XS banks take them from kInt8Tokens tokens: measured at 512 experts, top-10, on
@@ -44,6 +52,9 @@ struct Plan {  // byte offsets into the workspace
     size_t ximage, aimage, y;                                                // decode path
     size_t xq, xs, counts, offsets, perm, dispatch_ws, act16, aq, as, y16, rq, rs;   // grouped path
     bool blocks;            // int8 products with a scale per 32 activations
+    bool prepared;           // fp16 products on prepared rows
+    bool half_rows;          // their down product's rows are halves
+    size_t x16, xs16, items;
     size_t xbs, abks;        // their block scales
 };
 
@@ -60,16 +71,14 @@ constexpr size_t kLayerBlocksSize = offsetof(tqmoe_layer, swiglu_clamp);
 // the descriptor's request for the int8 grouped products: 0 none (the library chooses), 1 a scale per 32 activations, 2 a scale per token
 int int8_mode_of(const tqmoe_layer & L) { return L.struct_size >= kLayerBlocksSize ? (L.act_blocks == 1 ? 1 : L.act_blocks == 2 ? 2 : 0) : 0; }
 bool act_blocks_of(const tqmoe_layer & L) { return int8_mode_of(L) == 1; }
-// Formats whose 8-bit grouped products are the faster ones at n tokens (measured against the fp16 grouped products at 256
-// experts top-8 and at 64 experts top-8, 256 to 4096 tokens, uniform and Zipf routing): the lattice formats of two and three
-// bits (a tenth faster), NVFP4G on its fp8 products, IQ4_XS from kInt8Tokens tokens, Q4_K from 2048 tokens (with fp32 input
-// rows, which the fp16 kernel converts block by block, int8 is a tenth faster there; with 16-bit rows the two are level).
-// IQ3_S, Q5_K, IQ4_NL, Q4_0 and Q8_0 run 5 to 25 % faster on the fp16 products (their row-major codes reach the int8 kernel's
-// lanes in 8-byte pieces of 32 different rows, and two int8 planes cost the matrix pipe what one fp16 operand does).
+// Formats whose 8-bit grouped products are the faster ones at n tokens: the lattice formats of two and three bits that have
+// no fp16 products on prepared rows (a tenth faster than the fp16 kernel that takes every format), NVFP4G on its fp8
+// products, IQ4_XS from kInt8Tokens tokens. Q4_K, Q6_K and IQ3_S run on prepared fp16 rows at every size (Q4_K at 4096
+// tokens 576 us a layer against 855 on its three int8 planes; IQ3_S at 512 tokens 260 against 393 on the general fp16
+// kernel), the others on the general fp16 kernel, 5 to 25 % faster than int8 there.
 bool int8_faster(uint32_t type, int n) {
     switch (type) {
         case TQMOE_IQ4_XS: return n >= kInt8Tokens;
-        case TQMOE_Q4_K: return n >= 2 * kInt8Tokens;
         case TQMOE_NVFP4G: case TQMOE_IQ3_XXS: case TQMOE_IQ2_XXS: case TQMOE_IQ2_XS: case TQMOE_IQ2_S: case TQMOE_IQ1_S: return true;
         default: return false;
     }
@@ -124,7 +133,16 @@ Plan plan_for(const tqmoe_layer & L, int n) {
             p.xbs = take(size_t(tqmoe_grouped_block_scale_words(int64_t(a), banks, L.hidden)) * 4);
             p.abks = take(size_t(tqmoe_grouped_block_scale_words(int64_t(a), banks, L.ff)) * 4);
         }
-    } else if (!p.grouped) {
+    } else if (p.grouped) {
+        // both products of one kind: the gate / up product leaves its rows in the order the prepared down product reads
+        p.prepared = grouped_f16_takes(L.gate.type, L.ff, L.hidden) && grouped_f16_takes(L.down.type, L.hidden, L.ff) && (!L.has_shared || L.shared_ff % 64 == 0);
+        p.half_rows = L.gate.type == TQMOE_Q4_K && L.down.type == TQMOE_Q4_K && n >= kQ4kHalfRows;
+        if (p.prepared) {
+            p.x16 = take(c * L.hidden * 2);
+            p.xs16 = take(c * 4);
+            p.items = take(size_t(1 + grouped_f16_items(int64_t(a), banks)) * sizeof(int4));
+        }
+    } else {
         p.ximage = take(tqmoe_act_image_bytes(n, L.hidden));
         p.aimage = take(tqmoe_act_image_bytes(int32_t(a), L.ff));
         p.y = take(a * L.hidden * 4);
@@ -228,6 +246,22 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
             uint16_t * act16 = reinterpret_cast<uint16_t *>(ws + p.act16), * y16 = reinterpret_cast<uint16_t *>(ws + p.y16);
             if (int32_t rc = tqmoe_dispatch(cid, counts, offsets, perm, nullptr, 0, banks, c, slots, ws + p.dispatch_ws,
                                             tqmoe_dispatch_workspace_bytes(banks, c, slots), stream, err)) return rc;
+            if (p.prepared) {
+                const hipStream_t st = static_cast<hipStream_t>(stream);
+                uint16_t * x16 = reinterpret_cast<uint16_t *>(ws + p.x16);
+                float * xs16 = reinterpret_cast<float *>(ws + p.xs16);
+                int4 * items = reinterpret_cast<int4 *>(ws + p.items);
+                const int shared_expert = L.has_shared ? banks - 1 : -1;
+                const int64_t a = int64_t(c) * slots;
+                enqueue_prepare_rows(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, x16, xs16, st);
+                enqueue_grouped_plan(counts, offsets, banks, items, st);
+                enqueue_grouped_f16(L.gate, &L.up, x16, xs16, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, st);
+                enqueue_grouped_f16(L.down, nullptr, act16, nullptr, perm, items, a, 1, y16, !p.half_rows, shared_expert, L.shared_ff, Glu{0.f, 0}, st);
+                if (int32_t rc = launched(err, "tqmoe_layer_forward (grouped products)")) return rc;
+                const uint8_t * yb = ws + p.y16;
+                if (int32_t rc = combine(yb, p.half_rows ? TQMOE_F16 : TQMOE_F32, L.has_shared ? yb + size_t(L.topk) * L.hidden * (p.half_rows ? 2 : 4) : nullptr)) return rc;
+                continue;
+            }
             if (!p.int8) {
                 if (int32_t rc = gemm_f16_common(&L.gate, &L.up, xb + size_t(t0) * L.hidden * xbytes, xtype, counts, offsets, perm, c, slots, L.topk, L.shared_ff, slots,
                                                  act16, TQMOE_F16, 1, stream, err, "tqmoe_layer_forward (gate / up)", glu)) return rc;
