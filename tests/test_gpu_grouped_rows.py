@@ -1,5 +1,5 @@
-"""The grouped fp16 products on prepared rows (IQ4_XS, Q4_K, Q6_K, IQ3_S) inside the layer, against the fp32 oracle, at the
-row counts where items and row tiles begin and end."""
+"""The grouped products on prepared rows inside the layer, at the row counts where items and row tiles begin and end: fp16
+(IQ4_XS, Q4_K, Q6_K, IQ3_S) against the fp32 oracle, NVFP4G against the oracle of its E4M3 operands."""
 import numpy as np
 import pytest
 import torch
@@ -16,7 +16,7 @@ def tq():
     return tqllm_amd
 
 
-@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "Q6_K", "IQ3_S"])
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "Q6_K", "IQ3_S", "NVFP4G"])
 @pytest.mark.parametrize("n,hidden,ff,shared_ff", [(32, 256, 256, 0), (33, 512, 256, 256), (64, 256, 512, 256), (65, 1280, 256, 0), (128, 256, 768, 512),
                                                   (129, 512, 512, 512), (700, 768, 512, 0)])
 def test_layer_on_prepared_rows(tq, oracle, fmt, n, hidden, ff, shared_ff):
@@ -31,10 +31,12 @@ def test_layer_on_prepared_rows(tq, oracle, fmt, n, hidden, ff, shared_ff):
         x[:, 0] = 4.0
         router[:, 0] = [0, 3, 0, 0, 4, 0, 0]
     layer = tq.MoeLayer(torch.from_numpy(router).cuda(), dev(inp["shared_gate"]) if shared_ff else None, gate, up, down, 2, shared_ff=shared_ff)
-    assert layer.path(n) == "grouped_f16"
+    fp8 = fmt == "NVFP4G"
+    assert layer.path(n) == ("grouped_fp8" if fp8 else "grouped_f16")
     out, ids, w, logits = (t.cpu().numpy() for t in layer.forward(torch.from_numpy(x).cuda(), return_routing=True))
-    want, want_ids, _ = oracle.layer_forward(x, logits, *raws, cfg["wtype"], hidden, ff, 7, 2, shared_ff=shared_ff, act_mode=0, threads=16)
+    want, want_ids, _ = oracle.layer_forward(x, logits, *raws, cfg["wtype"], hidden, ff, 7, 2, shared_ff=shared_ff, act_mode=2 if fp8 else 0, threads=16)
     clear = clear_tokens(oracle, logits, 7, 2, ids, want_ids)
     assert n == 700 or (np.bincount(ids.reshape(-1), minlength=7) == [0, n, 0, 0, n, 0, 0]).all()
     mx, rel = synth.errors(out[clear], want[clear])
-    assert mx < 1e-2 and rel < 1e-3, (mx, rel)
+    top = float(np.abs(want[clear]).max())     # E4M3's coarse steps amplify last-bit differences of the act rows
+    assert mx < 1e-2 * (max(1.0, top) if fp8 else 1.0) and rel < (3e-3 if fp8 else 1e-3), (mx, rel)

@@ -1,0 +1,499 @@
+// Grouped products of the tile-major bank formats at prefill sizes, on prepared rows: fp16 operands (IQ4_XS, Q4_K, Q6_K,
+// IQ3_S) or E4M3 operands (NVFP4G).
+//
+// A block of four waves takes one item of the plan (an expert and up to 128 of its input rows) and eight tiles of 32 weight
+// rows, two a wave: the same tile of the gate and the up bank, or two tiles of one bank. Per stage (128 bytes of an input row:
+// 64 halves or 128 E4M3 values):
+//  * input rows (in the order the weight operands come in) and the weights' code bytes go straight from memory to LDS one
+//    stage ahead of their use (16 bytes a lane, no registers, no vector instructions); one barrier a stage;
+//  * lane (n, g) of a wave turns the codes of sub-block g (E4M3: sub-blocks g and 2 + g) of weight row n into the sixteen
+//    dwords that are operand B of the stage's four (two) matrix instructions per row tile: decoded weights never pass
+//    through LDS;
+//  * the matrix instructions of operand piece j are followed by the decode of piece j of the next stage into the same
+//    registers, six or so vector instructions to a matrix instruction.
+//
+// Weight values. A code's table value (or the code itself) lands in the low byte of the half 1024 + u by one byte permute
+// or mask per pair; one mixed-precision multiply-add per weight takes the bias off and puts the fp32 scale (and minimum)
+// on, one conversion per pair rounds to fp16: 19 (Q4_K) to 27 (IQ4_XS) vector instructions for eight weights, one rounding.
+// (Packed fp16 multiply-adds take four fewer and round twice: a quarter more error in the layer's result.)
+// NVFP4G: the sixteen products of a scale byte, rounded to E4M3, are a table in LDS (4 KB for all scales); eleven instructions
+// for eight weights.
+//
+// Rows per item: a weight is decoded once per item and wave, so 128 rows spread its instructions over four matrix
+// instructions; with the two banks' eight accumulators (128 registers) two waves fit a SIMD, and one of them decodes while
+// the other's products run. Items of one and two row tiles have loops of their own with fewer products.
+//
+// What bounds it: Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 260 us, 0.8 PFLOP/s, matrix pipe 40 % busy;
+// NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 1.0 ms. A stage of an item with four row tiles takes 5300 cycles
+// where its SIMD's two waves have 2048 of matrix and 1300 to 2000 of vector work. Items of one row tile are bound by the
+// decode (IQ3_S, 512 tokens: 2.5 TB/s of codes).
+#pragma once
+#include "decode_api.cuh"
+#include "decode_table.cuh"
+#include "formats.cuh"
+#include "grouped_rows_api.cuh"
+
+namespace tqmoe {
+namespace {
+
+typedef _Float16 v8h __attribute__((ext_vector_type(8)));
+typedef _Float16 v2h __attribute__((ext_vector_type(2)));
+typedef float v16f __attribute__((ext_vector_type(16)));
+
+// 16 bytes a lane from memory to LDS at `lds` (a wave-uniform byte address) + 16 * lane. The compiler does not count these:
+// dma_wait() says when they are there.
+__device__ __forceinline__ void dma16(const void * p, uint32_t lds) {
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(p), "s"(lds) : "memory");
+}
+// all but the last N transfers of this wave are here (they finish in order); with BARRIER every wave's are
+template <int N, bool BARRIER> __device__ __forceinline__ void dma_wait() {
+    if constexpr (BARRIER) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "i"(N) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" :: "i"(N) : "memory");
+}
+__device__ __forceinline__ uint32_t lds_address(const void * p) {
+    return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t *)(p)));
+}
+
+typedef int v8i __attribute__((ext_vector_type(8)));
+__device__ __forceinline__ v8i join(uint4 a, uint4 b) { return v8i{int(a.x), int(a.y), int(a.z), int(a.w), int(b.x), int(b.y), int(b.z), int(b.w)}; }
+__device__ __forceinline__ v2h as_h2(uint32_t v) { return __builtin_bit_cast(v2h, v); }
+__device__ __forceinline__ uint32_t bits_of(v2h v) { return __builtin_bit_cast(uint32_t, v); }
+__device__ __forceinline__ v2h both(float v) { const _Float16 h = _Float16(v); return v2h{h, h}; }
+__device__ __forceinline__ v2h both_bits(uint32_t h16) { return as_h2(h16 | h16 << 16); }
+// both halves of u times s plus c, in fp32, rounded to halves: two v_fma_mix_f32 and a packed conversion (v_fma_mixlo_f16 and
+// v_fma_mixhi_f16 do it in two, at half the rate)
+__device__ __forceinline__ uint32_t mix2(v2h u, float s, float c) {
+    const float lo = fmaf(float(u[0]), s, c), hi = fmaf(float(u[1]), s, c);
+    return bits_of(v2h{_Float16(lo), _Float16(hi)});
+}
+// bytes 0, 2 and bytes 1, 3 of u as halves 1024 + byte
+__device__ __forceinline__ v2h bias_even(uint32_t u) { return as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04020400u)); }
+__device__ __forceinline__ v2h bias_odd(uint32_t u) { return as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04030401u)); }
+
+// What the kernel needs of a format.
+// kCodes: 1 KB transfers a bank and stage (64 lanes x 16 bytes): code() the lane's source, code_at() what to add
+// for a transfer and stage. kRecs transfers for both banks' records: rec(), rec_at(). Prep: what decoding a stage needs in registers;
+// slice(): piece j (16 bytes) of operand B. kTab bytes of lookup table in LDS, filled by tables(). row_factor(): a factor
+// of a whole weight row.
+template <uint32_t FMT> struct GroupedFormat;
+
+struct GroupedHalves {
+    static constexpr bool kFp8 = false;
+    static constexpr int kTab = 16;
+    static __device__ __forceinline__ void tables(uint8_t *, int) {}
+    static __device__ __forceinline__ float row_factor(const BankView &, int64_t) { return 1.f; }
+};
+struct GroupedNibbles : GroupedHalves {   // 16 code bytes a sub-block in the canonical order
+    static constexpr int kCodes = 1, kRecs = 1;
+    static __device__ __forceinline__ const uint8_t * code(const BankView & b, int64_t tile, int S, int lane) { return b.codes + tile * S * 512 + lane * 16; }
+    static __device__ __forceinline__ int code_at(int, int st) { return st * 1024; }
+};
+
+template <> struct GroupedFormat<TQMOE_IQ4_XS> : GroupedNibbles {
+    static __device__ __forceinline__ const uint8_t * rec(const BankView & b0, const BankView & b1, int64_t tile0, int64_t tile1, int S, int, int lane) {
+        const int l = lane & 31;   // sixteen lanes a bank; the upper half of the wave repeats the lower
+        return (l < 16 ? b0.aux + tile0 * (S / 8) * 256 : b1.aux + tile1 * (S / 8) * 256) + (l & 15) * 16;
+    }
+    static __device__ __forceinline__ int rec_at(int, int st) { return (st >> 2) * 256; }
+    struct Prep { uint32_t c[4]; float s, off; };
+    static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int st, int n, int g, const uint8_t *, Prep & p) {
+        const uint4 c = *reinterpret_cast<const uint4 *>(w + nb * 1024 + g * 512 + n * 16);
+        const uint2 r = *reinterpret_cast<const uint2 *>(w + 2048 + nb * 256 + n * 8);
+        p.c[0] = c.x; p.c[1] = c.y; p.c[2] = c.z; p.c[3] = c.w;
+        p.s = half_bits_to_float(iq4xs_d_bits(r)) * float(iq4xs_lsm32(r, (2 * st + g) & 7));   // 17 bits: exact
+        p.off = p.s * -1152.f;                                                                 // four more: exact
+    }
+    static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
+        constexpr Table16 t = table16({1, 24, 45, 63, 79, 93, 106, 118, 129, 141, 153, 166, 181, 197, 217, 241});   // the values + 128
+        const uint32_t c = p.c[j], lo = pick(t, c & 0x0F0F0F0Fu), hi = pick(t, (c >> 4) & 0x0F0F0F0Fu);
+        return make_uint4(mix2(bias_even(lo), p.s, p.off), mix2(bias_odd(lo), p.s, p.off), mix2(bias_even(hi), p.s, p.off), mix2(bias_odd(hi), p.s, p.off));
+    }
+};
+
+template <> struct GroupedFormat<TQMOE_Q4_K> : GroupedNibbles {
+    static __device__ __forceinline__ const uint8_t * rec(const BankView & b0, const BankView & b1, int64_t tile0, int64_t tile1, int S, int, int lane) {
+        return (lane < 32 ? b0.aux + tile0 * (S / 8) * 512 : b1.aux + tile1 * (S / 8) * 512) + (lane & 31) * 16;
+    }
+    static __device__ __forceinline__ int rec_at(int, int st) { return (st >> 2) * 512; }
+    struct Prep { uint32_t c[4]; float s, off; };
+    static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int st, int n, int g, const uint8_t *, Prep & p) {
+        const uint4 c = *reinterpret_cast<const uint4 *>(w + nb * 1024 + g * 512 + n * 16);
+        const uint4 r = *reinterpret_cast<const uint4 *>(w + 2048 + nb * 512 + n * 16);
+        p.c[0] = c.x; p.c[1] = c.y; p.c[2] = c.z; p.c[3] = c.w;
+        int sc, mn;
+        q4k_scale_min_flat(r.y, r.z, r.w, (2 * st + g) & 7, sc, mn);
+        p.s = half_bits_to_float(uint16_t(r.x & 0xFFFFu)) * float(sc);
+        // the bias and the minimum in one constant: its rounding is 2^-15 of a code step
+        p.off = -fmaf(p.s, 1024.f, half_bits_to_float(uint16_t(r.x >> 16)) * float(mn));
+    }
+    static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
+        const uint32_t c = p.c[j];
+        uint32_t mask = 0x000F000Fu;
+        asm("" : "+v"(mask));                      // in a register, so that mask and bias are one instruction
+        auto val = [&](uint32_t x) { return mix2(as_h2((x & mask) | 0x64006400u), p.s, p.off); };
+        return make_uint4(val(c), val(c >> 8), val(c >> 4), val(c >> 12));
+    }
+};
+
+template <> struct GroupedFormat<TQMOE_Q6_K> : GroupedHalves {
+    static constexpr int kCodes = 1, kRecs = 3;   // low nibbles; then both banks' upper bits (512 bytes each) and each bank's records
+    static __device__ __forceinline__ const uint8_t * code(const BankView & b, int64_t tile, int S, int lane) { return b.codes + tile * (S / 8) * 6144 + lane * 16; }
+    static __device__ __forceinline__ int code_at(int, int st) { return (st >> 2) * 6144 + (st & 3) * 1024; }
+    static __device__ __forceinline__ const uint8_t * rec(const BankView & b0, const BankView & b1, int64_t tile0, int64_t tile1, int S, int i, int lane) {
+        if (i == 0) return (lane < 32 ? b0.codes + tile0 * (S / 8) * 6144 : b1.codes + tile1 * (S / 8) * 6144) + 4096 + (lane & 31) * 16;
+        return (i == 1 ? b0.aux + tile0 * (S / 8) * 1024 : b1.aux + tile1 * (S / 8) * 1024) + lane * 16;
+    }
+    static __device__ __forceinline__ int rec_at(int i, int st) { return i == 0 ? (st >> 2) * 6144 + (st & 3) * 512 : (st >> 2) * 1024; }
+    struct Prep { uint32_t lo[4], hi[2]; float s[2], off[2]; };
+    static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int st, int n, int g, const uint8_t *, Prep & p) {
+        const uint4 c = *reinterpret_cast<const uint4 *>(w + nb * 1024 + g * 512 + n * 16);
+        p.lo[0] = c.x; p.lo[1] = c.y; p.lo[2] = c.z; p.lo[3] = c.w;
+        p.hi[0] = *reinterpret_cast<const uint32_t *>(w + 2048 + nb * 512 + n * 16 + g * 4);
+        p.hi[1] = *reinterpret_cast<const uint32_t *>(w + 2048 + nb * 512 + n * 16 + 8 + g * 4);
+        const uint8_t * r = w + 3072 + nb * 1024 + n * 32;
+        const uint32_t s2 = *reinterpret_cast<const uint16_t *>(r + 2 * ((2 * st + g) & 7));
+        const float d = 0.25f * half_bits_to_float(*reinterpret_cast<const uint16_t *>(r + 16));   // the operand byte is four times the value
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            p.s[i] = d * float(int(__builtin_amdgcn_sbfe(int(s2), 8 * i, 8)));
+            p.off[i] = p.s[i] * -1152.f;           // 18 bits and four: exact
+        }
+    }
+    static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
+        // dword j of the low nibbles: half j / 2 of the sub-block, its operand dwords 2 (j % 2) and + 1
+        const uint32_t lo = p.lo[j], hi = p.hi[j >> 1] >> (4 * (j & 1));
+        const uint32_t a = ((lo << 2) & 0x3C3C3C3Cu) | ((hi << 6) & 0xC0C0C0C0u), b = ((lo >> 2) & 0x3C3C3C3Cu) | ((hi << 4) & 0xC0C0C0C0u);
+        auto val = [&](v2h u, int i) { return mix2(u, p.s[i], p.off[i]); };
+        const uint32_t ua = a ^ 0x80808080u, ub = b ^ 0x80808080u;
+        return make_uint4(val(bias_even(ua), 0), val(bias_odd(ua), 0), val(bias_even(ub), 1), val(bias_odd(ub), 1));
+    }
+};
+
+template <> struct GroupedFormat<TQMOE_IQ3_S> : GroupedHalves {
+    static constexpr int kCodes = 1, kRecs = 1, kTab = 512 * 8;
+    static __device__ __forceinline__ void tables(uint8_t * tab, int tid) {   // a lattice point's magnitudes as halves, weights 0, 2, 1, 3
+        for (int i = tid; i < 512; i += 256) {
+            const v2h bias = as_h2(0xE400E400u);       // -1024
+            const uint32_t m = d_iq3s_grid.v[i];
+            reinterpret_cast<uint2 *>(tab)[i] = make_uint2(bits_of(bias_even(m) + bias), bits_of(bias_odd(m) + bias));
+        }
+    }
+    static __device__ __forceinline__ const uint8_t * code(const BankView & b, int64_t tile, int S, int lane) {   // the pair's indices, then the signs
+        return b.codes + tile * (S / 8) * 3072 + (lane < 32 ? 0 : 2048) + (lane & 31) * 16;
+    }
+    // (indices: 512 bytes a pair, signs: 512 bytes two pairs; the lane's own step)
+    static __device__ __forceinline__ int code_at(int, int st) { return (st >> 2) * 3072 + ((threadIdx.x & 32) ? ((st & 3) >> 1) * 512 : (st & 3) * 512); }
+    static __device__ __forceinline__ const uint8_t * rec(const BankView & b0, const BankView & b1, int64_t tile0, int64_t tile1, int S, int, int lane) {
+        return (lane < 32 ? b0.aux + tile0 * (S / 8) * 512 : b1.aux + tile1 * (S / 8) * 512) + (lane & 31) * 16;
+    }
+    static __device__ __forceinline__ int rec_at(int, int st) { return (st >> 2) * 512; }
+    struct Prep { uint32_t qs[2], sg, qh; v2h sc, d; const uint2 * lat; };
+    static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int st, int n, int g, const uint8_t * tab, Prep & p) {
+        const uint8_t * q = w + nb * 1024 + n * 16;
+        p.qs[0] = *reinterpret_cast<const uint32_t *>(q + g * 4);
+        p.qs[1] = *reinterpret_cast<const uint32_t *>(q + 8 + g * 4);
+        const int ib = (2 * st + g) & 7;
+        p.sg = *reinterpret_cast<const uint32_t *>(q + 512 + (ib & 3) * 4);
+        const uint4 r = *reinterpret_cast<const uint4 *>(w + 2048 + nb * 512 + n * 16);
+        p.qh = (ib < 4 ? r.y : r.z) >> (8 * (ib & 3));
+        const uint32_t ls = (ib < 4 ? r.x >> (16 + 4 * ib) : r.w >> (4 * (ib - 4))) & 15u;
+        p.sc = both(float(1 + 2 * int(ls)));
+        p.d = both_bits(r.x & 0xFFFFu);
+        p.lat = reinterpret_cast<const uint2 *>(tab);
+    }
+    static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
+        const int h = j >> 1, q = 2 * (j & 1);     // operand dwords q and q + 1 of half h: weights 4 j .. and 16 + 4 j ..
+        uint32_t v[4];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const uint32_t idx = ((p.qs[h] >> (8 * (q + i))) & 0xFFu) | ((p.qh << (8 - 4 * h - q - i)) & 0x100u);
+            const uint2 mag = p.lat[idx];          // the four magnitudes as halves, weights 0, 2 and 1, 3
+            const int s = 4 * h + q + i;           // bit 8 t + s: the sign of weight t
+            // times the integer scale (exact), times d (the one rounding)
+            v[2 * i] = bits_of(as_h2(mag.x ^ ((p.sg << (15 - s)) & 0x80008000u)) * p.sc * p.d);
+            v[2 * i + 1] = bits_of(as_h2(mag.y ^ ((p.sg << (7 - s)) & 0x80008000u)) * p.sc * p.d);
+        }
+        return make_uint4(v[0], v[1], v[2], v[3]);
+    }
+};
+
+template <> struct GroupedFormat<TQMOE_NVFP4G> {
+    static constexpr bool kFp8 = true;
+    static constexpr int kCodes = 2, kRecs = 1, kTab = 256 * 16;
+    // Per scale byte the 16 products e2m1(code) * e4m3(scale) / 8, rounded to E4M3 (nearest even; an eighth keeps the largest
+    // inside the format, row_factor gives it back), as the two pools of pick().
+    static __device__ __forceinline__ void tables(uint8_t * tab, int tid) {
+        const float sc = e4m3_to_float(uint32_t(tid));
+        uint32_t v[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float f[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint32_t twice = ((q == 0 ? kFp4T0 : q == 1 ? kFp4T1 : q == 2 ? kFp4T2 : kFp4T3) >> (8 * j)) & 0xFFu;
+                f[j] = fminf(fmaxf(float(int8_t(twice)) * 0.0625f * sc, -448.f), 448.f);
+            }
+            int w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+            v[q] = uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w, true));
+        }
+        reinterpret_cast<uint4 *>(tab)[tid] = table16_pools(v);
+    }
+    static __device__ __forceinline__ const uint8_t * code(const BankView & b, int64_t tile, int S, int lane) { return b.codes + tile * S * 512 + lane * 16; }
+    static __device__ __forceinline__ int code_at(int i, int st) { return st * 2048 + i * 1024; }
+    static __device__ __forceinline__ const uint8_t * rec(const BankView & b0, const BankView & b1, int64_t tile0, int64_t tile1, int S, int, int lane) {
+        const int l = lane & 31;   // eight bytes a row and stage: sixteen lanes a bank, the upper half of the wave repeats the lower
+        return (l < 16 ? b0.aux + tile0 * (S / 4) * 256 : b1.aux + tile1 * (S / 4) * 256) + (l & 15) * 16;
+    }
+    static __device__ __forceinline__ int rec_at(int, int st) { return st * 256; }
+    struct Prep { uint32_t c[2][4], sc[2]; uint4 t0, t1; const uint8_t * tab; };
+    static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int, int n, int g, const uint8_t * tab, Prep & p) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {   // sub-blocks g and 2 + g
+            const uint4 c = *reinterpret_cast<const uint4 *>(w + nb * 2048 + i * 1024 + g * 512 + n * 16);
+            p.c[i][0] = c.x; p.c[i][1] = c.y; p.c[i][2] = c.z; p.c[i][3] = c.w;
+        }
+        const uint2 r = *reinterpret_cast<const uint2 *>(w + 4096 + nb * 256 + n * 8);
+        p.sc[0] = r.x >> (16 * g);
+        p.sc[1] = r.y >> (16 * g);
+        p.tab = tab;
+    }
+    static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
+        const int i = j >> 1, h = j & 1;
+        if (h == 0) {
+            p.t0 = *reinterpret_cast<const uint4 *>(p.tab + (p.sc[i] & 0xFFu) * 16);
+            p.t1 = *reinterpret_cast<const uint4 *>(p.tab + ((p.sc[i] >> 8) & 0xFFu) * 16);
+        }
+        const Table16 lo{p.t0.x, p.t0.y, p.t0.z, p.t0.w}, hi{p.t1.x, p.t1.y, p.t1.z, p.t1.w};
+        const uint32_t a = p.c[i][2 * h], b = p.c[i][2 * h + 1], m = 0x0F0F0F0Fu;
+        return make_uint4(pick(lo, a & m), pick(hi, (a >> 4) & m), pick(lo, b & m), pick(hi, (b >> 4) & m));
+    }
+    static __device__ __forceinline__ float row_factor(const BankView & b, int64_t row) {
+        return 8.f * *reinterpret_cast<const float *>(b.aux + nvfp4_global_offset(b.rows_total, b.cols) + row * 4);
+    }
+};
+
+// bytes of a wave's codes and records of one stage
+template <class W> constexpr int kStageW = 2 * W::kCodes * 1024 + W::kRecs * 1024;
+template <class W> constexpr int kStageCols = W::kFp8 ? 128 : 64;   // columns of a stage: 128 bytes of a row
+// blocks a compute unit holds (four waves each, so waves a SIMD): the accumulators of MAX row tiles set the registers, longer
+// codes the LDS
+template <class W, int MAX> constexpr int kGroupedWaves = MAX == 4 || kStageW<W> > 4096 ? 2 : 3;
+// Stages of input rows and of codes in LDS for MT row tiles, in the part of a compute unit's 160 KB that one of its blocks may
+// take. Codes come from HBM and may be two and more stages on their way; rows come from the L2 (an item's other blocks read
+// the same). (Q4_K at 4096 tokens: 554 us a layer with one stage of codes under way, 521 with two.)
+template <class W, int MT, int MAX> struct Rings {
+    static constexpr int kLds = 163840 / kGroupedWaves<W, MAX> - W::kTab - 1280;   // what one of the unit's blocks may take
+    static constexpr int kRows = MT == 4 || MAX == 2 ? 2 : MT == 2 || kStageW<W> > 4096 ? 3 : 4;
+    static constexpr int kRoom = (kLds - kRows * MT * 4096) / (4 * kStageW<W>);
+    static constexpr int kCodes = kRoom < 5 ? kRoom : 5;
+    static_assert(kCodes >= 2, "two stages of codes");
+    static constexpr int kBytes = kRows * MT * 4096 + 4 * kCodes * kStageW<W>;
+};
+template <class W, int MAX> constexpr int grouped_lds() {
+    const int a = Rings<W, 1, MAX>::kBytes, b = Rings<W, 2, MAX>::kBytes, c = Rings<W, MAX, MAX>::kBytes;
+    return a > b ? (a > c ? a : c) : (b > c ? b : c);
+}
+
+template <uint32_t FMT, int MAX, bool GATEUP, class OT>   // MAX: row tiles of an item at most
+__global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void grouped_rows_k(GroupedArgs k) {
+    using W = GroupedFormat<FMT>;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [kRows][MT * 4096] input rows | [4 waves][kCodes][kStageW] codes and records
+    __shared__ __attribute__((aligned(16))) uint8_t s_tab[W::kTab];
+    constexpr int kItemRows = 32 * MAX;
+    __shared__ int s_asg[kItemRows];
+    __shared__ float s_scale[kItemRows];
+    // Items that share input rows (an item of the plan, all its groups of weight tiles) run on one XCD, one after the other.
+    const int xcd = int(blockIdx.x) & 7, at = int(blockIdx.x) >> 3;
+    const int chunk = at / k.groups * 8 + xcd, grp = at % k.groups;
+    if (chunk >= k.plan[0].x) return;
+    const int4 item = k.plan[1 + chunk];           // expert, its first row in perm, rows, first row tile
+    const int e = item.x, cnt = item.z;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 31, g = lane >> 5;
+    const int rows = k.b0.rows, cols = k.b0.cols, S = cols / 32, tiles = rows / 32;
+    const bool is_shared = e == k.shared_expert;
+    const int row_lim = GATEUP && is_shared ? k.shared_lim : rows;
+    const int stages = (!GATEUP && is_shared ? k.shared_lim : cols) / kStageCols<W>;
+    W::tables(s_tab, tid);
+    if (tid < kItemRows) {
+        s_asg[tid] = tid < cnt ? k.perm[item.y + tid] : -1;
+        s_scale[tid] = 1.f;
+        if (k.xs && tid < cnt) s_scale[tid] = k.xs[W::kFp8 && k.row_tiles ? item.w * 32 + tid : s_asg[tid] / k.xdiv];
+    }
+    __syncthreads();
+    // weight tiles of this wave (past the last one: it once more, not stored)
+    int wt[2];
+#pragma unroll
+    for (int b = 0; b < 2; ++b) wt[b] = GATEUP ? grp * 4 + wave : grp * 8 + wave * 2 + b;
+
+    auto body = [&](auto tag) {
+        constexpr int MT = decltype(tag)::value;
+        v16f acc[2][MT];
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int i = 0; i < 16; ++i) acc[b][m][i] = 0.f;
+        const bool any = GATEUP ? grp * 128 < row_lim : true;
+        if (any) {
+            using R = Rings<W, MT, MAX>;
+            constexpr int LA = R::kRows - 1, LW = R::kCodes, LM = LA > LW ? LA : LW;   // stages ahead: stage t sends the rows of t + LA and the codes of t + LW
+            constexpr int NA = MT, NW = 2 * W::kCodes + W::kRecs;   // transfers a wave sends for a stage
+            // input rows: transfer q of a wave is rows 8 (4 q + wave) .. + 7 of the stage's 128 bytes, a row's piece p in slot
+            // p ^ (row & 7), so that the operand reads (a row a lane) find eight rows' pieces in eight different bank groups
+            const uint8_t * a_src[MT];
+#pragma unroll
+            for (int q = 0; q < MT; ++q) {
+                const int row = (4 * q + wave) * 8 + (lane >> 3), piece = (lane & 7) ^ (row & 7);
+                if (W::kFp8 && k.row_tiles)   // operand-major tiles of 32 rows: 1 KB a sub-block, the rows' first halves, then their second
+                    a_src[q] = static_cast<const uint8_t *>(k.x) + (int64_t(item.w) + (row >> 5)) * 32 * cols + (piece >> 1) * 1024 + (piece & 1) * 512 + (row & 31) * 16;
+                else
+                    a_src[q] = static_cast<const uint8_t *>(k.x) + (int64_t(max(s_asg[row], 0)) / k.xdiv * cols) * (W::kFp8 ? 1 : 2) + piece * 16;
+            }
+            const int a_step = W::kFp8 && k.row_tiles ? 4096 : 128;
+            const uint32_t lds0 = lds_address(lds);
+            uint8_t * const w_lds = lds + R::kRows * MT * 4096 + wave * R::kCodes * kStageW<W>;
+            const uint32_t w_lds0 = lds_address(w_lds);
+            const int64_t t0 = int64_t(e) * tiles + min(wt[0], tiles - 1), t1 = int64_t(e) * tiles + min(wt[1], tiles - 1);
+            const uint8_t * c_src[2] = {W::code(k.b0, t0, S, lane), W::code(k.b1, t1, S, lane)}, * r_src[W::kRecs];
+#pragma unroll
+            for (int i = 0; i < W::kRecs; ++i) r_src[i] = W::rec(k.b0, k.b1, t0, t1, S, i, lane);
+            auto send_a = [&](int st, int slot) {
+                if (st >= stages) return;
+#pragma unroll
+                for (int q = 0; q < MT; ++q) dma16(a_src[q] + st * a_step, lds0 + slot * MT * 4096 + (4 * q + wave) * 1024);
+            };
+            auto send_w = [&](int st, int slot) {
+                if (st >= stages) return;
+                const uint32_t to = w_lds0 + slot * kStageW<W>;
+#pragma unroll
+                for (int b = 0; b < 2; ++b)
+#pragma unroll
+                    for (int i = 0; i < W::kCodes; ++i) dma16(c_src[b] + W::code_at(i, st), to + (b * W::kCodes + i) * 1024);
+#pragma unroll
+                for (int i = 0; i < W::kRecs; ++i) dma16(r_src[i] + W::rec_at(i, st), to + (2 * W::kCodes + i) * 1024);
+            };
+            const uint8_t * a_row = lds + n * 128;
+            uint4 bw[2][4];
+            typename W::Prep pr[2];
+#pragma unroll
+            for (int t = -LM; t < 0; ++t) {   // what the stages before the first would have sent
+                if (t + LA >= 0) send_a(t + LA, t + LA);
+                if (t + LW >= 0) send_w(t + LW, t + LW);
+            }
+            if (LM <= stages) dma_wait<(LW - 1) * NW + (LA < LW ? LA : LW - 1) * NA, false>(); else dma_wait<0, false>();
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                W::prep(w_lds, b, 0, n, g, s_tab, pr[b]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) bw[b][j] = W::slice(pr[b], j);
+            }
+            int a_at = 0, w_at = 0;           // slots of this stage's rows and codes
+            for (int st = 0; st < stages; ++st) {
+                // this stage's rows and the next one's codes are here (what the stages since have sent may be under way, where
+                // they have sent all), and every wave is done with the slots that are filled now
+                constexpr int kSinceA = NW + (LA - 1) * (NA + NW), kSinceW = (LW - 2) * (NA + NW);
+                if (st + LM <= stages) dma_wait<(kSinceA < kSinceW ? kSinceA : kSinceW), true>(); else dma_wait<0, true>();
+                send_a(st + LA, a_at == 0 ? LA : a_at - 1);
+                send_w(st + LW, w_at);
+                w_at = w_at + 1 == LW ? 0 : w_at + 1;
+                const bool more = st + 1 < stages;   // (past the last stage: its own codes again, not used)
+                const int w_next = more ? w_at : w_at == 0 ? LW - 1 : w_at - 1;
+#pragma unroll
+                for (int b = 0; b < 2; ++b) W::prep(w_lds + w_next * kStageW<W>, b, more ? st + 1 : st, n, g, s_tab, pr[b]);
+                const uint8_t * a_buf = a_row + a_at * MT * 4096;
+                a_at = a_at + 1 == LA + 1 ? 0 : a_at + 1;
+                uint4 a[2][MT];
+                // piece j of a row is the 16 bytes that go with piece j of operand B (E4M3: two pieces are one operand)
+                auto read_a = [&](int j) {
+                    const int piece = W::kFp8 ? 4 * (j >> 1) + 2 * g + (j & 1) : 4 * g + j;
+#pragma unroll
+                    for (int m = 0; m < MT; ++m) a[j & 1][m] = *reinterpret_cast<const uint4 *>(a_buf + m * 4096 + ((piece ^ (n & 7)) * 16));
+                };
+                read_a(0);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if constexpr (W::kFp8) {
+                        if (j & 1) continue;
+                        read_a(j + 1);
+#pragma unroll
+                        for (int b = 0; b < 2; ++b)
+#pragma unroll
+                            for (int m = 0; m < MT; ++m)
+                                acc[b][m] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(join(a[0][m], a[1][m]), join(bw[b][j], bw[b][j + 1]), acc[b][m], 0, 0, 0, 0, 0, 0);
+                        if (j < 2) read_a(j + 2);
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) { bw[b][j] = W::slice(pr[b], j); bw[b][j + 1] = W::slice(pr[b], j + 1); }
+                    } else {
+                        if (j < 3) read_a(j + 1);
+#pragma unroll
+                        for (int b = 0; b < 2; ++b)
+#pragma unroll
+                            for (int m = 0; m < MT; ++m)
+                                acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[j & 1][m]), __builtin_bit_cast(v8h, bw[b][j]), acc[b][m], 0, 0, 0);
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) bw[b][j] = W::slice(pr[b], j);
+                    }
+                }
+            }
+        }
+        if constexpr (W::kFp8) {
+#pragma unroll
+            for (int b = 0; b < 2; ++b) {
+                const float f = W::row_factor(b ? k.b1 : k.b0, (int64_t(e) * tiles + min(wt[b], tiles - 1)) * 32 + n);
+#pragma unroll
+                for (int m = 0; m < MT; ++m)
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) acc[b][m][i] *= f;
+            }
+        }
+        // result register i of lane half g: input row 8 (i / 4) + 4 g + i % 4 of the row tile, weight row n of the weight tile
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            int asg[16];
+            float scl[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) { const int r = m * 32 + 8 * (i >> 2) + 4 * g + (i & 3); asg[i] = s_asg[r]; scl[i] = s_scale[r]; }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if (asg[i] < 0) continue;
+                OT * o = static_cast<OT *>(k.out) + int64_t(asg[i]) * rows;
+                auto put = [&](int col, float v) {
+                    if constexpr (sizeof(OT) == 4) o[col] = v;
+                    else o[col] = W::kFp8 && k.out_bf16 ? float_to_bf16_bits(v) : __half_as_ushort(__float2half_rn(v));
+                };
+                if constexpr (GATEUP) {
+                    if (wt[0] >= tiles) continue;
+                    float gv = acc[0][m][i] * scl[i], uv = acc[1][m][i] * scl[i];
+                    glu_clamp_inputs(k.glu, gv, uv);
+                    const float v = glu_clamp_silu(k.glu, gv * __builtin_amdgcn_rcpf(1.f + __expf(-gv))) * uv;
+                    put(wt[0] * 32 + (W::kFp8 ? n : operand_pos(n)), wt[0] * 32 < row_lim ? v : 0.f);
+                } else {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) if (wt[b] < tiles) put(wt[b] * 32 + n, acc[b][m][i] * scl[i]);
+                }
+            }
+        }
+    };
+    if (cnt <= 32) body(std::integral_constant<int, 1>{});
+    else if (MAX == 2 || cnt <= 64) body(std::integral_constant<int, 2>{});
+    else body(std::integral_constant<int, MAX>{});
+}
+
+template <uint32_t FMT, int MAX> void grouped_rows_launch_max(const GroupedArgs & k, bool gateup, bool f32_out, unsigned blocks, hipStream_t s) {
+    constexpr int bytes = grouped_lds<GroupedFormat<FMT>, MAX>();
+    auto go = [&](auto kernel) {
+        allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes);
+        kernel<<<blocks, 256, bytes, s>>>(k);
+    };
+    if (gateup) go(&grouped_rows_k<FMT, MAX, true, uint16_t>);
+    else if (f32_out) go(&grouped_rows_k<FMT, MAX, false, float>);
+    else go(&grouped_rows_k<FMT, MAX, false, uint16_t>);
+}
+template <uint32_t FMT> void grouped_rows_launch(const GroupedArgs & k, int item_rows, bool gateup, bool f32_out, unsigned blocks, hipStream_t s) {
+    if (item_rows == 64) grouped_rows_launch_max<FMT, 2>(k, gateup, f32_out, blocks, s);
+    else grouped_rows_launch_max<FMT, 4>(k, gateup, f32_out, blocks, s);
+}
+
+}  // namespace
+}  // namespace tqmoe

@@ -2,13 +2,9 @@
 #include <algorithm>
 
 #include "formats.cuh"
-#include "grouped_f16_api.cuh"
+#include "grouped_rows_api.cuh"
 
 namespace tqmoe {
-void enqueue_prepare_rows(const void * x, uint32_t xtype, int64_t rows, int cols, uint16_t * out, float * xs, hipStream_t s);
-void enqueue_grouped_plan(const int * counts, const int * offsets, int experts, int4 * plan, hipStream_t s);
-void enqueue_grouped_f16(const tqmoe_bank & b0, const tqmoe_bank * b1, const uint16_t * x, const float * xs, const int * perm, const int4 * plan, int64_t assignments,
-                         int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s);
 int32_t check_bank(const tqmoe_bank * b, const char * what, tqmoe_error * err);
 int32_t enqueue_topk(const float * logits, int32_t * ids, float * weights, float * shared_weights, int32_t * ext_ids, int32_t extra, const void * x,
                      uint32_t xtype, int32_t cols, void * image, int32_t experts, int32_t topk, int32_t n, float scale, int32_t gating,
@@ -54,6 +50,7 @@ struct Plan {  // byte offsets into the workspace
     bool blocks;            // int8 products with a scale per 32 activations
     bool prepared;           // fp16 products on prepared rows
     bool half_rows;          // their down product's rows are halves
+    int item_rows;           // rows of their items at most
     size_t x16, xs16, items;
     size_t xbs, abks;        // their block scales
 };
@@ -119,7 +116,17 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         p.act16 = take(a * L.ff * 2);
         p.y16 = take(a * L.hidden * 4);   // fp16 rows (int8 products) or fp32 rows (fp16 products)
     }
-    if (p.int8) {
+    // the products on prepared rows take both banks: the gate / up product leaves its rows in the order the down product reads
+    const bool rows_ok = grouped_rows_takes(L.gate.type, L.ff, L.hidden) && grouped_rows_takes(L.down.type, L.hidden, L.ff) && (!L.has_shared || L.shared_ff % 128 == 0);
+    p.item_rows = grouped_rows_per_item(L.gate.type, int64_t(a), banks);
+    if (p.int8 && plane_gemm_is_fp8(L.gate.type)) {
+        p.prepared = rows_ok;    // int8_ok's conditions are the stricter ones
+        p.rq = take(c * L.hidden);
+        p.rs = take(c * 4);
+        p.aq = take(a * L.ff);
+        p.as = take(a * 4);
+        p.items = take(size_t(1 + grouped_rows_items(int64_t(a), banks, p.item_rows)) * sizeof(int4));
+    } else if (p.int8) {
         const size_t grows = size_t(tqmoe_grouped_rows(int64_t(a), banks));
         p.xq = take(grows * L.hidden);
         const size_t gwords = size_t(tqmoe_grouped_scale_words(int64_t(a), banks));
@@ -134,13 +141,12 @@ Plan plan_for(const tqmoe_layer & L, int n) {
             p.abks = take(size_t(tqmoe_grouped_block_scale_words(int64_t(a), banks, L.ff)) * 4);
         }
     } else if (p.grouped) {
-        // both products of one kind: the gate / up product leaves its rows in the order the prepared down product reads
-        p.prepared = grouped_f16_takes(L.gate.type, L.ff, L.hidden) && grouped_f16_takes(L.down.type, L.hidden, L.ff) && (!L.has_shared || L.shared_ff % 64 == 0);
+        p.prepared = rows_ok && !plane_gemm_is_fp8(L.gate.type) && !plane_gemm_is_fp8(L.down.type);
         p.half_rows = L.gate.type == TQMOE_Q4_K && L.down.type == TQMOE_Q4_K && n >= kQ4kHalfRows;
         if (p.prepared) {
             p.x16 = take(c * L.hidden * 2);
             p.xs16 = take(c * 4);
-            p.items = take(size_t(1 + grouped_f16_items(int64_t(a), banks)) * sizeof(int4));
+            p.items = take(size_t(1 + grouped_rows_items(int64_t(a), banks, p.item_rows)) * sizeof(int4));
         }
     } else {
         p.ximage = take(tqmoe_act_image_bytes(n, L.hidden));
@@ -246,6 +252,22 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
             uint16_t * act16 = reinterpret_cast<uint16_t *>(ws + p.act16), * y16 = reinterpret_cast<uint16_t *>(ws + p.y16);
             if (int32_t rc = tqmoe_dispatch(cid, counts, offsets, perm, nullptr, 0, banks, c, slots, ws + p.dispatch_ws,
                                             tqmoe_dispatch_workspace_bytes(banks, c, slots), stream, err)) return rc;
+            if (p.prepared && p.int8) {   // E4M3 rows
+                const hipStream_t st = static_cast<hipStream_t>(stream);
+                uint8_t * rq = ws + p.rq, * aq = ws + p.aq;
+                float * rs = reinterpret_cast<float *>(ws + p.rs), * as = reinterpret_cast<float *>(ws + p.as);
+                int4 * items = reinterpret_cast<int4 *>(ws + p.items);
+                const int shared_expert = L.has_shared ? banks - 1 : -1;
+                const int64_t a = int64_t(c) * slots;
+                if (int32_t rc = tqmoe_quant_rows_fp8(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, stream, err)) return rc;
+                enqueue_grouped_plan(counts, offsets, banks, p.item_rows, items, RowIndex{}, st);
+                enqueue_grouped_products(L.gate, &L.up, rq, rs, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, st, p.item_rows);
+                if (int32_t rc = tqmoe_quant_rows_fp8(act16, TQMOE_F16, a, L.ff, aq, as, stream, err)) return rc;
+                enqueue_grouped_products(L.down, nullptr, aq, as, perm, items, a, 1, y16, false, shared_expert, L.shared_ff, Glu{0.f, 0}, st, p.item_rows);
+                if (int32_t rc = launched(err, "tqmoe_layer_forward (grouped products)")) return rc;
+                if (int32_t rc = combine(y16, TQMOE_F16, L.has_shared ? y16 + size_t(L.topk) * L.hidden : nullptr)) return rc;
+                continue;
+            }
             if (p.prepared) {
                 const hipStream_t st = static_cast<hipStream_t>(stream);
                 uint16_t * x16 = reinterpret_cast<uint16_t *>(ws + p.x16);
@@ -254,9 +276,9 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
                 const int shared_expert = L.has_shared ? banks - 1 : -1;
                 const int64_t a = int64_t(c) * slots;
                 enqueue_prepare_rows(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, x16, xs16, st);
-                enqueue_grouped_plan(counts, offsets, banks, items, st);
-                enqueue_grouped_f16(L.gate, &L.up, x16, xs16, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, st);
-                enqueue_grouped_f16(L.down, nullptr, act16, nullptr, perm, items, a, 1, y16, !p.half_rows, shared_expert, L.shared_ff, Glu{0.f, 0}, st);
+                enqueue_grouped_plan(counts, offsets, banks, p.item_rows, items, RowIndex{}, st);
+                enqueue_grouped_products(L.gate, &L.up, x16, xs16, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, st, p.item_rows);
+                enqueue_grouped_products(L.down, nullptr, act16, nullptr, perm, items, a, 1, y16, !p.half_rows, shared_expert, L.shared_ff, Glu{0.f, 0}, st, p.item_rows);
                 if (int32_t rc = launched(err, "tqmoe_layer_forward (grouped products)")) return rc;
                 const uint8_t * yb = ws + p.y16;
                 if (int32_t rc = combine(yb, p.half_rows ? TQMOE_F16 : TQMOE_F32, L.has_shared ? yb + size_t(L.topk) * L.hidden * (p.half_rows ? 2 : 4) : nullptr)) return rc;
@@ -272,16 +294,7 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
             } else {
             int8_t * rq = reinterpret_cast<int8_t *>(ws + p.rq);
             float * rs = reinterpret_cast<float *>(ws + p.rs);
-            if (plane_gemm_is_fp8(L.gate.type)) {
-                if (int32_t rc = tqmoe_quant_rows_fp8(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, reinterpret_cast<uint8_t *>(rq), rs, stream, err)) return rc;
-                if (int32_t rc = tqmoe_gather_rows_i8(rq, rs, L.hidden, counts, offsets, perm, banks, int64_t(c) * slots, slots, xq, xs, stream, err)) return rc;
-                if (int32_t rc = gemm_8bit_common(&L.gate, &L.up, xq, xs, counts, offsets, perm, c, slots, L.topk, L.shared_ff, act16, 1, stream, err,
-                                                  "tqmoe_layer_forward (gate / up)", true, nullptr, false, glu, 0, nullptr)) return rc;
-                if (int32_t rc = group_rows_common(act16, TQMOE_F16, L.ff, counts, offsets, perm, banks, int64_t(c) * slots, 1, aq, as, stream, err, true,
-                                                   "tqmoe_layer_forward (act rows)", nullptr, false, xs)) return rc;
-                if (int32_t rc = gemm_8bit_common(&L.down, nullptr, aq, as, counts, offsets, perm, c, slots, L.topk, L.shared_ff, y16, 0, stream, err,
-                                                  "tqmoe_layer_forward (down)", true, nullptr, false, Glu{0.f, 0}, 0, xs)) return rc;
-            } else if (p.blocks) {
+            if (p.blocks) {
             float * xbs = reinterpret_cast<float *>(ws + p.xbs), * abks = reinterpret_cast<float *>(ws + p.abks);
             if (int32_t rc = tqmoe_quant_rows_i8_blocks(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, nullptr, stream, err)) return rc;
             if (int32_t rc = tqmoe_gather_rows_i8_blocks(rq, rs, L.hidden, counts, offsets, perm, banks, int64_t(c) * slots, slots, xq, xs, xbs, stream, err)) return rc;

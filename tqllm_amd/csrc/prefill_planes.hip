@@ -70,45 +70,6 @@ __global__ __launch_bounds__(256) void quant_rows_k(const void * __restrict__ x,
     }
 }
 
-// inclusive prefix sum over the wave's 64 lanes with DPP moves (rows of 16, then the rows' totals handed on)
-template <int N> __device__ __forceinline__ int dpp_row_shr(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x110 + N, 0xF, 0xF, true); }
-__device__ __forceinline__ int wave_prefix_sum(int v) {
-    v += dpp_row_shr<1>(v);
-    v += dpp_row_shr<2>(v);
-    v += dpp_row_shr<4>(v);
-    v += dpp_row_shr<8>(v);
-    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xA, 0xF, false);   // row_bcast:15 into rows 1 and 3
-    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xC, 0xF, false);   // row_bcast:31 into rows 2 and 3
-    return v;
-}
-
-__global__ __launch_bounds__(64) void plan_k(const int * __restrict__ counts, int experts, Plan plan) {
-    const int lane = threadIdx.x;
-    int * tile_base = const_cast<int *>(plan.tile_base), * chunk_base = const_cast<int *>(plan.chunk_base), * chunk_base2 = const_cast<int *>(plan.chunk_base2);
-    if (lane < kPlanCounters) plan.counters[lane] = 0;
-    int tbase = 0, cbase = 0, cbase2 = 0;
-    constexpr int kAhead = 16;   // counts of 16 x 64 experts are loaded in one trip to memory, then scanned 64 at a time
-    for (int eb = 0; eb < experts; eb += 64 * kAhead) {
-        int cnt[kAhead];
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) cnt[i] = counts[min(eb + 64 * i + lane, experts - 1)];
-#pragma unroll
-        for (int i = 0; i < kAhead; ++i) {
-            const int e0 = eb + 64 * i;
-            if (e0 >= experts) break;
-            const int e = e0 + lane;
-            const int tiles = e < experts ? (max(cnt[i], 0) + 31) >> 5 : 0;
-            const int chunks = (tiles + kChunkTiles - 1) / kChunkTiles, chunks2 = (tiles + 2 * kChunkTiles - 1) / (2 * kChunkTiles);
-            const int ti = wave_prefix_sum(tiles), ci = wave_prefix_sum(chunks), c2 = wave_prefix_sum(chunks2);
-            if (e < experts) { tile_base[e] = tbase + ti - tiles; chunk_base[e] = cbase + ci - chunks; chunk_base2[e] = cbase2 + c2 - chunks2; }
-            tbase += __builtin_amdgcn_readlane(ti, 63);
-            cbase += __builtin_amdgcn_readlane(ci, 63);
-            cbase2 += __builtin_amdgcn_readlane(c2, 63);
-        }
-    }
-    if (lane == 0) { tile_base[experts] = tbase; chunk_base[experts] = cbase; chunk_base2[experts] = cbase2; }
-}
-
 // Rows of the grouped operand: block b takes rows [8 (b % 4), +8) of row tile b / 4, one wave per two rows. Row i of
 // expert e's tiles is assignment perm[offsets[e] + i], its source row a / xdiv. Rows past the expert's count are left as
 // they are (their products are never stored).
@@ -320,7 +281,13 @@ int32_t enqueue_quant_rows_i8_blocks(const void * x, uint32_t xtype, int64_t row
     return 0;
 }
 
-int64_t grouped_scale_words(int64_t assignments, int experts) { return grouped_row_tiles(assignments, experts) * 32 + 3 * (int64_t(experts) + 1) + kPlanCounters; }
+int64_t grouped_scale_words(int64_t assignments, int experts) {
+    return grouped_row_tiles(assignments, experts) * 32 + 2 * (int64_t(experts) + 1) + kPlanCounters + 4 * (2 + grouped_rows_items(assignments, experts, grouped_rows_per_item(TQMOE_NVFP4G, assignments, experts)));
+}
+static void enqueue_index(const int * counts, const int * offsets, int experts, int64_t assignments, const Plan & plan, hipStream_t s) {
+    enqueue_grouped_plan(counts, offsets, experts, grouped_rows_per_item(TQMOE_NVFP4G, assignments, experts), plan.items,
+                         RowIndex{const_cast<int *>(plan.tile_base), const_cast<int *>(plan.chunk_base), plan.counters, kPlanCounters, kChunkTiles}, s);
+}
 
 template <int XT, bool F8, bool BLK>
 static void group_rows_launch(const void * x, int cols, const int * counts, const int * offsets, const int * perm, int experts, int64_t tiles, int xdiv, int8_t * q,
@@ -347,7 +314,7 @@ int32_t enqueue_group_rows_i8(const void * x, uint32_t xtype, int cols, const in
                               int64_t assignments, int xdiv, int8_t * q, float * scale, hipStream_t s, bool f8, float * block_scale, const float * plan_from) {
     const int64_t tiles = grouped_row_tiles(assignments, experts);
     const Plan plan = plan_at(plan_from ? plan_from : scale, tiles * 32, experts);
-    if (!plan_from) plan_k<<<1, 64, 0, s>>>(counts, experts, plan);
+    if (!plan_from) enqueue_index(counts, offsets, experts, assignments, plan, s);
 #define TQMOE_GROUP(XT) (f8 ? group_rows_launch<XT, true, false>(x, cols, counts, offsets, perm, experts, tiles, xdiv, q, scale, plan, s, nullptr) \
                          : block_scale ? group_rows_launch<XT, false, true>(x, cols, counts, offsets, perm, experts, tiles, xdiv, q, scale, plan, s, block_scale) \
                                        : group_rows_launch<XT, false, false>(x, cols, counts, offsets, perm, experts, tiles, xdiv, q, scale, plan, s, nullptr))
@@ -364,7 +331,7 @@ int32_t enqueue_gather_rows_i8(const int8_t * rq, const float * rs, int cols, co
                                int64_t assignments, int xdiv, int8_t * q, float * scale, hipStream_t s, float * block_scale) {
     const int64_t tiles = grouped_row_tiles(assignments, experts);
     const Plan plan = plan_at(scale, tiles * 32, experts);
-    plan_k<<<1, 64, 0, s>>>(counts, experts, plan);
+    enqueue_index(counts, offsets, experts, assignments, plan, s);
     gather_rows_i8_k<<<unsigned(tiles), 256, 0, s>>>(rq, rs, cols, counts, offsets, perm, experts, xdiv, q, scale, plan, block_scale);
     return 0;
 }
@@ -373,7 +340,7 @@ int32_t enqueue_gather_rows_natural(const int8_t * rq, const float * rs, int col
                                     int64_t assignments, int xdiv, int8_t * q, float * scale, hipStream_t s, float * block_scale) {
     const int64_t tiles = grouped_row_tiles(assignments, experts);
     const Plan plan = plan_at(scale, tiles * 32, experts);
-    plan_k<<<1, 64, 0, s>>>(counts, experts, plan);
+    enqueue_index(counts, offsets, experts, assignments, plan, s);
     gather_rows_natural_k<<<unsigned(tiles), 256, 0, s>>>(rq, rs, cols, counts, offsets, perm, experts, xdiv, q, scale, plan, block_scale);
     return 0;
 }
@@ -394,6 +361,12 @@ int32_t plane_gemm_legacy(uint32_t type, int nb, bool gateup, bool blk, const Ge
 int32_t enqueue_plane_gemm(const tqmoe_bank & b0, const tqmoe_bank * b1, const int8_t * xq, const float * xs, const int * counts, const int * offsets,
                            const int * perm, int experts, int64_t assignments, void * out_f16, int gateup, int shared_expert, int shared_lim, hipStream_t s,
                            const float * xbs, Glu glu, int out_bf16, const float * plan_from) {
+    if (plane_gemm_is_fp8(b0.type)) {   // on the same gathered rows, by the kernels that also take them ungathered
+        const Plan plan = plan_at(plan_from ? plan_from : xs, grouped_row_tiles(assignments, experts) * 32, experts);
+        enqueue_grouped_products(b0, gateup ? b1 : nullptr, xq, xs, perm, plan.items, assignments, 1, out_f16, false, shared_expert, shared_lim, glu, s,
+                                 grouped_rows_per_item(TQMOE_NVFP4G, assignments, experts), true, out_bf16 != 0);
+        return 0;
+    }
     const int nb = gateup || b0.rows % 64 == 0 ? 2 : 1;
     const int units = gateup ? b0.rows / 32 : b0.rows / (32 * nb);
     const int64_t tiles = grouped_row_tiles(assignments, experts);
@@ -412,7 +385,6 @@ int32_t enqueue_plane_gemm(const tqmoe_bank & b0, const tqmoe_bank * b1, const i
         case TQMOE_IQ4_XS: plane_gemm_launch<WIq4xs>(nb, gateup != 0, k, blocks, s); break;
         case TQMOE_IQ3_S: plane_gemm_launch<WIq3s>(nb, gateup != 0, k, blocks, s); break;
         case TQMOE_Q4_K: plane_gemm_launch<WQ4k>(nb, gateup != 0, k, blocks, s); break;
-        case TQMOE_NVFP4G: plane_gemm_launch<WNvfp4>(nb, gateup != 0, k, blocks, s); break;
         case TQMOE_IQ3_XXS: plane_gemm_launch<WIq3xxs>(nb, gateup != 0, k, blocks, s); break;
         case TQMOE_IQ2_XXS: plane_gemm_launch<WIq2xxs>(nb, gateup != 0, k, blocks, s); break;
         case TQMOE_IQ2_XS: plane_gemm_launch<WIq2xs>(nb, gateup != 0, k, blocks, s); break;

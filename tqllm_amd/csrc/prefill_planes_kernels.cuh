@@ -1,14 +1,12 @@
-// Prefill-sized expert products on the matrix pipe with 8-bit operands: grouped int8 x int8 -> int32 GEMMs for IQ4_XS,
-// IQ3_S and Q4_K banks (exact weights), and an fp8 x fp8 -> fp32 GEMM for NVFP4G banks (weights widened to E4M3).
+// Prefill-sized expert products on the matrix pipe with int8 operands: grouped int8 x int8 -> int32 GEMMs (exact weights).
 //
-// Operands. Activations are 8 bits per input row with one fp32 scale per row: int8 (amax / 127) or E4M3 (amax / 448). The
+// Operands. Activations are int8 per input row with one fp32 scale per row (amax / 127). The
 // rows of every expert's assignments are gathered into tiles of 32 rows, experts in order, each expert padded to whole
 // tiles, and stored operand-major: the 1 KB that the 64 lanes of a wave feed to one v_mfma_i32_32x32x32_i8 as operand A
 // (lane = 32 g + r holds, for row r and 32-weight sub-block j, the 16 values {8g..8g+7} and {16+8g..16+8g+7} in the byte
 // order of the bank's code bytes) is contiguous, sub-blocks in order. A wave then loads its operand with one fully
-// coalesced instruction and no shuffle. The two 8-byte halves of that operand are the operands of two
-// v_mfma_f32_32x32x16_fp8_fp8, and two sub-blocks' 32 bytes the operand of one
-// v_mfma_f32_32x32x64_f8f6f4 (which is what the fp8 path issues), so the fp8 path shares the layout.
+// coalesced instruction and no shuffle. (NVFP4G's E4M3 rows have the same layout; their products are in
+// grouped_rows_kernels.cuh.)
 // Integer weights stay exact. A value is d * p with an integer p per weight of up to 13 bits (IQ4_XS: (ls - 32) * kv[q];
 // IQ3_S: (1 + 2 ls) * (+-lattice magnitude); Q4_K: sc * q, with the minimum's coefficient mn as a further plane that
 // is constant over a sub-block). p is split as 64 * h + l with h, l int8, taken per sub-block from 16-entry lookup
@@ -18,9 +16,6 @@
 // With a scale per row and 32-value sub-block in place of one per row (the reference's other int8 mode) the integer sums
 // cannot ride through the super-block: every sub-block's MFMAs start from zero and its sums are scaled by the weights'
 // scale and the row's scale of that sub-block as they join the fp32 result (the BLK instances of the kernel).
-// NVFP4G weights are e2m1 * E4M3 scale (per 16 weights) * fp32 global (per row): the product of the first two is rounded
-// to E4M3 (a declared lossy operand: six significant bits into four), again through a 16-entry table per scale byte; the
-// fp8 MFMA accumulates in fp32 over the whole row and the global multiplies the result.
 //
 // Blocks. A work item is one expert, a chunk of up to kChunkTiles row tiles of its assignments and one unit of weight
 // rows: 32 rows of both banks (gate / up, SwiGLU fused) or 64 rows of one bank (down). Resident blocks of eight waves
@@ -35,6 +30,7 @@
 #include "act_image.cuh"
 #include "decode_api.cuh"
 #include "formats.cuh"
+#include "grouped_rows_api.cuh"
 
 #include <algorithm>
 #include <type_traits>
@@ -43,14 +39,15 @@ namespace tqmoe {
 
 // (types that cross translation units)
 // Index of the grouped rows, kept behind the row scales: tile_base[e] = row tiles of the experts before e
-// (tiles_e = ceil(count_e / 32)), chunk_base[e] = chunks of kChunkTiles row tiles before e, chunk_base2[e] = chunks of twice
-// as many, all with a total at [experts].
+// (tiles_e = ceil(count_e / 32)), chunk_base[e] = chunks of kChunkTiles row tiles before e, both with a total at [experts].
 // Behind them 16 counters the product kernel hands work out with (zero between launches).
 constexpr int kPlanCounters = 16;
-struct Plan { const int * tile_base, * chunk_base, * chunk_base2; int * counters; };
+// and behind those the items of the fp8 products (grouped_rows_api.cuh), from the next multiple of 16 bytes on.
+struct Plan { const int * tile_base, * chunk_base; int * counters; int4 * items; };
 __host__ __device__ inline Plan plan_at(const float * scale, int64_t grouped_rows, int experts) {
     const int * p = reinterpret_cast<const int *>(scale + grouped_rows);
-    return Plan{p, p + experts + 1, p + 2 * (experts + 1), const_cast<int *>(p) + 3 * (experts + 1)};
+    int * counters = const_cast<int *>(p) + 2 * (experts + 1);
+    return Plan{p, p + experts + 1, counters, reinterpret_cast<int4 *>((reinterpret_cast<uintptr_t>(counters + kPlanCounters) + 15) & ~uintptr_t(15))};
 }
 
 struct GemmArgs {
@@ -77,7 +74,7 @@ namespace {
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
 
-constexpr int kChunkTiles = 8;                // row tiles (of 32 assignments) per chunk; formats with registers to spare take chunks of twice that
+constexpr int kChunkTiles = 8;                // row tiles (of 32 assignments) per chunk
 constexpr int kPlanExperts = 1024;              // experts whose index a block keeps in LDS
 
 // four scaled values -> four operand bytes: int8 (round to nearest) or E4M3 (round to nearest even; the values are
@@ -167,9 +164,8 @@ __device__ const int8_t kIq4Values[16] = {-127, -104, -83, -65, -49, -35, -22, -
 // planes() turns a Code into kPlanes operand registers; tables() fills the lookup tables (and the lattice) in LDS.
 struct WIq4xs {   // tile-major codes (512 B per sub-block of a tile), 8-byte records (256 B per super-block of a tile)
     static constexpr bool kFoldSub = false;     // one scale per 32 weights: every sub-block's product is folded on its own
-    static constexpr bool kWideChunks = false;   // chunks of sixteen row tiles on eight waves (two row tiles a wave)
     static constexpr int kPlanes = 2, kTabBytes = 64 * 32, kLattice = 1;
-    static constexpr bool kFp8 = false, kMin = false, kRowMul = false;
+    static constexpr bool kMin = false;
     struct Code { uint2 c; };
     typedef uint2 Rec;
     typedef uint2 DRec;
@@ -191,7 +187,6 @@ struct WIq4xs {   // tile-major codes (512 B per sub-block of a tile), 8-byte re
     }
     static __device__ __forceinline__ float d(const DRec & r) { return half_bits_to_float(iq4xs_d_bits(r)); }
     static __device__ __forceinline__ float dmin(const DRec &) { return 0.f; }
-    static __device__ __forceinline__ float rowmul(const BankView &, int, int, int) { return 1.f; }
 };
 
 // IQ4_XS for rows with a scale per sub-block: the sub-block scale no longer needs to ride inside the operand (every
@@ -215,9 +210,8 @@ struct WIq4xsSub : WIq4xs {
 
 struct WQ4k {   // tile-major: 16 code bytes per sub-block, a 16-byte record (d | dmin << 16, twelve bytes of 6-bit scales and minimums) per super-block
     static constexpr bool kFoldSub = false;     // one scale per 32 weights: every sub-block's product is folded on its own
-    static constexpr bool kWideChunks = false;   // chunks of sixteen row tiles on eight waves (two row tiles a wave)
     static constexpr int kPlanes = 3, kTabBytes = 64 * 32, kLattice = 1;
-    static constexpr bool kFp8 = false, kMin = true, kRowMul = false;
+    static constexpr bool kMin = true;
     struct Code { uint2 c; };
     typedef uint4 Rec;
     typedef uint32_t DRec;
@@ -244,7 +238,6 @@ struct WQ4k {   // tile-major: 16 code bytes per sub-block, a 16-byte record (d 
     }
     static __device__ __forceinline__ float d(const DRec & r) { return half_bits_to_float(uint16_t(r & 0xFFFFu)); }
     static __device__ __forceinline__ float dmin(const DRec & r) { return half_bits_to_float(uint16_t(r >> 16)); }
-    static __device__ __forceinline__ float rowmul(const BankView &, int, int, int) { return 1.f; }
 };
 
 // Q4_K for rows with a scale per sub-block, likewise: the 4-bit codes themselves as one plane (no lookup), a plane of ones
@@ -273,9 +266,8 @@ struct WQ4kSub : WQ4k {
 
 struct WIq3s {   // tile-major: per half of a sub-block four lattice index bytes, a dword of signs for both, a 16-byte record per super-block
     static constexpr bool kFoldSub = false;     // one scale per 32 weights: every sub-block's product is folded on its own
-    static constexpr bool kWideChunks = false;   // chunks of sixteen row tiles on eight waves (two row tiles a wave)
     static constexpr int kPlanes = 2, kTabBytes = 16 * 32, kLattice = 512;
-    static constexpr bool kFp8 = false, kMin = false, kRowMul = false;
+    static constexpr bool kMin = false;
     struct Code { uint32_t qs, sg; };
     typedef uint4 Rec;       // see iq3s_qs_offset
     typedef uint32_t DRec;
@@ -316,7 +308,6 @@ struct WIq3s {   // tile-major: per half of a sub-block four lattice index bytes
     }
     static __device__ __forceinline__ float d(const DRec & r) { return half_bits_to_float(uint16_t(r & 0xFFFFu)); }
     static __device__ __forceinline__ float dmin(const DRec &) { return 0.f; }
-    static __device__ __forceinline__ float rowmul(const BankView &, int, int, int) { return 1.f; }
 };
 
 // ---- the other lattice formats of the reference's MMQ list: magnitudes of 4 or 8 weights per lattice point (LDS copy of the
@@ -336,7 +327,7 @@ template <class LEVEL> __device__ __forceinline__ void lattice_tables(uint8_t * 
 }
 struct WLatticeBase {   // row-major, a 16-byte record per super-block whose first 16 bits are d
     static constexpr int kPlanes = 2, kTabBytes = 16 * 32;
-    static constexpr bool kFp8 = false, kMin = false, kRowMul = false, kWideChunks = false, kFoldSub = false;
+    static constexpr bool kMin = false, kRowMul = false, kFoldSub = false;
     typedef uint32_t Rec;    // unused by the decode (the scales sit in the code bytes)
     typedef uint32_t DRec;
     struct Src { const uint8_t * codes, * aux; };
@@ -348,7 +339,6 @@ struct WLatticeBase {   // row-major, a 16-byte record per super-block whose fir
     static __device__ __forceinline__ Rec rec(const Src &, int) { return 0; }
     static __device__ __forceinline__ DRec drec(const Src & s, int sb) { return *reinterpret_cast<const uint32_t *>(s.aux + int64_t(sb) * 16); }
     static __device__ __forceinline__ float dmin(const DRec &) { return 0.f; }
-    static __device__ __forceinline__ float rowmul(const BankView &, int, int, int) { return 1.f; }
 };
 
 struct WIq3xxs : WLatticeBase {   // 12 code bytes: 8 lattice indices (4 weights each), a word of 4 x 7 sign bits + the scale
@@ -483,7 +473,7 @@ struct WIq1s : WLatticeBase {   // 8 code bytes: 4 low index bytes (8 weights ea
 
 struct WIq4nl {   // row-major: 16 code bytes per sub-block (nibbles as IQ4_XS), one fp16 scale per 32 weights (eight per 256 in the aux plane)
     static constexpr int kPlanes = 1, kTabBytes = 16, kLattice = 1;
-    static constexpr bool kFp8 = false, kMin = false, kRowMul = false, kWideChunks = false;
+    static constexpr bool kMin = false;
     static constexpr bool kFoldSub = true;
     struct Code { uint2 c; };
     typedef uint32_t Rec;    // unused by the decode
@@ -511,7 +501,6 @@ struct WIq4nl {   // row-major: 16 code bytes per sub-block (nibbles as IQ4_XS),
     }
     static __device__ __forceinline__ float d(const DRec &) { return 1.f; }
     static __device__ __forceinline__ float dmin(const DRec &) { return 0.f; }
-    static __device__ __forceinline__ float rowmul(const BankView &, int, int, int) { return 1.f; }
 };
 
 // Q4_0: IQ4_NL's layout; the weight is the nibble minus 8 (no lookup)
@@ -543,9 +532,9 @@ struct WQ8_0 : WIq4nl {
 // 48-byte record). The products sc * q of a 5-bit code q are looked up as for Q4_K, from two pairs of 16-entry tables per
 // scale (q below 16, q from 16 on), and the fifth bit chooses between the two results bit by bit.
 struct WQ5k {
-    static constexpr bool kFoldSub = false, kWideChunks = false;
+    static constexpr bool kFoldSub = false;
     static constexpr int kPlanes = 3, kTabBytes = 64 * 64, kLattice = 1;
-    static constexpr bool kFp8 = false, kMin = true, kRowMul = false;
+    static constexpr bool kMin = true;
     struct Code { uint2 c; uint32_t hb; };
     typedef uint4 Rec;
     typedef uint32_t DRec;
@@ -588,7 +577,6 @@ struct WQ5k {
     }
     static __device__ __forceinline__ float d(const DRec & r) { return half_bits_to_float(uint16_t(r & 0xFFFFu)); }
     static __device__ __forceinline__ float dmin(const DRec & r) { return half_bits_to_float(uint16_t(r >> 16)); }
-    static __device__ __forceinline__ float rowmul(const BankView &, int, int, int) { return 1.f; }
 };
 
 // Q5_K for rows with a scale per sub-block: the 5-bit codes themselves as one plane, a plane of ones, d * sc and dmin * mn
@@ -617,81 +605,20 @@ struct WQ5kSub : WQ5k {
     }
 };
 
-struct WNvfp4 {   // row-major: 16 code bytes per sub-block, one E4M3 scale byte per 16 weights, one fp32 global per row
-    static constexpr bool kFoldSub = false;     // one scale per 32 weights: every sub-block's product is folded on its own
-    static constexpr bool kWideChunks = true;   // chunks of sixteen row tiles on eight waves (two row tiles a wave)
-    static constexpr int kPlanes = 1, kTabBytes = 256 * 16, kLattice = 1;
-    static constexpr bool kFp8 = true, kRowMul = true;
-    struct Code { uint2 c; };
-    typedef uint4 Rec;       // the 16 scale bytes of the row's super-block
-    typedef uint32_t DRec;   // unused: nothing is folded
-    struct Src { const uint8_t * codes, * aux; int h; };
-    // per scale byte the 16 products e2m1(code) * e4m3(scale) / 8, rounded to E4M3 (nearest even); the division keeps the
-    // largest product (6 * 448) inside the format, and rowmul() gives the 8 back
-    static __device__ __forceinline__ void tables(uint8_t * tab, uint32_t *, int tid, int threads) {
-        uint32_t * t32 = reinterpret_cast<uint32_t *>(tab);
-        for (int i = tid; i < 256 * 4; i += threads) {
-            const float sc = e4m3_to_float(uint32_t(i >> 2));
-            float v[4];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int c = 4 * (i & 3) + j;
-                const uint32_t tb = ((c < 4 ? kFp4T0 : c < 8 ? kFp4T1 : c < 12 ? kFp4T2 : kFp4T3) >> (8 * (c & 3))) & 0xFFu;   // twice the e2m1 value
-                v[j] = float(int8_t(tb)) * 0.0625f * sc;
-            }
-            t32[i] = pack4_q<true>(v[0], v[1], v[2], v[3]);
-        }
-    }
-    static __device__ __forceinline__ Src src(const BankView & b, int e, int wtile, int n, int g) {
-        const int S = b.cols / 32;
-        const int64_t row = int64_t(e) * b.rows + wtile * 32 + n;
-        const int h = tile_rows(row, b.rows_total);
-        return Src{b.codes + tiled(row, h, S, 0, 16) + g * 8, b.aux + nvfp4_scale_offset(row, h, S, 0), h};
-    }
-    static __device__ __forceinline__ Code code(const Src & s, int sub) { return Code{*reinterpret_cast<const uint2 *>(s.codes + int64_t(sub) * s.h * 16)}; }
-    static __device__ __forceinline__ Rec rec(const Src & s, int sb) {   // two pieces of four sub-blocks' scales
-        const uint2 a = *reinterpret_cast<const uint2 *>(s.aux + int64_t(sb) * s.h * 16), b = *reinterpret_cast<const uint2 *>(s.aux + int64_t(sb) * s.h * 16 + s.h * 8);
-        return make_uint4(a.x, a.y, b.x, b.y);
-    }
-    static __device__ __forceinline__ DRec drec(const Src &, int) { return 0; }
-    static __device__ __forceinline__ void planes(const Code & c, const Rec & r, int ib, int, const uint8_t * tab, const uint32_t *, v4i * p) {
-        const uint32_t pair = ((ib >> 1) == 0 ? r.x : (ib >> 1) == 1 ? r.y : (ib >> 1) == 2 ? r.z : r.w) >> (16 * (ib & 1));
-        const uint4 t0 = *reinterpret_cast<const uint4 *>(tab + (pair & 0xFFu) * 16), t1 = *reinterpret_cast<const uint4 *>(tab + ((pair >> 8) & 0xFFu) * 16);
-        const uint32_t cw[2] = {c.c.x, c.c.y};
-#pragma unroll
-        for (int w = 0; w < 2; ++w) {   // low nibbles: the sub-block's first 16 weights (first scale), high nibbles: the other 16
-            const NibbleKeys k = nibble_keys(cw[w]);
-            p[0][2 * w] = pick16(t0, k.i_lo, k.s_lo);
-            p[0][2 * w + 1] = pick16(t1, k.i_hi, k.s_hi);
-        }
-    }
-    static __device__ __forceinline__ float d(const DRec &) { return 1.f; }
-    static __device__ __forceinline__ float dmin(const DRec &) { return 0.f; }
-    static __device__ __forceinline__ float rowmul(const BankView & b, int e, int wtile, int n) {
-        return 8.f * *reinterpret_cast<const float *>(b.aux + nvfp4_global_offset(b.rows_total, b.cols) + (int64_t(e) * b.rows + wtile * 32 + n) * 4);
-    }
-};
-
 // one sub-block's products of a row tile with the planes of a weight tile
 template <class W> struct Acc {
-    v16i plane[W::kFp8 || W::kFoldSub ? 1 : W::kPlanes];   // int32 sums of the current super-block (unused by the fp8 path and by per-sub-block folds)
+    v16i plane[W::kFoldSub ? 1 : W::kPlanes];   // int32 sums of the current super-block (unused by per-sub-block folds)
     v16f sum;                               // fp32 result so far
 };
 template <class W> __device__ __forceinline__ void acc_clear(Acc<W> & a) {
 #pragma unroll
     for (int i = 0; i < 16; ++i) a.sum[i] = 0.f;
 }
-// two consecutive sub-blocks (64 weights of the rows) of operand A and of the weight planes. int8: one
-// v_mfma_i32_32x32x32_i8 per sub-block and plane. fp8: one v_mfma_f32_32x32x64_f8f6f4 (both operands E4M3, no block
-// scales) for the pair: twice the rate of the 32x32x16 fp8 instruction on this part.
-typedef int v8i __attribute__((ext_vector_type(8)));
+// two consecutive sub-blocks (64 weights of the rows) of operand A and of the weight planes: one v_mfma_i32_32x32x32_i8 per
+// sub-block and plane
 template <class W> __device__ __forceinline__ void acc_step2(Acc<W> & a, v4i x0, v4i x1, const v4i * w0, const v4i * w1, bool first_of_sb, const typename W::DRec & r,
                                                             int ib0) {
-    if constexpr (W::kFp8) {
-        const v8i x = {x0[0], x0[1], x0[2], x0[3], x1[0], x1[1], x1[2], x1[3]};
-        const v8i w = {w0[0][0], w0[0][1], w0[0][2], w0[0][3], w1[0][0], w1[0][1], w1[0][2], w1[0][3]};
-        a.sum = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(x, w, a.sum, 0, 0, 0, 0, 0, 0);
-    } else if constexpr (W::kFoldSub) {   // a scale per sub-block: each sub-block's integer sums (exact) go into the fp32 result at once
+    if constexpr (W::kFoldSub) {   // a scale per sub-block: each sub-block's integer sums (exact) go into the fp32 result at once
         const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
         const v16i s0 = __builtin_amdgcn_mfma_i32_32x32x32_i8(x0, w0[0], zero, 0, 0, 0);
         const v16i s1 = __builtin_amdgcn_mfma_i32_32x32x32_i8(x1, w1[0], zero, 0, 0, 0);
@@ -743,7 +670,6 @@ template <class W> __device__ __forceinline__ void acc_block_fold(Acc<W> & a, co
 // through the second while the vector pipe scales the first
 template <class W> __device__ __forceinline__ void acc_step2_blocks(Acc<W> & a, v4i x0, v4i x1, const v4i * w0, const v4i * w1, const typename W::DRec & r, int ib0,
                                                                    const float4 * sc0, const float4 * sc1) {
-    static_assert(!W::kFp8, "a scale per sub-block: int8 operands only");
     const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     v16i s0[W::kPlanes], s1[W::kPlanes];
 #pragma unroll
@@ -760,7 +686,7 @@ template <class W> __device__ __forceinline__ void acc_step2_blocks(Acc<W> & a, 
 }
 // |64 acc_h + acc_l| <= 256 * 127 * 2^12 < 2^28: exact in int32, then one rounding into fp32
 template <class W> __device__ __forceinline__ void acc_fold(Acc<W> & a, const typename W::DRec & r) {
-    if constexpr (!W::kFp8 && !W::kFoldSub) {
+    if constexpr (!W::kFoldSub) {
         const float d = W::d(r);
 #pragma unroll
         for (int i = 0; i < 16; ++i) a.sum[i] = fold_sb(a.sum[i], a.plane[0][i], a.plane[1][i], d);
@@ -782,26 +708,23 @@ template <class W> __device__ __forceinline__ void acc_fold(Acc<W> & a, const ty
 template <int NB, class W, int WAVES, bool GATEUP, bool BLK = false>
 __global__ __launch_bounds__(64 * WAVES) void plane_gemm_k(GemmArgs k) {
     constexpr int THREADS = 64 * WAVES, P = W::kPlanes;
-    constexpr int TPW = (WAVES == 8 && W::kWideChunks ? 16 : 8) / WAVES;   // row tiles per wave of a shared chunk
+    constexpr int TPW = 8 / WAVES;   // row tiles per wave of a shared chunk
     constexpr int PIECES = 8 * NB / WAVES;   // (slot, sub-block) pieces a wave decodes per super-block
     constexpr int SPW = 4 * NB / WAVES;      // operand slots per wave on a lone row tile
-    // row tiles per chunk: twice the usual with eight waves where the format's accumulators leave the registers for two row
-    // tiles a wave (a chunk's weights are decoded once for twice the rows, and an expert with nine to sixteen row tiles is one
-    // item per unit group instead of a full chunk and a lone tile)
-    constexpr int CT = WAVES == 8 && W::kWideChunks ? 2 * kChunkTiles : kChunkTiles;
+    constexpr int CT = kChunkTiles;          // row tiles per chunk
     static_assert((PIECES == 2 || PIECES == 4) && (SPW == 1 || SPW == 2), "wave arrangement");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
     v4i * bs = reinterpret_cast<v4i *>(lds);
     __shared__ __attribute__((aligned(16))) uint8_t s_tab[W::kTabBytes];
     __shared__ uint32_t s_lat[W::kLattice];
-    __shared__ int s_asg[(WAVES == 8 && W::kWideChunks ? 16 : 8) * 32];
-    __shared__ float s_scale[(WAVES == 8 && W::kWideChunks ? 16 : 8) * 32];
+    __shared__ int s_asg[8 * 32];
+    __shared__ float s_scale[8 * 32];
     // the experts' index (chunk and tile prefix sums, counts, offsets), copied once: every item looks its expert up, and a
     // binary search is a chain of dependent reads
     __shared__ int s_cbase[kPlanExperts + 1], s_tbase[kPlanExperts + 1], s_cnt[kPlanExperts + 1], s_off[kPlanExperts + 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, n = lane & 31, g = lane >> 5;
     const int mg = wave & 3, nbw = wave >> 2;     // lone row tile: weight tile of the wave within the item, operand slot (SPW == 1)
-    const int * plan_chunks = (WAVES == 8 && W::kWideChunks) ? k.plan.chunk_base2 : k.plan.chunk_base;
+    const int * plan_chunks = k.plan.chunk_base;
     const bool cached = k.experts <= kPlanExperts;
     if (cached)
         for (int i = tid; i <= k.experts; i += THREADS) {
@@ -908,7 +831,7 @@ __global__ __launch_bounds__(64 * WAVES) void plane_gemm_k(GemmArgs k) {
 #pragma unroll
                 for (int q = 0; q < SPW; ++q) {
                     st.rec[q] = W::rec(wsrc[q], sb);
-                    if constexpr (!W::kFp8) st.drec[q] = W::drec(wsrc[q], sb);
+                    st.drec[q] = W::drec(wsrc[q], sb);
                 }
 #pragma unroll
                 for (int ib = 0; ib < 8; ++ib) {
@@ -959,14 +882,6 @@ __global__ __launch_bounds__(64 * WAVES) void plane_gemm_k(GemmArgs k) {
                 for (int sb = 0; sb < sbe; sb += 2) {
                     work1(sb, s0, s1);
                     if (sb + 1 < sbe) work1(sb + 1, s1, s0);
-                }
-            }
-            if constexpr (W::kRowMul) {
-#pragma unroll
-                for (int q = 0; q < SPW; ++q) {
-                    const float rm = W::rowmul((SPW == 1 ? nbw : q) ? k.b1 : k.b0, e, wt[q], n);
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[q].sum[i] = __fmul_rn(acc[q].sum[i], rm);
                 }
             }
             rows_to_lds();
@@ -1035,16 +950,6 @@ __global__ __launch_bounds__(64 * WAVES) void plane_gemm_k(GemmArgs k) {
             // row n. The rows' assignments and scales are read first, all at once: a read per element inside the store loop
             // would serialise on LDS latency.
             auto store_unit = [&](int u, bool zero) {
-                if constexpr (W::kRowMul) {
-#pragma unroll
-                    for (int b = 0; b < NB; ++b) {
-                        const float rm = W::rowmul(b ? k.b1 : k.b0, e, weight_tile(u, b), n);
-#pragma unroll
-                        for (int t = 0; t < MT; ++t)
-#pragma unroll
-                            for (int i = 0; i < 16; ++i) acc[t][b].sum[i] = __fmul_rn(acc[t][b].sum[i], rm);
-                    }
-                }
 #pragma unroll
                 for (int t = 0; t < MT; ++t) {
                     int asg[16];
@@ -1096,13 +1001,11 @@ __global__ __launch_bounds__(64 * WAVES) void plane_gemm_k(GemmArgs k) {
                 for (int j = 0; j < PIECES; ++j) f_code[j] = W::code(src, at * 8 + my_ib0 + j);
             };
             auto fetch_d = [&](int sb, int ahead) {
-                if constexpr (!W::kFp8) {
-                    const int t = sb + ahead;
-                    const bool here = t < sb_full || last;
-                    const int at = t < sb_full ? t : last ? sb_full - 1 : t - sb_full;
+                const int t = sb + ahead;
+                const bool here = t < sb_full || last;
+                const int at = t < sb_full ? t : last ? sb_full - 1 : t - sb_full;
 #pragma unroll
-                    for (int b = 0; b < NB; ++b) d_rec_next[b] = W::drec(here ? dsrc_cur[b] : dsrc_nxt[b], at);
-                }
+                for (int b = 0; b < NB; ++b) d_rec_next[b] = W::drec(here ? dsrc_cur[b] : dsrc_nxt[b], at);
             };
             auto decode_one = [&](int buf, int j) {
                 const int ib = my_ib0 + j;
