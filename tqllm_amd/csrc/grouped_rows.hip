@@ -83,7 +83,7 @@ __global__ __launch_bounds__(1024) void grouped_plan_k(const int * __restrict__ 
 #pragma unroll
     for (int i = 0; i < kScans; ++i) { at[i] += s_wave[i][wave] + (i < 4 ? base : 0); if (i < 4) base += s_total[i]; }
     if (tid == 0) {
-        plan[0] = make_int4(base, 0, 0, 0);
+        plan[0] = make_int4(s_total[0], s_total[1], s_total[2], s_total[3]);
         if (index.tile_base) { index.tile_base[experts] = s_total[4]; index.chunk_base[experts] = s_total[5]; }
     }
     if (index.tile_base && tid < index.counters_n) index.counters[tid] = 0;
@@ -133,7 +133,8 @@ void enqueue_grouped_products(const tqmoe_bank & b0, const tqmoe_bank * b1, cons
                          int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows, bool row_tiles, bool out_bf16) {
     const int tiles = b0.rows / 32, per = b1 ? 4 : 8, groups = (tiles + per - 1) / per;
     const GroupedArgs k{view(b0), b1 ? view(*b1) : view(b0), x, xs, perm, plan, xdiv, out, groups, shared_expert, shared_lim, glu, row_tiles, out_bf16};
-    const unsigned blocks = unsigned((grouped_rows_items(assignments, b0.experts, item_rows) + 7) / 8 * 8 * groups);
+    // (an XCD takes an eighth of every one of the four classes, rounded up)
+    const unsigned blocks = unsigned((grouped_rows_items(assignments, b0.experts, item_rows) + 28) / 8 * 8 * groups);
     switch (b0.type) {
         case TQMOE_IQ4_XS: grouped_rows_run<TQMOE_IQ4_XS>(k, item_rows, b1 != nullptr, f32_out, blocks, s); break;
         case TQMOE_Q4_K: grouped_rows_run<TQMOE_Q4_K>(k, item_rows, b1 != nullptr, f32_out, blocks, s); break;

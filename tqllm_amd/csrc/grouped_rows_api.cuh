@@ -14,7 +14,7 @@ struct GroupedArgs {
     const void * x;           // prepared rows: cols halves in operand_pos order, or (NVFP4G) cols E4M3 bytes in the order tqmoe_quant_rows_fp8 leaves
     const float * xs;         // their scales, or null (all 1)
     const int * perm;         // assignment indices grouped by expert
-    const int4 * plan;        // entry 0: number of items; then per item: expert, first index into perm, rows, first row tile
+    const int4 * plan;        // entry 0: items of each class (grouped_plan_k); then per item: expert, first index into perm, rows, first row tile
     int xdiv;                 // row of assignment a = a / xdiv
     void * out;               // gate / up: rows of halves [assignments][rows], in operand_pos order (NVFP4G: in natural order); else rows of fp32 or halves
     int groups;               // blocks per item: groups of weight tiles

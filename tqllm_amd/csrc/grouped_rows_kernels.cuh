@@ -302,10 +302,22 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
     constexpr int kItemRows = 32 * MAX;
     __shared__ int s_asg[kItemRows];
     __shared__ float s_scale[kItemRows];
-    // Items that share input rows (an item of the plan, all its groups of weight tiles) run on one XCD, one after the other.
-    const int xcd = int(blockIdx.x) & 7, at = int(blockIdx.x) >> 3;
-    const int chunk = at / k.groups * 8 + xcd, grp = at % k.groups;
-    if (chunk >= k.plan[0].x) return;
+    // An item's groups of weight tiles run on one XCD one after the other (its rows stay in that L2), and an XCD takes a run
+    // of consecutive items, an expert's items among them, of every class (its weights do too): see grouped_plan_k.
+    const int xcd = int(blockIdx.x) & 7, at = int(blockIdx.x) >> 3, grp = at % k.groups;
+    const int4 counts = k.plan[0];
+    int slot = at / k.groups, base = 0, chunk = -1;
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        const int items = c == 0 ? counts.x : c == 1 ? counts.y : c == 2 ? counts.z : counts.w, per = (items + 7) >> 3;
+        if (chunk < 0 && slot < per) {
+            if (xcd * per + slot >= items) return;
+            chunk = base + xcd * per + slot;
+        }
+        slot -= per;
+        base += items;
+    }
+    if (chunk < 0) return;
     const int4 item = k.plan[1 + chunk];           // expert, its first row in perm, rows, first row tile
     const int e = item.x, cnt = item.z;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), n = lane & 31, g = lane >> 5;
@@ -340,11 +352,12 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
             constexpr int LA = R::kRows - 1, LW = R::kCodes, LM = LA > LW ? LA : LW;   // stages ahead: stage t sends the rows of t + LA and the codes of t + LW
             constexpr int NA = MT, NW = 2 * W::kCodes + W::kRecs;   // transfers a wave sends for a stage
             // input rows: transfer q of a wave is rows 8 (4 q + wave) .. + 7 of the stage's 128 bytes, a row's piece p in slot
-            // p ^ (row & 7), so that the operand reads (a row a lane) find eight rows' pieces in eight different bank groups
+            // p ^ (row / 2 & 7): the operand reads (a row a lane) then find sixteen rows' pieces in the sixteen 16-byte groups of
+            // the 64 banks (rows are half as long as a line of banks)
             const uint8_t * a_src[MT];
 #pragma unroll
             for (int q = 0; q < MT; ++q) {
-                const int row = (4 * q + wave) * 8 + (lane >> 3), piece = (lane & 7) ^ (row & 7);
+                const int row = (4 * q + wave) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
                 if (W::kFp8 && k.row_tiles)   // operand-major tiles of 32 rows: 1 KB a sub-block, the rows' first halves, then their second
                     a_src[q] = static_cast<const uint8_t *>(k.x) + (int64_t(item.w) + (row >> 5)) * 32 * cols + (piece >> 1) * 1024 + (piece & 1) * 512 + (row & 31) * 16;
                 else
@@ -408,7 +421,7 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                 auto read_a = [&](int j) {
                     const int piece = W::kFp8 ? 4 * (j >> 1) + 2 * g + (j & 1) : 4 * g + j;
 #pragma unroll
-                    for (int m = 0; m < MT; ++m) a[j & 1][m] = *reinterpret_cast<const uint4 *>(a_buf + m * 4096 + ((piece ^ (n & 7)) * 16));
+                    for (int m = 0; m < MT; ++m) a[j & 1][m] = *reinterpret_cast<const uint4 *>(a_buf + m * 4096 + ((piece ^ ((n >> 1) & 7)) * 16));
                 };
                 read_a(0);
 #pragma unroll
@@ -420,7 +433,7 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                         for (int b = 0; b < 2; ++b)
 #pragma unroll
                             for (int m = 0; m < MT; ++m)
-                                acc[b][m] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(join(a[0][m], a[1][m]), join(bw[b][j], bw[b][j + 1]), acc[b][m], 0, 0, 0, 0, 0, 0);
+                                acc[b][m] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(join(bw[b][j], bw[b][j + 1]), join(a[0][m], a[1][m]), acc[b][m], 0, 0, 0, 0, 0, 0);
                         if (j < 2) read_a(j + 2);
 #pragma unroll
                         for (int b = 0; b < 2; ++b) { bw[b][j] = W::slice(pr[b], j); bw[b][j + 1] = W::slice(pr[b], j + 1); }
@@ -430,48 +443,75 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                         for (int b = 0; b < 2; ++b)
 #pragma unroll
                             for (int m = 0; m < MT; ++m)
-                                acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[j & 1][m]), __builtin_bit_cast(v8h, bw[b][j]), acc[b][m], 0, 0, 0);
+                                acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bw[b][j]), __builtin_bit_cast(v8h, a[j & 1][m]), acc[b][m], 0, 0, 0);
 #pragma unroll
                         for (int b = 0; b < 2; ++b) bw[b][j] = W::slice(pr[b], j);
                     }
                 }
             }
         }
-        if constexpr (W::kFp8) {
-#pragma unroll
-            for (int b = 0; b < 2; ++b) {
-                const float f = W::row_factor(b ? k.b1 : k.b0, (int64_t(e) * tiles + min(wt[b], tiles - 1)) * 32 + n);
-#pragma unroll
-                for (int m = 0; m < MT; ++m)
-#pragma unroll
-                    for (int i = 0; i < 16; ++i) acc[b][m][i] *= f;
-            }
-        }
-        // result register i of lane half g: input row 8 (i / 4) + 4 g + i % 4 of the row tile, weight row n of the weight tile
+        // The weights are the first operand: result register 4 c + i of lane (n, g) is weight row 8 c + 4 g + i of the tile and
+        // input row n of the row tile: a lane has four consecutive values of one row at a time. They go through the wave's own
+        // LDS (its codes are done with) and leave as 16 bytes a lane, a row's 64 or 128 bytes together.
+        constexpr int kPitch = 32 * sizeof(OT) + 16, kLanes = 32 * sizeof(OT) / 16, kStep = 64 / kLanes;   // lanes a row, rows a store
+        static_assert(32 * kPitch <= Rings<W, MT, MAX>::kCodes * kStageW<W>, "the tile's place");
+        uint8_t * const tile_lds = lds + Rings<W, MT, MAX>::kRows * MT * 4096 + wave * Rings<W, MT, MAX>::kCodes * kStageW<W>;
+        const bool clamp = k.glu.limit > 1e-6f;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
-            int asg[16];
-            float scl[16];
+            const float scl = s_scale[m * 32 + n];
 #pragma unroll
-            for (int i = 0; i < 16; ++i) { const int r = m * 32 + 8 * (i >> 2) + 4 * g + (i & 3); asg[i] = s_asg[r]; scl[i] = s_scale[r]; }
+            for (int b = 0; b < (GATEUP ? 1 : 2); ++b) {
+                if (wt[b] >= tiles) continue;
+                auto factors = [&](int bank, float (&v)[16]) {   // the weight rows' own factors, the input row's scale
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                if (asg[i] < 0) continue;
-                OT * o = static_cast<OT *>(k.out) + int64_t(asg[i]) * rows;
-                auto put = [&](int col, float v) {
-                    if constexpr (sizeof(OT) == 4) o[col] = v;
-                    else o[col] = W::kFp8 && k.out_bf16 ? float_to_bf16_bits(v) : __half_as_ushort(__float2half_rn(v));
+                    for (int i = 0; i < 16; ++i) {
+                        v[i] = acc[bank][m][i];
+                        if constexpr (W::kFp8) v[i] *= W::row_factor(bank ? k.b1 : k.b0, (int64_t(e) * tiles + wt[bank]) * 32 + 8 * (i >> 2) + 4 * g + (i & 3));
+                        v[i] *= scl;
+                    }
                 };
+                float v[16];
+                factors(b, v);
                 if constexpr (GATEUP) {
-                    if (wt[0] >= tiles) continue;
-                    float gv = acc[0][m][i] * scl[i], uv = acc[1][m][i] * scl[i];
-                    glu_clamp_inputs(k.glu, gv, uv);
-                    const float v = glu_clamp_silu(k.glu, gv * __builtin_amdgcn_rcpf(1.f + __expf(-gv))) * uv;
-                    put(wt[0] * 32 + (W::kFp8 ? n : operand_pos(n)), wt[0] * 32 < row_lim ? v : 0.f);
-                } else {
+                    float u[16];
+                    factors(1, u);
+                    if (clamp) {
 #pragma unroll
-                    for (int b = 0; b < 2; ++b) if (wt[b] < tiles) put(wt[b] * 32 + n, acc[b][m][i] * scl[i]);
+                        for (int i = 0; i < 16; ++i) glu_clamp_inputs(k.glu, v[i], u[i]);
+                    }
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[i] *= __builtin_amdgcn_rcpf(1.f + __expf(-v[i]));
+                    if (clamp) {
+#pragma unroll
+                        for (int i = 0; i < 16; ++i) v[i] = glu_clamp_silu(k.glu, v[i]);
+                    }
+                    const float live = wt[0] * 32 < row_lim ? 1.f : 0.f;
+#pragma unroll
+                    for (int i = 0; i < 16; ++i) v[i] *= live * u[i];
                 }
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const float * q = v + 4 * c;
+                    uint8_t * to = tile_lds + n * kPitch;
+                    auto half2 = [&](float x, float y) {
+                        if constexpr (W::kFp8) if (k.out_bf16) return float_to_bf16_bits(x) | uint32_t(float_to_bf16_bits(y)) << 16;
+                        return bits_of(v2h{_Float16(x), _Float16(y)});
+                    };
+                    if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4 *>(to + (8 * c + 4 * g) * 4) = make_float4(q[0], q[1], q[2], q[3]);
+                    else if constexpr (GATEUP && !W::kFp8)   // operand_pos: the four values stay together, 1 and 2 change places
+                        *reinterpret_cast<uint2 *>(to + operand_pos(8 * c + 4 * g) * 2) = make_uint2(half2(q[0], q[2]), half2(q[1], q[3]));
+                    else *reinterpret_cast<uint2 *>(to + (8 * c + 4 * g) * 2) = make_uint2(half2(q[0], q[1]), half2(q[2], q[3]));
+                }
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int q = 0; q < 32 / kStep; ++q) {
+                    const int row = q * kStep + lane / kLanes, asg = s_asg[m * 32 + row];
+                    const uint4 w = *reinterpret_cast<const uint4 *>(tile_lds + row * kPitch + (lane % kLanes) * 16);
+                    if (asg >= 0) *reinterpret_cast<uint4 *>(static_cast<OT *>(k.out) + int64_t(asg) * rows + wt[b] * 32 + (lane % kLanes) * (16 / sizeof(OT))) = w;
+                }
+                __builtin_amdgcn_wave_barrier();
             }
         }
     };
