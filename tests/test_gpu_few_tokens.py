@@ -1,0 +1,38 @@
+"""One to a few tokens: the launches that route for themselves and combine, against the oracle, at the edges of their ranges
+(one unit a block, experts at a power of two of the lanes, a shared expert narrower than the routed ones, the last batch that
+takes them and the first that does not)."""
+import numpy as np
+import pytest
+import torch
+
+import synth
+from gpu_util import banks_on_device, clear_tokens, dev
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.fixture(scope="module")
+def tq():
+    import tqllm_amd
+    return tqllm_amd
+
+
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "Q6_K", "IQ3_S", "NVFP4G"])
+@pytest.mark.parametrize("n,hidden,ff,experts,topk,shared_ff", [(1, 256, 256, 4, 1, 0), (2, 512, 768, 64, 6, 256), (5, 2304, 512, 128, 8, 512), (6, 1280, 512, 129, 10, 256),
+                                                               (7, 512, 256, 65, 3, 0), (1, 512, 1536, 513, 16, 512)])
+def test_layer_of_few_tokens(tq, oracle, fmt, n, hidden, ff, experts, topk, shared_ff):
+    cfg = dict(hidden=hidden, ff=ff, experts=experts, topk=topk, shared_ff=shared_ff, wtype=getattr(oracle, fmt), rtype="bf16", xtype="bf16")
+    raws = synth.make_banks(cfg, seed=n + hidden, distinct=min(experts + 1, 8))
+    gate, up, down = banks_on_device(cfg, raws)
+    inp = synth.make_inputs(cfg, n, seed=n)
+    layer = tq.MoeLayer(dev(inp["router"]), dev(inp["shared_gate"]) if shared_ff else None, gate, up, down, topk, shared_ff=shared_ff, weight_scale=2.5)
+    assert layer.path(n) == "decode"
+    x = dev(inp["x"])
+    out, ids, w, logits = (t.cpu().numpy() for t in layer.forward(x, return_routing=True))
+    want, want_ids, want_w = oracle.layer_forward(inp["x"][1], logits, *raws, cfg["wtype"], hidden, ff, experts, topk, shared_ff=shared_ff, act_mode=0, threads=16, scale=2.5)
+    clear = clear_tokens(oracle, logits, experts, topk, ids, want_ids)
+    assert np.array_equal(ids[clear], want_ids[clear]) and np.abs(w[clear] - want_w[clear]).max() < 3e-6
+    assert synth.errors(out[clear], want[clear])[1] < 1e-3
+    res = torch.randn_like(x)
+    got = layer.forward(x, residual=res)
+    assert torch.equal(got, (torch.from_numpy(out).cuda().bfloat16().float() + res.float()).bfloat16())

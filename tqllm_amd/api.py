@@ -154,10 +154,14 @@ def _ptr(t):
     return C.c_void_p(t.data_ptr()) if t is not None else None
 
 
+# (the raw handle of the current stream without a torch.cuda.Stream object around it: 2 us less a call)
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda device: torch.cuda.current_stream(device).cuda_stream)
+
+
 def _stream(t):
     if not t.is_cuda:
         raise TqmoeError(-3, "tensors must live on the GPU (there is no CPU path)")
-    return C.c_void_p(torch.cuda.current_stream(t.device).cuda_stream)
+    return C.c_void_p(_raw_stream(t.get_device()))
 
 
 def _ttype(t):
@@ -674,7 +678,7 @@ class MoeLayer:
         self.n_expert, self.hidden = router.shape
         self.ff, self.topk, self.shared_ff, self.weight_scale = gate.rows, topk, shared_ff, weight_scale
         self.gating, self.probs_bias, self.norm_weights = gating, probs_bias, norm_weights
-        self._ws = None
+        self._ws = self._desc = self._desc_key = None
 
     def desc(self):
         return _Layer(C.sizeof(_Layer), self.hidden, self.ff, self.n_expert, self.topk, int(self.shared_ff > 0), self.shared_ff,
@@ -682,6 +686,20 @@ class MoeLayer:
                       _ttype(self.router), self.gate.view(), self.up.view(), self.down.view(), int(self.gating), int(not self.norm_weights),
                       self.probs_bias.data_ptr() if self.probs_bias is not None else None, int(self.act_blocks), float(self.swiglu_clamp),
                       int(bool(self.clamp_gate)))
+
+    def _descriptor(self):
+        """desc(), built again only where something it holds has changed (a small batch's call is a few launches: building it
+        is a tenth of the host's time)."""
+        if "desc" in self.__dict__:
+            return self.desc()
+        g, u, d, bias, sg = self.gate, self.up, self.down, self.probs_bias, self.shared_gate
+        key = (self.router.data_ptr(), self.router.dtype, g.codes.data_ptr(), g.aux.data_ptr(), u.codes.data_ptr(), u.aux.data_ptr(), d.codes.data_ptr(), d.aux.data_ptr(),
+               sg.data_ptr() if sg is not None else 0, bias.data_ptr() if bias is not None else 0, g.type, u.type, d.type, g.experts, u.experts, d.experts, g.rows, u.rows,
+               d.rows, g.cols, u.cols, d.cols, self.hidden, self.ff, self.n_expert, self.topk, self.shared_ff, self.weight_scale, self.gating, self.norm_weights,
+               self.act_blocks, self.swiglu_clamp, self.clamp_gate)
+        if key != self._desc_key:
+            self._desc, self._desc_key = self.desc(), key
+        return self._desc
 
     def path(self, n):
         """'decode', 'grouped_i8', 'grouped_f16' or 'grouped_fp8': the expert products a batch of n tokens takes"""
@@ -692,7 +710,9 @@ class MoeLayer:
         return ("decode", "grouped_i8", "grouped_f16", "grouped_fp8")[rc]
 
     def workspace(self, n):
-        d = self.desc()
+        return self._workspace(self.desc(), n)
+
+    def _workspace(self, d, n):
         need = lib().tqmoe_layer_workspace_bytes(C.byref(d), n)
         if need == 0:
             raise TqmoeError(-1, "layer descriptor rejected (shapes of the banks do not match the layer)")
@@ -703,7 +723,8 @@ class MoeLayer:
     def forward(self, x, out_type=F32, return_routing=False, out=None, residual=None):
         """residual (bf16 [n][H]): added to the result, which is then bf16: bf16(bf16(layer(x)) + residual)."""
         n = x.shape[0]
-        ws = self.workspace(n)
+        d = self._descriptor()
+        ws = self._workspace(d, n)
         if residual is not None:
             out_type = BF16
         if out is None:
@@ -713,12 +734,13 @@ class MoeLayer:
             ids = torch.empty((n, self.topk), dtype=torch.int32, device=x.device)
             weights = torch.empty((n, self.topk), dtype=torch.float32, device=x.device)
             logits = torch.empty((n, self.n_expert + 1), dtype=torch.float32, device=x.device)
-        d = self.desc()
         err = _err()
+        stream = _stream(x)
+        routing = (ids.data_ptr(), weights.data_ptr(), logits.data_ptr()) if return_routing else (None, None, None)
         if residual is not None:
-            _check(lib().tqmoe_layer_forward_residual(C.byref(d), _ptr(x), _ttype(x), _ptr(residual), n, _ptr(out), _ptr(ids), _ptr(weights), _ptr(logits),
-                                                      _ptr(ws), ws.numel(), _stream(x), C.byref(err)), err)
+            rc = lib().tqmoe_layer_forward_residual(C.byref(d), x.data_ptr(), _ttype(x), residual.data_ptr(), n, out.data_ptr(), *routing, ws.data_ptr(), ws.numel(), stream,
+                                                    C.byref(err))
         else:
-            _check(lib().tqmoe_layer_forward(C.byref(d), _ptr(x), _ttype(x), n, _ptr(out), out_type, _ptr(ids), _ptr(weights), _ptr(logits),
-                                             _ptr(ws), ws.numel(), _stream(x), C.byref(err)), err)
+            rc = lib().tqmoe_layer_forward(C.byref(d), x.data_ptr(), _ttype(x), n, out.data_ptr(), out_type, *routing, ws.data_ptr(), ws.numel(), stream, C.byref(err))
+        _check(rc, err)
         return (out, ids, weights, logits) if return_routing else out

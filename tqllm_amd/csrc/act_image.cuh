@@ -126,6 +126,13 @@ template <int XT> __device__ __forceinline__ void load_block32(const void * __re
 }
 template <int XT> __device__ __forceinline__ void quantise_row_wave(const void * __restrict__ x, int64_t row, int cols, uint8_t * image_row, int lane) {
     const int S = cols / 32;
+    if (S <= 64) {   // a block per lane: read once
+        float v[32];
+        if (lane < S) load_block32<XT>(x, row * cols + 32 * lane, v);
+        const float amax = wave_max(lane < S ? block_amax(v) : 0.f);
+        if (lane < S) quantise_block(v, image_row, S, lane, amax);
+        return;
+    }
     float amax = 0.f;
     for (int s = lane; s < S; s += 64) {
         float v[32];

@@ -1,6 +1,7 @@
 // Entry points of the decode-sized expert products and the small element-wise steps around them.
 #include "act_image.cuh"
 #include "decode_api.cuh"
+#include "formats.cuh"
 
 namespace tqmoe {
 int32_t check_bank(const tqmoe_bank * b, const char * what, tqmoe_error * err);  // bank.hip
@@ -27,7 +28,7 @@ int32_t group_rows_common(const void * x, uint32_t xtype, int32_t cols, const in
                           float * block_scale = nullptr, bool blocks = false, const float * plan_from = nullptr);
 
 int32_t expert_gateup_glu(const tqmoe_bank * gate, const tqmoe_bank * up, const void * x_image, void * act_image, const int32_t * ids, int32_t n,
-                          int32_t slots, int32_t topk, int32_t shared_ff, Glu glu, void * stream, tqmoe_error * err);
+                          int32_t slots, int32_t topk, int32_t shared_ff, Glu glu, void * stream, tqmoe_error * err, const DecodeTopk & route = DecodeTopk{});
 int32_t gemm_8bit_common(const tqmoe_bank * b0, const tqmoe_bank * b1, const int8_t * xq, const float * xs, const int32_t * counts, const int32_t * offsets,
                          const int32_t * perm, int32_t n, int32_t slots, int32_t topk, int32_t shared_lim, void * out, int gateup, void * stream,
                          tqmoe_error * err, const char * what, bool fp8, const float * block_scale = nullptr, bool blocks = false, Glu glu = Glu{0.f, 0},
@@ -35,6 +36,10 @@ int32_t gemm_8bit_common(const tqmoe_bank * b0, const tqmoe_bank * b1, const int
 int32_t gemm_f16_common(const tqmoe_bank * b0, const tqmoe_bank * b1, const void * x, uint32_t xtype, const int32_t * counts, const int32_t * offsets,
                         const int32_t * perm, int32_t n, int32_t slots, int32_t topk, int32_t shared_lim, int32_t xdiv, void * out, uint32_t otype, int gateup,
                         void * stream, tqmoe_error * err, const char * what, Glu glu = Glu{0.f, 0});
+
+bool decode_few_takes(const tqmoe_bank & gate, const tqmoe_bank & down, int slots, int shared_ff);
+int32_t expert_down_combine(const tqmoe_bank & down, const void * act_image, const int32_t * ids, const float * weights, const float * shared_weights, int32_t n,
+                            int32_t slots, int32_t topk, int32_t shared_ff, void * out, uint32_t otype, const void * residual, void * stream, tqmoe_error * err);
 
 namespace {
 
@@ -197,6 +202,16 @@ void dispatch_gateup(uint32_t type, Split sp, const GateupArgs & k, hipStream_t 
         case TQMOE_IQ2_XXS: DecodeLaunch<TQMOE_IQ2_XXS>::gateup(sp, k, s); break;
         case TQMOE_IQ2_XS: DecodeLaunch<TQMOE_IQ2_XS>::gateup(sp, k, s); break;
         default: DecodeLaunch<TQMOE_NVFP4G>::gateup(sp, k, s); break;
+    }
+}
+
+void dispatch_down_combine(uint32_t type, const DownCombineArgs & k, hipStream_t s) {   // tile-major formats only (decode_few_takes)
+    switch (type) {
+        case TQMOE_IQ4_XS: DecodeLaunch<TQMOE_IQ4_XS>::down_combine(k, s); break;
+        case TQMOE_Q4_K: DecodeLaunch<TQMOE_Q4_K>::down_combine(k, s); break;
+        case TQMOE_Q6_K: DecodeLaunch<TQMOE_Q6_K>::down_combine(k, s); break;
+        case TQMOE_IQ3_S: DecodeLaunch<TQMOE_IQ3_S>::down_combine(k, s); break;
+        default: DecodeLaunch<TQMOE_NVFP4G>::down_combine(k, s); break;
     }
 }
 
@@ -363,22 +378,34 @@ extern "C" int32_t tqmoe_extend_ids(const int32_t * ids, int32_t * out, int32_t 
 // The gate / up products of the three paths with the optional clamp of the SwiGLU inputs (the layer's swiglu_clamp); the
 // C entry points are these without a clamp.
 int32_t tqmoe::expert_gateup_glu(const tqmoe_bank * gate, const tqmoe_bank * up, const void * x_image, void * act_image, const int32_t * ids, int32_t n,
-                                 int32_t slots, int32_t topk, int32_t shared_ff, Glu glu, void * stream, tqmoe_error * err) {
+                                 int32_t slots, int32_t topk, int32_t shared_ff, Glu glu, void * stream, tqmoe_error * err, const DecodeTopk & route) {
     const char * what = "tqmoe_expert_gateup";
     if (int32_t rc = check_bank(gate, what, err)) return rc;
     if (int32_t rc = check_bank(up, what, err)) return rc;
     if (up->type != gate->type || up->rows != gate->rows || up->cols != gate->cols || up->experts != gate->experts)
         return fail(err, TQMOE_E_ARG, "%s: the two banks differ in format or shape", what);
-    if (!x_image || !act_image || !ids || n <= 0 || topk <= 0 || slots < topk || gate->rows % 32) return fail(err, TQMOE_E_ARG, "%s: invalid shape or pointer", what);
+    if (!x_image || !act_image || (!ids && !route.logits) || n <= 0 || topk <= 0 || slots < topk || gate->rows % 32) return fail(err, TQMOE_E_ARG, "%s: invalid shape or pointer", what);
     if (slots > topk && (shared_ff <= 0 || shared_ff > gate->rows || shared_ff % 32)) return fail(err, TQMOE_E_ARG, "%s: invalid shared_ff", what);
     const int64_t A = int64_t(n) * slots;
     if (A > 65535) return fail(err, TQMOE_E_ARG, "%s: more than 65535 assignments in one call", what);
     const Split sp = split_for(gate->cols / 32, A);
     if (sp.m == 0) return fail(err, TQMOE_E_UNSUPPORTED, "%s: cols %d is too wide for the decode kernels", what, gate->cols);
     if (int32_t rc = need_device(err, what)) return rc;
-    GateupArgs k{view(*gate), view(*up), static_cast<const uint8_t *>(x_image), static_cast<uint8_t *>(act_image), ids, int(A), slots, topk, shared_ff, dedup_mode(A, slots), glu};
+    GateupArgs k{view(*gate), view(*up), static_cast<const uint8_t *>(x_image), static_cast<uint8_t *>(act_image), ids, int(A), slots, topk, shared_ff, route.logits ? 0 : dedup_mode(A, slots), glu, route};
     dispatch_gateup(gate->type, sp, k, static_cast<hipStream_t>(stream));
     return launched(err, what);
+}
+
+// The formats and shapes whose few-token products route and combine in their own launches.
+bool tqmoe::decode_few_takes(const tqmoe_bank & gate, const tqmoe_bank & down, int slots, int shared_ff) {
+    auto fits = [](const tqmoe_bank & b) { return is_tile_major(b.type) && b.rows % 32 == 0 && b.cols % 256 == 0; };
+    return fits(gate) && fits(down) && shared_ff % 256 == 0 && split_for(gate.cols / 32).m && size_t(slots) * size_t(down.cols / 256 + 1) * 128 <= 49152;
+}
+int32_t tqmoe::expert_down_combine(const tqmoe_bank & down, const void * act_image, const int32_t * ids, const float * weights, const float * shared_weights,
+                                   int32_t n, int32_t slots, int32_t topk, int32_t shared_ff, void * out, uint32_t otype, const void * residual, void * stream, tqmoe_error * err) {
+    dispatch_down_combine(down.type, DownCombineArgs{view(down), static_cast<const uint8_t *>(act_image), ids, weights, shared_weights, n, slots, topk, shared_ff, out, otype,
+                                                     static_cast<const uint16_t *>(residual)}, static_cast<hipStream_t>(stream));
+    return launched(err, "tqmoe_layer_forward (down)");
 }
 
 extern "C" int32_t tqmoe_expert_gateup(const tqmoe_bank * gate, const tqmoe_bank * up, const void * x_image, void * act_image, const int32_t * ids,

@@ -31,6 +31,26 @@ struct MatvecArgs {
     const int * ids;
     int A, xdiv, mode, slots, topk, shared_cols;
 };
+// Routing done by the gate / up blocks themselves (one to a few tokens): every block selects its own assignment's expert from
+// the logits, and one block per token writes the token's ids and weights.
+struct DecodeTopk {
+    const float * logits;     // [n][experts + 1], or null: the ids are given
+    int experts, topk, shared_ungated;
+    float scale;
+    int * ids;                // [n][topk]
+    float * weights, * shared_weights;
+};
+// The down product of one to a few tokens with the weighted sum over their experts in the same launch.
+struct DownCombineArgs {
+    BankView b;
+    const uint8_t * image;    // the act rows' images, [n * slots]
+    const int * ids;          // [n][topk]
+    const float * weights, * shared_weights;
+    int n, slots, topk, shared_cols;
+    void * out;
+    uint32_t otype;
+    const uint16_t * residual;
+};
 struct GateupArgs {
     BankView bg, bu;
     const uint8_t * ximage;
@@ -38,6 +58,7 @@ struct GateupArgs {
     const int * ids;
     int A, slots, topk, shared_ff, mode;
     Glu glu;                  // the optional clamp of the SwiGLU inputs
+    DecodeTopk route;
 };
 
 // arguments of the grouped fp16 products (prefill_f16_kernels.cuh)
@@ -66,9 +87,11 @@ template <uint32_t FMT> struct F16Launch {
 template <uint32_t FMT> struct DecodeLaunch {
     static void matvec(Split sp, int nb, const MatvecArgs & k, hipStream_t s);
     static void gateup(Split sp, const GateupArgs & k, hipStream_t s);
+    static void down_combine(const DownCombineArgs & k, hipStream_t s);   // tile-major formats, whole tiles and super-blocks
 };
 template <> void DecodeLaunch<TQMOE_IQ4_XS>::matvec(Split sp, int nb, const MatvecArgs & k, hipStream_t s);   // its own kernels (decode_iq4xs.hip)
 template <> void DecodeLaunch<TQMOE_IQ4_XS>::gateup(Split sp, const GateupArgs & k, hipStream_t s);
+template <> void DecodeLaunch<TQMOE_IQ4_XS>::down_combine(const DownCombineArgs & k, hipStream_t s);
 extern template struct DecodeLaunch<TQMOE_Q4_K>;
 extern template struct DecodeLaunch<TQMOE_IQ3_S>;
 extern template struct DecodeLaunch<TQMOE_NVFP4G>;

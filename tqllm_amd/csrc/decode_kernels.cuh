@@ -672,10 +672,13 @@ template <uint32_t FMT> void DecodeLaunch<FMT>::matvec(Split sp, int nb, const M
 template <uint32_t FMT> void DecodeLaunch<FMT>::gateup(Split sp, const GateupArgs & k, hipStream_t s) {
     if constexpr (is_tile_major(FMT))
         if (mfma_takes(k.bg.rows, k.bg.cols, 0))
-            return mfma_launch<FMT>(2, k.bg, k.bu, k.ximage, k.aimage, nullptr, TQMOE_F32, k.ids, k.A, k.slots, k.mode, k.slots, k.topk, k.shared_ff, 1, true, k.glu, s);
+            return mfma_launch<FMT>(2, k.bg, k.bu, k.ximage, k.aimage, nullptr, TQMOE_F32, k.ids, k.A, k.slots, k.mode, k.slots, k.topk, k.shared_ff, 1, true, k.glu, s, k.route);
 #define X(L, MM) if (sp.lpr == L && sp.m == MM) return launch_one_gateup<FMT, L, MM>(k, s);
     TQMOE_FOR_SPLITS(X)
 #undef X
+}
+template <uint32_t FMT> void DecodeLaunch<FMT>::down_combine(const DownCombineArgs & k, hipStream_t s) {
+    if constexpr (is_tile_major(FMT)) down_combine_launch<FMT>(k, s);
 }
 
 }  // namespace tqmoe

@@ -23,6 +23,7 @@
 #include "decode_api.cuh"
 #include "decode_table.cuh"
 #include "formats.cuh"
+#include "topk_select.cuh"
 
 namespace tqmoe {
 namespace {
@@ -187,12 +188,13 @@ template <> struct MfmaFormat<TQMOE_Q6_K> : MfmaBase {
 // MODE 0: input rows read straight from the image; 1: staged in LDS; 2: staged, and a wave takes tl_count row tiles in turn
 // Three waves a SIMD (168 registers) where that does not spill; two for the two-bank kernels of the formats with more codes or
 // scales in registers.
+// ROUTE (MODE 0): the block selects its own expert from the token's logits (up to 64 ROUTE experts); see DecodeTopk.
 template <uint32_t FMT, int NB, bool UNI, int MODE>
 constexpr int kDecodeWaves = NB == 2 && (FMT == TQMOE_Q6_K || (MODE == 0 && (FMT == TQMOE_Q4_K || (!UNI && FMT != TQMOE_IQ4_XS)))) ? 2 : 3;
-template <uint32_t FMT, int NB, bool UNI, int MODE>
+template <uint32_t FMT, int NB, bool UNI, int MODE, int ROUTE = 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWaves<FMT, NB, UNI, MODE>))) void decode_mfma_k(BankView b0, BankView b1, const uint8_t * __restrict__ image, void * out0, void * out1, uint32_t ytype,
                                                     const int * __restrict__ ids, int A, int xdiv, int mode, int slots, int topk, int shared_lim, int wk,
-                                                    int tpw, int gateup, int a_off, int tl_count, Glu glu) {
+                                                    int tpw, int gateup, int a_off, int tl_count, Glu glu, DecodeTopk route) {
     using F = MfmaFormat<FMT>;
     constexpr bool STAGED = MODE >= 1, MULTI = MODE == 2;
     extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
@@ -202,7 +204,34 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     __shared__ uint32_t lat[F::kLattice];
     if constexpr (FMT == TQMOE_IQ3_S)   // eight times the magnitudes (behind a barrier before the first use)
         for (int i = threadIdx.x; i < 512; i += blockDim.x) lat[i] = d_iq3s_grid.v[i] << 3;
-    const int a = blockIdx.y, e = fetch_ids(ids, A, a, mode, reinterpret_cast<int *>(stage));
+    const int a = blockIdx.y;
+    int e;
+    if constexpr (ROUTE > 0) {
+        // (one wave selects, for as many rounds as its assignment needs; the block that writes the token's routing for all)
+        const int token = a / slots, slot = a - token * slots;
+        const bool writer = blockIdx.x == 0 && slot == 0;
+        if (slot < topk) {
+            if (threadIdx.x < 64) {
+                const float * x = route.logits + int64_t(token) * (route.experts + 1);
+                const float shared_logit = route.shared_weights ? x[route.experts] : 0.f;
+                int my_id;
+                float my_w;
+                topk_select<ROUTE>(x, route.experts, writer ? topk : slot + 1, threadIdx.x, writer, my_id, my_w);
+                if (int(threadIdx.x) == slot) meta[0] = my_id;
+                if (writer) {
+                    const float v = topk_weight(my_w, topk, route.scale);
+                    if (int(threadIdx.x) < topk) { route.ids[int64_t(token) * topk + threadIdx.x] = my_id; route.weights[int64_t(token) * topk + threadIdx.x] = v; }
+                    if (threadIdx.x == 0 && route.shared_weights) route.shared_weights[token] = route.shared_ungated ? 1.f : 1.f / (1.f + expf(-shared_logit));
+                }
+            }
+            __syncthreads();
+            e = meta[0];
+        } else {
+            e = route.experts;
+        }
+    } else {
+        e = fetch_ids(ids, A, a, mode, reinterpret_cast<int *>(stage));
+    }
     if (e < 0 || int64_t(e) * b0.rows >= b0.rows_total) return;   // skipped assignment, or an id outside the bank
     int tok[kTP];
     const int n_tok = chunk_up(A, a, e, mode, kTP, reinterpret_cast<int *>(stage), meta, tok);   // the lists live in the dynamic space
@@ -487,7 +516,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
 
 template <uint32_t FMT>
 void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void * out0, void * out1, uint32_t ytype, const int * ids, int A, int xdiv, int mode,
-            int slots, int topk, int shared_lim, int gateup, bool uniform, Glu glu, hipStream_t s) {
+            int slots, int topk, int shared_lim, int gateup, bool uniform, Glu glu, hipStream_t s, DecodeTopk route = DecodeTopk{}) {
     const int NSB = b0.cols / 256, tiles = b0.rows / 32;
     // Waves that share a row's super-blocks: as many as it takes to put a few thousand waves in flight (a short batch
     // is bound by the latency of one wave's chain), fewer when the batch has the waves anyway (a longer chain per
@@ -516,11 +545,115 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl)), unsigned(A));
     const int a_off = int(lds);
     if (staged) lds += size_t(b0.cols / 32) * (256 + ((uniform ? 0 : 1) + (MfmaFormat<FMT>::kMin ? 1 : 0)) * kTP * sizeof(float));
-    auto go = [&](auto kernel) { kernel<<<grid, threads, lds, s>>>(b0, b1, image, out0, out1, ytype, ids, A, xdiv, mode, slots, topk, shared_lim, wk, tpw, gateup, a_off, tl, glu); };
+    auto go = [&](auto kernel) { kernel<<<grid, threads, lds, s>>>(b0, b1, image, out0, out1, ytype, ids, A, xdiv, mode, slots, topk, shared_lim, wk, tpw, gateup, a_off, tl, glu, route); };
+    if (route.logits) {   // few tokens: mode 0, nothing staged
+        if (route.experts <= 128) go(decode_mfma_k<FMT, 2, true, 0, 2>); else go(decode_mfma_k<FMT, 2, true, 0, 8>);
+        return;
+    }
     if (nb == 2 && uniform) staged ? go(decode_mfma_k<FMT, 2, true, 1>) : go(decode_mfma_k<FMT, 2, true, 0>);
     else if (nb == 2) staged ? go(decode_mfma_k<FMT, 2, false, 1>) : go(decode_mfma_k<FMT, 2, false, 0>);
     else if (tl > 1) go(decode_mfma_k<FMT, 1, false, 2>);
     else staged ? go(decode_mfma_k<FMT, 1, false, 1>) : go(decode_mfma_k<FMT, 1, false, 0>);
+}
+
+// The down product of one to a few tokens and the weighted sum over their experts. A block takes one token and 32 output columns
+// (a tile of 32 weight rows in every expert of the token); its waves take (slot, super-block) units in turn, leave each unit's
+// 32 sums in LDS, and the block adds a slot's super-blocks, then the slots in order. Against a product launch per assignment
+// and a launch that sums: one launch, one trip through memory and the [slots][hidden] fp32 rows less. Few blocks (hidden / 32
+// a token), each with all its loads in flight: a chain of one trip to memory and a few hundred instructions.
+constexpr int kDownWaves = 16;
+template <uint32_t FMT>
+__global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArgs k) {
+    using F = MfmaFormat<FMT>;
+    extern __shared__ float part[];   // [units][32] sums, then [slots][32] weighted rows
+    __shared__ uint32_t lat[F::kLattice];
+    const int token = blockIdx.y, tile = blockIdx.x, S = k.b.cols / 32, NSB = S / 8, tiles = k.b.rows / 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
+    const int shared_sb = k.slots > k.topk ? k.shared_cols / 256 : 0, units = k.topk * NSB + shared_sb;
+    const int extra = int(k.b.rows_total / k.b.rows) - 1;      // the shared expert's place
+    struct Unit { typename F::Codes code; typename F::Rec rec; v4i a[8]; float4 xs[2], xm[2]; float rf; };
+    auto expert_of = [&](int u) { const int slot = min(u / NSB, k.slots - 1); return slot < k.topk ? k.ids[token * k.topk + slot] : extra; };
+    auto fetch = [&](int u, int e, Unit & c) {
+        const int slot = min(u / NSB, k.slots - 1), sb = u - slot * NSB;
+        e = max(e, 0);
+        const int64_t at = (int64_t(e) * tiles + tile) * NSB + sb;
+        F::codes(k.b.codes + at * F::kCodeBytes, n, g, c.code);
+        c.rec = F::rec(k.b.aux + at * F::kRecBytes, n);
+        const uint8_t * row = image_row_ptr(k.image, int64_t(token) * k.slots + slot, S);
+        const uint8_t * a = row + sb * 512 + (n & 1) * 32 + g * 16;
+#pragma unroll
+        for (int ib = 0; ib < 8; ++ib) c.a[ib] = *reinterpret_cast<const v4i *>(a + ib * 64);
+        const float4 * xs = reinterpret_cast<const float4 *>(image_scales(row, S) + sb * 8);
+        c.xs[0] = xs[0]; c.xs[1] = xs[1];
+        if constexpr (F::kMin) { const float4 * xm = reinterpret_cast<const float4 *>(image_sums(row, S) + sb * 8); c.xm[0] = xm[0]; c.xm[1] = xm[1]; }
+        c.rf = F::row_factor(k.b, (int64_t(e) * k.b.rows) + tile * 32 + n);
+    };
+    auto multiply = [&](const Unit & c) {
+        const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+        const float xs[8] = {c.xs[0].x, c.xs[0].y, c.xs[0].z, c.xs[0].w, c.xs[1].x, c.xs[1].y, c.xs[1].z, c.xs[1].w};
+        float sum = 0.f, mins = 0.f;
+#pragma unroll
+        for (int ib = 0; ib < 8; ++ib) {
+            const v4i w = F::decode(c.code, c.rec, ib, g, lat);
+            // (every even row of operand A is the hi plane of the one input row, every odd one the lo plane)
+            auto add = [&](const v16i & acc, int grp) {
+                sum += float((acc[0] << 7) + acc[1]) * (F::d(c.rec) * float(F::scale(c.rec, ib, grp)) * xs[ib]);
+                asm volatile("" : : "v"(acc));   // (all sixteen registers in use until here: see decode_mfma_k)
+            };
+            if constexpr (F::kGroups == 1) add(__builtin_amdgcn_mfma_i32_32x32x32_i8(c.a[ib], w, zero, 0, 0, 0), 0);
+            else
+#pragma unroll
+                for (int grp = 0; grp < 2; ++grp) {
+                    const long a2 = long(uint64_t(uint32_t(c.a[ib][grp])) | uint64_t(uint32_t(c.a[ib][grp + 2])) << 32);
+                    const long w2 = long(uint64_t(uint32_t(w[grp])) | uint64_t(uint32_t(w[grp + 2])) << 32);
+                    add(__builtin_amdgcn_mfma_i32_32x32x16_i8(a2, w2, zero, 0, 0, 0), grp);
+                }
+            if constexpr (F::kGroups == 2) __builtin_amdgcn_sched_barrier(0);   // (sixteen results under way are more than the registers hold)
+            if constexpr (F::kMin) {
+                const float xm[8] = {c.xm[0].x, c.xm[0].y, c.xm[0].z, c.xm[0].w, c.xm[1].x, c.xm[1].y, c.xm[1].z, c.xm[1].w};
+                mins = fmaf(F::minimum(c.rec, ib), xm[ib], mins);
+            }
+        }
+        if constexpr (F::kMin) sum = fmaf(-F::dmin(c.rec), mins, sum);
+        return sum * c.rf;
+    };
+    if constexpr (FMT == TQMOE_IQ3_S) {
+        for (int i = threadIdx.x; i < 512; i += blockDim.x) lat[i] = d_iq3s_grid.v[i] << 3;
+        __syncthreads();
+    }
+    // (a second unit's loads in flight under the first's products: the registers of a block of sixteen waves spill, 7.9 -> 23.7 us
+    // for Q4_K at one token)
+    for (int u = wave; u < units; u += kDownWaves) {
+        const int e = expert_of(u);
+        Unit c;
+        fetch(u, e, c);
+        const float v = multiply(c);
+        if (g == 0) part[u * 32 + n] = e >= 0 && int64_t(e) * k.b.rows < k.b.rows_total ? v : 0.f;
+    }
+    __syncthreads();
+    float * rows = part + units * 32;
+    for (int i = threadIdx.x; i < k.slots * 32; i += blockDim.x) {
+        const int slot = i >> 5, nsb = slot < k.topk ? NSB : shared_sb;
+        float v = 0.f;
+        for (int sb = 0; sb < nsb; ++sb) v += part[(slot * NSB + sb) * 32 + (i & 31)];
+        rows[i] = (slot < k.topk ? k.weights[token * k.topk + slot] : k.shared_weights[token]) * v;
+    }
+    __syncthreads();
+    if (threadIdx.x < 32) {
+        float sum = 0.f;
+        for (int s = 0; s < k.slots; ++s) sum += rows[s * 32 + threadIdx.x];
+        const int64_t o = int64_t(token) * k.b.rows + tile * 32 + threadIdx.x;
+        if (k.otype == TQMOE_F32) static_cast<float *>(k.out)[o] = sum;
+        else {
+            if (k.residual) sum = bf16_bits_to_float(float_to_bf16_bits(sum)) + bf16_bits_to_float(k.residual[o]);
+            static_cast<uint16_t *>(k.out)[o] = float_to_bf16_bits(sum);
+        }
+    }
+}
+
+template <uint32_t FMT> void down_combine_launch(const DownCombineArgs & k, hipStream_t s) {
+    const int NSB = k.b.cols / 256, units = k.topk * NSB + (k.slots > k.topk ? k.shared_cols / 256 : 0);
+    down_combine_k<FMT><<<dim3(unsigned(k.b.rows / 32), unsigned(k.n)), 64 * kDownWaves, size_t(units + k.slots) * 32 * sizeof(float), s>>>(k);
 }
 
 // the shapes the kernel takes: whole tiles, whole super-blocks (a narrower shared expert included)

@@ -4,6 +4,7 @@
 
 #include "act_image.cuh"
 #include "common.cuh"
+#include "topk_select.cuh"
 
 namespace tqmoe {
 namespace {
@@ -14,11 +15,17 @@ namespace {
 // sum by ordinary fp32 rounding only.
 constexpr int kRouterTok = 4;       // tokens per pass of a wave: the router row is read once for them
 constexpr int kRouterTokFew = 1;    // decode-sized batches: a wave per (row, token), the latency of a wave's chain is what counts
-constexpr int kRouterFew = 7;       // batches up to here take kRouterTokFew
+constexpr int kRouterFew = 7;       // batches up to here take kRouterTokFew (enqueue_router_image is given no larger ones)
 template <int WT, int XT, int TOK>
 __global__ __launch_bounds__(256) void router_k(const void * __restrict__ w, const void * __restrict__ shared,
-                                                const void * __restrict__ x, float * __restrict__ logits, int h, int e, int n) {
+                                                const void * __restrict__ x, float * __restrict__ logits, int h, int e, int n, uint8_t * __restrict__ image) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if constexpr (TOK == 1) {   // with an activation image to write: a further block per token
+        if (image && blockIdx.x == gridDim.x - 1) {
+            if (wave == 0) quantise_row_wave<XT>(x, blockIdx.y, h, image + int64_t(blockIdx.y) * (h / 32) * kImageSubBytes, lane);
+            return;
+        }
+    }
     const int row = blockIdx.x * 4 + wave;  // 0..e (e = the shared gate)
     const int t0 = blockIdx.y * TOK;
     if (row > e) return;                     // whole waves leave together: reductions below see full waves
@@ -85,22 +92,22 @@ __global__ __launch_bounds__(256) void router_k(const void * __restrict__ w, con
 }
 
 template <int WT> int32_t launch_router_x(uint32_t xtype, const void * w, const void * sg, const void * x, float * logits,
-                                          int h, int e, int n, hipStream_t s) {
+                                          int h, int e, int n, hipStream_t s, uint8_t * image = nullptr) {
     const bool wide = n <= kRouterFew;   // the wide grid of one-token passes
     const int tok = wide ? kRouterTokFew : kRouterTok;
-    const dim3 grid(unsigned((e + 1 + 3) / 4), unsigned((n + tok - 1) / tok));
+    const dim3 grid(unsigned((e + 1 + 3) / 4 + (image ? 1 : 0)), unsigned((n + tok - 1) / tok));
     switch (xtype) {
         case TQMOE_F32:
-            if (wide) router_k<WT, TQMOE_F32, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n);
-            else router_k<WT, TQMOE_F32, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n);
+            if (wide) router_k<WT, TQMOE_F32, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
+            else router_k<WT, TQMOE_F32, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
             return 0;
         case TQMOE_F16:
-            if (wide) router_k<WT, TQMOE_F16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n);
-            else router_k<WT, TQMOE_F16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n);
+            if (wide) router_k<WT, TQMOE_F16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
+            else router_k<WT, TQMOE_F16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
             return 0;
         case TQMOE_BF16:
-            if (wide) router_k<WT, TQMOE_BF16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n);
-            else router_k<WT, TQMOE_BF16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n);
+            if (wide) router_k<WT, TQMOE_BF16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
+            else router_k<WT, TQMOE_BF16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
             return 0;
     }
     return -1;
@@ -249,53 +256,6 @@ __global__ __launch_bounds__(256 * KS) void router_gemm_k(const uint16_t * __res
 // One wave per token. Selection rule of the reference: larger probability first, equal probabilities to the lower
 // index. Up to 1024 experts the probabilities stay in registers (lane l owns entries l, l + 64, ...) and every
 // reduction is a DPP butterfly ending in a scalar broadcast; larger layers keep them in LDS.
-template <int CTRL, int ROWS> __device__ __forceinline__ float dpp_keep_f(float v) {   // lanes outside ROWS get their own value back
-    return __int_as_float(__builtin_amdgcn_update_dpp(__float_as_int(v), __float_as_int(v), CTRL, ROWS, 0xF, false));
-}
-template <int CTRL, int ROWS> __device__ __forceinline__ int dpp_keep_i(int v) { return __builtin_amdgcn_update_dpp(v, v, CTRL, ROWS, 0xF, false); }
-__device__ __forceinline__ float wave_max_all(float v) {   // the wave's maximum, the same in every lane
-    v = fmaxf(v, dpp_f<kDppXor1>(v));
-    v = fmaxf(v, dpp_f<kDppXor2>(v));
-    v = fmaxf(v, dpp_f<kDppHalfMirror>(v));
-    v = fmaxf(v, dpp_f<kDppMirror>(v));
-    v = fmaxf(v, dpp_keep_f<0x142, 0xA>(v));   // row_bcast:15 into rows 1 and 3
-    v = fmaxf(v, dpp_keep_f<0x143, 0xC>(v));   // row_bcast:31 into rows 2 and 3
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-__device__ __forceinline__ int wave_min_all(int v) {
-    v = min(v, dpp_i<kDppXor1>(v));
-    v = min(v, dpp_i<kDppXor2>(v));
-    v = min(v, dpp_i<kDppHalfMirror>(v));
-    v = min(v, dpp_i<kDppMirror>(v));
-    v = min(v, dpp_keep_i<0x142, 0xA>(v));
-    v = min(v, dpp_keep_i<0x143, 0xC>(v));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-__device__ __forceinline__ int wave_max_all_i(int v) {
-    v = max(v, dpp_i<kDppXor1>(v));
-    v = max(v, dpp_i<kDppXor2>(v));
-    v = max(v, dpp_i<kDppHalfMirror>(v));
-    v = max(v, dpp_i<kDppMirror>(v));
-    v = max(v, dpp_keep_i<0x142, 0xA>(v));
-    v = max(v, dpp_keep_i<0x143, 0xC>(v));
-    return __builtin_amdgcn_readlane(v, 63);
-}
-// Selection keys of the softmax top-k. The reference orders by rounded probability, ties to the lower index
-// (src/experts/moe.cpp:73-78); exp and the division by the common sum are monotone, so ordering by logit gives the same
-// choice whatever exp() the device has, except where two different logits round to one probability. Entries whose
-// probability underflowed to zero are all tied there and go by index: they share one key below every logit's.
-// A finite float maps to an integer with the same order (-0 counts as +0); the map is its own inverse.
-constexpr int kKeyGone = INT_MIN, kKeyZero = INT_MIN + 1;
-__device__ __forceinline__ int order_key(float x) { const int i = __float_as_int(x + 0.f); return i ^ ((i >> 31) & 0x7FFFFFFF); }
-__device__ __forceinline__ float key_value(int k) { return __int_as_float(k ^ ((k >> 31) & 0x7FFFFFFF)); }
-
-__device__ __forceinline__ float wave_sum_all(float v) {
-    v = row_sum16(v);
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x142, 0xA, 0xF, false));
-    v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x143, 0xC, 0xF, false));
-    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
-}
-
 struct TopkOut {
     int * ids; float * weights; float * shared_weights;
     int * ext_ids; int extra;          // optional [n][k + 1] copy of the ids with `extra` in the last slot
@@ -329,19 +289,27 @@ __device__ __forceinline__ void topk_reg_body(const float * __restrict__ logits,
     const int token = blockIdx.x, lane = threadIdx.x & 63;
     const float * x = logits + int64_t(token) * (e + 1);
     if (threadIdx.x >= 64) {
-        const int S = o.cols / 32;
-        if (S <= 64) {   // one block of 32 values per lane
-            float xv[32];
-            if (lane < S) load_block32<XT>(o.x, int64_t(token) * o.cols + 32 * lane, xv);
-            uint8_t * image_row = o.image + int64_t(token) * S * kImageSubBytes;
-            const float amax = wave_max(lane < S ? block_amax(xv) : 0.f);
-            if (lane < S) quantise_block(xv, image_row, S, lane, amax);
-        } else {
-            topk_quantise_row<XT>(o, token, lane);
-        }
+        topk_quantise_row<XT>(o, token, lane);
         return;
     }
     const float shared_logit = o.shared_weights ? x[e] : 0.f;
+    if (k <= 64) {
+        int my_id;
+        float my_w;
+        topk_select<R>(x, e, k, lane, true, my_id, my_w);
+        const float v = topk_weight(my_w, k, scale);
+        if (lane < k) {
+            o.ids[int64_t(token) * k + lane] = my_id;
+            o.weights[int64_t(token) * k + lane] = v;
+            if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + lane] = my_id;
+        }
+        if (lane == 0) {
+            if (o.shared_weights) o.shared_weights[token] = shared_weight_of(o, shared_logit);
+            if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + k] = o.extra;
+        }
+        return;
+    }
+    // more selections than lanes
     int key[R];
     float m = -INFINITY, sum = 0.f;
     {
@@ -360,25 +328,6 @@ __device__ __forceinline__ void topk_reg_body(const float * __restrict__ logits,
     }
     float selected = 0.f, my_w = 0.f;   // lane s keeps selection s
     int my_id = 0;
-    if (k <= 64) {
-        // Every round is a chain of dependent wave reductions, so the rounds carry only what the next round needs: the
-        // winner's key stays in lane s and the probabilities are computed for all selections at once afterwards. Equal
-        // keys are rare: one ballot tells whether the winner is alone, and only a tie pays for the index reduction.
-        int my_key = kKeyZero;
-        for (int s = 0; s < k; ++s) {
-            int bk = key[0], bi = lane;
-#pragma unroll
-            for (int r = 1; r < R; ++r) if (key[r] > bk) { bk = key[r]; bi = lane + 64 * r; }   // strict: the lowest index of equal keys
-            const int topkey = wave_max_all_i(bk);
-            const unsigned long long tie = __ballot(bk == topkey);
-            const int best = __popcll(tie) == 1 ? __builtin_amdgcn_readlane(bi, __builtin_ctzll(tie)) : wave_min_all(bk == topkey ? bi : 0x7FFFFFFF);
-            if (lane == s) { my_id = best; my_key = topkey; }
-#pragma unroll
-            for (int r = 0; r < R; ++r) if (lane + 64 * r == best) key[r] = kKeyGone;
-        }
-        my_w = my_key == kKeyZero ? 0.f : expf(key_value(my_key) - m) / sum;   // the probability, as every entry's would be computed
-        for (int s = 0; s < k; ++s) selected += __int_as_float(__builtin_amdgcn_readlane(__float_as_int(my_w), s));   // slot order, as the host sums them
-    } else
     for (int s = 0; s < k; ++s) {
         int bk = key[0], bi = lane;
 #pragma unroll
@@ -387,7 +336,7 @@ __device__ __forceinline__ void topk_reg_body(const float * __restrict__ logits,
         const int best = wave_min_all(bk == topkey ? bi : 0x7FFFFFFF);
         const float top = topkey == kKeyZero ? 0.f : expf(key_value(topkey) - m) / sum;   // the probability, as every entry's would be computed
         if (lane == (s & 63)) { my_id = best; my_w = top; }
-        if (k > 64 && (s & 63) == 63) {   // more selections than lanes: a full set goes out before the lanes are reused
+        if ((s & 63) == 63) {   // a full set goes out before the lanes are reused
             o.ids[int64_t(token) * k + s - 63 + lane] = my_id;
             o.weights[int64_t(token) * k + s - 63 + lane] = my_w;   // divided below
             if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + s - 63 + lane] = my_id;
@@ -396,30 +345,14 @@ __device__ __forceinline__ void topk_reg_body(const float * __restrict__ logits,
 #pragma unroll
         for (int r = 0; r < R; ++r) if (lane + 64 * r == best) key[r] = kKeyGone;
     }
-    if (k <= 64) {
-        // the host divides by the clamped sum, then multiplies by the scale
-        const float total = fmaxf(selected, 6.103515625e-5f);
-        if (lane < k) {
-            float v = my_w / total;
-            if (scale != 0.f && scale != 1.f) v *= scale;
-            o.ids[int64_t(token) * k + lane] = my_id;
-            o.weights[int64_t(token) * k + lane] = v;
-            if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + lane] = my_id;
-        }
-        if (lane == 0) {
-            if (o.shared_weights) o.shared_weights[token] = shared_weight_of(o, shared_logit);
-            if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + k] = o.extra;
-        }
-    } else {
-        const int done = k & ~63;             // the last partial set
-        if (lane < k - done) {
-            o.ids[int64_t(token) * k + done + lane] = my_id;
-            o.weights[int64_t(token) * k + done + lane] = my_w;
-            if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + done + lane] = my_id;
-        }
-        __threadfence_block();
-        topk_finish(o, x, token, lane, e, k, scale, selected);
+    const int done = k & ~63;             // the last partial set
+    if (lane < k - done) {
+        o.ids[int64_t(token) * k + done + lane] = my_id;
+        o.weights[int64_t(token) * k + done + lane] = my_w;
+        if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + done + lane] = my_id;
     }
+    __threadfence_block();
+    topk_finish(o, x, token, lane, e, k, scale, selected);
 }
 
 template <int R, int XT>
@@ -829,6 +762,15 @@ extern "C" int32_t tqmoe_router(const void * router, uint32_t wtype, const void 
     else launch_router_x<TQMOE_BF16>(xtype, router, shared_gate, x, logits, hidden, experts, n, s);
     return launched(err, "tqmoe_router");
 }
+
+// router logits and activation images of up to kRouterFew tokens in one launch
+namespace tqmoe {
+void enqueue_router_image(const void * router, uint32_t wtype, const void * shared_gate, const void * x, uint32_t xtype, float * logits, int hidden, int experts,
+                          int n, void * image, hipStream_t s) {
+    if (wtype == TQMOE_F32) launch_router_x<TQMOE_F32>(xtype, router, shared_gate, x, logits, hidden, experts, n, s, static_cast<uint8_t *>(image));
+    else launch_router_x<TQMOE_BF16>(xtype, router, shared_gate, x, logits, hidden, experts, n, s, static_cast<uint8_t *>(image));
+}
+}  // namespace tqmoe
 
 // top-k with the optional extras of the whole-layer path: extended ids and the input rows' activation image
 namespace tqmoe {
