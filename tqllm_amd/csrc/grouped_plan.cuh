@@ -1,0 +1,64 @@
+// The items of the grouped products from the experts' counts, by one block of 1024 threads.
+#pragma once
+#include "grouped_rows_api.cuh"
+
+namespace tqmoe {
+namespace {
+
+// Items of the products: an expert's rows cut into runs of item_rows, the full runs of all experts first, then the rests by
+// row tiles (four and three, two, one): the last blocks of a launch are its short ones. Where index is given, the index of
+// the gathered row tiles (RowIndex) too.
+constexpr int kScans = 6;   // full runs, rests of three classes; row tiles, chunks of chunk_tiles of them
+__device__ __forceinline__ void plan_items(const int * __restrict__ counts, const int * __restrict__ offsets, int experts, int item_rows, int4 * __restrict__ plan, RowIndex index) {
+    __shared__ int s_wave[kScans][16];
+    __shared__ int s_total[kScans];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int per = (experts + 1023) / 1024, lo = min(tid * per, experts), hi = min(lo + per, experts);
+    auto rest_class = [](int rest) { return rest > 64 ? 1 : rest > 32 ? 2 : rest > 0 ? 3 : -1; };
+    auto add = [&](int c, int (&v)[kScans]) {
+        const int k = rest_class(c % item_rows), t = (c + 31) / 32;
+        v[0] += c / item_rows;
+#pragma unroll
+        for (int i = 1; i < 4; ++i) v[i] += k == i;
+        v[4] += t;
+        if (index.tile_base) v[5] += (t + index.chunk_tiles - 1) / index.chunk_tiles;
+    };
+    int mine[kScans] = {};
+    for (int e = lo; e < hi; ++e) add(max(counts[e], 0), mine);
+    int at[kScans];
+#pragma unroll
+    for (int i = 0; i < kScans; ++i) {
+        int v = mine[i];
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) { const int u = __shfl_up(v, d, 64); if (lane >= d) v += u; }
+        at[i] = v - mine[i];
+        if (lane == 63) s_wave[i][wave] = v;
+    }
+    __syncthreads();
+    if (tid < kScans) {
+        int sum = 0;
+        for (int w = 0; w < 16; ++w) { const int v = s_wave[tid][w]; s_wave[tid][w] = sum; sum += v; }
+        s_total[tid] = sum;
+    }
+    __syncthreads();
+    int base = 0;
+#pragma unroll
+    for (int i = 0; i < kScans; ++i) { at[i] += s_wave[i][wave] + (i < 4 ? base : 0); if (i < 4) base += s_total[i]; }
+    if (tid == 0) {
+        plan[0] = make_int4(s_total[0], s_total[1], s_total[2], s_total[3]);
+        if (index.tile_base) { index.tile_base[experts] = s_total[4]; index.chunk_base[experts] = s_total[5]; }
+    }
+    if (index.tile_base && tid < index.counters_n) index.counters[tid] = 0;
+    for (int e = lo; e < hi; ++e) {
+        const int c = max(counts[e], 0), first = offsets[e], full = c / item_rows, rest = c % item_rows;
+        for (int f = 0; f < full; ++f) plan[1 + at[0] + f] = make_int4(e, first + f * item_rows, item_rows, at[4] + f * (item_rows / 32));
+        const int k = rest_class(rest);
+#pragma unroll
+        for (int i = 1; i < 4; ++i) if (k == i) plan[1 + at[i]] = make_int4(e, first + full * item_rows, rest, at[4] + full * (item_rows / 32));
+        if (index.tile_base) { index.tile_base[e] = at[4]; index.chunk_base[e] = at[5]; }
+        add(c, at);
+    }
+}
+
+}  // namespace
+}  // namespace tqmoe

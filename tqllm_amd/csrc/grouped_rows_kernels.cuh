@@ -32,6 +32,7 @@
 #include "decode_table.cuh"
 #include "formats.cuh"
 #include "grouped_rows_api.cuh"
+#include "lds_dma.cuh"
 
 namespace tqmoe {
 namespace {
@@ -39,20 +40,6 @@ namespace {
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 typedef float v16f __attribute__((ext_vector_type(16)));
-
-// 16 bytes a lane from memory to LDS at `lds` (a wave-uniform byte address) + 16 * lane. The compiler does not count these:
-// dma_wait() says when they are there.
-__device__ __forceinline__ void dma16(const void * p, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(p), "s"(lds) : "memory");
-}
-// all but the last N transfers of this wave are here (they finish in order); with BARRIER every wave's are
-template <int N, bool BARRIER> __device__ __forceinline__ void dma_wait() {
-    if constexpr (BARRIER) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "i"(N) : "memory");
-    else asm volatile("s_waitcnt vmcnt(%0)" :: "i"(N) : "memory");
-}
-__device__ __forceinline__ uint32_t lds_address(const void * p) {
-    return uint32_t(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) const uint8_t *)(p)));
-}
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ v8i join(uint4 a, uint4 b) { return v8i{int(a.x), int(a.y), int(a.z), int(a.w), int(b.x), int(b.y), int(b.z), int(b.w)}; }

@@ -3,14 +3,13 @@
 
 #include "formats.cuh"
 #include "grouped_rows_api.cuh"
+#include "routing_api.cuh"
 
 namespace tqmoe {
 int32_t check_bank(const tqmoe_bank * b, const char * what, tqmoe_error * err);
-int32_t enqueue_topk(const float * logits, int32_t * ids, float * weights, float * shared_weights, int32_t * ext_ids, int32_t extra, const void * x,
-                     uint32_t xtype, int32_t cols, void * image, int32_t experts, int32_t topk, int32_t n, float scale, int32_t gating,
-                     const float * bias, int32_t norm, hipStream_t s, int32_t shared_ungated);
-void enqueue_router_image(const void * router, uint32_t wtype, const void * shared_gate, const void * x, uint32_t xtype, float * logits, int hidden, int experts,
-                          int n, void * image, hipStream_t s);
+RowIndex grouped_index(float * scale, int64_t assignments, int experts, int4 ** items);
+int32_t enqueue_gather_rows_i8(const int8_t * rq, const float * rs, int cols, const int * counts, const int * offsets, const int * perm, int experts,
+                               int64_t assignments, int xdiv, int8_t * q, float * scale, hipStream_t s, float * block_scale, bool indexed);
 bool decode_few_takes(const tqmoe_bank & gate, const tqmoe_bank & down, int slots, int shared_ff);
 int32_t expert_down_combine(const tqmoe_bank & down, const void * act_image, const int32_t * ids, const float * weights, const float * shared_weights, int32_t n,
                             int32_t slots, int32_t topk, int32_t shared_ff, void * out, uint32_t otype, const void * residual, void * stream, tqmoe_error * err);
@@ -131,7 +130,7 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         p.counts = take(size_t(banks) * 4);
         p.offsets = take(size_t(banks + 1) * 4);
         p.perm = take(a * 4);
-        p.dispatch_ws = take(tqmoe_dispatch_workspace_bytes(banks, p.chunk, slots));
+        p.dispatch_ws = take(size_t((a + kDispatchChunk - 1) / kDispatchChunk) * banks * sizeof(int));   // the assignments of each chunk's experts
         p.act16 = take(a * L.ff * 2);
         p.y16 = take(a * L.hidden * 4);   // fp16 rows (int8 products) or fp32 rows (fp16 products)
     }
@@ -237,18 +236,40 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
 
     if (p.routes) {
         const hipStream_t st = static_cast<hipStream_t>(stream);
-        enqueue_router_image(L.router, L.router_type, L.shared_gate, x, xtype, logits, L.hidden, L.n_expert, n, ws + p.ximage, st);
+        RouterSide side;
+        side.image = ws + p.ximage;
+        if (int32_t rc = enqueue_router(L.router, L.router_type, L.shared_gate, x, xtype, logits, L.hidden, L.n_expert, n, side, st, err)) return rc;
         const DecodeTopk route{logits, L.n_expert, L.topk, L.has_shared && !L.shared_gate, L.weight_scale, ids, weights, L.has_shared ? shared_w : nullptr};
         if (int32_t rc = expert_gateup_glu(&L.gate, &L.up, ws + p.ximage, ws + p.aimage, nullptr, n, slots, L.topk, L.shared_ff, glu_of(L), stream, err, route)) return rc;
         return expert_down_combine(L.down, ws + p.aimage, ids, weights, shared_w, n, slots, L.topk, L.shared_ff, out, otype, residual, stream, err);
     }
-    if (int32_t rc = tqmoe_router(L.router, L.router_type, L.shared_gate, x, xtype, logits, L.hidden, L.n_expert, n, stream, err)) return rc;
-    // one launch: top-k, the ids extended by the shared expert, and (decode path) the input rows' activation image
+    if (L.hidden % 8) return fail(err, TQMOE_E_ARG, "tqmoe_layer_forward: hidden must be a multiple of 8");
+    if ((n + 3) / 4 > 65535) return fail(err, TQMOE_E_ARG, "tqmoe_layer_forward: too many tokens for one call");
+    // Beside the routing, in its launches: the rows in the form the products read (a batch that is one pass), the assignments
+    // of every dispatch chunk (cleared by the router launch, counted by the top-k launch), the ids extended by the shared expert.
+    const hipStream_t hs = static_cast<hipStream_t>(stream);
+    const bool whole = p.chunk >= n, counted = p.grouped && whole && banks <= kDispatchWide && L.topk <= 64;
+    int * chunk_counts = reinterpret_cast<int *>(ws + p.dispatch_ws);
+    RouterSide rside;
+    TopkSide side;
+    if (counted) {
+        rside.zero = side.chunk_counts = chunk_counts;
+        rside.zero_n = int((int64_t(n) * slots + kDispatchChunk - 1) / kDispatchChunk) * banks;
+        side.banks = banks;
+    }
+    if (!p.grouped || whole) {
+        side.rows = !p.grouped ? kRowsImage : !p.int8 ? (p.prepared ? kRowsHalves : kRowsNone) : p.prepared ? kRowsFp8 : p.blocks ? kRowsInt8Blocks : kRowsInt8;
+        side.x = x;
+        side.xtype = xtype;
+        side.cols = L.hidden;
+        side.q = ws + (!p.grouped ? p.ximage : p.int8 ? p.rq : p.x16);
+        side.scale = reinterpret_cast<float *>(ws + (p.int8 ? p.rs : p.xs16));
+    }
+    if (int32_t rc = enqueue_router(L.router, L.router_type, L.shared_gate, x, xtype, logits, L.hidden, L.n_expert, n, rside, hs, err)) return rc;
     int32_t * ext = L.has_shared ? reinterpret_cast<int32_t *>(ws + p.ids_ext) : nullptr;
     const Routing rt = routing_of(L);
     const Glu glu = glu_of(L);
-    enqueue_topk(logits, ids, weights, shared_w, ext, L.n_expert, x, xtype, L.hidden, p.grouped ? nullptr : ws + p.ximage, L.n_expert, L.topk, n,
-                 L.weight_scale, rt.gating, rt.bias, rt.norm, static_cast<hipStream_t>(stream), L.has_shared && !L.shared_gate);
+    enqueue_topk(logits, ids, weights, shared_w, ext, L.n_expert, L.n_expert, L.topk, n, L.weight_scale, rt.gating, rt.bias, rt.norm, L.has_shared && !L.shared_gate, side, hs);
     if (int32_t rc = launched(err, "tqmoe_layer_forward (top-k)")) return rc;
     const int32_t * ids_ext = ext ? ext : ids;
 
@@ -273,8 +294,16 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
             int32_t * counts = reinterpret_cast<int32_t *>(ws + p.counts), * offsets = reinterpret_cast<int32_t *>(ws + p.offsets),
                     * perm = reinterpret_cast<int32_t *>(ws + p.perm);
             uint16_t * act16 = reinterpret_cast<uint16_t *>(ws + p.act16), * y16 = reinterpret_cast<uint16_t *>(ws + p.y16);
-            if (int32_t rc = tqmoe_dispatch(cid, counts, offsets, perm, nullptr, 0, banks, c, slots, ws + p.dispatch_ws,
-                                            tqmoe_dispatch_workspace_bytes(banks, c, slots), stream, err)) return rc;
+            DispatchSide lists;
+            lists.counted = counted;
+            if (p.prepared) {
+                lists.item_rows = p.item_rows;
+                lists.items = reinterpret_cast<int4 *>(ws + p.items);
+            } else if (p.int8) {
+                lists.item_rows = 128;
+                lists.index = grouped_index(xs, int64_t(c) * slots, banks, &lists.items);
+            }
+            if (int32_t rc = enqueue_layer_dispatch(cid, counts, offsets, perm, banks, c, slots, chunk_counts, lists, hs, err)) return rc;
             if (p.prepared && p.int8) {   // E4M3 rows
                 const hipStream_t st = static_cast<hipStream_t>(stream);
                 uint8_t * rq = ws + p.rq, * aq = ws + p.aq;
@@ -282,8 +311,8 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
                 int4 * items = reinterpret_cast<int4 *>(ws + p.items);
                 const int shared_expert = L.has_shared ? banks - 1 : -1;
                 const int64_t a = int64_t(c) * slots;
-                if (int32_t rc = tqmoe_quant_rows_fp8(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, stream, err)) return rc;
-                enqueue_grouped_plan(counts, offsets, banks, p.item_rows, items, RowIndex{}, st);
+                if (!whole)
+                    if (int32_t rc = tqmoe_quant_rows_fp8(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, stream, err)) return rc;
                 enqueue_grouped_products(L.gate, &L.up, rq, rs, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, st, p.item_rows);
                 if (int32_t rc = tqmoe_quant_rows_fp8(act16, TQMOE_F16, a, L.ff, aq, as, stream, err)) return rc;
                 enqueue_grouped_products(L.down, nullptr, aq, as, perm, items, a, 1, y16, false, shared_expert, L.shared_ff, Glu{0.f, 0}, st, p.item_rows);
@@ -298,8 +327,7 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
                 int4 * items = reinterpret_cast<int4 *>(ws + p.items);
                 const int shared_expert = L.has_shared ? banks - 1 : -1;
                 const int64_t a = int64_t(c) * slots;
-                enqueue_prepare_rows(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, x16, xs16, st);
-                enqueue_grouped_plan(counts, offsets, banks, p.item_rows, items, RowIndex{}, st);
+                if (!whole) enqueue_prepare_rows(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, x16, xs16, st);
                 enqueue_grouped_products(L.gate, &L.up, x16, xs16, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, st, p.item_rows);
                 enqueue_grouped_products(L.down, nullptr, act16, nullptr, perm, items, a, 1, y16, !p.half_rows, shared_expert, L.shared_ff, Glu{0.f, 0}, st, p.item_rows);
                 if (int32_t rc = launched(err, "tqmoe_layer_forward (grouped products)")) return rc;
@@ -319,8 +347,9 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
             float * rs = reinterpret_cast<float *>(ws + p.rs);
             if (p.blocks) {
             float * xbs = reinterpret_cast<float *>(ws + p.xbs), * abks = reinterpret_cast<float *>(ws + p.abks);
-            if (int32_t rc = tqmoe_quant_rows_i8_blocks(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, nullptr, stream, err)) return rc;
-            if (int32_t rc = tqmoe_gather_rows_i8_blocks(rq, rs, L.hidden, counts, offsets, perm, banks, int64_t(c) * slots, slots, xq, xs, xbs, stream, err)) return rc;
+            if (!whole)
+                if (int32_t rc = tqmoe_quant_rows_i8_blocks(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, nullptr, stream, err)) return rc;
+            enqueue_gather_rows_i8(rq, rs, L.hidden, counts, offsets, perm, banks, int64_t(c) * slots, slots, xq, xs, hs, xbs, true);
             if (int32_t rc = gemm_8bit_common(&L.gate, &L.up, xq, xs, counts, offsets, perm, c, slots, L.topk, L.shared_ff, act16, 1, stream, err,
                                               "tqmoe_layer_forward (gate / up)", false, xbs, true, glu, 0, nullptr)) return rc;
             if (int32_t rc = group_rows_common(act16, TQMOE_F16, L.ff, counts, offsets, perm, banks, int64_t(c) * slots, 1, aq, as, stream, err, false,
@@ -328,8 +357,9 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
             if (int32_t rc = gemm_8bit_common(&L.down, nullptr, aq, as, counts, offsets, perm, c, slots, L.topk, L.shared_ff, y16, 0, stream, err,
                                               "tqmoe_layer_forward (down)", false, abks, true, Glu{0.f, 0}, 0, xs)) return rc;
             } else {
-            if (int32_t rc = tqmoe_quant_rows_i8(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, stream, err)) return rc;
-            if (int32_t rc = tqmoe_gather_rows_i8(rq, rs, L.hidden, counts, offsets, perm, banks, int64_t(c) * slots, slots, xq, xs, stream, err)) return rc;
+            if (!whole)
+                if (int32_t rc = tqmoe_quant_rows_i8(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, stream, err)) return rc;
+            enqueue_gather_rows_i8(rq, rs, L.hidden, counts, offsets, perm, banks, int64_t(c) * slots, slots, xq, xs, hs, nullptr, true);
             if (int32_t rc = gemm_8bit_common(&L.gate, &L.up, xq, xs, counts, offsets, perm, c, slots, L.topk, L.shared_ff, act16, 1, stream, err,
                                               "tqmoe_layer_forward (gate / up)", false, nullptr, false, glu, 0, nullptr)) return rc;
             if (int32_t rc = group_rows_common(act16, TQMOE_F16, L.ff, counts, offsets, perm, banks, int64_t(c) * slots, 1, aq, as, stream, err, false,

@@ -4,70 +4,11 @@
 namespace tqmoe {
 namespace {
 
-// the largest magnitude over the four lanes that hold a 32-value block (eight values each)
-__device__ __forceinline__ float quad_max(float v) {
-    v = fmaxf(v, dpp_f<kDppXor1>(v));
-    return fmaxf(v, dpp_f<kDppXor2>(v));
-}
-__device__ __forceinline__ int byte_sum_i8(uint32_t w) { return int(int8_t(w)) + int(int8_t(w >> 8)) + int(int8_t(w >> 16)) + int(int8_t(w >> 24)); }
-
-// rows of 8-bit activations: q = rint(x * 127 / amax) per row, scale = amax / 127 (E4M3: 448 in place of 127); one wave per row.
-// BLK: amax and scale per block of 32 values (scale [rows][cols / 32]) and, when asked for, the sums of q over each 16
-// values (qsum [rows][cols / 32][2]).
 template <int XT, bool F8, bool BLK = false>
 __global__ __launch_bounds__(256) void quant_rows_k(const void * __restrict__ x, int64_t rows, int cols, int8_t * __restrict__ q, float * __restrict__ scale,
                                                     int16_t * __restrict__ qsum = nullptr) {
-    const int lane = threadIdx.x & 63;
     const int64_t row = int64_t(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    if (row >= rows) return;
-    const int groups = cols / 8;   // 8 consecutive values = natural dwords 2j, 2j + 1 of a 32-block
-    if constexpr (BLK) {           // (a block's four lanes enter or leave the loop together: cols is a multiple of 32)
-        uint32_t * out = reinterpret_cast<uint32_t *>(q + row * cols);
-        for (int gi = lane; gi < groups; gi += 64) {
-            float v[8];
-            load8<XT>(x, row * cols + gi * 8, v);
-            float amax = 0.f;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-            amax = quad_max(amax);
-            const float mul = amax > 0.f ? 127.f / amax : 0.f;
-            const uint32_t w[2] = {pack4_q<false>(v[0] * mul, v[1] * mul, v[2] * mul, v[3] * mul), pack4_q<false>(v[4] * mul, v[5] * mul, v[6] * mul, v[7] * mul)};
-            const int blk = gi >> 2, d0 = 2 * (gi & 3);
-            out[blk * 8 + plane_pos(d0)] = w[0];
-            out[blk * 8 + plane_pos(d0 + 1)] = w[1];
-            if ((gi & 3) == 0) scale[row * (cols / 32) + blk] = amax / 127.f;
-            if (qsum) {
-                int sum = byte_sum_i8(w[0]) + byte_sum_i8(w[1]);
-                sum += dpp_i<kDppXor1>(sum);
-                if ((gi & 1) == 0) qsum[(row * (cols / 32) + blk) * 2 + ((gi & 3) >> 1)] = int16_t(sum);
-            }
-        }
-        return;
-    }
-    float amax = 0.f;
-    for (int gi = lane; gi < groups; gi += 64) {
-        float v[8];
-        load8<XT>(x, row * cols + gi * 8, v);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) amax = fmaxf(amax, fabsf(v[j]));
-    }
-    amax = fmaxf(amax, dpp_f<kDppXor1>(amax));
-    amax = fmaxf(amax, dpp_f<kDppXor2>(amax));
-    amax = fmaxf(amax, dpp_f<kDppHalfMirror>(amax));
-    amax = fmaxf(amax, dpp_f<kDppMirror>(amax));
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
-    amax = fmaxf(amax, __shfl_xor(amax, 32, 64));
-    const float mul = amax > 0.f ? kOperandMax<F8> / amax : 0.f;
-    if (lane == 0) scale[row] = amax / kOperandMax<F8>;
-    uint32_t * out = reinterpret_cast<uint32_t *>(q + row * cols);
-    for (int gi = lane; gi < groups; gi += 64) {
-        float v[8];
-        load8<XT>(x, row * cols + gi * 8, v);
-        const uint32_t w[2] = {pack4_q<F8>(v[0] * mul, v[1] * mul, v[2] * mul, v[3] * mul), pack4_q<F8>(v[4] * mul, v[5] * mul, v[6] * mul, v[7] * mul)};
-        const int blk = gi >> 2, d0 = 2 * (gi & 3);
-        out[blk * 8 + plane_pos(d0)] = w[0];
-        out[blk * 8 + plane_pos(d0 + 1)] = w[1];
-    }
+    if (row < rows) quant_row_wave<XT, F8, BLK>(x, row, cols, q, scale, qsum, threadIdx.x & 63);
 }
 
 // Rows of the grouped operand: block b takes rows [8 (b % 4), +8) of row tile b / 4, one wave per two rows. Row i of
@@ -284,6 +225,12 @@ int32_t enqueue_quant_rows_i8_blocks(const void * x, uint32_t xtype, int64_t row
 int64_t grouped_scale_words(int64_t assignments, int experts) {
     return grouped_row_tiles(assignments, experts) * 32 + 2 * (int64_t(experts) + 1) + kPlanCounters + 4 * (2 + grouped_rows_items(assignments, experts, grouped_rows_per_item(TQMOE_NVFP4G, assignments, experts)));
 }
+// where the index of rows grouped into `scale` goes, for a launch that writes it beside other work
+RowIndex grouped_index(float * scale, int64_t assignments, int experts, int4 ** items) {
+    const Plan plan = plan_at(scale, grouped_row_tiles(assignments, experts) * 32, experts);
+    *items = plan.items;
+    return RowIndex{const_cast<int *>(plan.tile_base), const_cast<int *>(plan.chunk_base), plan.counters, kPlanCounters, kChunkTiles};
+}
 static void enqueue_index(const int * counts, const int * offsets, int experts, int64_t assignments, const Plan & plan, hipStream_t s) {
     enqueue_grouped_plan(counts, offsets, experts, grouped_rows_per_item(TQMOE_NVFP4G, assignments, experts), plan.items,
                          RowIndex{const_cast<int *>(plan.tile_base), const_cast<int *>(plan.chunk_base), plan.counters, kPlanCounters, kChunkTiles}, s);
@@ -328,10 +275,10 @@ int32_t enqueue_group_rows_i8(const void * x, uint32_t xtype, int cols, const in
 }
 
 int32_t enqueue_gather_rows_i8(const int8_t * rq, const float * rs, int cols, const int * counts, const int * offsets, const int * perm, int experts,
-                               int64_t assignments, int xdiv, int8_t * q, float * scale, hipStream_t s, float * block_scale) {
+                               int64_t assignments, int xdiv, int8_t * q, float * scale, hipStream_t s, float * block_scale, bool indexed) {
     const int64_t tiles = grouped_row_tiles(assignments, experts);
     const Plan plan = plan_at(scale, tiles * 32, experts);
-    enqueue_index(counts, offsets, experts, assignments, plan, s);
+    if (!indexed) enqueue_index(counts, offsets, experts, assignments, plan, s);
     gather_rows_i8_k<<<unsigned(tiles), 256, 0, s>>>(rq, rs, cols, counts, offsets, perm, experts, xdiv, q, scale, plan, block_scale);
     return 0;
 }

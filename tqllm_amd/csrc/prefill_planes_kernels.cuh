@@ -31,6 +31,7 @@
 #include "decode_api.cuh"
 #include "formats.cuh"
 #include "grouped_rows_api.cuh"
+#include "row_quant.cuh"
 
 #include <algorithm>
 #include <type_traits>
@@ -76,21 +77,6 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kChunkTiles = 8;                // row tiles (of 32 assignments) per chunk
 constexpr int kPlanExperts = 1024;              // experts whose index a block keeps in LDS
-
-// four scaled values -> four operand bytes: int8 (round to nearest) or E4M3 (round to nearest even; the values are
-// clamped to +-448 first, so the conversion never leaves the finite codes)
-template <bool F8> __device__ __forceinline__ uint32_t pack4_q(float a, float b, float c, float d) {
-    if constexpr (F8) {
-        auto clamp = [](float v) { return fminf(fmaxf(v, -448.f), 448.f); };
-        int w = __builtin_amdgcn_cvt_pk_fp8_f32(clamp(a), clamp(b), 0, false);
-        w = __builtin_amdgcn_cvt_pk_fp8_f32(clamp(c), clamp(d), w, true);
-        return uint32_t(w);
-    } else {
-        return uint32_t(__float2int_rn(a) & 0xFF) | uint32_t(__float2int_rn(b) & 0xFF) << 8 | uint32_t(__float2int_rn(c) & 0xFF) << 16 |
-               uint32_t(__float2int_rn(d) & 0xFF) << 24;
-    }
-}
-template <bool F8> constexpr float kOperandMax = F8 ? 448.f : 127.f;
 
 // largest e in [0, experts) with base[e] <= unit, for unit < base[experts] (experts with no unit share their successor's
 // base and are skipped by taking the last of equal entries)

@@ -3,7 +3,11 @@
 #include <mutex>
 
 #include "act_image.cuh"
+#include "lds_dma.cuh"
 #include "common.cuh"
+#include "grouped_plan.cuh"
+#include "routing_api.cuh"
+#include "row_quant.cuh"
 #include "topk_select.cuh"
 
 namespace tqmoe {
@@ -18,13 +22,15 @@ constexpr int kRouterTokFew = 1;    // decode-sized batches: a wave per (row, to
 constexpr int kRouterFew = 7;       // batches up to here take kRouterTokFew (enqueue_router_image is given no larger ones)
 template <int WT, int XT, int TOK>
 __global__ __launch_bounds__(256) void router_k(const void * __restrict__ w, const void * __restrict__ shared,
-                                                const void * __restrict__ x, float * __restrict__ logits, int h, int e, int n, uint8_t * __restrict__ image) {
+                                                const void * __restrict__ x, float * __restrict__ logits, int h, int e, int n, RouterSide side) {
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    if constexpr (TOK == 1) {   // with an activation image to write: a further block per token
-        if (image && blockIdx.x == gridDim.x - 1) {
-            if (wave == 0) quantise_row_wave<XT>(x, blockIdx.y, h, image + int64_t(blockIdx.y) * (h / 32) * kImageSubBytes, lane);
-            return;
+    if ((side.image || side.zero) && blockIdx.x == gridDim.x - 1) {   // a further block per pass for what stands beside the routing
+        if (blockIdx.y == 0)
+            for (int i = threadIdx.x; i < side.zero_n; i += 256) side.zero[i] = 0;
+        if constexpr (TOK == 1) {
+            if (side.image && wave == 0) quantise_row_wave<XT>(x, blockIdx.y, h, side.image + int64_t(blockIdx.y) * (h / 32) * kImageSubBytes, lane);
         }
+        return;
     }
     const int row = blockIdx.x * 4 + wave;  // 0..e (e = the shared gate)
     const int t0 = blockIdx.y * TOK;
@@ -92,164 +98,286 @@ __global__ __launch_bounds__(256) void router_k(const void * __restrict__ w, con
 }
 
 template <int WT> int32_t launch_router_x(uint32_t xtype, const void * w, const void * sg, const void * x, float * logits,
-                                          int h, int e, int n, hipStream_t s, uint8_t * image = nullptr) {
+                                          int h, int e, int n, const RouterSide & side, hipStream_t s) {
     const bool wide = n <= kRouterFew;   // the wide grid of one-token passes
     const int tok = wide ? kRouterTokFew : kRouterTok;
-    const dim3 grid(unsigned((e + 1 + 3) / 4 + (image ? 1 : 0)), unsigned((n + tok - 1) / tok));
+    const dim3 grid(unsigned((e + 1 + 3) / 4 + (side.image || side.zero ? 1 : 0)), unsigned((n + tok - 1) / tok));
     switch (xtype) {
         case TQMOE_F32:
-            if (wide) router_k<WT, TQMOE_F32, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
-            else router_k<WT, TQMOE_F32, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
+            if (wide) router_k<WT, TQMOE_F32, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, side);
+            else router_k<WT, TQMOE_F32, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, side);
             return 0;
         case TQMOE_F16:
-            if (wide) router_k<WT, TQMOE_F16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
-            else router_k<WT, TQMOE_F16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
+            if (wide) router_k<WT, TQMOE_F16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, side);
+            else router_k<WT, TQMOE_F16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, side);
             return 0;
         case TQMOE_BF16:
-            if (wide) router_k<WT, TQMOE_BF16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
-            else router_k<WT, TQMOE_BF16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, image);
+            if (wide) router_k<WT, TQMOE_BF16, kRouterTokFew><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, side);
+            else router_k<WT, TQMOE_BF16, kRouterTok><<<grid, 256, 0, s>>>(w, sg, x, logits, h, e, n, side);
             return 0;
     }
     return -1;
 }
 
-// Router logits of many tokens, bf16 rows on both sides or fp32 rows on both sides: a GEMM on the matrix pipe. bf16 x bf16
+// Router logits of more tokens, bf16 rows on both sides or fp32 rows on both sides: a GEMM on the matrix pipe. bf16 x bf16
 // products are exact in fp32, the fp32 instruction multiplies and adds in fp32, and both accumulate in fp32, so the result
-// differs from the scalar kernel's only by the order of the sum. A block of four waves takes 64 tokens x 64 router rows, every wave a 32 x 32 quadrant. The kernel is a
-// chain of stages (load from memory, store to LDS, multiply), and a stage costs a trip to memory however little it
-// multiplies: so a stage is 512 bytes of every row (256 bf16 columns: eight stages at hidden 2048; 128 fp32 columns), the next stage's loads are in registers while
-// this one is multiplied, and two blocks fit a compute unit. The shared expert's gate row rides along as a 65th row of the
-// last row block (one more matrix instruction per step for two of its waves), so that 512 experts are eight row blocks and
-// not nine.
+// differs from the scalar kernel's only by the order of the sum.
+// A block of eight waves takes 16 TA tokens x 64 router rows; every wave computes the whole tile over an eighth of the
+// columns, operands straight from memory (16 bytes a lane, 64 of a row together), a chunk of steps ahead of the matrix
+// instructions, and the eight partial tiles are added through LDS in a fixed order. No stage is waited for by the whole block:
+// a launch is one trip to memory and the bandwidth of the L2, where stages of 256 columns through LDS were a chain of eight
+// trips (512 experts, 2048 columns: 21 us for 333 tokens, 32 for 4096). TA is the largest tile that still gives every
+// compute unit a block. A token's sums do not depend on it, nor on the batch.
+// The last row of blocks takes the shared expert's gate row (or stores its zeros): a wave a token.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
-typedef float v16f __attribute__((ext_vector_type(16)));
-constexpr int kRouterGemmMin = 120000;   // tokens x router rows from which a bf16 router and input take the GEMM (the wave-per-row kernel
-                                         // takes 10 us up to 16,000 and grows with tokens x rows)
-constexpr int kRgTok = 64, kRgRows = 64, kRgK = 256, kRgPad = kRgK + 8;   // halves per staged row: 16-byte reads of consecutive rows spread over the banks
+typedef float v4f __attribute__((ext_vector_type(4)));
+constexpr int kRouterGemmMin = 30000;   // tokens x router rows from which a bf16 router and input take the GEMM
+constexpr int kRgWaves = 8, kRgRows = 64, kRgPitch = kRgRows + 4;   // floats of a token's row in the exchange space: four rows apart, other banks
+template <int TA> constexpr int kRgLds = 4 * TA * 16 * kRgPitch * int(sizeof(float));
 
-// F32: the rows are fp32 (h counts 2-byte units here: twice the columns); else bf16.
-// KS = 2: eight waves, the second four take the second half of every stage's steps and hand their sums to the first four
-// through LDS at the end (first half + second half, a fixed order): for grids that leave most compute units without a
-// block, where a block's own chain of stages is the whole time.
-template <bool F32, int KS = 1>
-__global__ __launch_bounds__(256 * KS) void router_gemm_k(const uint16_t * __restrict__ w, const uint16_t * __restrict__ shared, const uint16_t * __restrict__ x,
-                                                       float * __restrict__ logits, int h, int e, int n) {
-    __shared__ __attribute__((aligned(16))) uint16_t As[kRgTok][kRgPad];
-    __shared__ __attribute__((aligned(16))) uint16_t Bs[kRgRows + 1][kRgPad];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, r = lane & 31, g = lane >> 5;
-    const int t0 = int(blockIdx.x) * kRgTok, r0 = int(blockIdx.y) * kRgRows;
-    const bool last = blockIdx.y == gridDim.y - 1;     // this block also has row e (the shared gate, or zeros)
-    const int mq = wave & 1, nq = (wave >> 1) & 1;     // quadrant: tokens 32 mq.., router rows 32 nq..
-    const int kh = wave >> 2;                          // which part of every stage's steps (0 when KS == 1)
-    const bool extra = last && nq == 0;
-    // staging: thread -> 16-byte piece sp of rows sr, sr + 8 KS, ... of both tiles (a wave's loads cover two whole rows of 512 bytes)
-    constexpr int SR = 8 / KS;                         // rows of each tile a thread stages
-    const int sp = tid & 31, sr = tid >> 5;
-    const uint16_t * a_src[SR], * b_src[SR];
-    bool b_zero[SR];
+// the gate row's logits of tokens [t0, t1) (zeros without a gate row), a wave a token; and the grid's share of what is to be cleared
+template <int XT>
+__device__ __forceinline__ void router_shared_column(const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x, float * __restrict__ logits, int h, int e, int n,
+                                                     int t0, int t1, const RouterSide & side, int waves) {
+    const int lane = threadIdx.x & 63;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < side.zero_n; i += gridDim.x * blockDim.x) side.zero[i] = 0;
+    for (int t = t0 + (threadIdx.x >> 6); t < t1; t += waves) {
+        float acc = 0.f;
+        if (shared)
+            for (int c = lane * 8; c < h; c += 512) {
+                float wv[8], xv[8];
+                load8<XT>(shared, c, wv);
+                load8<XT>(x, int64_t(t) * h + c, xv);
 #pragma unroll
-    for (int i = 0; i < SR; ++i) {
-        a_src[i] = x + int64_t(min(t0 + sr + 8 * KS * i, n - 1)) * h + 8 * sp;   // rows past the end repeat a valid row (not stored)
-        const int row = r0 + sr + 8 * KS * i;
-        b_zero[i] = row >= e;
-        b_src[i] = w + int64_t(min(row, e - 1)) * h + 8 * sp;
+                for (int j = 0; j < 8; ++j) acc = fmaf(wv[j], xv[j], acc);
+            }
+        acc = group_sum<64>(acc);
+        if (lane == 0) logits[int64_t(t) * (e + 1) + e] = acc;
     }
-    uint4 a_st[SR], b_st[SR], x_st = make_uint4(0, 0, 0, 0);
-    auto fetch = [&](int k0) {
-        const bool in = k0 + 8 * sp < h;   // the last stage may be narrower
+}
+
+template <bool F32, int TA>
+__global__ __launch_bounds__(64 * kRgWaves) void router_gemm_k(const uint8_t * __restrict__ w, const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x,
+                                                              float * __restrict__ logits, int h, int e, int n, RouterSide side) {
+    extern __shared__ __attribute__((aligned(16))) float red[];   // [4][TA * 16][kRgPitch]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    constexpr int kBytes = F32 ? 4 : 2, TT = 16 * TA;
+    const int t0 = int(blockIdx.x) * TT, r0 = int(blockIdx.y) * kRgRows;
+    const int64_t pitch = int64_t(h) * kBytes;
+    if (blockIdx.y == gridDim.y - 1) {
+        router_shared_column<F32 ? TQMOE_F32 : TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + TT, n), side, kRgWaves);
+        return;
+    }
+    const uint8_t * ap[TA], * bp[4];   // rows past the end repeat a valid row (not stored)
 #pragma unroll
-        for (int i = 0; i < SR; ++i) {
-            a_st[i] = in ? *reinterpret_cast<const uint4 *>(a_src[i] + k0) : make_uint4(0, 0, 0, 0);
-            b_st[i] = in && !b_zero[i] ? *reinterpret_cast<const uint4 *>(b_src[i] + k0) : make_uint4(0, 0, 0, 0);
+    for (int i = 0; i < TA; ++i) ap[i] = x + int64_t(min(t0 + 16 * i + r, n - 1)) * pitch + 16 * g;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) bp[j] = w + int64_t(min(r0 + 16 * j + r, e - 1)) * pitch + 16 * g;
+    const int steps = int(pitch / 64), s0 = wave * steps / kRgWaves, s1 = (wave + 1) * steps / kRgWaves;   // 64 bytes of every row a step
+    v4f acc[TA][4];
+#pragma unroll
+    for (int i = 0; i < TA; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
+    constexpr int C = TA == 4 ? 2 : 4;   // steps of loads together, and as many under way
+    uint4 a[2][C][TA], b[2][C][4];
+    auto fetch = [&](int st, int buf) {
+#pragma unroll
+        for (int q = 0; q < C; ++q) {
+            const int64_t at = int64_t(min(st + q, s1 - 1)) * 64;
+#pragma unroll
+            for (int i = 0; i < TA; ++i) a[buf][q][i] = *reinterpret_cast<const uint4 *>(ap[i] + at);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b[buf][q][j] = *reinterpret_cast<const uint4 *>(bp[j] + at);
         }
-        if (last && tid < 32) x_st = in && shared ? *reinterpret_cast<const uint4 *>(shared + k0 + 8 * sp) : make_uint4(0, 0, 0, 0);
     };
-    auto stage = [&]() {
+    auto multiply = [&](int st, int buf) {
 #pragma unroll
-        for (int i = 0; i < SR; ++i) {
-            *reinterpret_cast<uint4 *>(&As[sr + 8 * KS * i][8 * sp]) = a_st[i];
-            *reinterpret_cast<uint4 *>(&Bs[sr + 8 * KS * i][8 * sp]) = b_st[i];
-        }
-        if (last && tid < 32) *reinterpret_cast<uint4 *>(&Bs[kRgRows][8 * sp]) = x_st;
-    };
-    v16f acc, accx, acc1, acc2, acc3;   // the last three: fp32 rows only
+        for (int q = 0; q < C; ++q) {
+            if (st + q >= s1) break;
 #pragma unroll
-    for (int q = 0; q < 16; ++q) acc[q] = accx[q] = acc1[q] = acc2[q] = acc3[q] = 0.f;
-    fetch(0);
-    for (int k0 = 0; k0 < h; k0 += kRgK) {
-        __syncthreads();          // the previous stage has been multiplied
-        stage();
-        __syncthreads();
-        if (k0 + kRgK < h) fetch(k0 + kRgK);
-        const int steps = min(kRgK, h - k0) / 16;
-        auto step = [&](int j) {  // operand of lane (r, g): row r, the 16 bytes at halves 16 j + 8 g
-            if constexpr (F32) {  // four fp32 columns a lane: four instructions of two columns each, lane half g's s-th with the other half's s-th
-                const float4 a = *reinterpret_cast<const float4 *>(&As[mq * 32 + r][16 * j + 8 * g]);
-                const float4 b = *reinterpret_cast<const float4 *>(&Bs[nq * 32 + r][16 * j + 8 * g]);
-                // four running sums (joined at the end): a quarter of the terms each, and no instruction waits for the one before it
-                acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, b.x, acc, 0, 0, 0);
-                acc1 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, b.y, acc1, 0, 0, 0);
-                acc2 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, b.z, acc2, 0, 0, 0);
-                acc3 = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, b.w, acc3, 0, 0, 0);
-                if (extra) {
-                    const float4 bx = *reinterpret_cast<const float4 *>(&Bs[kRgRows][16 * j + 8 * g]);
-                    accx = __builtin_amdgcn_mfma_f32_32x32x2f32(a.x, bx.x, accx, 0, 0, 0);
-                    accx = __builtin_amdgcn_mfma_f32_32x32x2f32(a.y, bx.y, accx, 0, 0, 0);
-                    accx = __builtin_amdgcn_mfma_f32_32x32x2f32(a.z, bx.z, accx, 0, 0, 0);
-                    accx = __builtin_amdgcn_mfma_f32_32x32x2f32(a.w, bx.w, accx, 0, 0, 0);
+            for (int i = 0; i < TA; ++i)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if constexpr (F32) {   // lane group g's four columns with the other groups' four, one of each a time
+                        const v4f av = __builtin_bit_cast(v4f, a[buf][q][i]), bv = __builtin_bit_cast(v4f, b[buf][q][j]);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[c], bv[c], acc[i][j], 0, 0, 0);
+                    } else {
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a[buf][q][i]), __builtin_bit_cast(v8bf, b[buf][q][j]), acc[i][j], 0, 0, 0);
+                    }
                 }
-            } else {
-                const v8bf a = *reinterpret_cast<const v8bf *>(&As[mq * 32 + r][16 * j + 8 * g]);
-                const v8bf b = *reinterpret_cast<const v8bf *>(&Bs[nq * 32 + r][16 * j + 8 * g]);
-                acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
-                if (extra) {      // every column of this product is row e: lane r = 0 keeps it
-                    const v8bf bx = *reinterpret_cast<const v8bf *>(&Bs[kRgRows][16 * j + 8 * g]);
-                    accx = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, bx, accx, 0, 0, 0);
+        }
+    };
+    if (s0 < s1) {
+        fetch(s0, 0);
+        for (int st = s0; st < s1; st += 2 * C) {
+            if (st + C < s1) fetch(st + C, 1);
+            multiply(st, 0);
+            if (st + C >= s1) break;
+            if (st + 2 * C < s1) fetch(st + 2 * C, 0);
+            multiply(st + C, 1);
+        }
+    }
+    // result register q of lane group g: token 4 g + q of the 16, router row r
+    auto at = [&](int slot, int i, int q) { return (slot * TT + 16 * i + 4 * g + q) * kRgPitch + r; };
+    if (wave >= 4) {
+#pragma unroll
+        for (int i = 0; i < TA; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) red[at(wave - 4, i, q) + 16 * j] = acc[i][j][q];
+    }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+        for (int i = 0; i < TA; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) red[at(wave, i, q) + 16 * j] += acc[i][j][q];
+    }
+    __syncthreads();
+    for (int i = tid; i < TT * kRgRows; i += 64 * kRgWaves) {
+        const int t = i / kRgRows, c = i % kRgRows;
+        const float * p = red + t * kRgPitch + c;
+        const float v = (p[0] + p[TT * kRgPitch]) + (p[2 * TT * kRgPitch] + p[3 * TT * kRgPitch]);
+        if (t0 + t < n && r0 + c < e) logits[int64_t(t0 + t) * (e + 1) + r0 + c] = v;
+    }
+}
+// The same for large batches of bf16 rows: 64 tokens x 128 router rows a block, operands through LDS, so that a row of x is
+// read by a quarter of the blocks. 128 bytes of every row a stage, from memory to LDS without registers, two stages under
+// way, two blocks a compute unit. The eight parts of the columns follow each other and join in the order the kernel above adds them: same bits.
+// (512 experts, 2048 columns, 4096 tokens: 24 us; 45 with every wave's operands from memory, 32 with stages of 512 bytes a
+// row that pass registers.)
+// Blocks from which it is the faster one (in us, this / operands from memory: 96 blocks 19 / 27, 64 blocks 15 / 22, 24 blocks
+// 19 / 12).
+constexpr int kRlBlocks = 48;
+constexpr int kRlFull = 224;    // blocks from which none are added for the gate row's column (256: 24 us against 33; 126: 26 against 20)
+constexpr int kRlTok = 64, kRlRows = 128, kRlRing = 3, kRlStage = (kRlTok + kRlRows) * 128, kRlLds = kRlRing * kRlStage, kRlWaves = 8;
+__global__ __launch_bounds__(64 * kRlWaves) void router_gemm_lds_k(const uint8_t * __restrict__ w, const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x,
+                                                         float * __restrict__ logits, int h, int e, int n, RouterSide side) {
+    constexpr int NQ = (kRlTok + kRlRows) / 8 / kRlWaves;
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    const int t0 = int(blockIdx.x) * kRlTok, r0 = int(blockIdx.y) * kRlRows;
+    const int64_t pitch = int64_t(h) * 2;
+    // The gate row's column: a last row of blocks where they find compute units free, else every block's share of its tokens.
+    const int cols = (e + kRlRows - 1) / kRlRows;
+    if (int(blockIdx.y) == cols) {
+        router_shared_column<TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + kRlTok, n), side, kRlWaves);
+        return;
+    }
+    // transfer q of a wave is eight rows of a stage: the tokens' rows, then the router's; a row's 16-byte piece p in slot
+    // p ^ (row / 2 & 7)
+    const uint8_t * src[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int row = (NQ * wave + q) * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+        src[q] = (row < kRlTok ? x + int64_t(min(t0 + row, n - 1)) * pitch : w + int64_t(min(r0 + row - kRlTok, e - 1)) * pitch) + piece * 16;
+    }
+    const uint32_t lds0 = lds_address(lds);
+    const int steps = int(pitch / 64);
+    auto part_of = [&](int k) { return (k & 1) * 4 + (k >> 1); };          // parts 0, 4, 1, 5, 2, 6, 3, 7
+    auto first = [&](int k) { return part_of(k) * steps / kRgWaves; };
+    auto last = [&](int k) { return (part_of(k) + 1) * steps / kRgWaves; };
+    int sk = 0, ss = first(0), slot_in = 0;                                // the next stage to send
+    while (sk < 8 && ss >= last(sk)) { ++sk; ss = sk < 8 ? first(sk) : 0; }
+    auto send = [&]() {
+        if (sk < 8) {
+            const int64_t at = min(int64_t(ss) * 64, pitch - 128);        // (a part's odd last step: half a stage is not used)
+#pragma unroll
+            for (int q = 0; q < NQ; ++q) dma16(src[q] + at, lds0 + slot_in * kRlStage + (NQ * wave + q) * 1024);
+            ss += 2;
+            while (sk < 8 && ss >= last(sk)) { ++sk; ss = sk < 8 ? first(sk) : 0; }
+        }
+        slot_in = slot_in + 1 == kRlRing ? 0 : slot_in + 1;
+    };
+    int total = 0;
+    for (int k = 0; k < 8; ++k) total += (last(k) - first(k) + 1) / 2;
+#pragma unroll
+    for (int i = 0; i < kRlRing - 1; ++i) send();
+    if (int(gridDim.y) == cols) {   // (under the first transfers)
+        const int share = (kRlTok + cols - 1) / cols, first_t = t0 + int(blockIdx.y) * share;
+        router_shared_column<TQMOE_BF16>(shared, x, logits, h, e, n, first_t, min(min(first_t + share, t0 + kRlTok), n), side, kRlWaves);
+    }
+    const int tq = wave & 1, rq = wave >> 1;
+    const uint8_t * a_row = lds + (tq * 32 + r) * 128, * b_row = lds + (kRlTok + rq * 32 + r) * 128;
+    const v4f zero = {0.f, 0.f, 0.f, 0.f};
+    v4f acc[2][2], pair[2][2], half[2][2], sum[2][2];
+    int slot = 0, done = 0;
+    for (int k = 0; k < 8; ++k) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[i][j] = zero;
+        for (int st = first(k); st < last(k); st += 2) {
+            if (done + kRlRing - 1 <= total) dma_wait<NQ * (kRlRing - 2), true>(); else dma_wait<0, true>();
+            send();
+            const int skip = int64_t(st) * 64 > pitch - 128 ? 1 : 0;      // the step is the stage's second half
+            const uint8_t * as = a_row + slot * kRlStage, * bs = b_row + slot * kRlStage;
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (q == 1 && st + 1 >= last(k)) break;
+                const int piece = (4 * (q + skip) + g) ^ ((r >> 1) & 7);   // (rows 16 further on have the same low bits)
+                v8bf a[2], b[2];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) {
+                    a[i] = *reinterpret_cast<const v8bf *>(as + i * 2048 + piece * 16);
+                    b[i] = *reinterpret_cast<const v8bf *>(bs + i * 2048 + piece * 16);
+                }
+#pragma unroll
+                for (int i = 0; i < 2; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+            }
+            slot = slot + 1 == kRlRing ? 0 : slot + 1;
+            ++done;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                if ((k & 1) == 0) pair[i][j] = acc[i][j];
+                else {
+                    pair[i][j] += acc[i][j];
+                    if (k == 1 || k == 5) half[i][j] = pair[i][j];
+                    else if (k == 3) sum[i][j] = half[i][j] + pair[i][j];
+                    else sum[i][j] = sum[i][j] + (half[i][j] + pair[i][j]);
                 }
             }
-        };
-        if (steps == kRgK / 16) {
-#pragma unroll
-            for (int j = 0; j < kRgK / 16 / KS; ++j) step(kh * (kRgK / 16 / KS) + j);
-        } else {
-            const int per = (steps + KS - 1) / KS;
-            for (int j = kh * per; j < min(steps, (kh + 1) * per); ++j) step(j);
-        }
     }
-    if constexpr (F32) {
 #pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] = (acc[q] + acc1[q]) + (acc2[q] + acc3[q]);
-    }
-    if constexpr (KS == 2) {   // the second part's sums to the first part's waves, through the space of the row tiles
-        __syncthreads();       // the last stage has been multiplied
-        float * ex = reinterpret_cast<float *>(&As[0][0]);   // [quadrant][17 registers][64 lanes] floats: 17.4 KB of As's 33.8 KB
-        static_assert(sizeof(As) >= 4 * 17 * 64 * sizeof(float), "exchange space");
-        if (kh == 1) {
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int q = 0; q < 16; ++q) ex[((wave & 3) * 17 + q) * 64 + lane] = acc[q];
-            if (extra) {
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int q = 0; q < 16; ++q) if (r == 0) ex[((wave & 3) * 17 + 16) * 64 + 16 * g + q] = accx[q];
+            for (int q = 0; q < 4; ++q) {
+                const int t = t0 + tq * 32 + 16 * i + 4 * g + q, c = r0 + rq * 32 + 16 * j + r;
+                if (t < n && c < e) logits[int64_t(t) * (e + 1) + c] = sum[i][j][q];
             }
-        }
-        __syncthreads();
-        if (kh == 1) return;
-#pragma unroll
-        for (int q = 0; q < 16; ++q) acc[q] += ex[((wave & 3) * 17 + q) * 64 + lane];
-        if (extra && r == 0) {
-#pragma unroll
-            for (int q = 0; q < 16; ++q) accx[q] += ex[((wave & 3) * 17 + 16) * 64 + 16 * g + q];
+}
+template <bool F32> void launch_router_gemm(const void * w, const void * sg, const void * x, float * logits, int h, int e, int n, const RouterSide & side, hipStream_t s) {
+    const int64_t rows = (e + kRgRows - 1) / kRgRows;
+    auto blocks = [&](int ta) { return ((n + 16 * ta - 1) / (16 * ta)) * rows; };
+    auto go = [&](auto kernel, int ta, int lds) {
+        allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds);
+        kernel<<<dim3(unsigned((n + 16 * ta - 1) / (16 * ta)), unsigned(rows + 1)), 64 * kRgWaves, lds, s>>>(
+            static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, side);
+    };
+    if constexpr (!F32) {
+        const int64_t tiles = (n + kRlTok - 1) / kRlTok, cols = (e + kRlRows - 1) / kRlRows;
+        if (tiles * cols >= kRlBlocks && h >= 512) {
+            allow_dynamic_lds(reinterpret_cast<const void *>(&router_gemm_lds_k), kRlLds);
+            router_gemm_lds_k<<<dim3(unsigned(tiles), unsigned(cols + (tiles * cols < kRlFull ? 1 : 0))), 64 * kRlWaves, kRlLds, s>>>(
+                static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, side);
+            return;
         }
     }
-    // result register q of lane half g: token row 8 (q / 4) + 4 g + q % 4 of the 32-row tile, router row r
-    const int row = r0 + nq * 32 + r;
-#pragma unroll
-    for (int q = 0; q < 16; ++q) {
-        const int t = t0 + mq * 32 + 8 * (q >> 2) + 4 * g + (q & 3);
-        if (t >= n) continue;
-        if (row < e) logits[int64_t(t) * (e + 1) + row] = acc[q];
-        if (extra && r == 0) logits[int64_t(t) * (e + 1) + e] = accx[q];
-    }
+    if (blocks(4) >= 384) go(&router_gemm_k<F32, 4>, 4, kRgLds<4>);
+    else if (blocks(2) >= 256) go(&router_gemm_k<F32, 2>, 2, kRgLds<2>);
+    else go(&router_gemm_k<F32, 1>, 1, kRgLds<1>);
 }
 
 // ------------------------------------------------------------------------------------------------------ top-k
@@ -259,9 +387,8 @@ __global__ __launch_bounds__(256 * KS) void router_gemm_k(const uint16_t * __res
 struct TopkOut {
     int * ids; float * weights; float * shared_weights;
     int * ext_ids; int extra;          // optional [n][k + 1] copy of the ids with `extra` in the last slot
-    const void * x; uint8_t * image;   // optional: the token's input row is written as an activation image row
-    int cols;
     int shared_ungated;                // the shared expert has no gate row: its weight is 1, not sigmoid(0)
+    TopkSide side;
 };
 __device__ __forceinline__ float shared_weight_of(const TopkOut & o, float logit) { return o.shared_ungated ? 1.f : 1.f / (1.f + expf(-logit)); }
 
@@ -278,18 +405,32 @@ __device__ __forceinline__ void topk_finish(const TopkOut & o, const float * x_l
     }
 }
 
-template <int XT> __device__ __forceinline__ void topk_quantise_row(const TopkOut & o, int token, int lane) {
-    quantise_row_wave<XT>(o.x, token, o.cols, o.image + int64_t(token) * (o.cols / 32) * kImageSubBytes, lane);
+// the token's input row in the form the products read
+template <int XT> __device__ __forceinline__ void topk_row(const TopkOut & o, int token, int lane) {
+    const TopkSide & d = o.side;
+    switch (d.rows) {
+        case kRowsImage: quantise_row_wave<XT>(d.x, token, d.cols, static_cast<uint8_t *>(d.q) + int64_t(token) * (d.cols / 32) * kImageSubBytes, lane); break;
+        case kRowsHalves: prepare_row_wave<XT>(d.x, token, d.cols, static_cast<uint16_t *>(d.q), d.scale, lane); break;
+        case kRowsFp8: quant_row_wave<XT, true, false>(d.x, token, d.cols, static_cast<int8_t *>(d.q), d.scale, nullptr, lane); break;
+        case kRowsInt8: quant_row_wave<XT, false, false>(d.x, token, d.cols, static_cast<int8_t *>(d.q), d.scale, nullptr, lane); break;
+        case kRowsInt8Blocks: quant_row_wave<XT, false, true>(d.x, token, d.cols, static_cast<int8_t *>(d.q), d.scale, nullptr, lane); break;
+    }
+}
+// selection s of the token is expert id (s = k: the shared one): one more assignment of it in the dispatch chunk
+__device__ __forceinline__ void topk_count(const TopkOut & o, int token, int k, int s, int id) {
+    if (!o.side.chunk_counts) return;
+    const int64_t a = int64_t(token) * (o.ext_ids ? k + 1 : k) + s;
+    atomicAdd(o.side.chunk_counts + a / kDispatchChunk * o.side.banks + id, 1);
 }
 
-// With an activation image to write the block has a second wave that does nothing else: the row's quantisation runs beside
-// the selection instead of after it.
+// With rows to write the block has a second wave that does nothing else: the row's quantisation runs beside the selection
+// instead of after it.
 template <int R, int XT>
 __device__ __forceinline__ void topk_reg_body(const float * __restrict__ logits, const TopkOut & o, int e, int k, float scale) {
     const int token = blockIdx.x, lane = threadIdx.x & 63;
     const float * x = logits + int64_t(token) * (e + 1);
     if (threadIdx.x >= 64) {
-        topk_quantise_row<XT>(o, token, lane);
+        topk_row<XT>(o, token, lane);
         return;
     }
     const float shared_logit = o.shared_weights ? x[e] : 0.f;
@@ -302,10 +443,11 @@ __device__ __forceinline__ void topk_reg_body(const float * __restrict__ logits,
             o.ids[int64_t(token) * k + lane] = my_id;
             o.weights[int64_t(token) * k + lane] = v;
             if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + lane] = my_id;
+            topk_count(o, token, k, lane, my_id);
         }
         if (lane == 0) {
             if (o.shared_weights) o.shared_weights[token] = shared_weight_of(o, shared_logit);
-            if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + k] = o.extra;
+            if (o.ext_ids) { o.ext_ids[int64_t(token) * (k + 1) + k] = o.extra; topk_count(o, token, k, k, o.extra); }
         }
         return;
     }
@@ -394,15 +536,15 @@ __global__ __launch_bounds__(64) void topk_lds_k(const float * __restrict__ logi
         if ((best & 63) == lane) keys[best] = kKeyGone;
     }
     topk_finish(o, x, token, lane, e, k, scale, selected);
-    if (o.image) topk_quantise_row<XT>(o, token, lane);
+    if (o.side.rows) topk_row<XT>(o, token, lane);
 }
 
 template <int XT> void launch_topk(const float * logits, const TopkOut & o, int e, int k, int n, float scale, hipStream_t s) {
-    if (e <= 64) topk_reg_k<1, XT><<<unsigned(n), o.image ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
-    else if (e <= 128) topk_reg_k<2, XT><<<unsigned(n), o.image ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
-    else if (e <= 256) topk_reg_k<4, XT><<<unsigned(n), o.image ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
-    else if (e <= 512) topk_reg_k<8, XT><<<unsigned(n), o.image ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
-    else if (e <= 1024) topk_reg_k<16, XT><<<unsigned(n), o.image ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
+    if (e <= 64) topk_reg_k<1, XT><<<unsigned(n), o.side.rows ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
+    else if (e <= 128) topk_reg_k<2, XT><<<unsigned(n), o.side.rows ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
+    else if (e <= 256) topk_reg_k<4, XT><<<unsigned(n), o.side.rows ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
+    else if (e <= 512) topk_reg_k<8, XT><<<unsigned(n), o.side.rows ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
+    else if (e <= 1024) topk_reg_k<16, XT><<<unsigned(n), o.side.rows ? 128 : 64, 0, s>>>(logits, o, e, k, scale);
     else topk_lds_k<XT><<<unsigned(n), 64, size_t(e) * sizeof(float), s>>>(logits, o, e, k, scale);
 }
 
@@ -513,6 +655,7 @@ __global__ __launch_bounds__(64) void topk_gated_k(const float * __restrict__ lo
             o.ids[int64_t(token) * k + lane] = my_id;
             o.weights[int64_t(token) * k + lane] = my_w;
             if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + lane] = my_id;
+            topk_count(o, token, k, lane, my_id);
         }
     } else {
         const int done = k & ~63;             // the last partial set
@@ -526,9 +669,9 @@ __global__ __launch_bounds__(64) void topk_gated_k(const float * __restrict__ lo
     }
     if (lane == 0) {
         if (o.shared_weights) o.shared_weights[token] = shared_weight_of(o, shared_logit);
-        if (o.ext_ids) o.ext_ids[int64_t(token) * (k + 1) + k] = o.extra;
+        if (o.ext_ids) { o.ext_ids[int64_t(token) * (k + 1) + k] = o.extra; topk_count(o, token, k, k, o.extra); }
     }
-    if (o.image) topk_quantise_row<XT>(o, token, lane);
+    if (o.side.rows) topk_row<XT>(o, token, lane);
 }
 
 template <int XT> void launch_topk_gated(const float * logits, const TopkOut & o, const Gate & g, int e, int k, int n, float scale, hipStream_t s) {
@@ -546,7 +689,7 @@ template <int XT> void launch_topk_gated(const float * logits, const TopkOut & o
 // places every assignment at offsets[e] + prefix[chunk][e] + its rank among the chunk's earlier assignments of the
 // same expert. Ranks come from ballots (lower lanes of the same expert) and a per-expert running count in LDS that
 // waves add to in wave order, so no ordering is left to atomics. A single chunk runs all three passes in one block.
-constexpr int kChunk = 1024;
+constexpr int kChunk = kDispatchChunk;
 
 __device__ __forceinline__ void zero_lds(int * a, int n) {
     for (int j = threadIdx.x; j < n; j += blockDim.x) a[j] = 0;
@@ -648,65 +791,67 @@ __global__ __launch_bounds__(256) void dispatch_place_k(const int * __restrict__
 }
 
 // Pass 2 and 3 in one launch for up to kWideExperts experts: a block of sixteen waves takes a chunk, one wave per 64
-// consecutive assignments. Every block sums the per-chunk counts itself (the chunks before it: where its assignments
-// start inside each expert; all chunks: the experts' offsets), the waves rank their assignments with ballots all at
-// once and leave their group sizes in a per-wave histogram, and a prefix over the waves in index order gives every
-// assignment its place. Nothing is left to the order of atomics.
-constexpr int kWideExperts = 1024, kWideWaves = kChunk / 64;
+// consecutive assignments, and thread j keeps expert j's sums. Every block adds up the per-chunk counts itself (the chunks
+// before it: where its assignments start inside each expert; all chunks: the experts' offsets); a wave finds each lane's equals
+// with a ballot per bit of the expert's number (a loop over the distinct experts of a wave's 64 assignments is 64 rounds at
+// worst), leaves its group sizes in a histogram of its own, and a prefix over the waves in index order gives every
+// assignment its place. Nothing is left to the order of atomics. The first block plans the products' items on the side.
+constexpr int kWideExperts = kDispatchWide, kWideWaves = kChunk / 64;
 
 __global__ __launch_bounds__(1024) void dispatch_place_wide_k(const int * __restrict__ ids, const int * __restrict__ chunk_counts, int * __restrict__ counts,
                                                               int * __restrict__ offsets, int * __restrict__ perm, int * __restrict__ groups, int capacity,
-                                                              int A, int E, int chunks) {
-    extern __shared__ int sm[];   // start E + 1 | total E | scratch 1024 | hist kWideWaves x E
-    int * start = sm, * total = sm + E + 1, * scratch = total + E, * hist = scratch + 1024;
+                                                              int A, int E, int chunks, DispatchSide side) {
+    extern __shared__ int hist[];   // kWideWaves x E: group sizes, then each wave's first place
+    __shared__ int s_start[kWideExperts], s_all[kWideExperts], s_wave[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, chunk = blockIdx.x;
-    for (int j = tid; j < E; j += 1024) {
-        int before = 0, all = 0;
-        for (int b0 = 0; b0 < chunks; b0 += 16) {   // sixteen loads in flight: the loop is latency, not bandwidth
-            int v[16];
-#pragma unroll
-            for (int q = 0; q < 16; ++q) v[q] = b0 + q < chunks ? chunk_counts[int64_t(b0 + q) * E + j] : 0;
-#pragma unroll
-            for (int q = 0; q < 16; ++q) { all += v[q]; before += b0 + q < chunk ? v[q] : 0; }
-        }
-        total[j] = all;
-        hist[j] = before;          // parked here until the offsets are known
-    }
-    for (int j = tid; j < kWideWaves * E; j += 1024) if (j >= E) hist[j] = 0;
-    __syncthreads();
-    // the assignment's rank among the wave's earlier lanes of the same expert, and the size of its group
     const int a = chunk * kChunk + tid;
     int e = a < A ? ids[a] : -1;
     if (e >= E) e = -1;
-    int rank = 0, size = 0;
-    bool last = false;
-    unsigned long long todo = __ballot(e >= 0);
-    while (todo) {
-        const int leader = __ffsll(todo) - 1;
-        const int v = __shfl(e, leader, 64);
-        const unsigned long long same = __ballot(e == v);
-        if (e == v) {
-            rank = __popcll(same & ((1ull << lane) - 1ull));
-            size = __popcll(same);
-            last = (63 - __clzll(same)) == lane;
+    int before = 0, all = 0;
+    if (tid < E)
+        for (int b0 = 0; b0 < chunks; b0 += 16) {   // sixteen loads in flight: the loop is latency, not bandwidth
+            int v[16];
+#pragma unroll
+            for (int q = 0; q < 16; ++q) v[q] = b0 + q < chunks ? chunk_counts[int64_t(b0 + q) * E + tid] : 0;
+#pragma unroll
+            for (int q = 0; q < 16; ++q) { all += v[q]; before += b0 + q < chunk ? v[q] : 0; }
         }
-        todo &= ~same;
+    for (int j = tid; j < kWideWaves * E; j += 1024) hist[j] = 0;
+    // the experts' first places: a prefix sum over the threads
+    int incl = all;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) { const int u = __shfl_up(incl, d, 64); if (lane >= d) incl += u; }
+    if (lane == 63) s_wave[wave] = incl;
+    // the lanes of this wave with the same expert
+    unsigned long long same = __ballot(e >= 0);
+    for (int bit = 0; (1 << bit) < E; ++bit) {
+        const unsigned long long m = __ballot((e >> bit) & 1);
+        same &= ((e >> bit) & 1) ? m : ~m;
     }
-    const int before_e = e >= 0 ? hist[e] : 0;   // row 0 of hist still holds the chunks before this one
+    const int rank = __popcll(same & ((1ull << lane) - 1ull)), size = __popcll(same);
     __syncthreads();
-    for (int j = tid; j < E; j += 1024) hist[j] = 0;
-    block_exclusive_scan(total, start, E, scratch);   // ends with a barrier
-    if (e >= 0 && last) hist[wave * E + e] = size;
+    int start = incl - all;
+    for (int w = 0; w < wave; ++w) start += s_wave[w];
+    if (e >= 0 && rank == size - 1) hist[wave * E + e] = size;
+    if (tid < E) { s_start[tid] = start; s_all[tid] = all; }
+    __syncthreads();
+    if (tid < E) {
+        int v[kWideWaves], at = start + before;
+#pragma unroll
+        for (int w = 0; w < kWideWaves; ++w) v[w] = hist[w * E + tid];
+#pragma unroll
+        for (int w = 0; w < kWideWaves; ++w) { hist[w * E + tid] = at; at += v[w]; }
+    }
     __syncthreads();
     if (e >= 0) {
-        int slot = before_e + rank;
-        for (int w = 0; w < wave; ++w) slot += hist[w * E + e];
-        if (perm) perm[start[e] + slot] = a;
+        const int place = hist[wave * E + e] + rank, slot = place - s_start[e];
+        if (perm) perm[place] = a;
         if (groups && slot < capacity) groups[int64_t(e) * capacity + slot] = a;
     }
     if (chunk == 0) {
-        for (int j = tid; j < E; j += 1024) { counts[j] = total[j]; if (offsets) offsets[j] = start[j]; }
-        if (tid == 0 && offsets) offsets[E] = start[E];
+        if (tid < E) { counts[tid] = all; if (offsets) offsets[tid] = start; }
+        if (tid == E - 1 && offsets) offsets[E] = start + all;
+        if (side.item_rows) plan_items(s_all, s_start, E, side.item_rows, side.items, side.index);
     }
 }
 
@@ -742,43 +887,25 @@ extern "C" int32_t tqmoe_router(const void * router, uint32_t wtype, const void 
     if ((wtype != TQMOE_F32 && wtype != TQMOE_BF16) || !is_act_type(xtype)) return fail(err, TQMOE_E_UNSUPPORTED, "tqmoe_router: unsupported element type");
     if ((n + kRouterTok - 1) / kRouterTok > 65535) return fail(err, TQMOE_E_ARG, "tqmoe_router: too many tokens for one call");
     if (int32_t rc = need_device(err, "tqmoe_router")) return rc;
-    const hipStream_t s = static_cast<hipStream_t>(stream);
-    if (wtype == xtype && (wtype == TQMOE_BF16 || wtype == TQMOE_F32) && int64_t(n) * (experts + 1) >= kRouterGemmMin && hidden % 64 == 0) {
-        const dim3 grid(unsigned((n + kRgTok - 1) / kRgTok), unsigned((experts + kRgRows - 1) / kRgRows));
-        const uint16_t * w16 = static_cast<const uint16_t *>(router), * s16 = static_cast<const uint16_t *>(shared_gate), * x16 = static_cast<const uint16_t *>(x);
-        // a layer of few experts has few blocks: eight waves a block then, the steps of every stage split between two sets
-        // of four (decided by the router rows alone, so that a token's logits do not depend on the batch around it)
-        const bool split = grid.y <= 2;
-        if (wtype == TQMOE_F32) {
-            if (split) router_gemm_k<true, 2><<<grid, 512, 0, s>>>(w16, s16, x16, logits, 2 * hidden, experts, n);
-            else router_gemm_k<true><<<grid, 256, 0, s>>>(w16, s16, x16, logits, 2 * hidden, experts, n);
-        } else {
-            if (split) router_gemm_k<false, 2><<<grid, 512, 0, s>>>(w16, s16, x16, logits, hidden, experts, n);
-            else router_gemm_k<false><<<grid, 256, 0, s>>>(w16, s16, x16, logits, hidden, experts, n);
-        }
-        return launched(err, "tqmoe_router");
-    }
-    if (wtype == TQMOE_F32) launch_router_x<TQMOE_F32>(xtype, router, shared_gate, x, logits, hidden, experts, n, s);
-    else launch_router_x<TQMOE_BF16>(xtype, router, shared_gate, x, logits, hidden, experts, n, s);
+    return enqueue_router(router, wtype, shared_gate, x, xtype, logits, hidden, experts, n, RouterSide{}, static_cast<hipStream_t>(stream), err);
+}
+
+int32_t tqmoe::enqueue_router(const void * router, uint32_t wtype, const void * shared_gate, const void * x, uint32_t xtype, float * logits, int hidden, int experts, int n,
+                              const RouterSide & side, hipStream_t s, tqmoe_error * err) {
+    if (wtype == xtype && (wtype == TQMOE_BF16 || wtype == TQMOE_F32) && int64_t(n) * (experts + 1) >= kRouterGemmMin && hidden % 64 == 0 && !side.image) {
+        if (wtype == TQMOE_F32) launch_router_gemm<true>(router, shared_gate, x, logits, hidden, experts, n, side, s);
+        else launch_router_gemm<false>(router, shared_gate, x, logits, hidden, experts, n, side, s);
+    } else if (wtype == TQMOE_F32) launch_router_x<TQMOE_F32>(xtype, router, shared_gate, x, logits, hidden, experts, n, side, s);
+    else launch_router_x<TQMOE_BF16>(xtype, router, shared_gate, x, logits, hidden, experts, n, side, s);
     return launched(err, "tqmoe_router");
 }
 
-// router logits and activation images of up to kRouterFew tokens in one launch
-namespace tqmoe {
-void enqueue_router_image(const void * router, uint32_t wtype, const void * shared_gate, const void * x, uint32_t xtype, float * logits, int hidden, int experts,
-                          int n, void * image, hipStream_t s) {
-    if (wtype == TQMOE_F32) launch_router_x<TQMOE_F32>(xtype, router, shared_gate, x, logits, hidden, experts, n, s, static_cast<uint8_t *>(image));
-    else launch_router_x<TQMOE_BF16>(xtype, router, shared_gate, x, logits, hidden, experts, n, s, static_cast<uint8_t *>(image));
-}
-}  // namespace tqmoe
-
 // top-k with the optional extras of the whole-layer path: extended ids and the input rows' activation image
 namespace tqmoe {
-int32_t enqueue_topk(const float * logits, int32_t * ids, float * weights, float * shared_weights, int32_t * ext_ids, int32_t extra, const void * x,
-                     uint32_t xtype, int32_t cols, void * image, int32_t experts, int32_t topk, int32_t n, float scale, int32_t gating,
-                     const float * bias, int32_t norm, hipStream_t s, int32_t shared_ungated) {
-    const TopkOut o{ids, weights, shared_weights, ext_ids, extra, x, static_cast<uint8_t *>(image), cols, shared_ungated};
-    const uint32_t xt = image ? xtype : uint32_t(TQMOE_F32);
+int32_t enqueue_topk(const float * logits, int32_t * ids, float * weights, float * shared_weights, int32_t * ext_ids, int32_t extra, int32_t experts, int32_t topk, int32_t n,
+                     float scale, int32_t gating, const float * bias, int32_t norm, int32_t shared_ungated, const TopkSide & side, hipStream_t s) {
+    const TopkOut o{ids, weights, shared_weights, ext_ids, extra, shared_ungated, side};
+    const uint32_t xt = side.rows ? side.xtype : uint32_t(TQMOE_F32);
     if (gating == TQMOE_GATE_SOFTMAX && !bias && norm) {   // the common case has its own kernel
         switch (xt) {
             case TQMOE_F32: launch_topk<TQMOE_F32>(logits, o, experts, topk, n, scale, s); break;
@@ -802,8 +929,7 @@ extern "C" int32_t tqmoe_topk(const float * logits, int32_t * ids, float * weigh
     if (!logits || !ids || !weights || experts <= 0 || experts > 4096 || topk <= 0 || topk > experts || n <= 0)
         return fail(err, TQMOE_E_ARG, "tqmoe_topk: invalid shape or pointer");
     if (int32_t rc = need_device(err, "tqmoe_topk")) return rc;
-    enqueue_topk(logits, ids, weights, shared_weights, nullptr, 0, nullptr, TQMOE_F32, 0, nullptr, experts, topk, n, scale, TQMOE_GATE_SOFTMAX, nullptr, 1,
-                 static_cast<hipStream_t>(stream), 0);
+    enqueue_topk(logits, ids, weights, shared_weights, nullptr, 0, experts, topk, n, scale, TQMOE_GATE_SOFTMAX, nullptr, 1, 0, TopkSide{}, static_cast<hipStream_t>(stream));
     return launched(err, "tqmoe_topk");
 }
 
@@ -815,7 +941,7 @@ extern "C" int32_t tqmoe_topk2(const float * logits, int32_t * ids, float * weig
     if (!logits || !ids || !weights || !logits2 || !ids2 || !weights2 || experts <= 0 || experts > 1024 || topk <= 0 || topk > experts || n <= 0)
         return fail(err, TQMOE_E_ARG, "tqmoe_topk2: invalid shape or pointer (at most 1024 experts)");
     if (int32_t rc = need_device(err, "tqmoe_topk2")) return rc;
-    const TopkOut o{ids, weights, shared_weights, nullptr, 0, nullptr, nullptr, 0, 0}, o2{ids2, weights2, shared_weights2, nullptr, 0, nullptr, nullptr, 0, 0};
+    const TopkOut o{ids, weights, shared_weights, nullptr, 0, 0, TopkSide{}}, o2{ids2, weights2, shared_weights2, nullptr, 0, 0, TopkSide{}};
     const dim3 grid(unsigned(n), 2);
     const hipStream_t s = static_cast<hipStream_t>(stream);
     if (experts <= 64) topk2_reg_k<1><<<grid, 64, 0, s>>>(logits, o, logits2, o2, experts, topk, scale);
@@ -832,8 +958,8 @@ extern "C" int32_t tqmoe_topk_gated(const float * logits, const float * probs_bi
         return fail(err, TQMOE_E_ARG, "tqmoe_topk_gated: invalid shape or pointer");
     if (gating < TQMOE_GATE_SOFTMAX || gating > TQMOE_GATE_SQRT_SOFTPLUS) return fail(err, TQMOE_E_UNSUPPORTED, "tqmoe_topk_gated: unsupported gating function %d", gating);
     if (int32_t rc = need_device(err, "tqmoe_topk_gated")) return rc;
-    enqueue_topk(logits, ids, weights, shared_weights, nullptr, 0, nullptr, TQMOE_F32, 0, nullptr, experts, topk, n, scale, gating, probs_bias, norm_weights != 0,
-                 static_cast<hipStream_t>(stream), 0);
+    enqueue_topk(logits, ids, weights, shared_weights, nullptr, 0, experts, topk, n, scale, gating, probs_bias, norm_weights != 0, 0, TopkSide{},
+                 static_cast<hipStream_t>(stream));
     return launched(err, "tqmoe_topk_gated");
 }
 
@@ -853,6 +979,11 @@ static __device__ __align__(256) int scratch[kStaticInts + kStaticOffsets];
 
 namespace tqmoe {
 namespace {
+void place_wide(const int32_t * ids, const int * cc, int32_t * counts, int32_t * offsets, int32_t * perm, int32_t * groups, int32_t capacity, int32_t experts, int A,
+                int chunks, const DispatchSide & side, hipStream_t s) {
+    allow_dynamic_lds(reinterpret_cast<const void *>(&dispatch_place_wide_k), int(kWideWaves * kWideExperts * sizeof(int)));
+    dispatch_place_wide_k<<<unsigned(chunks), 1024, size_t(kWideWaves) * experts * sizeof(int), s>>>(ids, cc, counts, offsets, perm, groups, capacity, A, experts, chunks, side);
+}
 // the launches of tqmoe_dispatch; cc: chunks x experts ints of scratch for more than one chunk. offsets and perm may be
 // null where the caller only wants counts and groups (spare_offsets: experts + 1 ints the scan may use instead).
 int32_t enqueue_dispatch(const int32_t * ids, int32_t * counts, int32_t * offsets, int32_t * perm, int32_t * groups, int32_t capacity, int32_t experts,
@@ -863,9 +994,7 @@ int32_t enqueue_dispatch(const int32_t * ids, int32_t * counts, int32_t * offset
     }
     dispatch_count_k<<<unsigned(chunks), 256, size_t(experts) * sizeof(int), s>>>(ids, cc, A, experts);
     if (experts <= kWideExperts) {
-        const size_t lds = size_t(2 * experts + 1 + 1024 + kWideWaves * experts) * sizeof(int);
-        allow_dynamic_lds(reinterpret_cast<const void *>(&dispatch_place_wide_k), int((2 * kWideExperts + 1 + 1024 + kWideWaves * kWideExperts) * sizeof(int)));
-        dispatch_place_wide_k<<<unsigned(chunks), 1024, lds, s>>>(ids, cc, counts, offsets, perm, groups, capacity, A, experts, chunks);
+        place_wide(ids, cc, counts, offsets, perm, groups, capacity, experts, A, chunks, DispatchSide{}, s);
         return launched(err, what);
     }
     int32_t * offs = offsets ? offsets : spare_offsets;
@@ -949,6 +1078,19 @@ __global__ __launch_bounds__(1024) void dedup_maps_k(const int * __restrict__ id
     }
 }
 }  // namespace
+
+int32_t enqueue_layer_dispatch(const int32_t * ids, int32_t * counts, int32_t * offsets, int32_t * perm, int32_t experts, int32_t n, int32_t topk, int * chunk_counts,
+                               const DispatchSide & side, hipStream_t s, tqmoe_error * err) {
+    const int A = n * topk, chunks = (A + kChunk - 1) / kChunk;
+    if (experts <= kWideExperts && (side.counted || chunks > 1)) {
+        if (!side.counted) dispatch_count_k<<<unsigned(chunks), 256, size_t(experts) * sizeof(int), s>>>(ids, chunk_counts, A, experts);
+        place_wide(ids, chunk_counts, counts, offsets, perm, nullptr, 0, experts, A, chunks, side, s);
+        return launched(err, "tqmoe_layer_forward (dispatch)");
+    }
+    if (int32_t rc = enqueue_dispatch(ids, counts, offsets, perm, nullptr, 0, experts, A, chunks, chunk_counts, nullptr, s, err, "tqmoe_layer_forward (dispatch)")) return rc;
+    if (side.item_rows) enqueue_grouped_plan(counts, offsets, experts, side.item_rows, side.items, side.index, s);
+    return launched(err, "tqmoe_layer_forward (plan)");
+}
 }  // namespace tqmoe
 
 extern "C" int32_t tqmoe_dispatch(const int32_t * ids, int32_t * counts, int32_t * offsets, int32_t * perm, int32_t * groups,
