@@ -537,11 +537,15 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     // other's waits, and what counts is that a wave's own weight loads stay in flight under its products); a short batch is
     // one chain of dependent steps per wave, and the extra stop at a barrier costs more than the exact waits return
     const bool staged = A >= 12 * slots;
-    // ... and a wave then takes up to four row tiles one after the other, as long as the grid keeps two blocks per compute
-    // unit: the block's search for its input rows and their staging are paid once for all of them
+    // ... and a wave then takes up to four row tiles one after the other, as long as the grid keeps five blocks per compute
+    // unit: the block's search for its input rows and their staging are paid once for all of them, but a grid of two or
+    // three blocks per unit, some of which find their expert taken by another and leave, ends in a round that most units
+    // sit out. A Q4_K/Q6_K layer of 23 tokens over 125 experts takes 99 us with two blocks as the least, 90 with five; IQ3_S with
+    // 20 tokens over 64 experts 94 and 78.
+    constexpr int kLeastBlocks = 1280;
     int tl = 1;
     if (staged && nb == 1 && shared_lim == (gateup ? b0.rows : b0.cols))
-        while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= 512) tl *= 2;
+        while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= kLeastBlocks) tl *= 2;
     const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl)), unsigned(A));
     const int a_off = int(lds);
     if (staged) lds += size_t(b0.cols / 32) * (256 + ((uniform ? 0 : 1) + (MfmaFormat<FMT>::kMin ? 1 : 0)) * kTP * sizeof(float));
