@@ -36,9 +36,10 @@ namespace {
 constexpr int kQ4kHalfRows = 2048;
 // Where the descriptor asks for the int8 grouped products (act_blocks nonzero), IQ4_XS banks take them from kGroupedMin tokens.
 constexpr int kGroupedMin = 64;
-// Left to the library (act_blocks zero), IQ4_XS banks take them from kInt8Tokens tokens: measured at 512 experts, top-10, on
-// uniform and on Zipf routing, the fp16 grouped products are level or up to a fifth faster below (most experts then hold a
-// row tile or two, which the fp16 kernel's one-expert blocks serve better), the int8 products a seventh faster at 4096.
+// Left to the library (act_blocks zero), IQ4_XS banks take them from kInt8Tokens tokens. The line is where the result changes,
+// not where the speed does: a scale per token on eight bits moves the layer's result by 2 % of its norm. fp16 products on
+// prepared rows are the faster ones on both sides (4096 tokens of 10 of 512 experts, Zipf / balanced: 569 / 620 us a layer
+// against 697 / 1012), so a caller whose results may change gains by a higher line.
 constexpr int kInt8Tokens = 1024;
 // Up to here the down blocks add a token's experts themselves, and with plain softmax routing the gate / up blocks select their
 // own experts: three launches a layer instead of five (of about 2 us each on the GPU and 3.5 us of host time). An expert that
@@ -82,7 +83,7 @@ int int8_mode_of(const tqmoe_layer & L) { return L.struct_size >= kLayerBlocksSi
 bool act_blocks_of(const tqmoe_layer & L) { return int8_mode_of(L) == 1; }
 // Formats whose 8-bit grouped products are the faster ones at n tokens: the lattice formats of two and three bits that have
 // no fp16 products on prepared rows (a tenth faster than the fp16 kernel that takes every format), NVFP4G on its fp8
-// products, IQ4_XS from kInt8Tokens tokens. Q4_K, Q6_K and IQ3_S run on prepared fp16 rows at every size (Q4_K at 4096
+// products; and IQ4_XS from kInt8Tokens tokens (see there). Q4_K, Q6_K and IQ3_S run on prepared fp16 rows at every size (Q4_K at 4096
 // tokens 576 us a layer against 855 on its three int8 planes; IQ3_S at 512 tokens 260 against 393 on the general fp16
 // kernel), the others on the general fp16 kernel, 5 to 25 % faster than int8 there.
 bool int8_faster(uint32_t type, int n) {
