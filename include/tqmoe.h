@@ -66,7 +66,8 @@ int32_t tqmoe_topk2(const float * logits, int32_t * ids, float * weights, float 
  *                 TQMOE_GATE_SOFTMAX_WEIGHT  p = logit; the weights are a softmax over the selected logits only
  *                 TQMOE_GATE_SQRT_SOFTPLUS   p = sqrt(log(1 + exp(logit)))
  *   probs_bias    device [experts] fp32 or NULL: added to p for the choice only (descending p + bias, ties to the lower
- *                 index); the weights come from the unbiased p
+ *                 index; a NaN is chosen as the lowest value, so the ids are distinct experts whatever the logits);
+ *                 the weights come from the unbiased p
  *   norm_weights  nonzero: weights divided by max(their sum, 6.103515625e-5); then * (scale == 0 ? 1 : scale)
  * The values are MoeGating's (src/experts/moe.hpp:20-26). shared_weights as in tqmoe_topk. experts <= 4096. */
 enum { TQMOE_GATE_SOFTMAX = 1, TQMOE_GATE_SIGMOID = 2, TQMOE_GATE_SOFTMAX_WEIGHT = 3, TQMOE_GATE_SQRT_SOFTPLUS = 4 };

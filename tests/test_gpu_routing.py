@@ -6,7 +6,7 @@ import pytest
 import torch
 
 import synth
-from gpu_util import clear_tokens, clear_tokens_gated, dev, oracle_type
+from gpu_util import clear_tokens, clear_tokens_gated, dev, oracle_type, selection_values
 
 pytestmark = pytest.mark.gpu
 
@@ -178,6 +178,30 @@ def test_topk_gated_closed_forms(tq, oracle):
     assert ids[0].tolist() == [1, 2] and np.abs(w[0] - np.array([np.e, 1]) / (np.e + 1)).max() < 1e-6
     with pytest.raises(tq.TqmoeError):
         tq.moe_topk(dev(lg), 4, 2, gating=7)
+
+
+@pytest.mark.parametrize("gating", [1, 2, 3, 4])
+@pytest.mark.parametrize("e,k,n", [(5, 5, 6), (64, 6, 33), (160, 70, 9), (512, 10, 16), (1500, 4, 8)])
+def test_topk_gated_of_values_without_order(tq, oracle, gating, e, k, n):
+    """NaN, infinite and lowest-value logits: every selection is another expert of the layer, a NaN comes after every number
+    (equal values, and NaNs, by index). One NaN makes every softmax probability NaN: the first k experts."""
+    rng = np.random.default_rng(e + k + gating)
+    logits = (rng.standard_normal((n, e + 1)) * 2).astype(np.float32)
+    logits[0, :e] = np.nan
+    logits[1, :e] = np.where(np.arange(e) % 3 == 0, np.nan, logits[1, :e])
+    logits[2, [0, e - 1]] = np.nan, np.inf
+    logits[3, :e] = -np.inf
+    logits[4, :e] = np.finfo(np.float32).min
+    logits[5, :e - 1] = np.nan
+    bias = np.zeros(e, np.float32)
+    for biased in (None, bias) if gating != 1 else (bias,):
+        ids, w, _ = (t.cpu().numpy() for t in tq.moe_topk(dev(logits), e, k, gating=gating, bias=dev(biased) if biased is not None else None, norm=False))
+        assert ids.min() >= 0 and ids.max() < e and all(len(set(row)) == k for row in ids.tolist())
+        with np.errstate(all="ignore"):
+            v = selection_values(logits[:, :e], gating, biased)
+        want = np.argsort(-np.where(np.isnan(v), -np.inf, v), axis=1, kind="stable")[:, :k]
+        assert np.array_equal(ids, want)
+        assert np.isfinite(w[6:]).all()      # the other tokens
 
 
 @pytest.mark.parametrize("e,n,k", [(64, 1, 8), (512, 16, 10), (512, 4096, 10), (256, 8192, 9), (7, 300, 3), (4096, 700, 2), (512, 102, 10)])

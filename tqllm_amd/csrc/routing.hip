@@ -615,7 +615,11 @@ __global__ __launch_bounds__(64) void topk_gated_k(const float * __restrict__ lo
         for (int r = 0; r < per_lane; ++r) P(r) = gate_value(g.gating, P(r));
     }
 #pragma unroll
-    for (int r = 0; r < per_lane; ++r) { const int j = lane + 64 * r; V(r) = g.bias && j < e ? P(r) + g.bias[j] : P(r); }
+    for (int r = 0; r < per_lane; ++r) {   // a NaN compares with nothing: it is chosen as the lowest value, so that every round finds an expert not yet taken
+        const int j = lane + 64 * r;
+        const float v = g.bias && j < e ? P(r) + g.bias[j] : P(r);
+        V(r) = v == v ? v : -INFINITY;
+    }
     uint64_t taken = 0;   // bit r: entry r of this lane is chosen already or lies past the end
 #pragma unroll
     for (int r = 0; r < per_lane; ++r) if (lane + 64 * r >= e) taken |= uint64_t(1) << r;
