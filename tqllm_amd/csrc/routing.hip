@@ -416,9 +416,10 @@ template <int XT> __device__ __forceinline__ void topk_row(const TopkOut & o, in
         case kRowsInt8Blocks: quant_row_wave<XT, false, true>(d.x, token, d.cols, static_cast<int8_t *>(d.q), d.scale, nullptr, lane); break;
     }
 }
-// selection s of the token is expert id (s = k: the shared one): one more assignment of it in the dispatch chunk
+// selection s of the token is expert id (s = k: the shared one): one more assignment of it in the dispatch chunk. An id
+// outside the banks is not counted, as the dispatch that reads the counts does not place it.
 __device__ __forceinline__ void topk_count(const TopkOut & o, int token, int k, int s, int id) {
-    if (!o.side.chunk_counts) return;
+    if (!o.side.chunk_counts || id < 0 || id >= o.side.banks) return;
     const int64_t a = int64_t(token) * (o.ext_ids ? k + 1 : k) + s;
     atomicAdd(o.side.chunk_counts + a / kDispatchChunk * o.side.banks + id, 1);
 }
