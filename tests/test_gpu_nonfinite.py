@@ -14,7 +14,7 @@ GATINGS = {"softmax": (1, False, True), "softmax_biased": (1, True, True), "soft
 
 
 @pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K"])
-@pytest.mark.parametrize("n", [800])
+@pytest.mark.parametrize("n", [5, 800])
 @pytest.mark.parametrize("gating", sorted(GATINGS))
 def test_neighbours_of_a_token_without_numbers(oracle, gating, n, fmt):
     import tqllm_amd as tq

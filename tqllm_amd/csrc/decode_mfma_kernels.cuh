@@ -579,7 +579,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
     auto expert_of = [&](int u) { const int slot = min(u / NSB, k.slots - 1); return slot < k.topk ? k.ids[token * k.topk + slot] : extra; };
     auto fetch = [&](int u, int e, Unit & c) {
         const int slot = min(u / NSB, k.slots - 1), sb = u - slot * NSB;
-        e = max(e, 0);
+        e = min(max(e, 0), extra);   // an id outside the bank: a bank's weights, not added below
         const int64_t at = (int64_t(e) * tiles + tile) * NSB + sb;
         F::codes(k.b.codes + at * F::kCodeBytes, n, g, c.code);
         c.rec = F::rec(k.b.aux + at * F::kRecBytes, n);
