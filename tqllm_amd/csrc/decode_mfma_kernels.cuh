@@ -33,6 +33,7 @@ typedef int v16i __attribute__((ext_vector_type(16)));
 
 constexpr int kTP = kChunkRowsMax;   // input rows per block
 constexpr int kMaxWaves = 8;
+constexpr int kStagedFrom = 12;      // assignments from which a block's input rows go through LDS (see mfma_launch)
 
 constexpr int kIq4Table[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
 constexpr int kFp4Table[16] = {0, 1, 2, 3, 4, 6, 8, 12, 0, -1, -2, -3, -4, -6, -8, -12};   // twice the E2M1 values
@@ -520,11 +521,17 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     const int NSB = b0.cols / 256, tiles = b0.rows / 32;
     // Waves that share a row's super-blocks: as many as it takes to put a few thousand waves in flight (a short batch
     // is bound by the latency of one wave's chain), fewer when the batch has the waves anyway (a longer chain per
-    // wave streams with its loads one super-block ahead and saves the cross-wave sums).
+    // wave streams with its loads one super-block ahead and saves the cross-wave sums), and fewer at once where registers
+    // leave a SIMD two waves. Shares may differ by a super-block: a row of 11 at one token takes 21 us a layer with four or
+    // eight waves and 33 with one (Q4_K, ff 512); with many units an uneven split only loses (nine super-blocks, 5120
+    // units: 111 us against 107). Blocks of five to seven waves fill a compute unit badly: only the smallest launches take more
+    // than four waves (12 super-blocks, ff 1536: one token, four waves 32 us, six 38; four tokens, two 80, four 79, six 95).
+    // One bank, eight tokens of 8 of 128 experts, ff 512 to 1536: one wave a row 55 to 92 us a layer, two 59 to 103.
     const int64_t units = int64_t(A) * tiles;
-    const int cap = units >= 8192 ? 1 : units >= 2048 ? 2 : units >= 512 ? 4 : kMaxWaves;
-    int wk = 1;
-    for (int w = 1; w <= kMaxWaves && w <= cap; ++w) if (NSB % w == 0) wk = w;
+    const int halves = kDecodeWaves<FMT, 2, true, 0> == 2 && NSB <= 12 ? 576 : 768;   // units of two banks from which two waves share a row
+    int wk = nb == 2 ? (units >= 8192 ? 1 : units >= 2048 ? (NSB >= 8 && (NSB % 2 == 0 || units < 3072) ? 2 : 1) : units > halves ? 2 : units >= 320 ? 4 : kMaxWaves)
+                     : (units >= 2048 ? 1 : units >= 1024 ? 2 : units >= 320 ? 4 : kMaxWaves);
+    if (wk > NSB) wk = NSB;
     const int waves = wk > 4 ? wk : 4;                    // per block: small blocks, a compute unit holds several and their phases interleave
     int tpw = waves / wk;                                                 // row tiles per block
     if (tpw > tiles) tpw = tiles;
@@ -533,10 +540,11 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     // rows' planes (256 bytes per sub-block) and, for rows with a scale per sub-block, the scales
     size_t lds = mode ? size_t(2) * kMaxList * sizeof(int) : 0;
     if (lds < size_t(wk * tpw) * nb * kTP * 32 * sizeof(float)) lds = size_t(wk * tpw) * nb * kTP * 32 * sizeof(float);
-    // the input rows go through LDS from a dozen tokens on (measured: 5 % at 16 and 32 tokens; the waves then overlap each
-    // other's waits, and what counts is that a wave's own weight loads stay in flight under its products); a short batch is
-    // one chain of dependent steps per wave, and the extra stop at a barrier costs more than the exact waits return
-    const bool staged = A >= 12 * slots;
+    // the input rows go through LDS from a dozen assignments on (the waves then overlap each other's waits, and what
+    // counts is that a wave's own weight loads stay in flight under its products: 10 tokens of 8 of 128 experts, Q4_K 71.5
+    // and 61.3 us a layer, NVFP4G 69.2 and 68.0, IQ3_S 67.7 and 64.7); a shorter batch is one chain of dependent steps per wave,
+    // and the extra stop at a barrier costs more than the exact waits return
+    const bool staged = A >= kStagedFrom;
     // ... and a wave then takes up to four row tiles one after the other, as long as the grid keeps five blocks per compute
     // unit: the block's search for its input rows and their staging are paid once for all of them, but a grid of two or
     // three blocks per unit, some of which find their expert taken by another and leave, ends in a round that most units
@@ -544,7 +552,7 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     // 20 tokens over 64 experts 94 and 78.
     constexpr int kLeastBlocks = 1280;
     int tl = 1;
-    if (staged && nb == 1 && shared_lim == (gateup ? b0.rows : b0.cols))
+    if (staged && nb == 1 && NSB % wk == 0 && shared_lim == (gateup ? b0.rows : b0.cols))
         while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= kLeastBlocks) tl *= 2;
     const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl)), unsigned(A));
     const int a_off = int(lds);

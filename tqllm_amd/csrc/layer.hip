@@ -41,12 +41,22 @@ constexpr int kGroupedMin = 64;
 // prepared rows are the faster ones on both sides (4096 tokens of 10 of 512 experts, Zipf / balanced: 569 / 620 us a layer
 // against 697 / 1012), so a caller whose results may change gains by a higher line.
 constexpr int kInt8Tokens = 1024;
-// Up to here the down blocks add a token's experts themselves, and with plain softmax routing the gate / up blocks select their
+// Few tokens: the down blocks add a token's experts themselves, and with plain softmax routing the gate / up blocks select their
 // own experts: three launches a layer instead of five (of about 2 us each on the GPU and 3.5 us of host time). An expert that
-// several tokens chose is read once for each of them, from the caches: layer in us at five / three launches, IQ4_XS (512
-// experts) 25.5 / 20.5 at one token, 38.0 / 27.5 at four, 46.6 / 42.0 at six; NVFP4G (1536 x 3072 experts) 92.3 / 91.8 at
-// four, 128.8 / 130.0 at seven.
-constexpr int kFewTokens = 6;
+// several tokens chose is read once for each of them, from the caches, and a block of the down launch walks all of a token's
+// weight rows: what a launch reads is the line (weights of one projection over all assignments), lower where the gate / up
+// kernel's registers leave a SIMD two waves. Layer in us, five / three launches, Q4_K and NVFP4G: 2048 x 768 experts, top-8
+// of 128, two tokens 32.6 / 26.1 and 34.7 / 28.7, seven (88 M) 49.1 / 51.2 and 55.8 / 51.2; 4096 x 1024, top-4, five (84 M)
+// 57.6 / 53.4 and 62.6 / 55.5, six (101 M) 55.7 / 58.4 and 63.5 / 64.2; 3072 x 1536, top-8 and a shared one, two (85 M) 54.4 /
+// 47.3 and 58.7 / 51.2, three (127 M) 60.2 / 78.3 and 71.8 / 77.5; and where all the down blocks find a compute unit of their
+// own (4096 x 8192, top-2 of 8, two tokens 58.0 / 52.7 and 69.4 / 59.2). A token with more than 64 units (super-blocks of its
+// experts' rows) keeps a block's sixteen waves too long (1024 x 4096, top-6, one token 28.9 / 36.7 and 29.7 / 37.8). At most
+// as many tokens as the router's one-token passes take (they write the activation images).
+bool few_tokens(uint32_t gate_type, int n, int slots, int hidden, int ff) {
+    const bool two_waves = gate_type == TQMOE_Q4_K || gate_type == TQMOE_Q6_K;
+    const bool one_round = int64_t(n) * (hidden / 32) <= 256;   // the down launch's blocks: one a compute unit
+    return n <= (two_waves ? 5 : kRouterFew) && slots * (ff / 256) <= 64 && (one_round || int64_t(n) * slots * hidden * ff <= (two_waves ? 85000000 : 90000000));
+}
 constexpr int kDecodeAssignments = 65535;   // per decode launch
 constexpr int kDecodeDedup = 2048;          // assignments up to which the decode kernels serve an expert's rows together
 constexpr int kGroupedPerBank = 3;          // assignments per expert from which the fp16 grouped products are the faster path
@@ -169,7 +179,7 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         }
     } else {
         const Routing rt = routing_of(L);
-        p.few = n <= kFewTokens && decode_few_takes(L.gate, L.down, slots, L.has_shared ? L.shared_ff : 0);
+        p.few = few_tokens(L.gate.type, n, slots, L.hidden, L.ff) && decode_few_takes(L.gate, L.down, slots, L.has_shared ? L.shared_ff : 0);
         p.routes = p.few && rt.gating == TQMOE_GATE_SOFTMAX && rt.norm && !rt.bias && L.n_expert <= 512 && L.topk <= 64;
         p.ximage = take(tqmoe_act_image_bytes(n, L.hidden));
         p.aimage = take(tqmoe_act_image_bytes(int32_t(a), L.ff));

@@ -19,7 +19,6 @@ namespace {
 // sum by ordinary fp32 rounding only.
 constexpr int kRouterTok = 4;       // tokens per pass of a wave: the router row is read once for them
 constexpr int kRouterTokFew = 1;    // decode-sized batches: a wave per (row, token), the latency of a wave's chain is what counts
-constexpr int kRouterFew = 7;       // batches up to here take kRouterTokFew
 template <int WT, int XT, int TOK>
 __global__ __launch_bounds__(256) void router_k(const void * __restrict__ w, const void * __restrict__ shared,
                                                 const void * __restrict__ x, float * __restrict__ logits, int h, int e, int n, RouterSide side) {

@@ -7,6 +7,7 @@ namespace tqmoe {
 
 constexpr int kDispatchChunk = 1024;        // consecutive assignments a dispatch block places
 constexpr int kDispatchWide = 1024;         // experts up to which it does so in one launch
+constexpr int kRouterFew = 7;               // tokens up to which the router takes them one a pass
 
 struct RouterSide {
     uint8_t * image = nullptr;              // activation images of the rows (batches of one-token passes only)
