@@ -100,6 +100,24 @@ def test_no_device_is_an_error_not_a_fallback(tq):
     assert rc == -3 and b"no CPU path" in err.message
 
 
+def fake_layer(tq, hidden, ff, experts, topk, shared, fmt, down=None):
+    """A descriptor whose pointers are never read: for the answers that come before any device work."""
+    bank = lambda f, rows, cols: tq.api._Bank(C.sizeof(tq.api._Bank), f, experts + int(shared), rows, cols, 4096, 4096)
+    return tq.api._Layer(C.sizeof(tq.api._Layer), hidden, ff, experts, topk, int(shared), ff if shared else 0, 1.0, 4096, 4096, tq.BF16, bank(fmt, ff, hidden),
+                         bank(fmt, ff, hidden), bank(down or fmt, hidden, ff), 1, 0, None, 0, 0.0, 0)
+
+
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "Q5_K", "NVFP4G", "IQ2_S"])
+def test_grouped_products_refuse_more_than_4096_experts(tq, fmt):
+    """4096 routed experts and a shared one are 4097 lists, one more than the dispatch takes: the layer refuses the batches that
+    need the lists before anything is enqueued, and takes the small ones (which here end at the missing workspace)."""
+    lib, err = tq.lib(), tq.api._err()
+    run = lambda d, n: lib.tqmoe_layer_forward(C.byref(d), 4096, tq.BF16, n, 4096, tq.F32, None, None, None, None, 0, None, C.byref(err))
+    over, most = (fake_layer(tq, 512, 256, experts, 8, True, getattr(tq, fmt)) for experts in (4096, 4095))
+    assert run(over, 2000) == -1 and b"4096 experts" in err.message
+    assert run(over, 4) == -4 and run(most, 2000) == -4
+
+
 def test_adapter_header_compiles(tmp_path):
     src = tmp_path / "use.cpp"
     src.write_text('#include "tqmoe_adapter.hpp"\n'

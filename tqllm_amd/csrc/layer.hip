@@ -234,6 +234,7 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
     if (!is_act_type(xtype) || (otype != TQMOE_F32 && otype != TQMOE_BF16)) return fail(err, TQMOE_E_UNSUPPORTED, "tqmoe_layer_forward: unsupported element type");
     const int slots = L.topk + (L.has_shared ? 1 : 0), banks = L.n_expert + (L.has_shared ? 1 : 0);
     const Plan p = plan_for(L, n);
+    if (p.grouped && banks > 4096) return fail(err, TQMOE_E_ARG, "tqmoe_layer_forward: the grouped products take at most 4096 experts, the shared one included");   // as tqmoe_dispatch does
     if (!workspace || workspace_bytes < p.total) return fail(err, TQMOE_E_WORKSPACE, "tqmoe_layer_forward: workspace of %zu bytes needed", p.total);
     if (int32_t rc = need_device(err, "tqmoe_layer_forward")) return rc;
     uint8_t * ws = static_cast<uint8_t *>(workspace);
