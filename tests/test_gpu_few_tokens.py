@@ -37,3 +37,19 @@ def test_layer_of_few_tokens(tq, oracle, fmt, n, hidden, ff, experts, topk, shar
     res = torch.randn_like(x)
     got = layer.forward(x, residual=res)
     assert torch.equal(got, (torch.from_numpy(out).cuda().bfloat16().float() + res.float()).bfloat16())
+
+
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K"])
+def test_down_rows_wider_than_the_decode_products_take(tq, oracle, fmt):
+    """8448 columns: batches of up to six tokens have the launches of few tokens whatever they read, the next is refused."""
+    cfg = dict(hidden=256, ff=8448, experts=8, topk=2, shared_ff=0, wtype=getattr(oracle, fmt), rtype="bf16", xtype="bf16")
+    raws = synth.make_banks(cfg, seed=5, distinct=2)
+    inp = synth.make_inputs(cfg, 7, seed=6)
+    layer = tq.MoeLayer(dev(inp["router"]), None, *banks_on_device(cfg, raws), 2)
+    x = dev(inp["x"])
+    for n in (1, 6):
+        out, ids, _, logits = (t.cpu().numpy() for t in layer.forward(x[:n], return_routing=True))
+        want, want_ids, _ = oracle.layer_forward(inp["x"][1][:n], logits, *raws, cfg["wtype"], 256, 8448, 8, 2, act_mode=0, threads=16)
+        assert np.array_equal(ids, want_ids) and synth.errors(out, want)[1] < 1e-3
+    with pytest.raises(tq.TqmoeError, match="too wide"):
+        layer.forward(x)

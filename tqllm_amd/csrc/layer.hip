@@ -179,7 +179,9 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         }
     } else {
         const Routing rt = routing_of(L);
-        p.few = few_tokens(L.gate.type, n, slots, L.hidden, L.ff) && decode_few_takes(L.gate, L.down, slots, L.has_shared ? L.shared_ff : 0);
+        // (rows too wide for the decode products' entry, which refuses them: up to six tokens have the three launches all the same)
+        const bool only = n <= 6 && !split_for(L.ff / 32).m;
+        p.few = (only || few_tokens(L.gate.type, n, slots, L.hidden, L.ff)) && decode_few_takes(L.gate, L.down, slots, L.has_shared ? L.shared_ff : 0);
         p.routes = p.few && rt.gating == TQMOE_GATE_SOFTMAX && rt.norm && !rt.bias && L.n_expert <= 512 && L.topk <= 64;
         p.ximage = take(tqmoe_act_image_bytes(n, L.hidden));
         p.aimage = take(tqmoe_act_image_bytes(int32_t(a), L.ff));
