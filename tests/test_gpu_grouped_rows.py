@@ -40,3 +40,26 @@ def test_layer_on_prepared_rows(tq, oracle, fmt, n, hidden, ff, shared_ff):
     mx, rel = synth.errors(out[clear], want[clear])
     top = float(np.abs(want[clear]).max())     # E4M3's coarse steps amplify last-bit differences of the act rows
     assert mx < 1e-2 * (max(1.0, top) if fp8 else 1.0) and rel < (3e-3 if fp8 else 1e-3), (mx, rel)
+
+
+@pytest.mark.parametrize("fmt,n,shared_ff", [("Q4_K", 2048, 128), ("Q4_K", 2047, 256), ("Q6_K", 2048, 256), ("IQ3_S", 2048, 128)])
+def test_down_rows_past_the_range_of_halves(tq, oracle, fmt, n, shared_ff):
+    """Results past 65504, the largest half, before the weighted sum: down rows are fp32 but where the int8 products, whose rows
+    are halves, would have taken the batch (Q4_K, 2048 tokens, whole super-blocks everywhere). Against float64 on the decoded weights."""
+    cfg = dict(hidden=256, ff=256, experts=7, topk=2, shared_ff=shared_ff, wtype=getattr(oracle, fmt), rtype="f32", xtype="f32")
+    raws = synth.make_banks(cfg, seed=11, sigma=0.5)
+    inp = synth.make_inputs(cfg, n, seed=12)
+    x = np.ascontiguousarray(inp["x"][1] * 6)
+    layer = tq.MoeLayer(dev(inp["router"]), dev(inp["shared_gate"]), *banks_on_device(cfg, raws), 2, shared_ff=shared_ff)
+    assert layer.path(n) == "grouped_f16"
+    out, ids, w, logits = (t.cpu().numpy() for t in layer.forward(torch.from_numpy(x).cuda(), return_routing=True))
+    g, u, d = (oracle.dequantize(cfg["wtype"], raw, 8 * 256 * 256).reshape(8, 256, 256).astype(np.float64) for raw in raws)
+
+    def expert(e, rows, lim):
+        a, b = rows @ g[e, :lim].T, rows @ u[e, :lim].T
+        return a / (1 + np.exp(-np.clip(a, -700, 700))) * b @ d[e, :, :lim].T
+
+    rows = np.stack([expert(e, x.astype(np.float64), 256) for e in range(7)], axis=1)[np.arange(n)[:, None], ids]
+    want = (rows * w[:, :, None]).sum(axis=1) + expert(7, x.astype(np.float64), shared_ff) / (1 + np.exp(-logits[:, 7:].astype(np.float64)))
+    assert np.abs(rows).max() > 65504 and np.isfinite(out).all()
+    assert synth.errors(out, want)[1] < 1e-3

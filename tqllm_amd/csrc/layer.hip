@@ -31,8 +31,9 @@ int32_t gemm_f16_common(const tqmoe_bank * b0, const tqmoe_bank * b1, const void
 
 namespace {
 
-// From here on the down product of Q4_K banks leaves its rows as halves, as its int8 products always have: the sum over a
-// token's experts reads half the bytes (4096 tokens: 45 us of the layer). Smaller batches and other formats keep fp32 rows.
+// From here on the down product of Q4_K banks leaves its rows as halves where the int8 products, which this batch ran on before it
+// had products on prepared rows, take the shape (int8_ok) and did the same: the sum over a token's experts reads half the bytes
+// (4096 tokens: 45 us of the layer). Everything else keeps fp32 rows: halves end at 65504.
 constexpr int kQ4kHalfRows = 2048;
 // Where the descriptor asks for the int8 grouped products (act_blocks nonzero), IQ4_XS banks take them from kGroupedMin tokens.
 constexpr int kGroupedMin = 64;
@@ -171,7 +172,7 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         }
     } else if (p.grouped) {
         p.prepared = rows_ok && !plane_gemm_is_fp8(L.gate.type) && !plane_gemm_is_fp8(L.down.type);
-        p.half_rows = L.gate.type == TQMOE_Q4_K && L.down.type == TQMOE_Q4_K && n >= kQ4kHalfRows;
+        p.half_rows = L.gate.type == TQMOE_Q4_K && L.down.type == TQMOE_Q4_K && n >= kQ4kHalfRows && int8_ok(L);
         if (p.prepared) {
             p.x16 = take(c * L.hidden * 2);
             p.xs16 = take(c * 4);
