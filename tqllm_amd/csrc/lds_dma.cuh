@@ -7,9 +7,12 @@ namespace {
 
 // 16 bytes a lane from memory to LDS at `lds` (a wave-uniform byte address) + 16 * lane. The compiler does not count these:
 // dma_wait() says when they are there.
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"   // m0 is a register the compiler reserves: what it keeps there itself must know of the write
 __device__ __forceinline__ void dma16(const void * p, uint32_t lds) {
-    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(p), "s"(lds) : "memory");
+    asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" :: "v"(p), "s"(lds) : "memory", "m0");
 }
+#pragma clang diagnostic pop
 // all but the last N transfers of this wave are here (they finish in order); with BARRIER every wave's are
 template <int N, bool BARRIER> __device__ __forceinline__ void dma_wait() {
     if constexpr (BARRIER) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "i"(N) : "memory");
