@@ -63,3 +63,19 @@ def test_down_rows_past_the_range_of_halves(tq, oracle, fmt, n, shared_ff):
     want = (rows * w[:, :, None]).sum(axis=1) + expert(7, x.astype(np.float64), shared_ff) / (1 + np.exp(-logits[:, 7:].astype(np.float64)))
     assert np.abs(rows).max() > 65504 and np.isfinite(out).all()
     assert synth.errors(out, want)[1] < 1e-3
+
+
+def test_rows_past_the_shared_expert_are_zero_whatever_the_bank_holds(tq, oracle):
+    """The shared expert has 256 of the bank's 512 rows; the others are infinite in the gate bank and NaN in the up bank."""
+    cfg = dict(hidden=256, ff=512, experts=3, topk=1, shared_ff=256, wtype=oracle.NVFP4G, rtype="f32", xtype="f32")
+    raws = synth.make_banks(cfg, seed=21)
+    inp = synth.make_inputs(cfg, 70, seed=22)
+    x = dev(inp["x"])
+    for raw, value in zip(raws[:2], (np.inf, np.nan)):
+        elems, nbytes = oracle.BLOCK[cfg["wtype"]]
+        raw.reshape(4, 512, 256 // elems, nbytes)[3, 256:, :, 0:4] = np.frombuffer(np.float32(value).tobytes(), np.uint8)
+    gate, up, down = banks_on_device(cfg, raws)
+    ids = tq.moe_extend_ids(torch.randint(0, 3, (70, 1), dtype=torch.int32, device="cuda"), 3)
+    lists = tq.moe_dispatch(ids, 4)[:3]
+    act = tq.expert_gemm_gateup_fp8(gate, up, *tq.gather_rows_i8(*tq.quant_rows_fp8(x), lists, 140, 2), lists, 70, 2, 1, 256).view(70, 2, 512)
+    assert not act[:, 1, 256:].any() and torch.isfinite(act).all() and act[:, 1, :256].any()

@@ -473,9 +473,9 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
 #pragma unroll
                         for (int i = 0; i < 16; ++i) v[i] = glu_clamp_silu(k.glu, v[i]);
                     }
-                    const float live = wt[0] * 32 < row_lim ? 1.f : 0.f;
+                    const bool live = wt[0] * 32 < row_lim;   // (zeros past the shared expert's rows, whatever the bank holds there)
 #pragma unroll
-                    for (int i = 0; i < 16; ++i) v[i] *= live * u[i];
+                    for (int i = 0; i < 16; ++i) v[i] = live ? v[i] * u[i] : 0.f;
                 }
 #pragma unroll
                 for (int c = 0; c < 4; ++c) {
