@@ -162,6 +162,9 @@ int32_t tqmoe_dedup_maps(const int32_t * ids, const int32_t * slot_of, int32_t c
  *   IQ4_NL  codes 16 B, GGUF's own nibble order; aux 2 B per sub-block: its d (f16).
  *   Q4_0    as IQ4_NL (the weight is the nibble minus 8).
  *   Q8_0    codes 32 B: the int8 values; aux 2 B per sub-block: its d (f16).
+ * codes and aux are 16-byte aligned where the fastest grouped products are wanted: those of IQ4_XS, Q4_K, Q6_K, IQ3_S and
+ * NVFP4G on prepared rows move 16-byte pieces from memory to LDS. tqmoe_layer_forward runs the general fp16 products on
+ * planes that start elsewhere (NVFP4G too, where it has fp8 products otherwise), the fp8 entry points refuse them.
  * cols must be a multiple of 256 (128 for NVFP4G). Every format has the decode products and the fp16 grouped products
  * (tqmoe_expert_gemm, tqmoe_expert_gemm_gateup). The grouped int8 products take the formats with one scale per 32 weights
  * (IQ4_XS, IQ4_NL, IQ3_S, IQ3_XXS, IQ2_XXS, IQ2_XS, IQ2_S, IQ1_S, Q4_K, Q5_K, Q4_0, Q8_0), the grouped fp8 products NVFP4G;
@@ -373,6 +376,7 @@ int32_t tqmoe_quant_rows_fp8(const void * x, uint32_t xtype, int64_t rows, int32
 int32_t tqmoe_group_rows_fp8(const void * x, uint32_t xtype, int32_t cols, const int32_t * counts, const int32_t * offsets,
                              const int32_t * perm, int32_t experts, int64_t assignments, int32_t xdiv, uint8_t * q,
                              float * scale, void * stream, tqmoe_error * err);
+/* xq and the banks' planes 16-byte aligned, else TQMOE_E_ARG */
 int32_t tqmoe_expert_gemm_gateup_fp8(const tqmoe_bank * gate, const tqmoe_bank * up, const uint8_t * xq, const float * xs,
                                      const int32_t * counts, const int32_t * offsets, const int32_t * perm, int32_t n,
                                      int32_t slots, int32_t topk, int32_t shared_lim, void * act_f16, void * stream,
@@ -491,6 +495,7 @@ size_t  tqmoe_layer_workspace_bytes(const tqmoe_layer * layer, int32_t n);
  * bank formats only, never on the data, so that a token's result does not depend on what else is routed; the reference
  * makes its switch slot-independent for the same reason, src/models/qwen/qwen4exp/fn_layer_forward.cpp:408-414):
  * the decode kernels (one read of every distinct expert), the grouped 8-bit products, or the grouped fp16 products.
+ * (NVFP4G: also on the alignment of the bank planes, see tqmoe_bank.)
  * With act_blocks zero the grouped products are the ones measured faster for the formats: int8 for IQ4_XS from 1024
  * tokens and for the two- and three-bit lattice formats other than IQ3_S, fp8 for NVFP4G, fp16 otherwise.
  * Negative: the descriptor is invalid. */

@@ -118,6 +118,17 @@ def test_grouped_products_refuse_more_than_4096_experts(tq, fmt):
     assert run(over, 4) == -4 and run(most, 2000) == -4
 
 
+def test_planes_that_are_not_aligned_take_the_general_products(tq):
+    """The fp8 products move 16-byte pieces to LDS: a layer whose planes start elsewhere runs on the fp16 products."""
+    d = fake_layer(tq, 512, 256, 16, 4, False, tq.NVFP4G)
+    assert tq.lib().tqmoe_layer_path(C.byref(d), 500) == 3
+    for bank in (d.gate, d.up, d.down):
+        for plane in ("codes", "aux"):
+            setattr(bank, plane, 4104)
+            assert tq.lib().tqmoe_layer_path(C.byref(d), 500) == 2
+            setattr(bank, plane, 4096)
+
+
 def test_adapter_header_compiles(tmp_path):
     src = tmp_path / "use.cpp"
     src.write_text('#include "tqmoe_adapter.hpp"\n'

@@ -79,3 +79,43 @@ def test_rows_past_the_shared_expert_are_zero_whatever_the_bank_holds(tq, oracle
     lists = tq.moe_dispatch(ids, 4)[:3]
     act = tq.expert_gemm_gateup_fp8(gate, up, *tq.gather_rows_i8(*tq.quant_rows_fp8(x), lists, 140, 2), lists, 70, 2, 1, 256).view(70, 2, 512)
     assert not act[:, 1, 256:].any() and torch.isfinite(act).all() and act[:, 1, :256].any()
+
+
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "NVFP4G"])
+def test_layer_on_operands_that_are_not_aligned(tq, oracle, fmt):
+    """Bank planes eight bytes, input rows one element and the workspace three bytes past a multiple of 16: the router's and the
+    products' transfers to LDS need that multiple, and the kernels that load into registers take over."""
+    cfg = dict(hidden=512, ff=256, experts=60, topk=4, shared_ff=0, wtype=getattr(oracle, fmt), rtype="bf16", xtype="bf16")
+    raws = synth.make_banks(cfg, seed=31, distinct=4)
+    banks = banks_on_device(cfg, raws)
+    n = 3100                                     # 49 x 1 blocks of the router's kernel for large batches
+    inp = synth.make_inputs(cfg, n, seed=32)
+    x, router = dev(inp["x"]), dev(inp["router"])
+    want, ids, _, logits = tq.MoeLayer(router, None, *banks, 4, act_blocks=2 if fmt == "IQ4_XS" else 0).forward(x, return_routing=True)
+
+    def moved(t, elements):
+        raw = torch.empty(t.numel() + 64, dtype=t.dtype, device="cuda")
+        out = raw[elements:elements + t.numel()].view(t.shape)
+        out.copy_(t)
+        return out
+
+    for b in banks:
+        b.codes, b.aux = moved(b.codes.view(torch.uint8), 8), moved(b.aux.view(torch.uint8), 8)
+    layer = tq.MoeLayer(moved(router, 1), None, *banks, 4, act_blocks=2 if fmt == "IQ4_XS" else 0)
+    layer._ws = moved(layer.workspace(n), 3)
+    out, ids2, _, logits2 = layer.forward(moved(x, 1), return_routing=True)
+    assert torch.equal(logits, logits2) and torch.equal(ids, ids2)
+    if fmt == "NVFP4G":      # the fp16 products in place of the fp8 ones: within their bar of fp32 activations
+        assert layer.path(n) == "grouped_f16"
+        out, want = out[:64], torch.from_numpy(oracle.layer_forward(inp["x"][1][:64], logits.cpu().numpy()[:64], *raws, cfg["wtype"], 512, 256, 60, 4, act_mode=0, threads=16)[0])
+    assert synth.errors(out.cpu().numpy(), want.cpu().numpy())[1] < 1e-3
+
+
+def test_fp8_products_refuse_operands_that_are_not_aligned(tq, oracle):
+    cfg = dict(hidden=256, ff=256, experts=3, topk=1, shared_ff=0, wtype=oracle.NVFP4G, rtype="f32", xtype="f32")
+    gate, up, down = banks_on_device(cfg, synth.make_banks(cfg, seed=41))
+    lists = tq.moe_dispatch(torch.zeros((64, 1), dtype=torch.int32, device="cuda"), 3)[:3]
+    q, s = tq.gather_rows_i8(*tq.quant_rows_fp8(torch.randn((64, 256), device="cuda")), lists, 64, 1)
+    assert tq.expert_gemm_fp8(down, q, s, lists, 64, 1, 1).shape[0] == 64
+    with pytest.raises(tq.TqmoeError, match="16 bytes"):
+        tq.expert_gemm_fp8(down, torch.empty(q.numel() + 16, dtype=q.dtype, device="cuda")[8:8 + q.numel()].view(q.shape), s, lists, 64, 1, 1)

@@ -82,6 +82,8 @@ inline bool is_bank_type(uint32_t t) { return t == TQMOE_Q2_K || t == TQMOE_IQ1_
            t == TQMOE_Q5_K || t == TQMOE_Q6_K || t == TQMOE_IQ3_XXS || t == TQMOE_IQ2_S;
 }
 inline size_t elem_bytes(uint32_t t) { return t == TQMOE_F32 ? 4 : 2; }
+// sources of 16-byte transfers from memory to LDS
+inline bool aligned16(const void * p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; }
 inline size_t align_up(size_t v, size_t a) { return (v + a - 1) / a * a; }
 
 // ----------------------------------------------------------------------------------------------- device side

@@ -596,6 +596,8 @@ int32_t tqmoe::gemm_8bit_common(const tqmoe_bank * b0, const tqmoe_bank * b1, co
                     fp8 ? "fp8" : "int8", b0->type);
     if (b0->cols % 256 || b0->rows % 32) return fail(err, TQMOE_E_UNSUPPORTED, "%s: the bank's rows must be a multiple of 32 and its columns of 256", what);
     if (!xq || !xs || !counts || !offsets || !perm || !out || n <= 0 || topk <= 0 || slots < topk) return fail(err, TQMOE_E_ARG, "%s: invalid shape or pointer", what);
+    if (fp8 && !(aligned16(xq) && aligned16(b0->codes) && aligned16(b0->aux) && (!b1 || (aligned16(b1->codes) && aligned16(b1->aux)))))
+        return fail(err, TQMOE_E_ARG, "%s: rows and bank planes must start at multiples of 16 bytes", what);
     const int lim_max = gateup ? b0->rows : b0->cols;
     if (slots > topk && (shared_lim <= 0 || shared_lim > lim_max || shared_lim % 256)) return fail(err, TQMOE_E_ARG, "%s: shared_lim must be a multiple of 256 within the bank", what);
     if (b0->experts > 4096) return fail(err, TQMOE_E_ARG, "%s: more than 4096 experts", what);

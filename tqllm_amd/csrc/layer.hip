@@ -79,10 +79,11 @@ struct Plan {  // byte offsets into the workspace
     size_t xbs, abks;        // their block scales
 };
 
+bool banks_aligned(const tqmoe_layer & L) { return grouped_rows_aligned(L.gate) && grouped_rows_aligned(L.up) && grouped_rows_aligned(L.down); }
 // the 8-bit grouped products: both banks' formats have one with the same operand type (int8, or E4M3 for NVFP4G)
 bool int8_ok(const tqmoe_layer & L) {
     return plane_gemm_has(L.gate.type) && plane_gemm_has(L.down.type) && plane_gemm_is_fp8(L.gate.type) == plane_gemm_is_fp8(L.down.type) &&
-           L.hidden % 256 == 0 && L.ff % 256 == 0 && (!L.has_shared || L.shared_ff % 256 == 0);
+           (!plane_gemm_is_fp8(L.gate.type) || banks_aligned(L)) && L.hidden % 256 == 0 && L.ff % 256 == 0 && (!L.has_shared || L.shared_ff % 256 == 0);
 }
 
 // The descriptor grew three times: one that ends before the routing fields means softmax, normalised, no bias; one that
@@ -147,7 +148,7 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         p.y16 = take(a * L.hidden * 4);   // fp16 rows (int8 products) or fp32 rows (fp16 products)
     }
     // the products on prepared rows take both banks: the gate / up product leaves its rows in the order the down product reads
-    const bool rows_ok = grouped_rows_takes(L.gate.type, L.ff, L.hidden) && grouped_rows_takes(L.down.type, L.hidden, L.ff) && (!L.has_shared || L.shared_ff % 128 == 0);
+    const bool rows_ok = banks_aligned(L) && grouped_rows_takes(L.gate.type, L.ff, L.hidden) && grouped_rows_takes(L.down.type, L.hidden, L.ff) && (!L.has_shared || L.shared_ff % 128 == 0);
     p.item_rows = grouped_rows_per_item(L.gate.type, int64_t(a), banks);
     if (p.int8 && plane_gemm_is_fp8(L.gate.type)) {
         p.prepared = rows_ok;    // int8_ok's conditions are the stricter ones
@@ -219,7 +220,7 @@ using namespace tqmoe;
 
 extern "C" size_t tqmoe_layer_workspace_bytes(const tqmoe_layer * layer, int32_t n) {
     if (!layer || n <= 0 || check_layer(layer, nullptr)) return 0;
-    return plan_for(*layer, n).total;
+    return plan_for(*layer, n).total + 256;   // (room to move the areas to a multiple of 16 bytes in a workspace that starts elsewhere)
 }
 
 extern "C" int32_t tqmoe_layer_path(const tqmoe_layer * layer, int32_t n) {
@@ -238,9 +239,10 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
     const int slots = L.topk + (L.has_shared ? 1 : 0), banks = L.n_expert + (L.has_shared ? 1 : 0);
     const Plan p = plan_for(L, n);
     if (p.grouped && banks > 4096) return fail(err, TQMOE_E_ARG, "tqmoe_layer_forward: the grouped products take at most 4096 experts, the shared one included");   // as tqmoe_dispatch does
-    if (!workspace || workspace_bytes < p.total) return fail(err, TQMOE_E_WORKSPACE, "tqmoe_layer_forward: workspace of %zu bytes needed", p.total);
+    const size_t pad = size_t(-reinterpret_cast<uintptr_t>(workspace)) & 15;
+    if (!workspace || workspace_bytes < p.total + pad) return fail(err, TQMOE_E_WORKSPACE, "tqmoe_layer_forward: workspace of %zu bytes needed", p.total + pad);
     if (int32_t rc = need_device(err, "tqmoe_layer_forward")) return rc;
-    uint8_t * ws = static_cast<uint8_t *>(workspace);
+    uint8_t * ws = static_cast<uint8_t *>(workspace) + pad;
     float * logits = logits_out ? logits_out : reinterpret_cast<float *>(ws + p.logits);
     int32_t * ids = ids_out ? ids_out : reinterpret_cast<int32_t *>(ws + p.ids);
     float * weights = weights_out ? weights_out : reinterpret_cast<float *>(ws + p.weights);

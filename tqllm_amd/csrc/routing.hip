@@ -367,7 +367,7 @@ template <bool F32> void launch_router_gemm(const void * w, const void * sg, con
     };
     if constexpr (!F32) {
         const int64_t tiles = (n + kRlTok - 1) / kRlTok, cols = (e + kRlRows - 1) / kRlRows;
-        if (tiles * cols >= kRlBlocks && h >= 512) {
+        if (tiles * cols >= kRlBlocks && h >= 512 && aligned16(w) && aligned16(x)) {
             allow_dynamic_lds(reinterpret_cast<const void *>(&router_gemm_lds_k), kRlLds);
             router_gemm_lds_k<<<dim3(unsigned(tiles), unsigned(cols + (tiles * cols < kRlFull ? 1 : 0))), 64 * kRlWaves, kRlLds, s>>>(
                 static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, side);
