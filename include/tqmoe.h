@@ -21,7 +21,10 @@
 extern "C" {
 #endif
 
-#define TQMOE_ABI_VERSION 1u
+/* What a caller built against this header relies on: the functions, the structures and the bank planes as described below.
+ * 2: the planes of Q4_K, Q6_K, IQ3_S and NVFP4G banks are tile-major (version 1: row-major, IQ3_S 12 bytes and Q6_K 24 bytes
+ *    a sub-block). Planes packed or kept by a program of version 1 are loaded again from their GGUF blocks. */
+#define TQMOE_ABI_VERSION 2u
 
 /* error record, shaped as plugin.h:9 `tq_error` */
 typedef struct tqmoe_error { uint32_t struct_size; int32_t code; char message[256]; } tqmoe_error;

@@ -2,6 +2,9 @@
 (moe_dedup_maps) and the routing histogram (moe_count) bit for bit against the oracle's restatements, moe_group with the
 reference's arguments, the clamp of the SwiGLU inputs (MoeConfig::swiglu_clamp) on every path of the layer against the
 oracle, and the int8 grouped product on natural-order rows (WeightFormat::expert_gemm_i8's operands)."""
+import ctypes as C
+import zlib
+
 import numpy as np
 import pytest
 import torch
@@ -218,3 +221,28 @@ def test_expert_gemm_i8_reference_operands(tq, oracle, wtype_name, per_expert_in
         with pytest.raises(tq.TqmoeError) as ex:
             tq.expert_gemm_i8_ref(q6, xq_nat, xs_ref, counts, groups, topk, A, per_expert_input)
         assert ex.value.code == -2
+
+
+# crc32 of the planes of 96 rows of 512 columns filled with a fixed byte sequence: what a bank kept by a program of this version holds
+PLANES = {2: (0x37dd7d8b, 0x7004b165), 8: (0xe2d3dbb9, 0x4eaa00af), 10: (0x0e7cf40c, 0x3dd79d79), 11: (0x9d737ae9, 0x2986c187),
+          12: (0xc7c24cdc, 0xd60eccba), 13: (0x0663a3bc, 0xfeb3dbc8), 14: (0xcdbf0f01, 0x111f62c7), 16: (0x0faa6a38, 0x1b00d6bd),
+          17: (0x24a5e439, 0x5cc060df), 18: (0x0c26a6e8, 0x3ba2462c), 19: (0xcceaf6d5, 0x9f79ee2f), 20: (0x37dd7d8b, 0x7004b165),
+          21: (0x196f4c98, 0x8bc5063a), 22: (0xca55733a, 0x6511829d), 23: (0x3e1b71fe, 0xbd16e1c5), 323: (0x6ea3389e, 0x0ced4617)}
+
+
+def test_bank_planes_are_those_of_the_version(tq):
+    """A caller may pack planes by the header's description or keep them: they change only with TQMOE_ABI_VERSION."""
+    assert tq.abi_version() == 2
+    got = {}
+    for wtype, (elems, nbytes) in sorted(tq.api.BLOCK.items()):
+        n = 96 * 512 // elems
+        raw = (np.arange(n * nbytes, dtype=np.uint64) * 2654435761 >> 11).astype(np.uint8).reshape(n, nbytes)
+        if wtype == tq.NVFP4G:
+            raw[:, 0:4] = raw[0, 0:4]            # one global a row
+        bank = tq.ExpertBank(wtype, raw.reshape(-1), 3, 32, 512)
+        bank.codes.zero_(), bank.aux.zero_()     # (padding is left as it was)
+        err = tq.api._err()
+        src = torch.from_numpy(raw.reshape(-1)).cuda()
+        assert tq.lib().tqmoe_bank_load(wtype, src.data_ptr(), 96, 512, bank.codes.data_ptr(), bank.aux.data_ptr(), None, torch.cuda.current_stream().cuda_stream, C.byref(err)) == 0
+        got[wtype] = tuple(zlib.crc32(t.cpu().numpy().tobytes()) for t in (bank.codes, bank.aux))
+    assert got == PLANES, got
