@@ -34,11 +34,13 @@ def test_router_logits(tq, oracle, name, n):
 
 @pytest.mark.parametrize("n,e,h,shared", [(32, 512, 2048, True), (100, 33, 512, False), (4096, 512, 2048, True), (77, 64, 192, True),
                                           (250, 600, 512, False), (1000, 130, 192, True), (9000, 1100, 256, True),
-                                          (2100, 64, 320, True), (4096, 100, 2048, False)])   # few router rows: eight waves a block
+                                          (2100, 64, 320, True), (4096, 100, 2048, False),     # few router rows
+                                          (87, 512, 512, True), (88, 512, 512, True), (4096, 64, 512, False), (8190, 60, 256, True)])
 def test_router_gemm_path(tq, oracle, n, e, h, shared):
-    """bf16 router rows and bf16 inputs take the matrix-pipe kernel from about 120,000 tokens x rows (64-token blocks, 128-token
-    blocks for the largest grids), the wave-per-row kernel below: same logits to the same bar, ragged token and row counts,
-    with and without the shared-gate row; on the matrix-pipe kernel the rows of a large batch equal those of a smaller one."""
+    """bf16 router rows and bf16 inputs take the matrix-pipe kernels from 45,000 tokens x rows (16 to 64 tokens a block; through
+    LDS for more than 64 rows and many blocks), the wave-per-row kernel below: same logits to the same bar, ragged token and
+    row counts, with and without the shared-gate row; on the matrix-pipe kernels the rows of a large batch equal those of a
+    smaller one."""
     rng = np.random.default_rng(n + e)
     wb, wv = oracle.to_bf16((rng.standard_normal((e, h)) * 0.02).astype(np.float32))
     gb, gv = oracle.to_bf16((rng.standard_normal(h) * 0.02).astype(np.float32))
@@ -58,10 +60,10 @@ def test_router_gemm_path(tq, oracle, n, e, h, shared):
         assert torch.equal(part, logits[5:5 + m])
 
 
-@pytest.mark.parametrize("n,e,h,shared", [(4096, 64, 2048, False), (3000, 130, 192, True), (2100, 64, 320, True), (1000, 64, 2048, False)])
+@pytest.mark.parametrize("n,e,h,shared", [(4096, 64, 2048, False), (3000, 130, 192, True), (2100, 64, 320, True), (1000, 64, 2048, False), (861, 64, 512, True), (862, 64, 512, True), (8192, 120, 64, False)])
 def test_router_gemm_path_f32(tq, oracle, n, e, h, shared):
-    """fp32 router rows and fp32 inputs take the matrix-pipe kernel from the same size on (the last case stays on the
-    wave-per-row kernel): fp32 products and sums, ragged shapes, with and without the shared-gate row."""
+    """fp32 router rows and fp32 inputs take the matrix-pipe kernel from 56,000 tokens x rows, the wave-per-row kernel below: fp32
+    products and sums, ragged shapes, with and without the shared-gate row."""
     rng = np.random.default_rng(n + e + h)
     w = (rng.standard_normal((e, h)) * 0.02).astype(np.float32)
     gate = (rng.standard_normal(h) * 0.02).astype(np.float32)

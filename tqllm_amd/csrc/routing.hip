@@ -130,7 +130,9 @@ template <int WT> int32_t launch_router_x(uint32_t xtype, const void * w, const 
 // The last row of blocks takes the shared expert's gate row (or stores its zeros): a wave a token.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-constexpr int kRouterGemmMin = 30000;   // tokens x router rows from which a bf16 router and input take the GEMM
+// Tokens x router rows from which a router and input of one type take the GEMM (us, wave per row / GEMM, 2048 columns: bf16 32768
+// 8.4 / 10.8, 62464 14.3 / 10.7; fp32 33000 14.4 / 24.5, 62464 28.2 / 24.5; 1024 to 4096 columns cross at the same sizes).
+template <bool F32> constexpr int kRouterGemmMin = F32 ? 56000 : 45000;
 constexpr int kRgWaves = 8, kRgRows = 64, kRgPitch = kRgRows + 4;   // floats of a token's row in the exchange space: four rows apart, other banks
 template <int TA> constexpr int kRgLds = 4 * TA * 16 * kRgPitch * int(sizeof(float));
 
@@ -250,10 +252,11 @@ __global__ __launch_bounds__(64 * kRgWaves) void router_gemm_k(const uint8_t * _
 // way, two blocks a compute unit. The eight parts of the columns follow each other and join in the order the kernel above adds them: same bits.
 // (512 experts, 2048 columns, 4096 tokens: 24 us; 45 with every wave's operands from memory, 32 with stages of 512 bytes a
 // row that pass registers.)
-// Blocks from which it is the faster one (in us, this / operands from memory: 96 blocks 19 / 27, 64 blocks 15 / 22, 24 blocks
-// 19 / 12).
+// Blocks from which it is the faster one (in us, this / operands from memory, 2048 columns: 64 blocks over 256 or 512 router
+// rows 18.7 / 17.4, 128 blocks 19.2 / 27; 32 blocks 18.6 / 13.4; 1024 and 4096 columns cross at the same numbers). Up to 64
+// router rows half the tile would be empty (60 rows, 4096 tokens: 18.6 / 13.5).
 constexpr int kRlBlocks = 48;
-constexpr int kRlFull = 224;    // blocks from which none are added for the gate row's column (256: 24 us against 33; 126: 26 against 20)
+constexpr int kRlFull = 224;    // blocks from which none are added for the gate row's column (256: 23 us against 31; 128: 32 against 19)
 constexpr int kRlTok = 64, kRlRows = 128, kRlRing = 3, kRlStage = (kRlTok + kRlRows) * 128, kRlLds = kRlRing * kRlStage, kRlWaves = 8;
 __global__ __launch_bounds__(64 * kRlWaves) void router_gemm_lds_k(const uint8_t * __restrict__ w, const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x,
                                                          float * __restrict__ logits, int h, int e, int n, RouterSide side) {
@@ -367,15 +370,17 @@ template <bool F32> void launch_router_gemm(const void * w, const void * sg, con
     };
     if constexpr (!F32) {
         const int64_t tiles = (n + kRlTok - 1) / kRlTok, cols = (e + kRlRows - 1) / kRlRows;
-        if (tiles * cols >= kRlBlocks && h >= 512 && aligned16(w) && aligned16(x)) {
+        if (tiles * cols >= kRlBlocks && e > kRgRows && h >= 512 && aligned16(w) && aligned16(x)) {
             allow_dynamic_lds(reinterpret_cast<const void *>(&router_gemm_lds_k), kRlLds);
             router_gemm_lds_k<<<dim3(unsigned(tiles), unsigned(cols + (tiles * cols < kRlFull ? 1 : 0))), 64 * kRlWaves, kRlLds, s>>>(
                 static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, side);
             return;
         }
     }
-    if (blocks(4) >= 384) go(&router_gemm_k<F32, 4>, 4, kRgLds<4>);
-    else if (blocks(2) >= 256) go(&router_gemm_k<F32, 2>, 2, kRgLds<2>);
+    // (2048 columns, us with 16 / 32 / 64 tokens a block: bf16, 128 blocks of 32 tokens 14.9 / 13.5 / 17.6, 128 of 64 28 / 21 / 19; fp32, 128
+    // blocks of 32 tokens 30 / 43 / 71, 256 of 64 106 / 85 / 79)
+    if (blocks(4) >= (F32 ? 256 : 128)) go(&router_gemm_k<F32, 4>, 4, kRgLds<4>);
+    else if (blocks(2) >= (F32 ? 256 : 128)) go(&router_gemm_k<F32, 2>, 2, kRgLds<2>);
     else go(&router_gemm_k<F32, 1>, 1, kRgLds<1>);
 }
 
@@ -896,7 +901,7 @@ extern "C" int32_t tqmoe_router(const void * router, uint32_t wtype, const void 
 
 int32_t tqmoe::enqueue_router(const void * router, uint32_t wtype, const void * shared_gate, const void * x, uint32_t xtype, float * logits, int hidden, int experts, int n,
                               const RouterSide & side, hipStream_t s, tqmoe_error * err) {
-    if (wtype == xtype && (wtype == TQMOE_BF16 || wtype == TQMOE_F32) && int64_t(n) * (experts + 1) >= kRouterGemmMin && hidden % 64 == 0 && !side.image) {
+    if (wtype == xtype && (wtype == TQMOE_BF16 || wtype == TQMOE_F32) && int64_t(n) * (experts + 1) >= (wtype == TQMOE_F32 ? kRouterGemmMin<true> : kRouterGemmMin<false>) && hidden % 64 == 0 && !side.image) {
         if (wtype == TQMOE_F32) launch_router_gemm<true>(router, shared_gate, x, logits, hidden, experts, n, side, s);
         else launch_router_gemm<false>(router, shared_gate, x, logits, hidden, experts, n, side, s);
     } else if (wtype == TQMOE_F32) launch_router_x<TQMOE_F32>(xtype, router, shared_gate, x, logits, hidden, experts, n, side, s);
