@@ -292,7 +292,7 @@ def measure_point(torch, tq, cfg, key, trios, gen, T, args, traffic):
 
     gu_s, dn_s, step_s = kernels["gateup"] * 1e-3, kernels["down"] * 1e-3, ms_step * 1e-3
     if path == "decode":
-        kname = "iq4xs_mfma_k<2> (gate + up + SwiGLU)" if cfg["wtype"] == IQ4_XS else "gateup_k<%s> (gate + up + SwiGLU)" % cfg["fmt"]
+        kname = "decode_mfma_k<%s, 2> (gate + up + SwiGLU)" % cfg["fmt"]
         roofline = {"bound": "hbm", "kernel": kname, "achieved": round(gu_bytes / gu_s / 1e9, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",
                     "frac": round(gu_bytes / gu_s / HBM_PEAK, 4), "traffic": None, "algorithmic_bytes_per_launch": int(gu_bytes),
                     "us_per_launch": round(gu_s * 1e6, 2)}
@@ -302,8 +302,8 @@ def measure_point(torch, tq, cfg, key, trios, gen, T, args, traffic):
     else:
         op = {"grouped_i8": "int8", "grouped_f16": "fp16", "grouped_fp8": "fp8"}[path]
         kname = {"grouped_i8": "plane_gemm_k<2, %s> (grouped gate + up int8 MFMA product + SwiGLU)" % cfg["fmt"],
-                 "grouped_f16": "expert_gemm_f16_k<%s,2> (grouped gate + up fp16 MFMA product + SwiGLU)" % cfg["fmt"],
-                 "grouped_fp8": "plane_gemm_k<2, %s> (grouped gate + up fp8 MFMA product + SwiGLU)" % cfg["fmt"]}[path]
+                 "grouped_f16": "expert_gemm_f16_k<%s,2> (the general entry's grouped gate + up fp16 MFMA product + SwiGLU; the layer runs grouped_rows_k on prepared rows)" % cfg["fmt"],
+                 "grouped_fp8": "grouped_rows_k<%s> (grouped gate + up fp8 MFMA product + SwiGLU)" % cfg["fmt"]}[path]
         roofline = {"bound": "mfma", "kernel": kname, "achieved": round(gu_ops / gu_s / 1e12, 2), "peak": PEAK[op] / 1e12, "unit": "TFLOP/s",
                     "frac": round(gu_ops / gu_s / PEAK[op], 4), "traffic": None,
                     "ops": "multiply-add = 2 operations; peak = dense %s %.1f POP/s" % (op, PEAK[op] / 1e15),

@@ -164,7 +164,7 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         p.xs = take(gwords * 4);
         p.aq = take(grows * L.ff);
         p.as = take(gwords * 4);
-        p.blocks = act_blocks_of(L) && !plane_gemm_is_fp8(L.gate.type);
+        p.blocks = act_blocks_of(L);
         p.rq = take(c * L.hidden);        // the chunk's input rows as int8, quantised once, then gathered per assignment
         p.rs = take(c * 4 * (p.blocks ? size_t(L.hidden / 32) : 1));
         if (p.blocks) {

@@ -313,7 +313,7 @@ template <class LEVEL> __device__ __forceinline__ void lattice_tables(uint8_t * 
 }
 struct WLatticeBase {   // row-major, a 16-byte record per super-block whose first 16 bits are d
     static constexpr int kPlanes = 2, kTabBytes = 16 * 32;
-    static constexpr bool kMin = false, kRowMul = false, kFoldSub = false;
+    static constexpr bool kMin = false, kFoldSub = false;
     typedef uint32_t Rec;    // unused by the decode (the scales sit in the code bytes)
     typedef uint32_t DRec;
     struct Src { const uint8_t * codes, * aux; };
