@@ -23,10 +23,11 @@
 // instructions; with the two banks' eight accumulators (128 registers) two waves fit a SIMD, and one of them decodes while
 // the other's products run. Items of one and two row tiles have loops of their own with fewer products.
 //
-// What bounds it: Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 260 us, 0.8 PFLOP/s, matrix pipe 40 % busy;
-// NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 1.0 ms. A stage of an item with four row tiles takes 5300 cycles
-// where its SIMD's two waves have 2048 of matrix and 1300 to 2000 of vector work. Items of one row tile are bound by the
-// decode (IQ3_S, 512 tokens: 2.5 TB/s of codes).
+// What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 262 us, 0.8
+// PFLOP/s, matrix pipe 43 % busy, vector pipe 52 %; NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 985 us, 40 % and
+// 51 %. A stage of an item with four row tiles takes about 4800 cycles where its SIMD's two waves have 2048 of matrix work.
+// Items of one row tile are bound by the decode (IQ3_S, 512 tokens: 2.6 TB/s of codes, vector pipe 69 %, LDS 51 %, three
+// fifths of that bank conflicts of the lattice's look-ups).
 #pragma once
 #include "decode_api.cuh"
 #include "decode_table.cuh"
