@@ -96,8 +96,8 @@ bool act_blocks_of(const tqmoe_layer & L) { return int8_mode_of(L) == 1; }
 // Formats whose 8-bit grouped products are the faster ones at n tokens: the lattice formats of two and three bits that have
 // no fp16 products on prepared rows (a tenth faster than the fp16 kernel that takes every format), NVFP4G on its fp8
 // products; and IQ4_XS from kInt8Tokens tokens (see there). Q4_K, Q6_K and IQ3_S run on prepared fp16 rows at every size (Q4_K at 4096
-// tokens 576 us a layer against 855 on its three int8 planes; IQ3_S at 512 tokens 260 against 393 on the general fp16
-// kernel), the others on the general fp16 kernel, 5 to 25 % faster than int8 there.
+// tokens 479 us a layer against 827 on its three int8 planes; IQ3_S at 512 tokens 240 against 391 on its int8
+// planes), the others on the general fp16 kernel, 5 to 25 % faster than int8 there.
 bool int8_faster(uint32_t type, int n) {
     switch (type) {
         case TQMOE_IQ4_XS: return n >= kInt8Tokens;
