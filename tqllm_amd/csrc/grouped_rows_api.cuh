@@ -23,6 +23,7 @@ struct GroupedArgs {
     Glu glu;
     int row_tiles;            // NVFP4G: x is in operand-major row tiles (each expert's rows padded to whole tiles), xs by row of those
     int out_bf16;             // NVFP4G: 16-bit results are bf16
+    float * out_scale;        // int8 gate / up with a scale per 32 values: the scales of the act rows, [assignments][rows / 32]
 };
 
 // index of the gathered row tiles, written beside the items where tile_base is not null
@@ -38,5 +39,11 @@ void enqueue_grouped_plan(const int * counts, const int * offsets, int experts, 
 // assignments: total entries of perm (it bounds the items)
 void enqueue_grouped_products(const tqmoe_bank & b0, const tqmoe_bank * b1, const void * x, const float * xs, const int * perm, const int4 * plan, int64_t assignments,
                               int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows, bool row_tiles = false, bool out_bf16 = false);
+
+// int8 products on rows in quantiser order (a row per token or per assignment); blocks: a scale per 32 values
+bool grouped_i8_takes(uint32_t type, int rows, int cols);
+int grouped_i8_per_item(bool blocks, int64_t assignments, int experts);   // input rows of an item at most: 32 or 64
+void enqueue_grouped_i8(const tqmoe_bank & b0, const tqmoe_bank * b1, const int8_t * x, const float * xs, bool blocks, const int * perm, const int4 * plan, int64_t assignments,
+                        int xdiv, void * out, float * out_scale, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows);
 
 }  // namespace tqmoe

@@ -149,6 +149,7 @@ Plan plan_for(const tqmoe_layer & L, int n) {
     }
     // the products on prepared rows take both banks: the gate / up product leaves its rows in the order the down product reads
     const bool rows_ok = banks_aligned(L) && grouped_rows_takes(L.gate.type, L.ff, L.hidden) && grouped_rows_takes(L.down.type, L.hidden, L.ff) && (!L.has_shared || L.shared_ff % 128 == 0);
+    const bool rows_i8 = banks_aligned(L) && grouped_i8_takes(L.gate.type, L.ff, L.hidden) && grouped_i8_takes(L.down.type, L.hidden, L.ff);
     p.item_rows = grouped_rows_per_item(L.gate.type, int64_t(a), banks);
     if (p.int8 && plane_gemm_is_fp8(L.gate.type)) {
         p.prepared = rows_ok;    // int8_ok's conditions are the stricter ones
@@ -156,6 +157,15 @@ Plan plan_for(const tqmoe_layer & L, int n) {
         p.rs = take(c * 4);
         p.aq = take(a * L.ff);
         p.as = take(a * 4);
+        p.items = take(size_t(1 + grouped_rows_items(int64_t(a), banks, p.item_rows)) * sizeof(int4));
+    } else if (p.int8 && rows_i8) {
+        p.prepared = true;
+        p.blocks = act_blocks_of(L);
+        p.item_rows = grouped_i8_per_item(p.blocks, int64_t(a), banks);
+        p.rq = take(c * L.hidden);
+        p.rs = take(c * 4 * (p.blocks ? size_t(L.hidden / 32) : 1));
+        p.aq = take(a * L.ff);
+        p.as = take(a * 4 * (p.blocks ? size_t(L.ff / 32) : 1));
         p.items = take(size_t(1 + grouped_rows_items(int64_t(a), banks, p.item_rows)) * sizeof(int4));
     } else if (p.int8) {
         const size_t grows = size_t(tqmoe_grouped_rows(int64_t(a), banks));
@@ -275,7 +285,7 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
         side.banks = banks;
     }
     if (!p.grouped || whole) {
-        side.rows = !p.grouped ? kRowsImage : !p.int8 ? (p.prepared ? kRowsHalves : kRowsNone) : p.prepared ? kRowsFp8 : p.blocks ? kRowsInt8Blocks : kRowsInt8;
+        side.rows = !p.grouped ? kRowsImage : !p.int8 ? (p.prepared ? kRowsHalves : kRowsNone) : plane_gemm_is_fp8(L.gate.type) ? kRowsFp8 : p.blocks ? kRowsInt8Blocks : kRowsInt8;
         side.x = x;
         side.xtype = xtype;
         side.cols = L.hidden;
@@ -321,18 +331,34 @@ static int32_t layer_forward(const tqmoe_layer * layer, const void * x, uint32_t
                 lists.index = grouped_index(xs, int64_t(c) * slots, banks, &lists.items);
             }
             if (int32_t rc = enqueue_layer_dispatch(cid, counts, offsets, perm, banks, c, slots, chunk_counts, lists, hs, err)) return rc;
-            if (p.prepared && p.int8) {   // E4M3 rows
-                const hipStream_t st = static_cast<hipStream_t>(stream);
+            if (p.prepared && p.int8) {   // 8-bit rows: E4M3 or int8
                 uint8_t * rq = ws + p.rq, * aq = ws + p.aq;
                 float * rs = reinterpret_cast<float *>(ws + p.rs), * as = reinterpret_cast<float *>(ws + p.as);
                 int4 * items = reinterpret_cast<int4 *>(ws + p.items);
                 const int shared_expert = L.has_shared ? banks - 1 : -1;
                 const int64_t a = int64_t(c) * slots;
-                if (!whole)
-                    if (int32_t rc = tqmoe_quant_rows_fp8(xb + size_t(t0) * L.hidden * xbytes, xtype, c, L.hidden, rq, rs, stream, err)) return rc;
-                enqueue_grouped_products(L.gate, &L.up, rq, rs, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, st, p.item_rows);
-                if (int32_t rc = tqmoe_quant_rows_fp8(act16, TQMOE_F16, a, L.ff, aq, as, stream, err)) return rc;
-                enqueue_grouped_products(L.down, nullptr, aq, as, perm, items, a, 1, y16, false, shared_expert, L.shared_ff, Glu{0.f, 0}, st, p.item_rows);
+                const void * xc = xb + size_t(t0) * L.hidden * xbytes;
+                const Glu none{0.f, 0};
+                if (plane_gemm_is_fp8(L.gate.type)) {
+                    if (!whole)
+                        if (int32_t rc = tqmoe_quant_rows_fp8(xc, xtype, c, L.hidden, rq, rs, stream, err)) return rc;
+                    enqueue_grouped_products(L.gate, &L.up, rq, rs, perm, items, a, slots, act16, false, shared_expert, L.shared_ff, glu, hs, p.item_rows);
+                    if (int32_t rc = tqmoe_quant_rows_fp8(act16, TQMOE_F16, a, L.ff, aq, as, stream, err)) return rc;
+                    enqueue_grouped_products(L.down, nullptr, aq, as, perm, items, a, 1, y16, false, shared_expert, L.shared_ff, none, hs, p.item_rows);
+                } else {
+                    int8_t * rq8 = reinterpret_cast<int8_t *>(rq), * aq8 = reinterpret_cast<int8_t *>(aq);
+                    if (!whole) {
+                        const int32_t rc = p.blocks ? tqmoe_quant_rows_i8_blocks(xc, xtype, c, L.hidden, rq8, rs, nullptr, stream, err) : tqmoe_quant_rows_i8(xc, xtype, c, L.hidden, rq8, rs, stream, err);
+                        if (rc) return rc;
+                    }
+                    if (p.blocks) {   // (a weight tile's act values are one block: the gate / up product quantises them)
+                        enqueue_grouped_i8(L.gate, &L.up, rq8, rs, true, perm, items, a, slots, aq8, as, shared_expert, L.shared_ff, glu, hs, p.item_rows);
+                    } else {
+                        enqueue_grouped_i8(L.gate, &L.up, rq8, rs, false, perm, items, a, slots, act16, nullptr, shared_expert, L.shared_ff, glu, hs, p.item_rows);
+                        if (int32_t rc = tqmoe_quant_rows_i8(act16, TQMOE_F16, a, L.ff, aq8, as, stream, err)) return rc;
+                    }
+                    enqueue_grouped_i8(L.down, nullptr, aq8, as, p.blocks, perm, items, a, 1, y16, nullptr, shared_expert, L.shared_ff, none, hs, p.item_rows);
+                }
                 if (int32_t rc = launched(err, "tqmoe_layer_forward (grouped products)")) return rc;
                 if (int32_t rc = combine(y16, TQMOE_F16, L.has_shared ? y16 + size_t(L.topk) * L.hidden : nullptr)) return rc;
                 continue;

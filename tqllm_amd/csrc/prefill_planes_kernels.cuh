@@ -31,6 +31,7 @@
 #include "decode_api.cuh"
 #include "formats.cuh"
 #include "grouped_rows_api.cuh"
+#include "int8_fold.cuh"
 #include "row_quant.cuh"
 
 #include <algorithm>
@@ -121,25 +122,8 @@ __device__ __forceinline__ void split_planes(int v, uint8_t & hi, uint8_t & lo) 
     hi = uint8_t((v - l) >> 6);
 }
 
-// The two ways through the kernel (a lone row tile, a shared chunk) must give a row the same bits: the fold of a
-// super-block and the epilogue are spelled with explicitly rounded operations, and the product that is converted to fp16
-// passes through an opaque register, so that no path turns multiply + convert into one mixed-precision instruction
-// (one rounding instead of two: different bits at ties).
+// acc + (64 h + l) d: the two ways through the kernel (a lone row tile, a shared chunk) must give a row the same bits (int8_fold.cuh)
 __device__ __forceinline__ float fold_sb(float acc, int h, int l, float d) { return __fmaf_rn(float((h << 6) + l), d, acc); }
-__device__ __forceinline__ uint16_t to_half_bits(float v) {
-    asm volatile("" : "+v"(v));
-    return __half_as_ushort(__float2half_rn(v));
-}
-__device__ __forceinline__ uint16_t swiglu_half(float g_acc, float u_acc, float sc, const Glu glu) {
-    float gv = __fmul_rn(g_acc, sc), uv = __fmul_rn(u_acc, sc);
-    glu_clamp_inputs(glu, gv, uv);
-    const float den = __fadd_rn(1.f, __expf(-gv));
-    return to_half_bits(__fmul_rn(glu_clamp_silu(glu, __fdiv_rn(gv, den)), uv));
-}
-__device__ __forceinline__ uint16_t scaled_half(float acc, float sc, int bf16) {
-    const float v = __fmul_rn(acc, sc);
-    return bf16 ? float_to_bf16_bits(v) : to_half_bits(v);
-}
 
 __device__ const int8_t kIq4Values[16] = {-127, -104, -83, -65, -49, -35, -22, -10, 1, 13, 25, 38, 53, 69, 89, 113};
 
