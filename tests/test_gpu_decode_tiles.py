@@ -1,5 +1,5 @@
 """GPU parity of the decode products of the tile-major formats where their split can go wrong: a row cut over waves into
-equal and unequal shares (eleven super-blocks over eight, four and two waves), ragged last tiles (the row-wise kernels take them), batches that stage their input rows and that walk several
+equal and unequal shares (eleven super-blocks over eight, four and two waves), ragged last tiles (the row-wise kernels take them), batches that stage their input rows and that walk several (two, four)
 row tiles a wave, more input rows of one expert than a block serves. Against float64 on the decoded weights."""
 import numpy as np
 import pytest
@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 
 FORMATS = {"iq4_xs": 23, "q4_k": 12, "q6_k": 14, "iq3_s": 21, "nvfp4": 323}
 SHAPES = [(64, 1280, 1, 3), (96, 1536, 2, 3), (32, 1792, 1, 2), (40, 512, 5, 3), (33, 768, 14, 3), (1024, 512, 40, 4), (160, 2304, 13, 1),
-          (64, 2816, 1, 3), (64, 2816, 6, 3), (320, 2816, 18, 4), (1024, 2816, 17, 4), (2048, 1792, 30, 2)]
+          (64, 2816, 1, 3), (64, 2816, 6, 3), (320, 2816, 18, 4), (1024, 2816, 17, 4), (2048, 1792, 30, 2), (2048, 512, 80, 4), (2048, 256, 160, 3)]
 
 
 @pytest.mark.parametrize("fmt", sorted(FORMATS))

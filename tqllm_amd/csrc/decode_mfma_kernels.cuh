@@ -549,10 +549,11 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     // unit: the block's search for its input rows and their staging are paid once for all of them, but a grid of two or
     // three blocks per unit, some of which find their expert taken by another and leave, ends in a round that most units
     // sit out. A Q4_K/Q6_K layer of 23 tokens over 125 experts takes 99 us with two blocks as the least, 90 with five; IQ3_S with
-    // 20 tokens over 64 experts 94 and 78.
+    // 20 tokens over 64 experts 94 and 78. (Not where a shared expert has fewer columns than the others: the waves' steps then
+    // differ. 64 tokens, top-8 of 256, without a shared expert: 170 us a layer with one row tile a wave, 164 with four.)
     constexpr int kLeastBlocks = 1280;
     int tl = 1;
-    if (staged && nb == 1 && NSB % wk == 0 && shared_lim == (gateup ? b0.rows : b0.cols))
+    if (staged && nb == 1 && NSB % wk == 0 && (slots <= topk || shared_lim == (gateup ? b0.rows : b0.cols)))
         while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= kLeastBlocks) tl *= 2;
     const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl)), unsigned(A));
     const int a_off = int(lds);
