@@ -124,7 +124,7 @@ template <> struct MfmaFormat<TQMOE_NVFP4G> : MfmaNibbles {
     }
 };
 template <> struct MfmaFormat<TQMOE_IQ3_S> : MfmaBase {
-    static constexpr int kCodeBytes = 3072, kRecBytes = 512, kLattice = 512;
+    static constexpr int kCodeBytes = 3072, kRecBytes = 512, kLattice = 2304;
     struct Codes { uint2 qs[4]; uint4 sg[2]; };
     typedef uint4 Rec;
     static __device__ __forceinline__ void codes(const uint8_t * p, int n, int g, Codes & c) {
@@ -136,24 +136,39 @@ template <> struct MfmaFormat<TQMOE_IQ3_S> : MfmaBase {
     static __device__ __forceinline__ Rec rec(const uint8_t * p, int n) { return *reinterpret_cast<const uint4 *>(p + n * 16); }
     // The lattice in LDS holds eight times the odd magnitudes: 8 (2 k + 1) is the byte k << 4 | 8, and its negative the same
     // byte with the upper four bits inverted, so that a sign is one exclusive or.
+    // Points 0..255 are the first 1 KB; the others follow 1, 2, 4 and 8 KB behind it, so that an index's ninth bit q of the four at
+    // a time is an address bit where it stands (and a sign bit is a selector where it stands: seven of 45 instructions a sub-block
+    // less; 64 tokens, top-8 of 256: 163.9 -> 157.2 us a layer).
+    static __device__ __forceinline__ void lattice(uint32_t * lat, int tid, int threads) {
+        for (int i = tid; i < 512; i += threads) {
+            const uint32_t m = d_iq3s_grid.v[i] << 3;
+            if (i < 256) lat[i] = m;
+            else for (int q = 0; q < 4; ++q) lat[(256 << q) + i - 256] = m;
+        }
+    }
     // lookup: the four points' magnitudes, on their way from LDS; signed_of: with the signs
     static __device__ __forceinline__ v4i lookup(const Codes & c, const Rec & r, int ib, int g, const uint32_t * lat) {
         const uint32_t qs = (ib & 1) ? c.qs[ib >> 1].y : c.qs[ib >> 1].x;
-        const uint32_t qh = ((ib < 4 ? r.y : r.z) >> (8 * (ib & 3))) >> (4 * g);
+        const uint32_t qh = (((ib < 4 ? r.y : r.z) >> (8 * (ib & 3))) >> (4 * g)) << 10;
         v4i w;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             uint32_t low = ((qs >> (8 * q)) & 0xFFu) << 2;   // (a byte shifted: one instruction, where nothing is merged into it)
             asm("" : "+v"(low));
-            w[q] = *reinterpret_cast<const int *>(reinterpret_cast<const uint8_t *>(lat) + (low | ((qh << (10 - q)) & 0x400u)));
+            w[q] = *reinterpret_cast<const int *>(reinterpret_cast<const uint8_t *>(lat) + (low | (qh & (0x400u << q))));
         }
         return w;
     }
     static __device__ __forceinline__ v4i signed_of(v4i w, const Codes & c, int ib, int g) {
         const uint4 s4 = c.sg[ib >> 2];
         const uint32_t sg = ((ib & 3) == 0 ? s4.x : (ib & 3) == 1 ? s4.y : (ib & 3) == 2 ? s4.z : s4.w) >> (4 * g);
+        // A sign bit where it stands (a byte 0 or 1 << q) picks from a pool with 0x00 at 0 and 0xF0 at 1, 2 and 4; 8 picks the sign of
+        // the pool's byte 1 in all bits.
 #pragma unroll
-        for (int q = 0; q < 4; ++q) w[q] ^= int(__builtin_amdgcn_perm(0u, 0x0000F000u, (sg >> q) & 0x01010101u));   // 0xF0 where the sign bit is set
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t m = __builtin_amdgcn_perm(0x000000F0u, 0x00F0F000u, sg & (0x01010101u << q));
+            w[q] ^= int(q < 3 ? m : m & 0xF0F0F0F0u);
+        }
         return w;
     }
     static __device__ __forceinline__ v4i decode(const Codes & c, const Rec & r, int ib, int g, const uint32_t * lat) { return signed_of(lookup(c, r, ib, g, lat), c, ib, g); }
@@ -211,7 +226,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     __shared__ int ql[kMaxWaves * 2][32];
     __shared__ uint32_t lat[F::kLattice];
     if constexpr (FMT == TQMOE_IQ3_S)   // eight times the magnitudes (behind a barrier before the first use)
-        for (int i = threadIdx.x; i < 512; i += blockDim.x) lat[i] = d_iq3s_grid.v[i] << 3;
+        F::lattice(lat, threadIdx.x, blockDim.x);
     const int a = blockIdx.y;
     int e;
     if constexpr (ROUTE > 0) {
@@ -424,7 +439,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                 const int ib = step / (NB * G), nb = step / G % NB, grp = step % G;
                 if (step % (kPart * NB * G) == 0) part_a(ib);
                 if constexpr (FMT == TQMOE_IQ3_S) {   // the next step's look-ups are under way while this step's signs are put on and the sums before are added
-                                                      // (64 tokens, top-8 of 256: 164.1 -> 161.6 us a layer)
+                                                      // (64 tokens, top-8 of 256: 164 -> 161.6 us a layer)
                     if (step == 0) found = F::lookup(cur.code[0], cur.rec[0], 0, g, lat);
                     w = F::signed_of(found, cur.code[nb], ib, g);
                     if (step + 1 < kSteps) found = F::lookup(cur.code[(step + 1) % NB], cur.rec[(step + 1) % NB], (step + 1) / NB, g, lat);
@@ -647,7 +662,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
         return sum * c.rf;
     };
     if constexpr (FMT == TQMOE_IQ3_S) {
-        for (int i = threadIdx.x; i < 512; i += blockDim.x) lat[i] = d_iq3s_grid.v[i] << 3;
+        F::lattice(lat, threadIdx.x, blockDim.x);
         __syncthreads();
     }
     // (a second unit's loads in flight under the first's products: the registers of a block of sixteen waves spill, 7.9 -> 23.7 us
