@@ -42,6 +42,8 @@ __device__ __forceinline__ v4i decode_table(const Table16 & t, uint2 c) {
     return v4i{int(pick(t, c.x & m)), int(pick(t, (c.x >> 4) & m)), int(pick(t, c.y & m)), int(pick(t, (c.y >> 4) & m))};
 }
 
+// Every other sub-block (down_combine_k with half tiles): half_codes loads sub-blocks odd, odd + 2, ... into the places of 0, 2, ...;
+// odd_rec moves their scales (minimums, index bits) there; d and dmin are read from the record as it was.
 // What the kernel needs of a format. A lane's part of a super-block: Codes and Rec, loaded from the tile's code and record
 // blocks (kCodeBytes, kRecBytes per tile and super-block). decode: operand B of sub-block ib. Scales: kGroups integer
 // scales per sub-block (kFloat: fp32 ones) with the super-block's d behind them; kMin: a minimum per sub-block times the
@@ -61,6 +63,11 @@ struct MfmaNibbles : MfmaBase {   // sixteen code bytes a sub-block in the canon
 #pragma unroll
         for (int ib = 0; ib < 8; ++ib) c.c[ib] = *reinterpret_cast<const uint2 *>(q + ib * 512);
     }
+    static __device__ __forceinline__ void half_codes(const uint8_t * p, int n, int g, int odd, Codes & c) {
+        const uint8_t * q = p + n * 16 + g * 8 + odd * 512;
+#pragma unroll
+        for (int ib = 0; ib < 8; ib += 2) c.c[ib] = *reinterpret_cast<const uint2 *>(q + ib * 512);
+    }
 };
 template <> struct MfmaFormat<TQMOE_IQ4_XS> : MfmaNibbles {
     static constexpr int kRecBytes = 256;
@@ -72,6 +79,9 @@ template <> struct MfmaFormat<TQMOE_IQ4_XS> : MfmaNibbles {
     }
     static __device__ __forceinline__ int scale(const Rec & r, int ib, int) { return iq4xs_lsm32(r, ib); }
     static __device__ __forceinline__ float d(const Rec & r) { return half_bits_to_float(iq4xs_d_bits(r)); }
+    static __device__ __forceinline__ Rec odd_rec(const Rec & r, int odd) {   // five fields in x, then three from bit 14 of y: the fifth's successor is y's first
+        return make_uint2(odd ? ((r.x >> 6) & 0x00FFFFFFu) | ((r.y << 10) & 0x3F000000u) : r.x, r.y >> (6 * odd));
+    }
 };
 template <> struct MfmaFormat<TQMOE_Q4_K> : MfmaNibbles {
     static constexpr int kRecBytes = 512;
@@ -96,6 +106,7 @@ template <> struct MfmaFormat<TQMOE_Q4_K> : MfmaNibbles {
     }
     static __device__ __forceinline__ float d(const Rec & r) { return half_bits_to_float(uint16_t(r.x & 0xFFFFu)); }
     static __device__ __forceinline__ float dmin(const Rec & r) { return half_bits_to_float(uint16_t(r.x >> 16)); }
+    static __device__ __forceinline__ Rec odd_rec(const Rec & r, int odd) { return make_uint4(r.x, r.y >> (8 * odd), r.z >> (8 * odd), r.w >> (8 * odd)); }
 };
 template <> struct MfmaFormat<TQMOE_NVFP4G> : MfmaNibbles {
     static constexpr int kRecBytes = 512, kGroups = 2;
@@ -119,6 +130,7 @@ template <> struct MfmaFormat<TQMOE_NVFP4G> : MfmaNibbles {
         }
     }
     static __device__ __forceinline__ float d(const Rec &) { return 1.f; }
+    static __device__ __forceinline__ Rec odd_rec(const Rec & r, int odd) { return make_uint4(r.x >> (16 * odd), r.y >> (16 * odd), r.z >> (16 * odd), r.w >> (16 * odd)); }
     static __device__ __forceinline__ float row_factor(const BankView & b, int64_t row) {   // half the row's global: the table holds twice the values
         return 0.5f * *reinterpret_cast<const float *>(b.aux + nvfp4_global_offset(b.rows_total, b.cols) + row * 4);
     }
@@ -172,6 +184,14 @@ template <> struct MfmaFormat<TQMOE_IQ3_S> : MfmaBase {
         return w;
     }
     static __device__ __forceinline__ v4i decode(const Codes & c, const Rec & r, int ib, int g, const uint32_t * lat) { return signed_of(lookup(c, r, ib, g, lat), c, ib, g); }
+    static __device__ __forceinline__ void half_codes(const uint8_t * p, int n, int g, int odd, Codes & c) {
+        codes(p, n, g, c);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c.qs[i].x = odd ? c.qs[i].y : c.qs[i].x;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) { c.sg[i].x = odd ? c.sg[i].y : c.sg[i].x; c.sg[i].z = odd ? c.sg[i].w : c.sg[i].z; }
+    }
+    static __device__ __forceinline__ Rec odd_rec(const Rec & r, int odd) { return make_uint4(r.x >> (4 * odd), r.y >> (8 * odd), r.z >> (8 * odd), r.w >> (4 * odd)); }
     static __device__ __forceinline__ int scale(const Rec & r, int ib, int) { return 1 + 2 * iq3s_ls(r, ib); }
     static __device__ __forceinline__ float d(const Rec & r) { return 0.125f * half_bits_to_float(uint16_t(r.x & 0xFFFFu)); }
 };
@@ -199,6 +219,16 @@ template <> struct MfmaFormat<TQMOE_Q6_K> : MfmaBase {
         return __builtin_amdgcn_sbfe(int(w), 8 * (2 * (ib & 1) + grp), 8);
     }
     static __device__ __forceinline__ float d(const Rec & r) { return 0.25f * half_bits_to_float(uint16_t(r.d)); }
+    static __device__ __forceinline__ void half_codes(const uint8_t * p, int n, int g, int odd, Codes & c) {
+        const uint8_t * q = p + n * 16 + g * 8;
+#pragma unroll
+        for (int ib = 0; ib < 8; ib += 2) c.lo[ib] = *reinterpret_cast<const uint2 *>(q + (ib + odd) * 512);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c.hi[i].x = *reinterpret_cast<const uint32_t *>(q + 4096 + i * 512 + odd * 4);
+    }
+    static __device__ __forceinline__ Rec odd_rec(const Rec & r, int odd) {
+        return Rec{make_uint4(r.sc.x >> (16 * odd), r.sc.y >> (16 * odd), r.sc.z >> (16 * odd), r.sc.w >> (16 * odd)), r.d};
+    }
 };
 
 // NB banks (gate and up, or one). gateup != 0: out0 is the activation image that receives silu(gate) * up; else out0 /
@@ -605,58 +635,73 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
 // 32 sums in LDS, and the block adds a slot's super-blocks, then the slots in order. Against a product launch per assignment
 // and a launch that sums: one launch, one trip through memory and the [slots][hidden] fp32 rows less. Few blocks (hidden / 32
 // a token), each with all its loads in flight: a chain of one trip to memory and a few hundred instructions.
-constexpr int kDownWaves = 16;
-template <uint32_t FMT>
+//
+// What bounds it is the vector work of a compute unit (a unit's decode serves one input row, and the blocks are few), so while
+// they still find compute units of their own, blocks take half a tile (HALF): the matrix instruction's columns are then sixteen weight rows
+// of two sub-blocks, its rows the planes of both sub-blocks' activations, and a lane decodes half as much.
+// (2048 columns out, us, whole / half tiles: one token of the 512-expert IQ4_XS layer 7.2 / 5.9, of Q4_K top-8 6.9 / 5.8, of NVFP4G 7.4 /
+// 6.1; two tokens, 256 half tiles, 7.0 / 5.8; three tokens, 384 half tiles on 256 compute units, 7.7 / 10.5.)
+constexpr int kHalfBlocks = 256, kDownWaves = 16;
+template <uint32_t FMT, bool HALF>
 __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArgs k) {
     using F = MfmaFormat<FMT>;
-    extern __shared__ float part[];   // [units][32] sums, then [slots][32] weighted rows
+    constexpr int kRows = HALF ? 16 : 32, kSub = HALF ? 4 : 8, kStep = HALF ? 2 : 1;   // weight rows of a block; products of a unit; sub-blocks of one
+    extern __shared__ float part[];   // [units][32] sums, then [slots][kRows] weighted rows
     __shared__ uint32_t lat[F::kLattice];
-    const int token = blockIdx.y, tile = blockIdx.x, S = k.b.cols / 32, NSB = S / 8, tiles = k.b.rows / 32;
+    const int token = blockIdx.y, tile = blockIdx.x / (32 / kRows), S = k.b.cols / 32, NSB = S / 8, tiles = k.b.rows / 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
+    const int odd = HALF ? n >> 4 : 0, row_n = HALF ? int(blockIdx.x & 1) * 16 + (n & 15) : n;   // the lane's sub-blocks, its weight row in the tile
     const int shared_sb = k.slots > k.topk ? k.shared_cols / 256 : 0, units = k.topk * NSB + shared_sb;
     const int extra = int(k.b.rows_total / k.b.rows) - 1;      // the shared expert's place
-    struct Unit { typename F::Codes code; typename F::Rec rec; v4i a[8]; float4 xs[2], xm[2]; float rf; };
+    struct Unit { typename F::Codes code; typename F::Rec rec; v4i a[kSub]; float4 xs[2], xm[2]; float rf; };
     auto expert_of = [&](int u) { const int slot = min(u / NSB, k.slots - 1); return slot < k.topk ? k.ids[token * k.topk + slot] : extra; };
     auto fetch = [&](int u, int e, Unit & c) {
         const int slot = min(u / NSB, k.slots - 1), sb = u - slot * NSB;
         e = min(max(e, 0), extra);   // an id outside the bank: a bank's weights, not added below
         const int64_t at = (int64_t(e) * tiles + tile) * NSB + sb;
-        F::codes(k.b.codes + at * F::kCodeBytes, n, g, c.code);
-        c.rec = F::rec(k.b.aux + at * F::kRecBytes, n);
+        if constexpr (HALF) F::half_codes(k.b.codes + at * F::kCodeBytes, row_n, g, odd, c.code);
+        else F::codes(k.b.codes + at * F::kCodeBytes, n, g, c.code);
+        c.rec = F::rec(k.b.aux + at * F::kRecBytes, row_n);
         const uint8_t * row = image_row_ptr(k.image, int64_t(token) * k.slots + slot, S);
-        const uint8_t * a = row + sb * 512 + (n & 1) * 32 + g * 16;
+        const uint8_t * a = row + sb * 512 + (HALF ? ((n >> 1) & 1) * 64 : 0) + (n & 1) * 32 + g * 16;
 #pragma unroll
-        for (int ib = 0; ib < 8; ++ib) c.a[ib] = *reinterpret_cast<const v4i *>(a + ib * 64);
+        for (int i = 0; i < kSub; ++i) c.a[i] = *reinterpret_cast<const v4i *>(a + i * kStep * 64);
         const float4 * xs = reinterpret_cast<const float4 *>(image_scales(row, S) + sb * 8);
         c.xs[0] = xs[0]; c.xs[1] = xs[1];
         if constexpr (F::kMin) { const float4 * xm = reinterpret_cast<const float4 *>(image_sums(row, S) + sb * 8); c.xm[0] = xm[0]; c.xm[1] = xm[1]; }
-        c.rf = F::row_factor(k.b, (int64_t(e) * k.b.rows) + tile * 32 + n);
+        c.rf = F::row_factor(k.b, (int64_t(e) * k.b.rows) + tile * 32 + row_n);
     };
     auto multiply = [&](const Unit & c) {
         const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-        const float xs[8] = {c.xs[0].x, c.xs[0].y, c.xs[0].z, c.xs[0].w, c.xs[1].x, c.xs[1].y, c.xs[1].z, c.xs[1].w};
+        auto of_lane = [&](const float4 (&v)[2], int i) {      // sub-block kStep i + odd
+            const float w[8] = {v[0].x, v[0].y, v[0].z, v[0].w, v[1].x, v[1].y, v[1].z, v[1].w};
+            return HALF ? (odd ? w[kStep * i + kStep - 1] : w[kStep * i]) : w[i];
+        };
+        typename F::Rec rec = c.rec;
+        if constexpr (HALF) rec = F::odd_rec(c.rec, odd);
         float sum = 0.f, mins = 0.f;
 #pragma unroll
-        for (int ib = 0; ib < 8; ++ib) {
-            const v4i w = F::decode(c.code, c.rec, ib, g, lat);
-            // (every even row of operand A is the hi plane of the one input row, every odd one the lo plane)
+        for (int i = 0; i < kSub; ++i) {
+            const int ib = kStep * i;
+            const float xs = of_lane(c.xs, i);
+            const v4i w = F::decode(c.code, rec, ib, g, lat);
+            // (every even row of operand A is the hi plane of the one input row, every odd one the lo plane; HALF: rows 0 and 1 those
+            // of the even sub-block, 2 and 3 those of the odd one)
             auto add = [&](const v16i & acc, int grp) {
-                sum += float((acc[0] << 7) + acc[1]) * (F::d(c.rec) * float(F::scale(c.rec, ib, grp)) * xs[ib]);
+                const int hi = odd ? acc[2] : acc[0], lo = odd ? acc[3] : acc[1];
+                sum += float((hi << 7) + lo) * (F::d(c.rec) * float(F::scale(rec, ib, grp)) * xs);
                 asm volatile("" : : "v"(acc));   // (all sixteen registers in use until here: see decode_mfma_k)
             };
-            if constexpr (F::kGroups == 1) add(__builtin_amdgcn_mfma_i32_32x32x32_i8(c.a[ib], w, zero, 0, 0, 0), 0);
+            if constexpr (F::kGroups == 1) add(__builtin_amdgcn_mfma_i32_32x32x32_i8(c.a[i], w, zero, 0, 0, 0), 0);
             else
 #pragma unroll
                 for (int grp = 0; grp < 2; ++grp) {
-                    const long a2 = long(uint64_t(uint32_t(c.a[ib][grp])) | uint64_t(uint32_t(c.a[ib][grp + 2])) << 32);
+                    const long a2 = long(uint64_t(uint32_t(c.a[i][grp])) | uint64_t(uint32_t(c.a[i][grp + 2])) << 32);
                     const long w2 = long(uint64_t(uint32_t(w[grp])) | uint64_t(uint32_t(w[grp + 2])) << 32);
                     add(__builtin_amdgcn_mfma_i32_32x32x16_i8(a2, w2, zero, 0, 0, 0), grp);
                 }
             if constexpr (F::kGroups == 2) __builtin_amdgcn_sched_barrier(0);   // (sixteen results under way are more than the registers hold)
-            if constexpr (F::kMin) {
-                const float xm[8] = {c.xm[0].x, c.xm[0].y, c.xm[0].z, c.xm[0].w, c.xm[1].x, c.xm[1].y, c.xm[1].z, c.xm[1].w};
-                mins = fmaf(F::minimum(c.rec, ib), xm[ib], mins);
-            }
+            if constexpr (F::kMin) mins = fmaf(F::minimum(rec, ib), of_lane(c.xm, i), mins);
         }
         if constexpr (F::kMin) sum = fmaf(-F::dmin(c.rec), mins, sum);
         return sum * c.rf;
@@ -676,17 +721,18 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
     }
     __syncthreads();
     float * rows = part + units * 32;
-    for (int i = threadIdx.x; i < k.slots * 32; i += blockDim.x) {
-        const int slot = i >> 5, nsb = slot < k.topk ? NSB : shared_sb;
+    for (int i = threadIdx.x; i < k.slots * kRows; i += blockDim.x) {
+        const int slot = i / kRows, nsb = slot < k.topk ? NSB : shared_sb;
         float v = 0.f;
-        for (int sb = 0; sb < nsb; ++sb) v += part[(slot * NSB + sb) * 32 + (i & 31)];
+        for (int sb = 0; sb < nsb; ++sb)
+            for (int h = 0; h < 32 / kRows; ++h) v += part[(slot * NSB + sb) * 32 + h * kRows + i % kRows];
         rows[i] = (slot < k.topk ? k.weights[token * k.topk + slot] : k.shared_weights[token]) * v;
     }
     __syncthreads();
-    if (threadIdx.x < 32) {
+    if (threadIdx.x < kRows) {
         float sum = 0.f;
-        for (int s = 0; s < k.slots; ++s) sum += rows[s * 32 + threadIdx.x];
-        const int64_t o = int64_t(token) * k.b.rows + tile * 32 + threadIdx.x;
+        for (int s = 0; s < k.slots; ++s) sum += rows[s * kRows + threadIdx.x];
+        const int64_t o = int64_t(token) * k.b.rows + int64_t(blockIdx.x) * kRows + threadIdx.x;
         if (k.otype == TQMOE_F32) static_cast<float *>(k.out)[o] = sum;
         else {
             if (k.residual) sum = bf16_bits_to_float(float_to_bf16_bits(sum)) + bf16_bits_to_float(k.residual[o]);
@@ -697,7 +743,9 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
 
 template <uint32_t FMT> void down_combine_launch(const DownCombineArgs & k, hipStream_t s) {
     const int NSB = k.b.cols / 256, units = k.topk * NSB + (k.slots > k.topk ? k.shared_cols / 256 : 0);
-    down_combine_k<FMT><<<dim3(unsigned(k.b.rows / 32), unsigned(k.n)), 64 * kDownWaves, size_t(units + k.slots) * 32 * sizeof(float), s>>>(k);
+    const size_t lds = size_t(units + k.slots) * 32 * sizeof(float);
+    if (int64_t(k.n) * (k.b.rows / 16) <= kHalfBlocks) down_combine_k<FMT, true><<<dim3(unsigned(k.b.rows / 16), unsigned(k.n)), 64 * kDownWaves, lds, s>>>(k);
+    else down_combine_k<FMT, false><<<dim3(unsigned(k.b.rows / 32), unsigned(k.n)), 64 * kDownWaves, lds, s>>>(k);
 }
 
 // the shapes the kernel takes: whole tiles, whole super-blocks (a narrower shared expert included)
