@@ -54,3 +54,22 @@ def test_down_rows_wider_than_the_decode_products_take(tq, oracle, fmt):
         assert np.array_equal(ids, want_ids) and synth.errors(out, want)[1] < 1e-3
     with pytest.raises(tq.TqmoeError, match="too wide"):
         layer.forward(x)
+
+
+@pytest.mark.parametrize("experts", [65, 300])
+@pytest.mark.parametrize("spread", [70, 100, 4000])
+def test_logits_far_apart(tq, oracle, experts, spread):
+    """Logits whose exponentials are all there, partly in the subnormal range, and zero for all but a few experts (which then
+    follow by index): every block of the first launch selects what the launch writes down as the routing."""
+    cfg = dict(hidden=256, ff=256, experts=experts, topk=8, shared_ff=0, wtype=oracle.IQ4_XS, rtype="f32", xtype="f32")
+    raws = synth.make_banks(cfg, seed=spread, distinct=5)
+    inp = synth.make_inputs(cfg, 2, seed=7)
+    x, router = (np.array(inp[k][1], dtype=np.float32) for k in ("x", "router"))
+    x[:, 0] = [1.0, 0.5]
+    router[:] = 0.0
+    router[:, 0] = -np.random.default_rng(spread).permutation(experts) * (spread / experts)
+    layer = tq.MoeLayer(torch.from_numpy(router).cuda(), None, *banks_on_device(cfg, raws), 8)
+    out, ids, w, logits = (t.cpu().numpy() for t in layer.forward(torch.from_numpy(x).cuda(), return_routing=True))
+    want, want_ids, want_w = oracle.layer_forward(x, logits, *raws, cfg["wtype"], 256, 256, experts, 8, act_mode=0, threads=4)
+    assert np.array_equal(ids, want_ids) and np.abs(w - want_w).max() < 3e-6
+    assert synth.errors(out, want)[1] < 1e-3

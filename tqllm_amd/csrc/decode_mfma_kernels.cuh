@@ -250,6 +250,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                                                     int tpw, int gateup, int a_off, int tl_count, Glu glu, DecodeTopk route) {
     using F = MfmaFormat<FMT>;
     constexpr bool STAGED = MODE >= 1, MULTI = MODE == 2;
+    constexpr int kIn = ROUTE > 0 ? 1 : 2;   // input rows a lane half has sums of (a block that routes serves one)
     extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
     __shared__ int meta[2], s_tok[kTP];
     __shared__ float s_x0[kTP];
@@ -257,25 +258,30 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     __shared__ uint32_t lat[F::kLattice];
     if constexpr (FMT == TQMOE_IQ3_S)   // eight times the magnitudes (behind a barrier before the first use)
         F::lattice(lat, threadIdx.x, blockDim.x);
-    const int a = blockIdx.y;
+    const int a = blockIdx.y, bx = int(blockIdx.x) - (ROUTE > 0 ? 1 : 0);   // bx: the block's group of row tiles
     int e;
     if constexpr (ROUTE > 0) {
-        // (one wave selects, for as many rounds as its assignment needs; the block that writes the token's routing for all)
+        // (one wave selects, for as many rounds as its assignment needs; a block of its own, of the grid's first column, does so for
+        // the token's whole routing and writes it: the weights' exponentials and divisions are then in nobody's way. One token of the
+        // 512-expert IQ4_XS layer, launch 10.0 -> 9.3 us)
         const int token = a / slots, slot = a - token * slots;
-        const bool writer = blockIdx.x == 0 && slot == 0;
+        const float * x = route.logits + int64_t(token) * (route.experts + 1);
+        int my_id;
+        float my_w;
+        if (blockIdx.x == 0) {
+            if (slot == 0 && threadIdx.x < 64) {
+                const float shared_logit = route.shared_weights ? x[route.experts] : 0.f;
+                topk_select<ROUTE>(x, route.experts, topk, threadIdx.x, true, my_id, my_w);
+                const float v = topk_weight(my_w, topk, route.scale);
+                if (int(threadIdx.x) < topk) { route.ids[int64_t(token) * topk + threadIdx.x] = my_id; route.weights[int64_t(token) * topk + threadIdx.x] = v; }
+                if (threadIdx.x == 0 && route.shared_weights) route.shared_weights[token] = route.shared_ungated ? 1.f : 1.f / (1.f + expf(-shared_logit));
+            }
+            return;
+        }
         if (slot < topk) {
             if (threadIdx.x < 64) {
-                const float * x = route.logits + int64_t(token) * (route.experts + 1);
-                const float shared_logit = route.shared_weights ? x[route.experts] : 0.f;
-                int my_id;
-                float my_w;
-                topk_select<ROUTE>(x, route.experts, writer ? topk : slot + 1, threadIdx.x, writer, my_id, my_w);
+                topk_select<ROUTE>(x, route.experts, slot + 1, threadIdx.x, false, my_id, my_w);
                 if (int(threadIdx.x) == slot) meta[0] = my_id;
-                if (writer) {
-                    const float v = topk_weight(my_w, topk, route.scale);
-                    if (int(threadIdx.x) < topk) { route.ids[int64_t(token) * topk + threadIdx.x] = my_id; route.weights[int64_t(token) * topk + threadIdx.x] = v; }
-                    if (threadIdx.x == 0 && route.shared_weights) route.shared_weights[token] = route.shared_ungated ? 1.f : 1.f / (1.f + expf(-shared_logit));
-                }
             }
             __syncthreads();
             e = meta[0];
@@ -293,7 +299,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
 
     const int S = b0.cols / 32, NSB = S / 8, rows = b0.rows, tiles = rows / 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
-    const int wk_i = wave % wk, rt_l = wave / wk, tile = blockIdx.x * tl_count * tpw + rt_l;   // the wave's first (or only) row tile
+    const int wk_i = wave % wk, rt_l = wave / wk, tile = bx * tl_count * tpw + rt_l;   // the wave's first (or only) row tile
     const bool shared_slot = (a % slots) >= topk;
     // the shared expert may have fewer rows (gate / up) or read a narrower input row (down)
     const int row_lim = gateup && shared_slot ? shared_lim : rows;
@@ -457,7 +463,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                     }
                 };
                 if constexpr (!UNI) { get(sc0, xs0); get(sc1, xs1); }       // activation scales of the sub-blocks
-                if constexpr (F::kMin) { get(sum0, xm0); get(sum1, xm1); }  // and their sums
+                if constexpr (F::kMin) { get(sum0, xm0); if constexpr (kIn == 2) get(sum1, xm1); }  // and their sums
             };
             // The products of step (sub-block, bank, scale group) + 1 are issued before the sums of this step are read: the
             // matrix pipe's latency passes under the next step's lookups instead of in front of this step's multiply-adds.
@@ -498,20 +504,20 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                 if constexpr (F::kFloat) {
                     const float sc = F::scale(rec, ib, grp);
                     accf[nb][0] = fmaf(float((acc[0] << 7) + acc[1]), UNI ? sc : sc * xs0[ip], accf[nb][0]);
-                    accf[nb][1] = fmaf(float((acc[2] << 7) + acc[3]), UNI ? sc : sc * xs1[ip], accf[nb][1]);
+                    if constexpr (kIn == 2) accf[nb][1] = fmaf(float((acc[2] << 7) + acc[3]), UNI ? sc : sc * xs1[ip], accf[nb][1]);
                 } else if constexpr (UNI) {
                     // |acc| <= 32 * 128 * 128 = 2^19 and |scale| <= 2^7: 24-bit products, and with a scale per sixteen weights
                     // half the |acc|: sixteen of them stay below 2^30
                     const int ls = F::scale(rec, ib, grp);
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
+                    for (int q = 0; q < 2 * kIn; ++q) {
                         si[nb][q] = (ib || grp ? si[nb][q] : 0) + __mul24(acc[q], ls);
                         asm("" : "+v"(si[nb][q]));   // (one multiply-add each: two steps' products are otherwise made apart and added in a third instruction)
                     }
                     if (ib == 7 && grp == G - 1) {
                         const float d = F::d(rec);
                         accf[nb][0] += (float(si[nb][0]) * 128.f + float(si[nb][1])) * d;
-                        accf[nb][1] += (float(si[nb][2]) * 128.f + float(si[nb][3])) * d;
+                        if constexpr (kIn == 2) accf[nb][1] += (float(si[nb][2]) * 128.f + float(si[nb][3])) * d;
                     }
                 } else {
                     const float ws = F::d(rec) * float(F::scale(rec, ib, grp));
@@ -521,11 +527,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                 if constexpr (F::kMin) {
                     const float mn = F::minimum(rec, ib);
                     sm[nb][0] = ib ? fmaf(mn, xm0[ip], sm[nb][0]) : mn * xm0[ip];
-                    sm[nb][1] = ib ? fmaf(mn, xm1[ip], sm[nb][1]) : mn * xm1[ip];
+                    if constexpr (kIn == 2) sm[nb][1] = ib ? fmaf(mn, xm1[ip], sm[nb][1]) : mn * xm1[ip];
                     if (ib == 7) {
                         const float dm = F::dmin(rec);
                         accm[nb][0] = fmaf(dm, sm[nb][0], accm[nb][0]);
-                        accm[nb][1] = fmaf(dm, sm[nb][1], accm[nb][1]);
+                        if constexpr (kIn == 2) accm[nb][1] = fmaf(dm, sm[nb][1], accm[nb][1]);
                     }
                 }
                 // only four of the sixteen result registers are read; the others count as in use until here, or they are handed
@@ -543,7 +549,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
             auto fetch_step = [&](int gs, Cold & c) { fetch_tile(gs / nsteps * tpw, wk_i + gs % nsteps * wk, c); };
             auto after = [&](int gs) {   // step gs is done: was it its tile's last?
                 if ((gs + 1) % nsteps) return;
-                finish((int(blockIdx.x) * tl_count + gs / nsteps) * tpw, true);
+                finish((bx * tl_count + gs / nsteps) * tpw, true);
                 clear();
             };
             for (int gs = 0; gs < total; gs += 2) {
@@ -573,7 +579,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
         }
     }
 
-    if constexpr (!MULTI) finish(blockIdx.x * tpw, valid);
+    if constexpr (!MULTI) finish(bx * tpw, valid);
 }
 
 template <uint32_t FMT>
@@ -616,7 +622,7 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     int tl = 1;
     if (staged && nb == 1 && NSB % wk == 0 && (slots <= topk || shared_lim == (gateup ? b0.rows : b0.cols)))
         while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= kLeastBlocks) tl *= 2;
-    const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl)), unsigned(A));
+    const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl) + (route.logits ? 1 : 0)), unsigned(A));
     const int a_off = int(lds);
     if (staged) lds += size_t(b0.cols / 32) * (256 + ((uniform ? 0 : 1) + (MfmaFormat<FMT>::kMin ? 1 : 0)) * kTP * sizeof(float));
     auto go = [&](auto kernel) { kernel<<<grid, threads, lds, s>>>(b0, b1, image, out0, out1, ytype, ids, A, xdiv, mode, slots, topk, shared_lim, wk, tpw, gateup, a_off, tl, glu, route); };

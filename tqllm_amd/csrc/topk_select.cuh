@@ -65,12 +65,21 @@ template <int R> __device__ __forceinline__ void topk_select(const float * __res
 #pragma unroll
         for (int r = 0; r < R; ++r) { const int j = lane + 64 * r; l[r] = j < e ? x[j] : -INFINITY; m = fmaxf(m, l[r]); }
         m = wave_max_all(m);
+        // (the order alone needs the exponentials only where one may be zero, or a logit is not finite)
+        bool far = false;
 #pragma unroll
-        for (int r = 0; r < R; ++r) {
-            const int j = lane + 64 * r;
-            const float ex = j < e ? expf(l[r] - m) : 0.f;
-            sum += ex;
-            key[r] = j < e ? (ex > 0.f ? order_key(l[r]) : kKeyZero) : kKeyGone;   // entries past the end never win
+        for (int r = 0; r < R; ++r) far |= lane + 64 * r < e && !(l[r] - m >= -80.f);
+        if (weights || __any(far)) {
+#pragma unroll
+            for (int r = 0; r < R; ++r) {
+                const int j = lane + 64 * r;
+                const float ex = j < e ? expf(l[r] - m) : 0.f;
+                sum += ex;
+                key[r] = j < e ? (ex > 0.f ? order_key(l[r]) : kKeyZero) : kKeyGone;   // entries past the end never win
+            }
+        } else {
+#pragma unroll
+            for (int r = 0; r < R; ++r) key[r] = lane + 64 * r < e ? order_key(l[r]) : kKeyGone;
         }
     }
     int my_key = kKeyZero;
