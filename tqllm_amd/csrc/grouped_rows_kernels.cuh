@@ -12,9 +12,10 @@
 //  * the matrix instructions of operand piece j are followed by the decode of piece j of the next stage into the same
 //    registers, six or so vector instructions to a matrix instruction.
 //
-// Weight values. A code's table value (or the code itself) lands in the low byte of the half 1024 + u by one byte permute
-// or mask per pair; one mixed-precision multiply-add per weight takes the bias off and puts the fp32 scale (and minimum)
-// on, one conversion per pair rounds to fp16: 19 (Q4_K) to 27 (IQ4_XS) vector instructions for eight weights, one rounding.
+// Weight values. A code's table value lands in the low byte of the half 1024 + u by one byte permute per pair; one
+// mixed-precision multiply-add per weight takes the bias off and puts the fp32 scale (and minimum) on, one conversion per
+// pair rounds to fp16: 17 (Q4_K, whose codes are halves where they stand) to 27 (IQ4_XS) vector instructions for eight
+// weights, one rounding.
 // (Packed fp16 multiply-adds take four fewer and round twice: a quarter more error in the layer's result.)
 // NVFP4G: the sixteen products of a scale byte, rounded to E4M3, are a table in LDS (4 KB for all scales); eleven instructions
 // for eight weights.
@@ -23,9 +24,11 @@
 // instructions; with the two banks' eight accumulators (128 registers) two waves fit a SIMD, and one of them decodes while
 // the other's products run. Items of one and two row tiles have loops of their own with fewer products.
 //
-// What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 262 us, 0.8
-// PFLOP/s, matrix pipe 43 % busy, vector pipe 52 %; NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 985 us, 40 % and
-// 51 %. A stage of an item with four row tiles takes about 4800 cycles where its SIMD's two waves have 2048 of matrix work.
+// What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 237 us, 0.87
+// PFLOP/s (262 us with biased codes, when the matrix pipe was 43 % busy and the vector pipe 52 %; then 211 without the decode,
+// 173 without the row reads as well, which is the rate of a large fp16 product on this card); NVFP4G, 8192 tokens, gate / up
+// (2.1 TFLOP with down): 873 us, 40 % and 51 %. A product holds its SIMD's vector issue for about 18 cycles besides its own
+// time, so a stage's decode does not pass under its products for free: that sum and not a wait is what is left.
 // Items of one row tile are bound by the decode (IQ3_S, 512 tokens: 2.6 TB/s of codes, vector pipe 69 %, LDS 51 %, three
 // fifths of that bank conflicts of the lattice's look-ups).
 #pragma once
@@ -48,10 +51,12 @@ __device__ __forceinline__ v2h as_h2(uint32_t v) { return __builtin_bit_cast(v2h
 __device__ __forceinline__ uint32_t bits_of(v2h v) { return __builtin_bit_cast(uint32_t, v); }
 __device__ __forceinline__ v2h both(float v) { const _Float16 h = _Float16(v); return v2h{h, h}; }
 __device__ __forceinline__ v2h both_bits(uint32_t h16) { return as_h2(h16 | h16 << 16); }
-// both halves of u times s plus c, in fp32, rounded to halves: two v_fma_mix_f32 and a packed conversion (v_fma_mixlo_f16 and
-// v_fma_mixhi_f16 do it in two, at half the rate)
+// both halves of u times s plus c, in fp32, rounded to halves: two v_fma_mix_f32 and a packed conversion, 6.1 ns a SIMD
+// (v_fma_mixlo_f16 and v_fma_mixhi_f16, 7.8 ns, are what the compiler makes of one pair in four where the sums are not
+// pinned: Q4_K's layer of 4096 tokens 439 us so, 429 pinned)
 __device__ __forceinline__ uint32_t mix2(v2h u, float s, float c) {
-    const float lo = fmaf(float(u[0]), s, c), hi = fmaf(float(u[1]), s, c);
+    float lo = fmaf(float(u[0]), s, c), hi = fmaf(float(u[1]), s, c);
+    asm("" : "+v"(lo), "+v"(hi));
     return bits_of(v2h{_Float16(lo), _Float16(hi)});
 }
 // bytes 0, 2 and bytes 1, 3 of u as halves 1024 + byte
@@ -103,23 +108,29 @@ template <> struct GroupedFormat<TQMOE_Q4_K> : GroupedNibbles {
         return (lane < 32 ? b0.aux + tile0 * (S / 8) * 512 : b1.aux + tile1 * (S / 8) * 512) + (lane & 31) * 16;
     }
     static __device__ __forceinline__ int rec_at(int, int st) { return (st >> 2) * 512; }
-    struct Prep { uint32_t c[4]; float s, off; };
+    struct Prep { uint32_t c[4]; float s[2], off; };
     static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int st, int n, int g, const uint8_t *, Prep & p) {
         const uint4 c = *reinterpret_cast<const uint4 *>(w + nb * 1024 + g * 512 + n * 16);
         const uint4 r = *reinterpret_cast<const uint4 *>(w + 2048 + nb * 512 + n * 16);
         p.c[0] = c.x; p.c[1] = c.y; p.c[2] = c.z; p.c[3] = c.w;
-        int sc, mn;
-        q4k_scale_min_flat(r.y, r.z, r.w, (2 * st + g) & 7, sc, mn);
-        p.s = half_bits_to_float(uint16_t(r.x & 0xFFFFu)) * float(sc);
-        // the bias and the minimum in one constant: its rounding is 2^-15 of a code step
-        p.off = -fmaf(p.s, 1024.f, half_bits_to_float(uint16_t(r.x >> 16)) * float(mn));
+        // bytes (2 st + g) % 4 of the record's three dwords; the upper sub-blocks' six bits are a nibble and two top bits
+        const bool upper = st & 2;
+        const int sh = 16 * (st & 1) + 8 * g;
+        const uint32_t low = upper ? 15u : 0u, six = upper ? 48u : 63u, from = upper ? 2u : 0u;
+        const int sc = int(((r.w >> sh) & low) | ((r.y >> (sh + from)) & six)), mn = int(((r.w >> (sh + 4)) & low) | ((r.z >> (sh + from)) & six));
+        const float s = half_bits_to_float(uint16_t(r.x & 0xFFFFu)) * float(sc);
+        // A nibble alone in a half, in its low or the next four bits, is the subnormal number code * 2^-24 or 2^-20: the
+        // multiply-add reads it as it is, and the scale takes the power of two (exact). (As the low bits of 1024 + code: an
+        // instruction more a pair, and the constant that takes the bias off rounds; 4096 tokens 451 us so, 439 without.)
+        p.s[0] = s * 0x1p24f;
+        p.s[1] = s * 0x1p20f;
+        p.off = -(half_bits_to_float(uint16_t(r.x >> 16)) * float(mn));
     }
     static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
-        const uint32_t c = p.c[j];
-        uint32_t mask = 0x000F000Fu;
-        asm("" : "+v"(mask));                      // in a register, so that mask and bias are one instruction
-        auto val = [&](uint32_t x) { return mix2(as_h2((x & mask) | 0x64006400u), p.s, p.off); };
-        return make_uint4(val(c), val(c >> 8), val(c >> 4), val(c >> 12));
+        const uint32_t c = p.c[j], c8 = c >> 8;
+        auto low = [&](uint32_t x) { return mix2(as_h2(x & 0x000F000Fu), p.s[0], p.off); };
+        auto high = [&](uint32_t x) { return mix2(as_h2(x & 0x00F000F0u), p.s[1], p.off); };
+        return make_uint4(low(c), low(c8), high(c), high(c8));
     }
 };
 
