@@ -29,8 +29,14 @@
 // 173 without the row reads as well, which is the rate of a large fp16 product on this card); NVFP4G, 8192 tokens, gate / up
 // (2.1 TFLOP with down): 873 us, 40 % and 51 %. A product holds its SIMD's vector issue for about 18 cycles besides its own
 // time, so a stage's decode does not pass under its products for free: that sum and not a wait is what is left.
-// Items of one row tile are bound by the decode (IQ3_S, 512 tokens: 2.6 TB/s of codes, vector pipe 69 %, LDS 51 %, three
-// fifths of that bank conflicts of the lattice's look-ups).
+// Items of one row tile are bound by the decode (IQ3_S, 512 tokens: gate / up 139 us, 2.5 TB/s of codes; without the look-ups'
+// bank conflicts and addresses 103, without signs and scales 104, without code transfers 116).
+//
+// One row tile of a format with kFold (IQ3_S): the operands are the codes times the integer scale, exact in fp16, and every 256
+// columns the fp32 sums are multiplied by the super-block's factor instead (the weights are the second operand there, so that a
+// lane's factor is its own weight row's): 32 of 224 vector instructions a stage less for 16 more, and a rounding fewer (512
+// tokens, 16 rows an expert: 222 us a layer so, 213 folded; the error against float64 5.2e-4 and 3.6e-4). Two row tiles have no
+// registers for the second set of sums.
 #pragma once
 #include "decode_api.cuh"
 #include "decode_table.cuh"
@@ -66,11 +72,16 @@ __device__ __forceinline__ v2h bias_odd(uint32_t u) { return as_h2(__builtin_amd
 // What the kernel needs of a format.
 // kCodes: 1 KB transfers a bank and stage (64 lanes x 16 bytes): code() the lane's source, code_at() what to add
 // for a transfer and stage. kRecs transfers for both banks' records: rec(), rec_at(). Prep: what decoding a stage needs in registers;
-// slice(): piece j (16 bytes) of operand B. kTab bytes of lookup table in LDS, filled by tables(). row_factor(): a factor
-// of a whole weight row.
+// slice(): piece j (16 bytes) of operand B; with kFold also whole(), the piece without the super-block's factor fold(). kTab
+// bytes of lookup table in LDS, filled by tables(). row_factor(): a factor of a whole weight row.
 template <uint32_t FMT> struct GroupedFormat;
 
-struct GroupedHalves {
+struct GroupedWhole {                     // no factor outside the operands
+    static constexpr bool kFold = false;
+    template <class P> static __device__ __forceinline__ float fold(const P &) { return 1.f; }
+    template <class P> static __device__ __forceinline__ uint4 whole(P &, int) { return uint4(); }
+};
+struct GroupedHalves : GroupedWhole {
     static constexpr bool kFp8 = false;
     static constexpr int kTab = 16;
     static __device__ __forceinline__ void tables(uint8_t *, int) {}
@@ -169,12 +180,20 @@ template <> struct GroupedFormat<TQMOE_Q6_K> : GroupedHalves {
 };
 
 template <> struct GroupedFormat<TQMOE_IQ3_S> : GroupedHalves {
-    static constexpr int kCodes = 1, kRecs = 1, kTab = 512 * 8;
+    static constexpr bool kFold = true;
+    // Points 0..255 are the table's first 2 KB; the others follow 2 and again 4 KB behind it, so that an index's ninth bit is an
+    // address bit after one shift for two of them.
+    static constexpr int kCodes = 1, kRecs = 1, kTab = 6144;
     static __device__ __forceinline__ void tables(uint8_t * tab, int tid) {   // a lattice point's magnitudes as halves, weights 0, 2, 1, 3
         for (int i = tid; i < 512; i += 256) {
             const v2h bias = as_h2(0xE400E400u);       // -1024
             const uint32_t m = d_iq3s_grid.v[i];
-            reinterpret_cast<uint2 *>(tab)[i] = make_uint2(bits_of(bias_even(m) + bias), bits_of(bias_odd(m) + bias));
+            const uint2 v = make_uint2(bits_of(bias_even(m) + bias), bits_of(bias_odd(m) + bias));
+            if (i < 256) reinterpret_cast<uint2 *>(tab)[i] = v;
+            else {
+#pragma unroll
+                for (int c = 1; c <= 2; ++c) reinterpret_cast<uint2 *>(tab)[c * 256 + i - 256] = v;
+            }
         }
     }
     static __device__ __forceinline__ const uint8_t * code(const BankView & b, int64_t tile, int S, int lane) {   // the pair's indices, then the signs
@@ -186,7 +205,7 @@ template <> struct GroupedFormat<TQMOE_IQ3_S> : GroupedHalves {
         return (lane < 32 ? b0.aux + tile0 * (S / 8) * 512 : b1.aux + tile1 * (S / 8) * 512) + (lane & 31) * 16;
     }
     static __device__ __forceinline__ int rec_at(int, int st) { return (st >> 2) * 512; }
-    struct Prep { uint32_t qs[2], sg, qh; v2h sc, d; const uint2 * lat; };
+    struct Prep { uint32_t qs[2], sg, qh; v2h sc, d; const uint8_t * lat; };
     static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int st, int n, int g, const uint8_t * tab, Prep & p) {
         const uint8_t * q = w + nb * 1024 + n * 16;
         p.qs[0] = *reinterpret_cast<const uint32_t *>(q + g * 4);
@@ -198,25 +217,31 @@ template <> struct GroupedFormat<TQMOE_IQ3_S> : GroupedHalves {
         const uint32_t ls = (ib < 4 ? r.x >> (16 + 4 * ib) : r.w >> (4 * (ib - 4))) & 15u;
         p.sc = both(float(1 + 2 * int(ls)));
         p.d = both_bits(r.x & 0xFFFFu);
-        p.lat = reinterpret_cast<const uint2 *>(tab);
+        p.lat = tab;
     }
-    static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
+    static __device__ __forceinline__ float fold(const Prep & p) { return float(p.d[0]); }
+    static __device__ __forceinline__ uint4 slice(Prep & p, int j) { return values<true>(p, j); }
+    static __device__ __forceinline__ uint4 whole(Prep & p, int j) { return values<false>(p, j); }
+    template <bool D> static __device__ __forceinline__ uint4 values(const Prep & p, int j) {
         const int h = j >> 1, q = 2 * (j & 1);     // operand dwords q and q + 1 of half h: weights 4 j .. and 16 + 4 j ..
         uint32_t v[4];
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
-            const uint32_t idx = ((p.qs[h] >> (8 * (q + i))) & 0xFFu) | ((p.qh << (8 - 4 * h - q - i)) & 0x100u);
-            const uint2 mag = p.lat[idx];          // the four magnitudes as halves, weights 0, 2 and 1, 3
             const int s = 4 * h + q + i;           // bit 8 t + s: the sign of weight t
+            uint32_t at = ((p.qs[h] >> (8 * (q + i))) & 0xFFu) << 3;   // (a byte shifted: one instruction, where nothing is merged into it)
+            asm("" : "+v"(at));
+            const uint2 mag = *reinterpret_cast<const uint2 *>(p.lat + (at | ((p.qh << (11 - (s & 6))) & (0x800u << (s & 1)))));   // the four magnitudes as halves, weights 0, 2 and 1, 3
             // times the integer scale (exact), times d (the one rounding)
-            v[2 * i] = bits_of(as_h2(mag.x ^ ((p.sg << (15 - s)) & 0x80008000u)) * p.sc * p.d);
-            v[2 * i + 1] = bits_of(as_h2(mag.y ^ ((p.sg << (7 - s)) & 0x80008000u)) * p.sc * p.d);
+            v2h a = as_h2(mag.x ^ ((p.sg << (15 - s)) & 0x80008000u)) * p.sc, b = as_h2(mag.y ^ ((p.sg << (7 - s)) & 0x80008000u)) * p.sc;
+            if constexpr (D) { a *= p.d; b *= p.d; }
+            v[2 * i] = bits_of(a);
+            v[2 * i + 1] = bits_of(b);
         }
         return make_uint4(v[0], v[1], v[2], v[3]);
     }
 };
 
-template <> struct GroupedFormat<TQMOE_NVFP4G> {
+template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
     static constexpr bool kFp8 = true;
     static constexpr int kCodes = 2, kRecs = 1, kTab = 256 * 16;
     // Per scale byte the 16 products e2m1(code) * e4m3(scale) / 8, rounded to E4M3 (nearest even; an eighth keeps the largest
@@ -341,13 +366,15 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
 
     auto body = [&](auto tag) {
         constexpr int MT = decltype(tag)::value;
-        v16f acc[2][MT];
+        constexpr bool FOLD = W::kFold && MT == 1;
+        v16f acc[2][MT], part[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[b][m][i] = 0.f;
+        if constexpr (FOLD) part[0] = part[1] = acc[0][0];
         const bool any = GATEUP ? grp * 128 < row_lim : true;
         if (any) {
             using R = Rings<W, MT, MAX>;
@@ -391,6 +418,10 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
             const uint8_t * a_row = lds + n * 128;
             uint4 bw[2][4];
             typename W::Prep pr[2];
+            auto operand = [&](typename W::Prep & p, int j) {
+                if constexpr (FOLD) return W::whole(p, j);
+                else return W::slice(p, j);
+            };
 #pragma unroll
             for (int t = -LM; t < 0; ++t) {   // what the stages before the first would have sent
                 if (t + LA >= 0) send_a(t + LA, t + LA);
@@ -401,7 +432,7 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
             for (int b = 0; b < 2; ++b) {
                 W::prep(w_lds, b, 0, n, g, s_tab, pr[b]);
 #pragma unroll
-                for (int j = 0; j < 4; ++j) bw[b][j] = W::slice(pr[b], j);
+                for (int j = 0; j < 4; ++j) bw[b][j] = operand(pr[b], j);
             }
             int a_at = 0, w_at = 0;           // slots of this stage's rows and codes
             for (int st = 0; st < stages; ++st) {
@@ -414,6 +445,14 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                 w_at = w_at + 1 == LW ? 0 : w_at + 1;
                 const bool more = st + 1 < stages;   // (past the last stage: its own codes again, not used)
                 const int w_next = more ? w_at : w_at == 0 ? LW - 1 : w_at - 1;
+                float d[2];
+                if constexpr (FOLD) {
+#pragma unroll
+                    for (int b = 0; b < 2; ++b) {
+                        d[b] = W::fold(pr[b]);
+                        asm("" : "+v"(d[b]));      // (in fp32: a mixed multiply-add takes half as long again)
+                    }
+                }
 #pragma unroll
                 for (int b = 0; b < 2; ++b) W::prep(w_lds + w_next * kStageW<W>, b, more ? st + 1 : st, n, g, s_tab, pr[b]);
                 const uint8_t * a_buf = a_row + a_at * MT * 4096;
@@ -442,12 +481,26 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                     } else {
                         if (j < 3) read_a(j + 1);
 #pragma unroll
+                        for (int b = 0; b < 2; ++b) {
+                            if constexpr (FOLD) part[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[j & 1][0]), __builtin_bit_cast(v8h, bw[b][j]), part[b], 0, 0, 0);
+                            else
+#pragma unroll
+                                for (int m = 0; m < MT; ++m)
+                                    acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bw[b][j]), __builtin_bit_cast(v8h, a[j & 1][m]), acc[b][m], 0, 0, 0);
+                        }
+#pragma unroll
+                        for (int b = 0; b < 2; ++b) bw[b][j] = operand(pr[b], j);
+                    }
+                }
+                if constexpr (FOLD) {
+                    if ((st & 3) == 3 || !more) {
+#pragma unroll
                         for (int b = 0; b < 2; ++b)
 #pragma unroll
-                            for (int m = 0; m < MT; ++m)
-                                acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bw[b][j]), __builtin_bit_cast(v8h, a[j & 1][m]), acc[b][m], 0, 0, 0);
-#pragma unroll
-                        for (int b = 0; b < 2; ++b) bw[b][j] = W::slice(pr[b], j);
+                            for (int i = 0; i < 16; ++i) {
+                                acc[b][0][i] = fmaf(part[b][i], d[b], acc[b][0][i]);
+                                part[b][i] = 0.f;
+                            }
                     }
                 }
             }
@@ -470,7 +523,7 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                     for (int i = 0; i < 16; ++i) {
                         v[i] = acc[bank][m][i];
                         if constexpr (W::kFp8) v[i] *= W::row_factor(bank ? k.b1 : k.b0, (int64_t(e) * tiles + wt[bank]) * 32 + 8 * (i >> 2) + 4 * g + (i & 3));
-                        v[i] *= scl;
+                        v[i] *= FOLD ? s_scale[8 * (i >> 2) + 4 * g + (i & 3)] : scl;
                     }
                 };
                 float v[16];
@@ -500,7 +553,14 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                         if constexpr (W::kFp8) if (k.out_bf16) return float_to_bf16_bits(x) | uint32_t(float_to_bf16_bits(y)) << 16;
                         return bits_of(v2h{_Float16(x), _Float16(y)});
                     };
-                    if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4 *>(to + (8 * c + 4 * g) * 4) = make_float4(q[0], q[1], q[2], q[3]);
+                    if constexpr (FOLD) {
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) {
+                            uint8_t * row = tile_lds + (8 * c + 4 * g + i) * kPitch;
+                            if constexpr (sizeof(OT) == 4) reinterpret_cast<float *>(row)[n] = q[i];
+                            else reinterpret_cast<_Float16 *>(row)[GATEUP ? operand_pos(n) : n] = _Float16(q[i]);
+                        }
+                    } else if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4 *>(to + (8 * c + 4 * g) * 4) = make_float4(q[0], q[1], q[2], q[3]);
                     else if constexpr (GATEUP && !W::kFp8)   // operand_pos: the four values stay together, 1 and 2 change places
                         *reinterpret_cast<uint2 *>(to + operand_pos(8 * c + 4 * g) * 2) = make_uint2(half2(q[0], q[2]), half2(q[1], q[3]));
                     else *reinterpret_cast<uint2 *>(to + (8 * c + 4 * g) * 2) = make_uint2(half2(q[0], q[1]), half2(q[2], q[3]));
