@@ -123,6 +123,31 @@ def test_topk2_equals_two_calls(tq, oracle, e, k, n):
         tq.moe_topk2(big, big, 1025, 2)
 
 
+@pytest.mark.parametrize("e,k", [(129, 1), (200, 64), (256, 8), (257, 10), (512, 10), (512, 64), (1000, 16)])
+def test_topk_by_bound_and_rank(tq, e, k):
+    """Beyond 128 experts the selection bounds the keys, ranks what reaches the bound and falls back to a round a selection where
+    two of those are equal, or there are more than lanes: by value, then by index, whatever the spacing."""
+    g = np.random.default_rng(e + k)
+    rows = g.standard_normal((12, e)).astype(np.float32)
+    order = np.argsort(-rows[1], kind="stable")
+    rows[1, order[k]] = rows[1, order[k - 1]]                    # equal across the last selection
+    rows[2, g.permutation(e)[:k + 1]] = 4.0                      # the selections all equal, and one more
+    rows[3] = np.round(rows[3])                                  # few different values
+    rows[4, g.integers(e)] = 60.0                                # one far above
+    rows[5] = np.linspace(0, 1, e)[g.permutation(e)]
+    rows[6] = np.nextafter(np.float32(1), np.float32(2)) + np.arange(e)[g.permutation(e)] * np.float32(2.0 ** -23)   # neighbouring keys
+    rows[7] = -np.abs(rows[7])                                   # negative keys
+    rows[8, ::64] += 5.0                                         # the large ones all in one lane
+    rows[9] = np.where(np.arange(e) % 2 == 0, np.float32(-0.0), np.float32(0.0))
+    rows[10, : e - k] = -30.0                                    # the selections at the end
+    logits = np.concatenate([rows, np.zeros((12, 1), np.float32)], axis=1)
+    ids, w, _ = (t.cpu().numpy() for t in tq.moe_topk(torch.from_numpy(logits).cuda(), e, k))
+    want = np.argsort(-rows, axis=1, kind="stable")[:, :k]
+    assert np.array_equal(ids, want)
+    p = np.exp(np.take_along_axis(rows, want, 1).astype(np.float64) - rows.max(axis=1, keepdims=True))
+    assert np.abs(w - p / p.sum(axis=1, keepdims=True)).max() < 1e-6
+
+
 def test_topk_ties_extremes_and_scale(tq, oracle):
     e, k = 96, 6
     rows = [np.full(e, 0.5, np.float32),                                   # all equal: lowest indices

@@ -50,6 +50,8 @@ struct DownCombineArgs {
     void * out;
     uint32_t otype;
     const uint16_t * residual;
+    int experts = 0;          // of the bank (the launcher's: a 64-bit division in the kernel was a tenth of its time)
+    uint32_t per_slot = 0;    // 2^32 / super-blocks of a row, rounded up: the product's upper half with a unit is the unit's slot
 };
 struct GateupArgs {
     BankView bg, bu;

@@ -254,53 +254,74 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
     __shared__ int meta[2], s_tok[kTP];
     __shared__ float s_x0[kTP];
-    __shared__ int ql[kMaxWaves * 2][32];
+    __shared__ __attribute__((aligned(16))) int ql[kMaxWaves * 2][32];
     __shared__ uint32_t lat[F::kLattice];
     if constexpr (FMT == TQMOE_IQ3_S)   // eight times the magnitudes (behind a barrier before the first use)
         F::lattice(lat, threadIdx.x, blockDim.x);
-    const int a = blockIdx.y, bx = int(blockIdx.x) - (ROUTE > 0 ? 1 : 0);   // bx: the block's group of row tiles
-    int e;
+    const int a = ROUTE > 0 ? int(blockIdx.z) * slots + int(blockIdx.y) : int(blockIdx.y), bx = int(blockIdx.x) - (ROUTE > 0 ? 1 : 0);   // bx: the block's group of row tiles
+    const int S = b0.cols / 32, NSB = S / 8, rows = b0.rows, tiles = rows / 32;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
+    // ROUTE: the block's one input row is known before its expert is: the row's first operands and its scale are loaded, and everything
+    // that does not depend on the expert is worked out, while that is selected (of 14600 cycles of the block 3700 passed before the
+    // expert was known, 1200 in setting up behind it, and the operands' trip began after the weights'; eight layers of one
+    // token over 512 experts 139 -> 128 us, four of 64 experts 63.9 -> 60)
+    constexpr bool EARLY = ROUTE > 0 && FMT != TQMOE_NVFP4G;   // (NVFP4G's scales leave no registers for them)
+    [[maybe_unused]] v4i a_row[EARLY ? 8 : 1];
+    [[maybe_unused]] float4 m_row[2];
+    [[maybe_unused]] float x_row = 0.f;
+    const uint8_t * const row_a = ROUTE > 0 ? image_row_ptr(image, blockIdx.z, S) : nullptr;
+    auto fetch_row = [&](int sb) {
+        if constexpr (EARLY) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a_row[i] = *reinterpret_cast<const v4i *>(row_a + (sb * 8 + i) * 64 + (n & 1) * 32 + g * 16);
+            if constexpr (F::kMin) {
+                m_row[0] = *reinterpret_cast<const float4 *>(image_sums(row_a, S) + sb * 8);
+                m_row[1] = *reinterpret_cast<const float4 *>(image_sums(row_a, S) + sb * 8 + 4);
+            }
+        }
+    };
+    int e, wk_i, rt_l;
     if constexpr (ROUTE > 0) {
         // (one wave selects, for as many rounds as its assignment needs; a block of its own, of the grid's first column, does so for
         // the token's whole routing and writes it: the weights' exponentials and divisions are then in nobody's way. One token of the
         // 512-expert IQ4_XS layer, launch 10.0 -> 9.3 us)
-        const int token = a / slots, slot = a - token * slots;
+        const int token = blockIdx.z, slot = blockIdx.y;
         const float * x = route.logits + int64_t(token) * (route.experts + 1);
         int my_id;
         float my_w;
         if (blockIdx.x == 0) {
             if (slot == 0 && threadIdx.x < 64) {
                 const float shared_logit = route.shared_weights ? x[route.experts] : 0.f;
-                topk_select<ROUTE>(x, route.experts, topk, threadIdx.x, true, my_id, my_w);
+                topk_select<ROUTE>(topk_logits<ROUTE>(x, route.experts, lane), route.experts, topk, lane, true, &ql[0][0], my_id, my_w);
                 const float v = topk_weight(my_w, topk, route.scale);
-                if (int(threadIdx.x) < topk) { route.ids[int64_t(token) * topk + threadIdx.x] = my_id; route.weights[int64_t(token) * topk + threadIdx.x] = v; }
-                if (threadIdx.x == 0 && route.shared_weights) route.shared_weights[token] = route.shared_ungated ? 1.f : 1.f / (1.f + expf(-shared_logit));
+                if (lane < topk) { route.ids[int64_t(token) * topk + lane] = my_id; route.weights[int64_t(token) * topk + lane] = v; }
+                if (lane == 0 && route.shared_weights) route.shared_weights[token] = route.shared_ungated ? 1.f : 1.f / (1.f + expf(-shared_logit));
             }
             return;
         }
-        if (slot < topk) {
-            if (threadIdx.x < 64) {
-                topk_select<ROUTE>(x, route.experts, slot + 1, threadIdx.x, false, my_id, my_w);
-                if (int(threadIdx.x) == slot) meta[0] = my_id;
-            }
-            __syncthreads();
-            e = meta[0];
-        } else {
-            e = route.experts;
+        TopkLogits<ROUTE> logits;
+        if (wave == 0) logits = topk_logits<ROUTE>(x, route.experts, lane);
+        rt_l = (wave >= wk) + (wave >= 2 * wk) + (wave >= 3 * wk), wk_i = wave - rt_l * wk;   // (at most four row tiles: divisions were a tenth of a short launch's instructions)
+        fetch_row(wk_i);
+        x_row = image_scales(row_a, S)[0];
+        if (wave == 0 && slot < topk) {
+            topk_select<ROUTE>(logits, route.experts, slot + 1, lane, false, &ql[0][0], my_id, my_w);
+            if (lane == slot) meta[0] = my_id;
         }
+        __syncthreads();
+        e = slot < topk ? meta[0] : route.experts;
     } else {
         e = fetch_ids(ids, A, a, mode, reinterpret_cast<int *>(stage));
+        rt_l = (wave >= wk) + (wave >= 2 * wk) + (wave >= 3 * wk), wk_i = wave - rt_l * wk;   // (at most four row tiles: divisions were a tenth of a short launch's instructions)
     }
     if (e < 0 || int64_t(e) * b0.rows >= b0.rows_total) return;   // skipped assignment, or an id outside the bank
     int tok[kTP];
-    const int n_tok = chunk_up(A, a, e, mode, kTP, reinterpret_cast<int *>(stage), meta, tok);   // the lists live in the dynamic space
+    const int n_tok = ROUTE > 0 ? 1 : chunk_up(A, a, e, mode, kTP, reinterpret_cast<int *>(stage), meta, tok);   // the lists live in the dynamic space
     if (n_tok == 0) return;
-    if (threadIdx.x < kTP) s_tok[threadIdx.x] = tok[threadIdx.x];
+    if (ROUTE == 0 && threadIdx.x < kTP) s_tok[threadIdx.x] = tok[threadIdx.x];
 
-    const int S = b0.cols / 32, NSB = S / 8, rows = b0.rows, tiles = rows / 32;
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
-    const int wk_i = wave % wk, rt_l = wave / wk, tile = bx * tl_count * tpw + rt_l;   // the wave's first (or only) row tile
-    const bool shared_slot = (a % slots) >= topk;
+    const int tile = bx * tl_count * tpw + rt_l;   // the wave's first (or only) row tile
+    const bool shared_slot = ROUTE > 0 ? int(blockIdx.y) >= topk : (a % slots) >= topk;
     // the shared expert may have fewer rows (gate / up) or read a narrower input row (down)
     const int row_lim = gateup && shared_slot ? shared_lim : rows;
     const int s_end = !gateup && shared_slot ? shared_lim / 32 : S;
@@ -373,7 +394,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                 if constexpr (F::kMin) sum_lds[i] = image_sums(row, S)[i - j * S];
             }
     }
-    __syncthreads();
+    if constexpr (ROUTE == 0) __syncthreads();
 
     float accf[NB][2], accm[NB][2];   // products; minimums times the activations' sums
     auto clear = [&]() {
@@ -386,8 +407,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     auto finish = [&](int tile0, bool wave_valid) {
         if constexpr (UNI) {
             if (wave_valid) {   // the rows' own scales, once
-                const float x0 = STAGED ? s_x0[2 * g] : image_scales(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S)[0];
-                const float x1 = STAGED ? s_x0[2 * g + 1] : image_scales(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S)[0];
+                const float x0 = ROUTE > 0 ? x_row : STAGED ? s_x0[2 * g] : image_scales(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S)[0];
+                const float x1 = ROUTE > 0 ? 0.f : STAGED ? s_x0[2 * g + 1] : image_scales(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S)[0];
 #pragma unroll
                 for (int nb = 0; nb < NB; ++nb) { accf[nb][0] *= x0; accf[nb][1] *= x1; }
             }
@@ -418,7 +439,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
             float v0 = 0.f, v1 = 0.f;
             if (live)
                 for (int w = 0; w < wk; ++w) { v0 += red[rt * wk + w][0][j][i]; if (NB == 2) v1 += red[rt * wk + w][NB - 1][j][i]; }
-            const int aj = live ? s_tok[j] : 0;
+            const int aj = ROUTE > 0 ? a : live ? s_tok[j] : 0;
             if (gateup) {
                 glu_clamp_inputs(glu, v0, v1);
                 const float act = glu_clamp_silu(glu, v0 / (1.f + expf(-v0))) * v1;
@@ -435,14 +456,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
         // this lane's part of operand A: plane row n of the MFMA = plane (n & 1) of input row n >> 1 (rows 8 and up repeat
         // rows 0..7: their sums land in result rows that nobody reads)
         // (not staged: straight from the image, a stride of 64 bytes per sub-block instead of the staged 256)
-        const int a_tok = max(s_tok[(n & 7) >> 1], s_tok[0]);
-        const uint8_t * a_lane = STAGED ? a_lds + ((n & 7) >> 1) * 64 + (n & 1) * 32 + g * 16 : image_row_ptr(image, a_tok / xdiv, S) + (n & 1) * 32 + g * 16;
+        const uint8_t * a_lane = ROUTE > 0 ? row_a + (n & 1) * 32 + g * 16 : STAGED ? a_lds + ((n & 7) >> 1) * 64 + (n & 1) * 32 + g * 16
+                                                : image_row_ptr(image, max(s_tok[(n & 7) >> 1], s_tok[0]) / xdiv, S) + (n & 1) * 32 + g * 16;
         constexpr int kStrideA = STAGED ? 256 : 64;
         // the two input rows whose sums land in this lane half's result registers
-        const float * sc0 = STAGED ? xs_lds + (2 * g) * S : image_scales(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S);
-        const float * sc1 = STAGED ? xs_lds + (2 * g + 1) * S : image_scales(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S);
-        const float * sum0 = STAGED ? sum_lds + (2 * g) * S : image_sums(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S);
-        const float * sum1 = STAGED ? sum_lds + (2 * g + 1) * S : image_sums(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S);
+        const float * sc0 = ROUTE > 0 ? nullptr : STAGED ? xs_lds + (2 * g) * S : image_scales(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S);
+        const float * sc1 = ROUTE > 0 ? nullptr : STAGED ? xs_lds + (2 * g + 1) * S : image_scales(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S);
+        const float * sum0 = ROUTE > 0 ? image_sums(row_a, S) : STAGED ? sum_lds + (2 * g) * S : image_sums(image_row_ptr(image, max(s_tok[2 * g], 0) / xdiv, S), S);
+        const float * sum1 = ROUTE > 0 ? nullptr : STAGED ? sum_lds + (2 * g + 1) * S : image_sums(image_row_ptr(image, max(s_tok[2 * g + 1], 0) / xdiv, S), S);
         auto multiply = [&](int sb, const Cold & cur) {
             // Staged rows: operand A and the scales of four sub-blocks at a time, right before their first use (an LDS read is
             // covered by the step in front of it; all eight at once are 16 to 32 registers more, which Q4_K and Q6_K spilled).
@@ -451,6 +472,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
             v4i areg[kPart];
             float xs0[kPart], xs1[kPart], xm0[kPart], xm1[kPart];
             auto part_a = [&](int ib0) {
+                if constexpr (!EARLY)
 #pragma unroll
                 for (int i = 0; i < kPart; ++i) areg[i] = *reinterpret_cast<const v4i *>(a_lane + (sb * 8 + ib0 + i) * kStrideA);
             };
@@ -463,7 +485,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                     }
                 };
                 if constexpr (!UNI) { get(sc0, xs0); get(sc1, xs1); }       // activation scales of the sub-blocks
-                if constexpr (F::kMin) { get(sum0, xm0); if constexpr (kIn == 2) get(sum1, xm1); }  // and their sums
+                if constexpr (F::kMin && EARLY) {
+                    const float4 f = m_row[0], h = m_row[1];
+                    xm0[0] = f.x; xm0[1] = f.y; xm0[2] = f.z; xm0[3] = f.w; xm0[4] = h.x; xm0[5] = h.y; xm0[6] = h.z; xm0[7] = h.w;
+                } else if constexpr (F::kMin) { get(sum0, xm0); get(sum1, xm1); }  // and their sums
             };
             // The products of step (sub-block, bank, scale group) + 1 are issued before the sums of this step are read: the
             // matrix pipe's latency passes under the next step's lookups instead of in front of this step's multiply-adds.
@@ -471,6 +496,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
             constexpr int G = F::kGroups, kSteps = 8 * NB * G;
             v4i w;
             [[maybe_unused]] v4i found;
+            auto operand = [&](int i) {
+                if constexpr (EARLY) return a_row[i];
+                else return areg[i];
+            };
             auto issue = [&](int step) {
                 const int ib = step / (NB * G), nb = step / G % NB, grp = step % G;
                 if (step % (kPart * NB * G) == 0) part_a(ib);
@@ -480,9 +509,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                     w = F::signed_of(found, cur.code[nb], ib, g);
                     if (step + 1 < kSteps) found = F::lookup(cur.code[(step + 1) % NB], cur.rec[(step + 1) % NB], (step + 1) / NB, g, lat);
                 } else if (grp == 0) w = F::decode(cur.code[nb], cur.rec[nb], ib, g, lat);
-                if constexpr (G == 1) return __builtin_amdgcn_mfma_i32_32x32x32_i8(areg[ib % kPart], w, zero, 0, 0, 0);
+                if constexpr (G == 1) return __builtin_amdgcn_mfma_i32_32x32x32_i8(operand(ib % kPart), w, zero, 0, 0, 0);
                 else {   // operand dwords 0 and 2 are the sub-block's first sixteen weights, 1 and 3 the others
-                    const long a2 = long(uint64_t(uint32_t(areg[ib % kPart][grp])) | uint64_t(uint32_t(areg[ib % kPart][grp + 2])) << 32);
+                    const v4i rows4 = operand(ib % kPart);
+                    const long a2 = long(uint64_t(uint32_t(rows4[grp])) | uint64_t(uint32_t(rows4[grp + 2])) << 32);
                     const long w2 = long(uint64_t(uint32_t(w[grp])) | uint64_t(uint32_t(w[grp + 2])) << 32);
                     return __builtin_amdgcn_mfma_i32_32x32x16_i8(a2, w2, zero, 0, 0, 0);
                 }
@@ -575,6 +605,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                 if (sb + wk < sb_end) fetch(sb + wk, c1);
                 multiply(sb, c0);
                 c0 = c1;
+                if constexpr (EARLY) if (sb + wk < sb_end) fetch_row(sb + wk);
             }
         }
     }
@@ -622,7 +653,8 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     int tl = 1;
     if (staged && nb == 1 && NSB % wk == 0 && (slots <= topk || shared_lim == (gateup ? b0.rows : b0.cols)))
         while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= kLeastBlocks) tl *= 2;
-    const dim3 grid(unsigned((tiles + tpw * tl - 1) / (tpw * tl) + (route.logits ? 1 : 0)), unsigned(A));
+    const unsigned groups = unsigned((tiles + tpw * tl - 1) / (tpw * tl));
+    const dim3 grid = route.logits ? dim3(groups + 1, unsigned(slots), unsigned(A / slots)) : dim3(groups, unsigned(A));
     const int a_off = int(lds);
     if (staged) lds += size_t(b0.cols / 32) * (256 + ((uniform ? 0 : 1) + (MfmaFormat<FMT>::kMin ? 1 : 0)) * kTP * sizeof(float));
     auto go = [&](auto kernel) { kernel<<<grid, threads, lds, s>>>(b0, b1, image, out0, out1, ytype, ids, A, xdiv, mode, slots, topk, shared_lim, wk, tpw, gateup, a_off, tl, glu, route); };
@@ -658,16 +690,11 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
     const int odd = HALF ? n >> 4 : 0, row_n = HALF ? int(blockIdx.x & 1) * 16 + (n & 15) : n;   // the lane's sub-blocks, its weight row in the tile
     const int shared_sb = k.slots > k.topk ? k.shared_cols / 256 : 0, units = k.topk * NSB + shared_sb;
-    const int extra = int(k.b.rows_total / k.b.rows) - 1;      // the shared expert's place
+    const int extra = k.experts - 1;                           // the shared expert's place
     struct Unit { typename F::Codes code; typename F::Rec rec; v4i a[kSub]; float4 xs[2], xm[2]; float rf; };
-    auto expert_of = [&](int u) { const int slot = min(u / NSB, k.slots - 1); return slot < k.topk ? k.ids[token * k.topk + slot] : extra; };
-    auto fetch = [&](int u, int e, Unit & c) {
-        const int slot = min(u / NSB, k.slots - 1), sb = u - slot * NSB;
-        e = min(max(e, 0), extra);   // an id outside the bank: a bank's weights, not added below
-        const int64_t at = (int64_t(e) * tiles + tile) * NSB + sb;
-        if constexpr (HALF) F::half_codes(k.b.codes + at * F::kCodeBytes, row_n, g, odd, c.code);
-        else F::codes(k.b.codes + at * F::kCodeBytes, n, g, c.code);
-        c.rec = F::rec(k.b.aux + at * F::kRecBytes, row_n);
+    auto slot_of = [&](int u) { return min(NSB == 1 ? u : int(__umulhi(uint32_t(u), k.per_slot)), k.slots - 1); };
+    auto fetch = [&](int u, int slot, int e, Unit & c) {
+        const int sb = u - slot * NSB;
         const uint8_t * row = image_row_ptr(k.image, int64_t(token) * k.slots + slot, S);
         const uint8_t * a = row + sb * 512 + (HALF ? ((n >> 1) & 1) * 64 : 0) + (n & 1) * 32 + g * 16;
 #pragma unroll
@@ -675,6 +702,11 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
         const float4 * xs = reinterpret_cast<const float4 *>(image_scales(row, S) + sb * 8);
         c.xs[0] = xs[0]; c.xs[1] = xs[1];
         if constexpr (F::kMin) { const float4 * xm = reinterpret_cast<const float4 *>(image_sums(row, S) + sb * 8); c.xm[0] = xm[0]; c.xm[1] = xm[1]; }
+        e = min(max(e, 0), extra);   // an id outside the bank: a bank's weights, not added below
+        const int64_t at = (int64_t(e) * tiles + tile) * NSB + sb;
+        if constexpr (HALF) F::half_codes(k.b.codes + at * F::kCodeBytes, row_n, g, odd, c.code);
+        else F::codes(k.b.codes + at * F::kCodeBytes, n, g, c.code);
+        c.rec = F::rec(k.b.aux + at * F::kRecBytes, row_n);
         c.rf = F::row_factor(k.b, (int64_t(e) * k.b.rows) + tile * 32 + row_n);
     };
     auto multiply = [&](const Unit & c) {
@@ -718,37 +750,44 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
     }
     // (a second unit's loads in flight under the first's products: the registers of a block of sixteen waves spill, 7.9 -> 23.7 us
     // for Q4_K at one token)
+    // what the sums need at the end, on its way meanwhile
+    const int sums = k.slots * kRows, first = threadIdx.x / kRows;
+    const float first_w = int(threadIdx.x) >= sums ? 0.f : first < k.topk ? k.weights[token * k.topk + first] : k.shared_weights[token];
+    const int64_t o = int64_t(token) * k.b.rows + int64_t(blockIdx.x) * kRows + threadIdx.x;
+    const uint16_t res = k.residual && k.otype != TQMOE_F32 && threadIdx.x < kRows ? k.residual[o] : uint16_t(0);
     for (int u = wave; u < units; u += kDownWaves) {
-        const int e = expert_of(u);
+        const int slot = slot_of(u), e = slot < k.topk ? k.ids[token * k.topk + slot] : extra;
         Unit c;
-        fetch(u, e, c);
+        fetch(u, slot, e, c);
         const float v = multiply(c);
-        if (g == 0) part[u * 32 + n] = e >= 0 && int64_t(e) * k.b.rows < k.b.rows_total ? v : 0.f;
+        if (g == 0) part[u * 32 + n] = e >= 0 && e <= extra ? v : 0.f;
     }
     __syncthreads();
     float * rows = part + units * 32;
-    for (int i = threadIdx.x; i < k.slots * kRows; i += blockDim.x) {
+    for (int i = threadIdx.x; i < sums; i += blockDim.x) {
         const int slot = i / kRows, nsb = slot < k.topk ? NSB : shared_sb;
         float v = 0.f;
         for (int sb = 0; sb < nsb; ++sb)
             for (int h = 0; h < 32 / kRows; ++h) v += part[(slot * NSB + sb) * 32 + h * kRows + i % kRows];
-        rows[i] = (slot < k.topk ? k.weights[token * k.topk + slot] : k.shared_weights[token]) * v;
+        rows[i] = (i == int(threadIdx.x) ? first_w : slot < k.topk ? k.weights[token * k.topk + slot] : k.shared_weights[token]) * v;
     }
     __syncthreads();
     if (threadIdx.x < kRows) {
         float sum = 0.f;
         for (int s = 0; s < k.slots; ++s) sum += rows[s * kRows + threadIdx.x];
-        const int64_t o = int64_t(token) * k.b.rows + int64_t(blockIdx.x) * kRows + threadIdx.x;
         if (k.otype == TQMOE_F32) static_cast<float *>(k.out)[o] = sum;
         else {
-            if (k.residual) sum = bf16_bits_to_float(float_to_bf16_bits(sum)) + bf16_bits_to_float(k.residual[o]);
+            if (k.residual) sum = bf16_bits_to_float(float_to_bf16_bits(sum)) + bf16_bits_to_float(res);
             static_cast<uint16_t *>(k.out)[o] = float_to_bf16_bits(sum);
         }
     }
 }
 
-template <uint32_t FMT> void down_combine_launch(const DownCombineArgs & k, hipStream_t s) {
-    const int NSB = k.b.cols / 256, units = k.topk * NSB + (k.slots > k.topk ? k.shared_cols / 256 : 0);
+template <uint32_t FMT> void down_combine_launch(DownCombineArgs k, hipStream_t s) {
+    const int NSB = k.b.cols / 256;
+    k.experts = int(k.b.rows_total / k.b.rows);
+    k.per_slot = 0xFFFFFFFFu / uint32_t(NSB) + 1;
+    const int units = k.topk * NSB + (k.slots > k.topk ? k.shared_cols / 256 : 0);
     const size_t lds = size_t(units + k.slots) * 32 * sizeof(float);
     if (int64_t(k.n) * (k.b.rows / 16) <= kHalfBlocks) down_combine_k<FMT, true><<<dim3(unsigned(k.b.rows / 16), unsigned(k.n)), 64 * kDownWaves, lds, s>>>(k);
     else down_combine_k<FMT, false><<<dim3(unsigned(k.b.rows / 32), unsigned(k.n)), 64 * kDownWaves, lds, s>>>(k);

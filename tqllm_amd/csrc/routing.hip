@@ -442,7 +442,8 @@ __device__ __forceinline__ void topk_reg_body(const float * __restrict__ logits,
     if (k <= 64) {
         int my_id;
         float my_w;
-        topk_select<R>(x, e, k, lane, true, my_id, my_w);
+        __shared__ __attribute__((aligned(16))) int cand[256];
+        topk_select<R>(topk_logits<R>(x, e, lane), e, k, lane, true, cand, my_id, my_w);
         const float v = topk_weight(my_w, k, scale);
         if (lane < k) {
             o.ids[int64_t(token) * k + lane] = my_id;

@@ -53,17 +53,28 @@ __device__ __forceinline__ float wave_sum_all(float v) {
 }
 
 // One wave, k <= 64 and e <= 64 R: lane s gets selection s (its expert, its softmax probability where `weights` asks for it) for the
-// first `rounds` selections. x: the token's logits; lane l owns entries l, l + 64, ...
-// Every round is a chain of dependent wave reductions, so the rounds carry only what the next round needs: the winner's key
-// stays in lane s and the probabilities are computed for all selections at once afterwards. Equal keys are rare: one ballot
-// tells whether the winner is alone, and only a tie pays for the index reduction.
-template <int R> __device__ __forceinline__ void topk_select(const float * __restrict__ x, int e, int rounds, int lane, bool weights, int & my_id, float & my_w) {
+// first `rounds` selections. cand: 256 ints in LDS of the wave's own, 16 bytes aligned.
+// A wave reduction for the maximum of every selection is a chain of 60 dependent instructions each with eight entries a lane (10 of 512:
+// 4900 cycles). So, beyond 128 entries: the `rounds`-th largest of the lanes' maxima is a bound that no selection lies below, and
+// few other entries lie above it. A search over the keys, eight parts a step, finds a bound that six maxima more reach at most;
+// what reaches it goes to a lane each and counts the larger ones (3000 cycles, more than half of them the fetch of instructions
+// that run once: the layer of one token 17.5 -> 17.2 us, 333 tokens 128.8 -> 126.6). Up to 128 entries the rounds are short: eight of 64 take
+// 2260 cycles, and the layer of one token 15.9 us with them against 16.4. Where two of what reaches the bound are equal, a
+// round for every selection.
+template <int R> struct TopkLogits { float l[R]; };   // lane l's entries l, l + 64, ... (-infinity past the end)
+template <int R> __device__ __forceinline__ TopkLogits<R> topk_logits(const float * __restrict__ x, int e, int lane) {
+    TopkLogits<R> v;
+#pragma unroll
+    for (int r = 0; r < R; ++r) { const int j = lane + 64 * r; v.l[r] = j < e ? x[j] : -INFINITY; }
+    return v;
+}
+template <int R> __device__ __forceinline__ void topk_select(const TopkLogits<R> & x, int e, int rounds, int lane, bool weights, int * cand, int & my_id, float & my_w) {
     int key[R];
     float m = -INFINITY, sum = 0.f;
     {
-        float l[R];
+        const float (&l)[R] = x.l;
 #pragma unroll
-        for (int r = 0; r < R; ++r) { const int j = lane + 64 * r; l[r] = j < e ? x[j] : -INFINITY; m = fmaxf(m, l[r]); }
+        for (int r = 0; r < R; ++r) m = fmaxf(m, l[r]);
         m = wave_max_all(m);
         // (the order alone needs the exponentials only where one may be zero, or a logit is not finite)
         bool far = false;
@@ -84,16 +95,68 @@ template <int R> __device__ __forceinline__ void topk_select(const float * __res
     }
     int my_key = kKeyZero;
     my_id = 0;
-    for (int s = 0; s < rounds; ++s) {
-        int bk = key[0], bi = lane;
+    bool alone = false;
+    if constexpr (R > 2) {
+        int most = key[0];
 #pragma unroll
-        for (int r = 1; r < R; ++r) if (key[r] > bk) { bk = key[r]; bi = lane + 64 * r; }   // strict: the lowest index of equal keys
-        const int topkey = wave_max_all_i(bk);
-        const unsigned long long tie = __ballot(bk == topkey);
-        const int best = __popcll(tie) == 1 ? __builtin_amdgcn_readlane(bi, __builtin_ctzll(tie)) : wave_min_all(bk == topkey ? bi : 0x7FFFFFFF);
-        if (lane == s) { my_id = best; my_key = topkey; }
+        for (int r = 1; r < R; ++r) most = max(most, key[r]);
+        int low = wave_min_all(most), high = order_key(m) + 1, reach = 64;   // `rounds` maxima or more reach low, fewer high
+        for (int i = 0; i < 4 && reach > rounds + 6; ++i) {
+            const uint32_t step = (uint32_t(high) - uint32_t(low)) >> 3;
+            if (step == 0) break;
+            unsigned long long mask[7];
 #pragma unroll
-        for (int r = 0; r < R; ++r) if (lane + 64 * r == best) key[r] = kKeyGone;
+            for (int q = 0; q < 7; ++q) mask[q] = __ballot(most >= int(uint32_t(low) + (q + 1) * step));
+            __builtin_amdgcn_sched_barrier(0);             // (seven comparisons, then seven counts: a chain each would be waited for in turn)
+            int parts = 0;
+#pragma unroll
+            for (int q = 0; q < 7; ++q) {
+                const int c = __popcll(mask[q]);
+                if (c >= rounds) { reach = c; parts = q + 1; }
+            }
+            low = int(uint32_t(low) + parts * step);
+            if (parts < 7) high = int(uint32_t(low) + step);
+        }
+        int total = 0;
+        cand[lane] = kKeyGone;
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const bool in = key[r] >= low;
+            const unsigned long long mask = __ballot(in);
+            const int to = __builtin_amdgcn_mbcnt_hi(uint32_t(mask >> 32), __builtin_amdgcn_mbcnt_lo(uint32_t(mask), total));
+            int * slot = cand + (in && to < 64 ? to : 64 + lane);
+            slot[0] = key[r];
+            slot[128] = lane + 64 * r + 1;
+            total += __popcll(mask);
+        }
+        alone = total <= 64;
+        if (alone) {
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int own = cand[lane], id1 = cand[128 + lane];
+            int before = 0;                            // larger keys; all of them for a lane without an entry
+            for (int c = 0; c < total; c += 8) {
+                const int4 u = *reinterpret_cast<const int4 *>(cand + c), v = *reinterpret_cast<const int4 *>(cand + c + 4);
+                before += (u.x > own) + (u.y > own) + (u.z > own) + (u.w > own) + (v.x > own) + (v.y > own) + (v.z > own) + (v.w > own);
+            }
+            my_key = __builtin_amdgcn_ds_permute(before * 4, own);
+            my_id = __builtin_amdgcn_ds_permute(before * 4, id1) - 1;
+            // (two equal keys leave the place behind them empty)
+            alone = !__any(lane <= rounds && lane < total && my_id < 0);
+        }
+    }
+    if (!alone) {                                  // equal keys: a round for every selection
+        for (int s = 0; s < rounds; ++s) {
+            int bk = key[0], bi = lane;
+#pragma unroll
+            for (int r = 1; r < R; ++r) if (key[r] > bk) { bk = key[r]; bi = lane + 64 * r; }   // strict: the lowest index of equal keys
+            const int topkey = wave_max_all_i(bk);
+            const unsigned long long tie = __ballot(bk == topkey);
+            const int best = __popcll(tie) == 1 ? __builtin_amdgcn_readlane(bi, __builtin_ctzll(tie)) : wave_min_all(bk == topkey ? bi : 0x7FFFFFFF);
+            if (lane == s) { my_id = best; my_key = topkey; }
+#pragma unroll
+            for (int r = 0; r < R; ++r) if (lane + 64 * r == best) key[r] = kKeyGone;
+        }
     }
     my_w = 0.f;
     if (weights) {
