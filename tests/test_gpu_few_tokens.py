@@ -56,6 +56,19 @@ def test_down_rows_wider_than_the_decode_products_take(tq, oracle, fmt):
         layer.forward(x)
 
 
+def test_batches_that_outgrow_the_workspace(tq, oracle):
+    """A layer's workspace grows with the batches it is given, with and without residual rows, and its results are those of a new layer."""
+    cfg = dict(hidden=512, ff=256, experts=8, topk=2, shared_ff=0, wtype=oracle.IQ4_XS, rtype="bf16", xtype="bf16")
+    banks = banks_on_device(cfg, synth.make_banks(cfg, seed=3))
+    inp = synth.make_inputs(cfg, 300, seed=4)
+    make = lambda: tq.MoeLayer(dev(inp["router"]), None, *banks, 2)
+    layer, x = make(), dev(inp["x"])
+    for n, residual in ((1, None), (40, None), (300, x), (2, x), (200, None)):
+        res = residual[:n].contiguous() if residual is not None else None
+        assert torch.equal(layer.forward(x[:n], residual=res), make().forward(x[:n], residual=res))
+    assert layer._ws.numel() == layer.workspace(300).numel()
+
+
 @pytest.mark.parametrize("experts", [65, 300])
 @pytest.mark.parametrize("spread", [70, 100, 4000])
 def test_logits_far_apart(tq, oracle, experts, spread):

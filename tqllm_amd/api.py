@@ -20,6 +20,7 @@ Q4_K, IQ3_S, IQ4_XS, NVFP4G = 12, 21, 23, 323
 Q8_0, IQ4_NL, Q5_K, Q6_K, IQ3_XXS, IQ2_S = 8, 20, 13, 14, 18, 22
 Q4_0, Q3_K, IQ2_XXS, IQ2_XS = 2, 11, 16, 17
 Q2_K, IQ1_S = 10, 19
+E_WORKSPACE = -4
 GATE_SOFTMAX, GATE_SIGMOID, GATE_SOFTMAX_WEIGHT, GATE_SQRT_SOFTPLUS = 1, 2, 3, 4   # MoeGating, src/experts/moe.hpp:20-26
 BLOCK = {Q4_K: (256, 144), IQ3_S: (256, 110), IQ4_XS: (256, 136), NVFP4G: (128, 76), IQ4_NL: (32, 18), Q8_0: (32, 34), Q5_K: (256, 176), Q6_K: (256, 210), IQ3_XXS: (256, 98), IQ2_S: (256, 82), Q4_0: (32, 18), Q3_K: (256, 110), IQ2_XXS: (256, 66), IQ2_XS: (256, 74), Q2_K: (256, 84), IQ1_S: (256, 50)}
 _TORCH_TYPE = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
@@ -724,11 +725,12 @@ class MoeLayer:
         """residual (bf16 [n][H]): added to the result, which is then bf16: bf16(bf16(layer(x)) + residual)."""
         n = x.shape[0]
         d = self._descriptor()
-        ws = self._workspace(d, n)
+        # (the library says where the workspace is too small: asking for the size first was a thirtieth of a small batch's host time)
+        ws = self._ws if self._ws is not None else self._workspace(d, n)
         if residual is not None:
             out_type = BF16
         if out is None:
-            out = torch.empty((n, self.hidden), dtype=_OUT_TYPE[out_type], device=x.device)
+            out = torch.empty(n, self.hidden, dtype=_OUT_TYPE[out_type], device=x.device)   # (a tuple costs 0.4 us)
         ids = weights = logits = None
         if return_routing:
             ids = torch.empty((n, self.topk), dtype=torch.int32, device=x.device)
@@ -737,10 +739,14 @@ class MoeLayer:
         err = _err()
         stream = _stream(x)
         routing = (ids.data_ptr(), weights.data_ptr(), logits.data_ptr()) if return_routing else (None, None, None)
-        if residual is not None:
-            rc = lib().tqmoe_layer_forward_residual(C.byref(d), x.data_ptr(), _ttype(x), residual.data_ptr(), n, out.data_ptr(), *routing, ws.data_ptr(), ws.numel(), stream,
-                                                    C.byref(err))
-        else:
-            rc = lib().tqmoe_layer_forward(C.byref(d), x.data_ptr(), _ttype(x), n, out.data_ptr(), out_type, *routing, ws.data_ptr(), ws.numel(), stream, C.byref(err))
+        while True:
+            if residual is not None:
+                rc = lib().tqmoe_layer_forward_residual(C.byref(d), x.data_ptr(), _ttype(x), residual.data_ptr(), n, out.data_ptr(), *routing, ws.data_ptr(), ws.numel(), stream,
+                                                        C.byref(err))
+            else:
+                rc = lib().tqmoe_layer_forward(C.byref(d), x.data_ptr(), _ttype(x), n, out.data_ptr(), out_type, *routing, ws.data_ptr(), ws.numel(), stream, C.byref(err))
+            if rc != E_WORKSPACE or self._workspace(d, n) is ws:
+                break
+            ws = self._ws
         _check(rc, err)
         return (out, ids, weights, logits) if return_routing else out
