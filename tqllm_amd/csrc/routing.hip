@@ -183,14 +183,19 @@ __global__ __launch_bounds__(64 * kRgWaves) void router_gemm_k(const uint8_t * _
     constexpr int C = TA == 4 ? 2 : 4;   // steps of loads together, and as many under way
     uint4 a[2][C][TA], b[2][C][4];
     auto fetch = [&](int st, int buf) {
+        // (a row's steps one after the other: both halves of a 128-byte line before other rows' lines push it out of the first-level
+        // cache. fp32, 64 experts, 4096 tokens: 30.4 -> 27.1 us; bf16 the same)
+        int64_t at[C];
 #pragma unroll
-        for (int q = 0; q < C; ++q) {
-            const int64_t at = int64_t(min(st + q, s1 - 1)) * 64;
+        for (int q = 0; q < C; ++q) at[q] = int64_t(min(st + q, s1 - 1)) * 64;
 #pragma unroll
-            for (int i = 0; i < TA; ++i) a[buf][q][i] = *reinterpret_cast<const uint4 *>(ap[i] + at);
+        for (int i = 0; i < TA; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) b[buf][q][j] = *reinterpret_cast<const uint4 *>(bp[j] + at);
-        }
+            for (int q = 0; q < C; ++q) a[buf][q][i] = *reinterpret_cast<const uint4 *>(ap[i] + at[q]);
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < C; ++q) b[buf][q][j] = *reinterpret_cast<const uint4 *>(bp[j] + at[q]);
     };
     auto multiply = [&](int st, int buf) {
 #pragma unroll
@@ -378,7 +383,7 @@ template <bool F32> void launch_router_gemm(const void * w, const void * sg, con
         }
     }
     // (2048 columns, us with 16 / 32 / 64 tokens a block: bf16, 128 blocks of 32 tokens 14.9 / 13.5 / 17.6, 128 of 64 28 / 21 / 19; fp32, 128
-    // blocks of 32 tokens 30 / 43 / 71, 256 of 64 106 / 85 / 79)
+    // blocks of 32 tokens 27 / 43 / 71, 256 of 64 106 / 85 / 79)
     if (blocks(4) >= (F32 ? 256 : 128)) go(&router_gemm_k<F32, 4>, 4, kRgLds<4>);
     else if (blocks(2) >= (F32 ? 256 : 128)) go(&router_gemm_k<F32, 2>, 2, kRgLds<2>);
     else go(&router_gemm_k<F32, 1>, 1, kRgLds<1>);
