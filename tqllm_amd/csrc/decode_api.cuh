@@ -39,6 +39,8 @@ struct DecodeTopk {
     float scale;
     int * ids;                // [n][topk]
     float * weights, * shared_weights;
+    int groups = 0, apart = 0;   // (the launcher's) groups of row tiles; 1: the grid's first block of a token writes the routing down
+    uint32_t per_group = 0;      // 2^32 / groups, rounded up
 };
 // The down product of one to a few tokens with the weighted sum over their experts in the same launch.
 struct DownCombineArgs {

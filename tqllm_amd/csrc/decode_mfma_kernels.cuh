@@ -258,7 +258,9 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     __shared__ uint32_t lat[F::kLattice];
     if constexpr (FMT == TQMOE_IQ3_S)   // eight times the magnitudes (behind a barrier before the first use)
         F::lattice(lat, threadIdx.x, blockDim.x);
-    const int a = ROUTE > 0 ? int(blockIdx.z) * slots + int(blockIdx.y) : int(blockIdx.y), bx = int(blockIdx.x) - (ROUTE > 0 ? 1 : 0);   // bx: the block's group of row tiles
+    // ROUTE: blockIdx.y is the token, blockIdx.x the slot and its group of row tiles (behind a block that only writes the routing down)
+    const int at = ROUTE > 0 ? int(blockIdx.x) - route.apart : 0, slot = ROUTE == 0 || at < 0 ? 0 : route.groups == 1 ? at : int(__umulhi(uint32_t(at), route.per_group));
+    const int a = ROUTE > 0 ? int(blockIdx.y) * slots + slot : int(blockIdx.y), bx = ROUTE > 0 ? at - slot * route.groups : int(blockIdx.x);   // bx: the block's group of row tiles
     const int S = b0.cols / 32, NSB = S / 8, rows = b0.rows, tiles = rows / 32;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), n = lane & 31, g = lane >> 5;
     // ROUTE: the block's one input row is known before its expert is: the row's first operands and its scale are loaded, and everything
@@ -269,7 +271,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     [[maybe_unused]] v4i a_row[EARLY ? 8 : 1];
     [[maybe_unused]] float4 m_row[2];
     [[maybe_unused]] float x_row = 0.f;
-    const uint8_t * const row_a = ROUTE > 0 ? image_row_ptr(image, blockIdx.z, S) : nullptr;
+    const uint8_t * const row_a = ROUTE > 0 ? image_row_ptr(image, blockIdx.y, S) : nullptr;
     auto fetch_row = [&](int sb) {
         if constexpr (EARLY) {
 #pragma unroll
@@ -282,32 +284,31 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     };
     int e, wk_i, rt_l;
     if constexpr (ROUTE > 0) {
-        // (one wave selects, for as many rounds as its assignment needs; a block of its own, of the grid's first column, does so for
-        // the token's whole routing and writes it: the weights' exponentials and divisions are then in nobody's way. One token of the
-        // 512-expert IQ4_XS layer, launch 10.0 -> 9.3 us)
-        const int token = blockIdx.z, slot = blockIdx.y;
+        // One wave selects, for as many rounds as its assignment needs. The token's whole routing is written down by a block of its own,
+        // so that the weights' exponentials and divisions are in nobody's way (one token of the 512-expert IQ4_XS layer, launch 10.0 ->
+        // 9.3 us), or, where such blocks would open another round of the compute units, by the last slot's first block (4096 x 512 experts, top-4,
+        // four tokens, 256 blocks: NVFP4G 25.5 us a layer so, 33 with blocks apart).
+        const int token = blockIdx.y;
         const float * x = route.logits + int64_t(token) * (route.experts + 1);
-        int my_id;
-        float my_w;
-        if (blockIdx.x == 0) {
-            if (slot == 0 && threadIdx.x < 64) {
-                const float shared_logit = route.shared_weights ? x[route.experts] : 0.f;
-                topk_select<ROUTE>(topk_logits<ROUTE>(x, route.experts, lane), route.experts, topk, lane, true, &ql[0][0], my_id, my_w);
+        const bool writes = route.apart ? at < 0 : bx == 0 && slot == slots - 1;
+        TopkLogits<ROUTE> logits;
+        if (wave == 0) logits = topk_logits<ROUTE>(x, route.experts, lane);
+        rt_l = (wave >= wk) + (wave >= 2 * wk) + (wave >= 3 * wk), wk_i = wave - rt_l * wk;
+        fetch_row(wk_i);
+        x_row = image_scales(row_a, S)[0];
+        if (wave == 0 && (writes || slot < topk)) {
+            const float shared_logit = writes && route.shared_weights ? x[route.experts] : 0.f;
+            int my_id;
+            float my_w;
+            topk_select<ROUTE>(logits, route.experts, writes ? topk : slot + 1, lane, writes, &ql[0][0], my_id, my_w);
+            if (lane == slot) meta[0] = my_id;
+            if (writes) {
                 const float v = topk_weight(my_w, topk, route.scale);
                 if (lane < topk) { route.ids[int64_t(token) * topk + lane] = my_id; route.weights[int64_t(token) * topk + lane] = v; }
                 if (lane == 0 && route.shared_weights) route.shared_weights[token] = route.shared_ungated ? 1.f : 1.f / (1.f + expf(-shared_logit));
             }
-            return;
         }
-        TopkLogits<ROUTE> logits;
-        if (wave == 0) logits = topk_logits<ROUTE>(x, route.experts, lane);
-        rt_l = (wave >= wk) + (wave >= 2 * wk) + (wave >= 3 * wk), wk_i = wave - rt_l * wk;   // (at most four row tiles: divisions were a tenth of a short launch's instructions)
-        fetch_row(wk_i);
-        x_row = image_scales(row_a, S)[0];
-        if (wave == 0 && slot < topk) {
-            topk_select<ROUTE>(logits, route.experts, slot + 1, lane, false, &ql[0][0], my_id, my_w);
-            if (lane == slot) meta[0] = my_id;
-        }
+        if (at < 0) return;
         __syncthreads();
         e = slot < topk ? meta[0] : route.experts;
     } else {
@@ -321,7 +322,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     if (ROUTE == 0 && threadIdx.x < kTP) s_tok[threadIdx.x] = tok[threadIdx.x];
 
     const int tile = bx * tl_count * tpw + rt_l;   // the wave's first (or only) row tile
-    const bool shared_slot = ROUTE > 0 ? int(blockIdx.y) >= topk : (a % slots) >= topk;
+    const bool shared_slot = ROUTE > 0 ? slot >= topk : (a % slots) >= topk;
     // the shared expert may have fewer rows (gate / up) or read a narrower input row (down)
     const int row_lim = gateup && shared_slot ? shared_lim : rows;
     const int s_end = !gateup && shared_slot ? shared_lim / 32 : S;
@@ -642,7 +643,7 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     // counts is that a wave's own weight loads stay in flight under its products: 10 tokens of 8 of 128 experts, Q4_K 71.5
     // and 61.3 us a layer, NVFP4G 69.2 and 68.0, IQ3_S 67.7 and 64.7); a shorter batch is one chain of dependent steps per wave,
     // and the extra stop at a barrier costs more than the exact waits return
-    const bool staged = A >= kStagedFrom;
+    const bool staged = A >= kStagedFrom && !route.logits;
     // ... and a wave then takes up to four row tiles one after the other, as long as the grid keeps five blocks per compute
     // unit: the block's search for its input rows and their staging are paid once for all of them, but a grid of two or
     // three blocks per unit, some of which find their expert taken by another and leave, ends in a round that most units
@@ -654,11 +655,17 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     if (staged && nb == 1 && NSB % wk == 0 && (slots <= topk || shared_lim == (gateup ? b0.rows : b0.cols)))
         while (tl < 4 && tiles % (tpw * tl * 2) == 0 && int64_t(tiles / (tpw * tl * 2)) * A >= kLeastBlocks) tl *= 2;
     const unsigned groups = unsigned((tiles + tpw * tl - 1) / (tpw * tl));
-    const dim3 grid = route.logits ? dim3(groups + 1, unsigned(slots), unsigned(A / slots)) : dim3(groups, unsigned(A));
+    if (route.logits) {
+        const int64_t work = int64_t(groups) * A;
+        route.groups = int(groups);
+        route.per_group = 0xFFFFFFFFu / groups + 1;
+        route.apart = (work + 255) / 256 == (work + A / slots + 255) / 256;
+    }
+    const dim3 grid = route.logits ? dim3(groups * unsigned(slots) + unsigned(route.apart), unsigned(A / slots)) : dim3(groups, unsigned(A));
     const int a_off = int(lds);
     if (staged) lds += size_t(b0.cols / 32) * (256 + ((uniform ? 0 : 1) + (MfmaFormat<FMT>::kMin ? 1 : 0)) * kTP * sizeof(float));
     auto go = [&](auto kernel) { kernel<<<grid, threads, lds, s>>>(b0, b1, image, out0, out1, ytype, ids, A, xdiv, mode, slots, topk, shared_lim, wk, tpw, gateup, a_off, tl, glu, route); };
-    if (route.logits) {   // few tokens: mode 0, nothing staged
+    if (route.logits) {   // few tokens
         if (route.experts <= 128) go(decode_mfma_k<FMT, 2, true, 0, 2>); else go(decode_mfma_k<FMT, 2, true, 0, 8>);
         return;
     }
@@ -750,15 +757,21 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
     }
     // (a second unit's loads in flight under the first's products: the registers of a block of sixteen waves spill, 7.9 -> 23.7 us
     // for Q4_K at one token)
-    // what the sums need at the end, on its way meanwhile
-    const int sums = k.slots * kRows, first = threadIdx.x / kRows;
-    const float first_w = int(threadIdx.x) >= sums ? 0.f : first < k.topk ? k.weights[token * k.topk + first] : k.shared_weights[token];
+    // what the sums need at the end, on its way meanwhile (Q6_K's whole tiles have no registers for it)
+    const int sums = k.slots * kRows;
+    auto weight_of = [&](int slot) { return slot < k.topk ? k.weights[token * k.topk + slot] : k.shared_weights[token]; };
     const int64_t o = int64_t(token) * k.b.rows + int64_t(blockIdx.x) * kRows + threadIdx.x;
-    const uint16_t res = k.residual && k.otype != TQMOE_F32 && threadIdx.x < kRows ? k.residual[o] : uint16_t(0);
+    [[maybe_unused]] float first_w = 0.f;
+    [[maybe_unused]] uint16_t res = 0;
+    if constexpr (HALF) {
+        if (int(threadIdx.x) < sums) first_w = weight_of(threadIdx.x / kRows);
+        if (k.residual && k.otype != TQMOE_F32 && threadIdx.x < kRows) res = k.residual[o];
+    }
     for (int u = wave; u < units; u += kDownWaves) {
         const int slot = slot_of(u), e = slot < k.topk ? k.ids[token * k.topk + slot] : extra;
         Unit c;
         fetch(u, slot, e, c);
+        if constexpr (!HALF && F::kGroups == 2) __builtin_amdgcn_sched_barrier(0);   // (or the decode is moved up between the loads, and Q6_K spills: one token 32 -> 82 us a layer)
         const float v = multiply(c);
         if (g == 0) part[u * 32 + n] = e >= 0 && e <= extra ? v : 0.f;
     }
@@ -769,7 +782,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
         float v = 0.f;
         for (int sb = 0; sb < nsb; ++sb)
             for (int h = 0; h < 32 / kRows; ++h) v += part[(slot * NSB + sb) * 32 + h * kRows + i % kRows];
-        rows[i] = (i == int(threadIdx.x) ? first_w : slot < k.topk ? k.weights[token * k.topk + slot] : k.shared_weights[token]) * v;
+        rows[i] = (HALF && i == int(threadIdx.x) ? first_w : weight_of(slot)) * v;
     }
     __syncthreads();
     if (threadIdx.x < kRows) {
@@ -777,7 +790,7 @@ __global__ __launch_bounds__(64 * kDownWaves) void down_combine_k(DownCombineArg
         for (int s = 0; s < k.slots; ++s) sum += rows[s * kRows + threadIdx.x];
         if (k.otype == TQMOE_F32) static_cast<float *>(k.out)[o] = sum;
         else {
-            if (k.residual) sum = bf16_bits_to_float(float_to_bf16_bits(sum)) + bf16_bits_to_float(res);
+            if (k.residual) sum = bf16_bits_to_float(float_to_bf16_bits(sum)) + bf16_bits_to_float(HALF ? res : k.residual[o]);
             static_cast<uint16_t *>(k.out)[o] = float_to_bf16_bits(sum);
         }
     }
