@@ -21,7 +21,8 @@ def tq():
 @pytest.mark.parametrize("n,hidden,ff,experts,topk,shared_ff", [(1, 256, 256, 4, 1, 0), (2, 512, 768, 64, 6, 256), (5, 2304, 512, 128, 8, 512), (6, 1280, 512, 129, 10, 256),
                                                                (7, 512, 256, 65, 3, 0), (8, 512, 256, 65, 3, 0), (1, 512, 1536, 513, 16, 512), (2, 2816, 256, 9, 2, 256),
                                                                (5, 2560, 1280, 33, 8, 256), (1, 512, 2816, 8, 5, 0), (1, 512, 2816, 8, 6, 0),
-                                                               (1, 4096, 256, 5, 2, 0), (1, 4352, 256, 5, 2, 256)])
+                                                               (1, 4096, 256, 5, 2, 0), (1, 4352, 256, 5, 2, 256),
+                                                               (12, 512, 256, 65, 3, 256), (13, 512, 256, 65, 3, 256), (9, 1024, 512, 300, 8, 0), (6, 2048, 768, 40, 10, 768)])
 def test_layer_of_few_tokens(tq, oracle, fmt, n, hidden, ff, experts, topk, shared_ff):
     cfg = dict(hidden=hidden, ff=ff, experts=experts, topk=topk, shared_ff=shared_ff, wtype=getattr(oracle, fmt), rtype="bf16", xtype="bf16")
     raws = synth.make_banks(cfg, seed=n + hidden, distinct=min(experts + 1, 8))

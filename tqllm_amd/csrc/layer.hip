@@ -37,26 +37,29 @@ namespace {
 constexpr int kQ4kHalfRows = 2048;
 // Where the descriptor asks for the int8 grouped products (act_blocks nonzero), IQ4_XS banks take them from kGroupedMin tokens.
 constexpr int kGroupedMin = 64;
-// Left to the library (act_blocks zero), IQ4_XS banks take them from kInt8Tokens tokens. The line is where the result changes,
-// not where the speed does: a scale per token on eight bits moves the layer's result by 2 % of its norm. fp16 products on
-// prepared rows are the faster ones on both sides (4096 tokens of 10 of 512 experts, Zipf / balanced: 569 / 620 us a layer
-// against 697 / 1012), so a caller whose results may change gains by a higher line.
+// Left to the library (act_blocks zero), IQ4_XS banks take them from kInt8Tokens tokens. The line is where the result changes:
+// a scale per token on eight bits moves the layer's result by 2 % of its norm. (4096 tokens of 10 of 512 experts, Zipf / balanced:
+// 525 / 611 us a layer with a scale per token, 569 / 620 with the fp16 products on prepared rows; 1500 tokens 315 with a scale per token.)
 constexpr int kInt8Tokens = 1024;
 // Few tokens: the down blocks add a token's experts themselves, and with plain softmax routing the gate / up blocks select their
 // own experts: three launches a layer instead of five (of about 2 us each on the GPU and 3.5 us of host time). An expert that
 // several tokens chose is read once for each of them, from the caches, and a block of the down launch walks all of a token's
-// weight rows: what a launch reads is the line (weights of one projection over all assignments), lower where the gate / up
-// kernel's registers leave a SIMD two waves. Layer in us, five / three launches, Q4_K and NVFP4G: 2048 x 768 experts, top-8
-// of 128, two tokens 32.6 / 26.1 and 34.7 / 28.7, seven (88 M) 49.1 / 51.2 and 55.8 / 51.2; 4096 x 1024, top-4, five (84 M)
-// 57.6 / 53.4 and 62.6 / 55.5, six (101 M) 55.7 / 58.4 and 63.5 / 64.2; 3072 x 1536, top-8 and a shared one, two (85 M) 54.4 /
-// 47.3 and 58.7 / 51.2, three (127 M) 60.2 / 78.3 and 71.8 / 77.5; and where all the down blocks find a compute unit of their
-// own (4096 x 8192, top-2 of 8, two tokens 58.0 / 52.7 and 69.4 / 59.2). A token with more than 64 units (super-blocks of its
-// experts' rows) keeps a block's sixteen waves too long (1024 x 4096, top-6, one token 28.9 / 36.7 and 29.7 / 37.8). At most
-// as many tokens as the router's one-token passes take (they write the activation images).
+// weight rows. Where all the down blocks find a compute unit of their own (256 blocks of 32 columns) the three launches are the
+// faster ones for every shape (layer in us, five / three, IQ4_XS: 2048 x 768 experts, top-8, two tokens 27.7 / 18.0, four 33.8 /
+// 26.2; 4096 x 1024, top-8, two 37.0 / 32.2; 512 x 1024, top-8, twelve 33.1 / 28.0; 7168 x 2048, top-8, one 55.0 / 49.6).
+// Beyond, what a launch reads is the line (weights of one projection over all assignments): 2048 x 768, top-8, eight tokens (101 M)
+// 44.0 / 36.7, nine (113 M) 45.7 / 47.9; 2048 x 512, top-10 and a shared one, eight (92 M) 49.0 / 38.9, nine (104 M) 49.4 / 49.3; 2048 x
+// 1024, top-8, six (101 M) 44.9 / 39.8, seven (117 M) 48.0 / 45.7 (IQ3_S 46.2 / 48.2); 4096 x 1024, top-4, six (101 M) 44.5 / 40.2, seven
+// (117 M) 49.3 / 48.2; 3072 x 1024, top-6, six (113 M) 50.1 / 49.7 (Q4_K with Q6_K 46.0 / 52.7); 2048 x 1536, top-6 and a shared one, five
+// (110 M) 46.2 / 47.8; 3072 x 1536, top-8 and a shared one, three (127 M) 53.0 / 54.7; 1024 x 512, top-8, twelve (50 M) 32.5 / 28.7. Q6_K's
+// gate / up kernel leaves a SIMD two waves: 1024 x 768, top-8 and a shared one, ten tokens 43.5 / 49.2 (2048 x 768, top-8, seven 60.9 / 51.9).
+// A token with more than 64 units (super-blocks of its experts' rows) keeps a block's sixteen waves too long (1024 x 4096, top-6, one
+// token 28.9 / 36.7).
+constexpr int kFewTokens = 12;
 bool few_tokens(uint32_t gate_type, int n, int slots, int hidden, int ff) {
-    const bool two_waves = gate_type == TQMOE_Q4_K || gate_type == TQMOE_Q6_K;
-    const bool one_round = int64_t(n) * (hidden / 32) <= 256;   // the down launch's blocks: one a compute unit
-    return n <= (two_waves ? 5 : kRouterFew) && slots * (ff / 256) <= 64 && (one_round || int64_t(n) * slots * hidden * ff <= (two_waves ? 85000000 : 90000000));
+    if (n > kFewTokens || slots * (ff / 256) > 64) return false;
+    if (int64_t(n) * (hidden / 32) <= 256) return true;           // the down launch's blocks: one a compute unit
+    return (gate_type != TQMOE_Q6_K || n <= 7) && int64_t(n) * slots * hidden * ff <= 102000000;
 }
 constexpr int kDecodeAssignments = 65535;   // per decode launch
 constexpr int kDecodeDedup = 2048;          // assignments up to which the decode kernels serve an expert's rows together

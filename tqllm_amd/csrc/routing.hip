@@ -98,7 +98,7 @@ __global__ __launch_bounds__(256) void router_k(const void * __restrict__ w, con
 
 template <int WT> int32_t launch_router_x(uint32_t xtype, const void * w, const void * sg, const void * x, float * logits,
                                           int h, int e, int n, const RouterSide & side, hipStream_t s) {
-    const bool wide = n <= kRouterFew;   // the wide grid of one-token passes
+    const bool wide = n <= kRouterFew || side.image;   // the wide grid of one-token passes (which write the activation images)
     const int tok = wide ? kRouterTokFew : kRouterTok;
     const dim3 grid(unsigned((e + 1 + 3) / 4 + (side.image || side.zero ? 1 : 0)), unsigned((n + tok - 1) / tok));
     switch (xtype) {
