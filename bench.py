@@ -301,7 +301,8 @@ def measure_point(torch, tq, cfg, key, trios, gen, T, args, traffic):
         dtype = "int8 x int8 -> int32 (weights exact, activations as two int8 planes), fp32 scales"
     else:
         op = {"grouped_i8": "int8", "grouped_f16": "fp16", "grouped_fp8": "fp8"}[path]
-        kname = {"grouped_i8": "plane_gemm_k<2, %s> (grouped gate + up int8 MFMA product + SwiGLU)" % cfg["fmt"],
+        kname = {"grouped_i8": "plane_gemm_k<2, %s> (%sgrouped gate + up int8 MFMA product + SwiGLU%s)" % (
+                     (cfg["fmt"],) + (("the general entry's ", "; the layer runs grouped_i8_k on rows in quantiser order") if cfg["fmt"] == "IQ4_XS" else ("", ""))),
                  "grouped_f16": "expert_gemm_f16_k<%s,2> (the general entry's grouped gate + up fp16 MFMA product + SwiGLU; the layer runs grouped_rows_k on prepared rows)" % cfg["fmt"],
                  "grouped_fp8": "grouped_rows_k<%s> (grouped gate + up fp8 MFMA product + SwiGLU)" % cfg["fmt"]}[path]
         roofline = {"bound": "mfma", "kernel": kname, "achieved": round(gu_ops / gu_s / 1e12, 2), "peak": PEAK[op] / 1e12, "unit": "TFLOP/s",

@@ -24,13 +24,14 @@
 // instructions; with the two banks' eight accumulators (128 registers) two waves fit a SIMD, and one of them decodes while
 // the other's products run. Items of one and two row tiles have loops of their own with fewer products.
 //
-// What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 237 us, 0.87
-// PFLOP/s (262 us with biased codes, when the matrix pipe was 43 % busy and the vector pipe 52 %; then 211 without the decode,
-// 173 without the row reads as well, which is the rate of a large fp16 product on this card); NVFP4G, 8192 tokens, gate / up
-// (2.1 TFLOP with down): 873 us, 40 % and 51 %. A product holds its SIMD's vector issue for about 18 cycles besides its own
-// time, so a stage's decode does not pass under its products for free: that sum and not a wait is what is left.
-// Items of one row tile are bound by the decode (IQ3_S, 512 tokens: gate / up 139 us, 2.5 TB/s of codes; without the look-ups'
-// bank conflicts and addresses 103, without signs and scales 104, without code transfers 116).
+// What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 228 us, 0.90
+// PFLOP/s, matrix pipe 48 % busy, vector pipe 53 % (262 us, 43 and 52 % with biased codes; then 211 without the decode, 173
+// without the row reads as well, which is the rate of a large fp16 product on this card); NVFP4G, 8192 tokens, gate / up (2.1
+// TFLOP with down): 886 us, 41 % and 53 %. A product holds its SIMD's vector issue for about 18 cycles besides its own time, so
+// a stage's decode does not pass under its products for free: that sum and not a wait is what is left.
+// Items of one row tile are bound by the decode (IQ3_S, 512 tokens: gate / up 118 us, 2.9 TB/s of codes, vector pipe 64 %, LDS 52 %,
+// three fifths of that bank conflicts of the lattice's look-ups; of 139 us on another day 103 without these and their addresses,
+// 104 without signs and scales, 116 without code transfers).
 //
 // One row tile of a format with kFold (IQ3_S): the operands are the codes times the integer scale, exact in fp16, and every 256
 // columns the fp32 sums are multiplied by the super-block's factor instead (the weights are the second operand there, so that a
