@@ -42,16 +42,13 @@ def test_layer_on_prepared_rows(tq, oracle, fmt, n, hidden, ff, shared_ff):
     assert mx < 1e-2 * (max(1.0, top) if fp8 else 1.0) and rel < (3e-3 if fp8 else 1e-3), (mx, rel)
 
 
-@pytest.mark.parametrize("shared_ff", [128, 384, 512])
-def test_iq3_s_items_of_one_row_tile(tq, oracle, shared_ff):
-    """One row tile's sums take IQ3_S's super-block factor themselves, every fourth stage and after the last: lists of a few
-    rows, the shared expert's of 32, its down product ending inside a super-block. Against float64 on the decoded weights: the
-    operands of each product are rounded to fp16 (2^-12 of a term at most, the sums' errors average), the weights are not."""
-    cfg = dict(hidden=512, ff=512, experts=7, topk=2, shared_ff=shared_ff, wtype=oracle.IQ3_S, rtype="f32", xtype="f32")
+def one_row_tile_error(tq, oracle, fmt, shared_ff, n=32):
+    """Error of a layer whose products are items of n rows and fewer, against float64 on the decoded weights."""
+    cfg = dict(hidden=512, ff=512, experts=7, topk=2, shared_ff=shared_ff, wtype=getattr(oracle, fmt), rtype="f32", xtype="f32")
     raws = synth.make_banks(cfg, seed=51)
-    inp = synth.make_inputs(cfg, 32, seed=52)
+    inp = synth.make_inputs(cfg, n, seed=52)
     layer = tq.MoeLayer(dev(inp["router"]), dev(inp["shared_gate"]), *banks_on_device(cfg, raws), 2, shared_ff=shared_ff)
-    assert layer.path(32) == "grouped_f16"
+    assert layer.path(n) == "grouped_f16"
     out, ids, w, logits = (t.cpu().numpy() for t in layer.forward(dev(inp["x"]), return_routing=True))
     g, u, d = (oracle.dequantize(cfg["wtype"], raw, 8 * 512 * 512).reshape(8, 512, 512).astype(np.float64) for raw in raws)
     x = inp["x"][1].astype(np.float64)
@@ -60,9 +57,24 @@ def test_iq3_s_items_of_one_row_tile(tq, oracle, shared_ff):
         a, b = x @ g[e, :lim].T, x @ u[e, :lim].T
         return a / (1 + np.exp(-a)) * b @ d[e, :, :lim].T
 
-    rows = np.stack([expert(e, 512) for e in range(7)], axis=1)[np.arange(32)[:, None], ids]
+    rows = np.stack([expert(e, 512) for e in range(7)], axis=1)[np.arange(n)[:, None], ids]
     want = (rows * w[:, :, None]).sum(axis=1) + expert(7, shared_ff) / (1 + np.exp(-logits[:, 7:].astype(np.float64)))
-    assert synth.errors(out, want)[1] < 2.0 ** -11
+    return synth.errors(out, want)[1]
+
+
+@pytest.mark.parametrize("shared_ff", [128, 384, 512])
+def test_iq3_s_items_of_one_row_tile(tq, oracle, shared_ff):
+    """One row tile's sums take IQ3_S's super-block factor themselves, every fourth stage and after the last: lists of a few
+    rows, the shared expert's of 32, its down product ending inside a super-block. Against float64 on the decoded weights: the
+    operands of each product are rounded to fp16 (2^-12 of a term at most, the sums' errors average), the weights are not."""
+    assert one_row_tile_error(tq, oracle, "IQ3_S", shared_ff) < 2.0 ** -11
+
+
+@pytest.mark.parametrize("shared_ff", [128, 384, 512])
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q6_K"])
+def test_items_of_one_row_tile(tq, oracle, fmt, shared_ff):
+    """The same with values times integer scales past fp16's eleven bits: rounded once (2^-12 of a term at most), as the input is."""
+    assert one_row_tile_error(tq, oracle, fmt, shared_ff) < 2.0 ** -11
 
 
 @pytest.mark.parametrize("fmt,n,shared_ff", [("Q4_K", 2048, 128), ("Q4_K", 2047, 256), ("Q6_K", 2048, 256), ("IQ3_S", 2048, 128)])
