@@ -56,3 +56,23 @@ def test_layer_equals_the_products_on_gathered_rows(tq, oracle, blocks, n, hidde
         assert synth.errors(out.cpu().numpy(), want.cpu().numpy())[1] < 1e-6
     else:
         assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("experts", [7, 60])
+def test_largest_sums_of_a_scale_per_32(tq, oracle, experts):
+    """A sub-block's integer sum at its bounds, 32 * 127 * 127 with either sign (every weight the table's first value, rows of one value):
+    the sums reach fp32 by another way than on the gathered rows, and with the same bits."""
+    n = 130
+    cfg = dict(hidden=512, ff=256, experts=experts, topk=2, shared_ff=0, wtype=oracle.IQ4_XS, rtype="f32", xtype="f32")
+    raws = [np.array(raw).reshape(-1, 136) for raw in synth.make_banks(cfg, seed=9, distinct=3)]
+    for raw in raws[:2]:
+        raw[:, 8:] = 0
+    banks = banks_on_device(cfg, [raw.reshape(-1) for raw in raws])
+    inp = synth.make_inputs(cfg, n, seed=n)
+    x = torch.ones((n, 512), device="cuda")
+    x[1::2] = -0.25
+    x[2::3] *= torch.linspace(0.0, 1.0, 512, device="cuda")
+    layer = tq.MoeLayer(dev(inp["router"]), None, *banks, 2, act_blocks=1)
+    assert layer.path(n) == "grouped_i8"
+    out, ids, w, logits = layer.forward(x, return_routing=True)
+    assert torch.isfinite(out).all() and torch.equal(out, on_gathered_rows(tq, layer, x, ids, w, logits, True, 0))

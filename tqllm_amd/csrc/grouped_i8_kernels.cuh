@@ -5,15 +5,15 @@
 //  * the rows go through registers into LDS a stage ahead, one barrier a stage; no gathered copy of them exists;
 //  * a lane loads eight code bytes of its weight row and sub-block a stage ahead, straight into registers (coalesced: the banks are
 //    tile-major), and turns them into the sixteen int8 table values that are its operand, 44 vector instructions;
-//  * one v_mfma_i32_32x32x32_i8 a (row tile, weight tile, sub-block), from zero: its sixteen sums a lane are scaled while the next
+//  * one v_mfma_i32_32x32x32_i8 a (row tile, weight tile, sub-block): its sixteen sums a lane are scaled while the next
 //    unit's product runs. A lane has one weight row, so that the weights' scales need no exchange.
 // The scale of a sub-block is applied to the sums and not inside the operand (where the 13-bit product of value and scale takes two
 // planes, two products and twice the look-ups): rows with one scale: a 24-bit integer multiply-add into the super-block's integer sum,
-// one fp32 multiply-add a super-block; rows with a scale per 32 values: sums to fp32, times the weight's scale, times the row's into the
-// fp32 result. Operations, order and roundings are those of plane_gemm_k: equal bits.
+// one fp32 multiply-add a super-block; rows with a scale per 32 values: sums to fp32, times the weight's scale (one multiply-add for
+// both), times the row's into the fp32 result. Order and roundings are those of plane_gemm_k: equal bits.
 //
 // Bound by vector instructions: a unit (65,536 operations) is one product (32 cycles of the matrix pipe, about 18 of the
-// vector issue) and 16 multiply-adds and 4 folds of 4 to 5 cycles each (a scale per 32 values: 48), the operand's decode (22) spread over
+// vector issue) and 16 multiply-adds and 4 folds of 4 to 5 cycles each (a scale per 32 values: 32), the operand's decode (22) spread over
 // the item's row tiles. 4096 tokens of 10 of 512 experts, Zipf: gate / up 336 -> 293 us, down 226 -> 179, and the two launches that
 // gathered rows (55 us) are one that quantises them (17); 1501 tokens, a scale per 32 values, balanced: gate / up 555 -> 227 us, down
 // 326 -> 145, no launch between (a weight tile's act values are one block of 32: the gate / up product quantises them itself).
@@ -100,6 +100,15 @@ __global__ __launch_bounds__(256, MAX == 1 ? 3 : 2) void grouped_i8_k(GroupedArg
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[b][m][i] = 0.f;
         if (GATEUP ? grp * 128 < row_lim : true) {
+            // Where sums go to fp32 one by one, a product starts from the bits of kBias = 1.5 * 2^23: its result p, read as a float, is
+            // kBias + p (|p| is at most 32 * 127 * 127), and one multiply-add to kBias * -d, which is exact (d has 17 bits), is p * d rounded
+            // once, as conversion and multiplication give it. (us a layer of 512 experts, converted / from the bits: 64 tokens 229 / 202, 1501
+            // 383 / 356, 8192 1302 / 1182.)
+            constexpr float kBias = 12582912.f;
+            v16i start;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) start[i] = BLK ? __builtin_bit_cast(int, kBias) : 0;
+            if constexpr (BLK) asm volatile("" : "+v"(start));   // (sixteen registers kept; they would be written for every product)
             int isum[2][MT][BLK ? 1 : 16];
             const uint8_t * x_src[MT];
             const float * s_src = nullptr;
@@ -152,19 +161,21 @@ __global__ __launch_bounds__(256, MAX == 1 ? 3 : 2) void grouped_i8_k(GroupedArg
                     asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
                     put_rows(1 - half);
                     load_rows(st + 2);
+                    constexpr bool kLate = BLK && MAX == 1;   // one set of sums and of the rows' scales: three waves a SIMD have no registers for two (31 spilled, 1501 tokens 378 -> 432)
                     v16i pend;
                     [[maybe_unused]] float4 pend_s[4];
                     auto fold = [&](int u) {   // unit u of the stage: sub-block u / (2 MT), row tile, weight tile
                         const int i = u / (2 * MT), m = u / 2 % MT, b = u & 1, ib = 4 * half + i;
                         if constexpr (BLK) {
-                            const float d = __fmul_rn(W::d(rec[b]), float(W::scale(rec[b], ib)));
+                            const float d = __fmul_rn(W::d(rec[b]), float(W::scale(rec[b], ib))), off = __fmul_rn(d, -kBias);
+                            auto scaled = [&](int q) { return __fmaf_rn(__builtin_bit_cast(float, int(pend[q])), d, off); };
 #pragma unroll
                             for (int c = 0; c < 4; ++c) {
                                 float * a = &acc[b][m][4 * c];
-                                a[0] = __fmaf_rn(__fmul_rn(float(pend[4 * c]), d), pend_s[c].x, a[0]);
-                                a[1] = __fmaf_rn(__fmul_rn(float(pend[4 * c + 1]), d), pend_s[c].y, a[1]);
-                                a[2] = __fmaf_rn(__fmul_rn(float(pend[4 * c + 2]), d), pend_s[c].z, a[2]);
-                                a[3] = __fmaf_rn(__fmul_rn(float(pend[4 * c + 3]), d), pend_s[c].w, a[3]);
+                                a[0] = __fmaf_rn(scaled(4 * c), pend_s[c].x, a[0]);
+                                a[1] = __fmaf_rn(scaled(4 * c + 1), pend_s[c].y, a[1]);
+                                a[2] = __fmaf_rn(scaled(4 * c + 2), pend_s[c].z, a[2]);
+                                a[3] = __fmaf_rn(scaled(4 * c + 3), pend_s[c].w, a[3]);
                             }
                         } else {
                             const int ls = W::scale(rec[b], ib);
@@ -187,19 +198,24 @@ __global__ __launch_bounds__(256, MAX == 1 ? 3 : 2) void grouped_i8_k(GroupedArg
                         for (int m = 0; m < MT; ++m) {
                             const v4i a = *reinterpret_cast<const v4i *>(&s_rows[half][m * 4096 + n * 128 + (((2 * i + g) ^ ((n >> 1) & 7)) * 16)]);
                             [[maybe_unused]] float4 sc[4];
-                            if constexpr (BLK) {
+                            auto scales = [&](float4 (&to)[4]) {
 #pragma unroll
-                                for (int c = 0; c < 4; ++c) sc[c] = *reinterpret_cast<const float4 *>(&s_bs[half][m * 128 + i * 32 + 8 * c + 4 * g]);
-                            }
+                                for (int c = 0; c < 4; ++c) to[c] = *reinterpret_cast<const float4 *>(&s_bs[half][m * 128 + i * 32 + 8 * c + 4 * g]);
+                            };
+                            if constexpr (BLK && !kLate) scales(sc);
 #pragma unroll
                             for (int b = 0; b < 2; ++b) {
-                                const v16i zero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
                                 const int u = (i * MT + m) * 2 + b;
-                                const v16i p = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w[b], zero, 0, 0, 0);
-                                if (u) fold(u - 1);
+                                if constexpr (kLate) {
+                                    if (u) fold(u - 1);
+                                    __builtin_amdgcn_sched_barrier(0);
+                                }
+                                const v16i p = __builtin_amdgcn_mfma_i32_32x32x32_i8(a, w[b], start, 0, 0, 0);
+                                if constexpr (kLate) { if (b == 0) scales(pend_s); }
+                                else if (u) fold(u - 1);
                                 __builtin_amdgcn_sched_barrier(0);
                                 pend = p;
-                                if constexpr (BLK) {
+                                if constexpr (BLK && !kLate) {
 #pragma unroll
                                     for (int c = 0; c < 4; ++c) pend_s[c] = sc[c];
                                 }
