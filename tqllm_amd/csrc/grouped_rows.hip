@@ -23,11 +23,14 @@ template <uint32_t FMT> void grouped_rows_run(const GroupedArgs & k, int item_ro
 
 // Rows of an item at most. 128 spread a weight's decode over four row tiles; 64 need 168 registers in place of 256, three waves
 // a SIMD in place of two, which is what counts where most experts have a row tile or two. fp16 products, layer in us at 64 /
-// 128 rows: 16 rows an expert (IQ3_S, 512 tokens) 245 / 266, 27 rows 376 / 395, 32 rows 108 / 110, 64 rows 143 / 137; 7 rows
-// an expert on average but Zipf routing (IQ4_XS, 333 tokens) 161 / 152, which the averages cannot tell. (32 rows and four
-// waves: 238, 382, 121, 160 and 173.) The fp8 products' codes leave LDS for two blocks either way: 128.
+// 128 rows, balanced and Zipf routing: IQ3_S, 256 experts with 16 rows 215 / 231 and 162 / 174, with 33 rows 273 / 296 and 235 / 236,
+// with 44 rows 296 / 320 and 276 / 279; IQ4_XS, 77 experts with 42 rows 189 / 197 and 201 / 203, 128 with 35 rows 166 / 168 and 164 / 162, with
+// 45 rows 187 / 185 and 187 / 178; Q4_K, 64 experts with 44 rows 98 / 102 and 109 / 126, with 60 rows 119 / 116 and 124 / 140; Q4_K / Q6_K, 128
+// experts with 45 rows 182 / 186 and 190 / 181, with 77 rows 244 / 233. Zipf routing of few tokens over many experts (IQ4_XS, 333 tokens, 7
+// rows an expert) has the other order, 124 / 116, which the averages cannot tell. (Items of 32 rows, four waves a SIMD: 238 us at IQ3_S's
+// 16 rows when 64 took 245, and slower from there.) The fp8 products' codes leave LDS for two blocks either way: 128.
 int grouped_rows_per_item(uint32_t type, int64_t assignments, int experts) {
-    return type != TQMOE_NVFP4G && assignments <= int64_t(experts) * 32 ? 64 : 128;
+    return type != TQMOE_NVFP4G && assignments <= int64_t(experts) * 40 ? 64 : 128;
 }
 
 bool grouped_rows_takes(uint32_t type, int rows, int cols) {
