@@ -40,7 +40,8 @@
 // Q6_K: bias and scale are whole numbers that halves hold, so that one packed multiply-add, rounded once, does for a pair of weights
 // what two mixed ones and a conversion do: eight instructions fewer for eight weights, 64 a stage for the 16 (us a layer without / with, IQ4_XS
 // on 512 experts: 200 tokens 299 / 267, Zipf 103 / 98, 1023 tokens 328 / 301; Q6_K on 77, 64 tokens 174 / 165; the error 5.2e-4 / 4.6e-4).
-// Two row tiles have no registers for the second set of sums.
+// Two row tiles have no registers for the second set of sums: a row's last bits say whether its item had one row tile or more. Items of
+// up to 128 rows, whose rests of one row tile are few, keep whole weights in IQ4_XS and Q6_K, and a row's bits with them.
 #pragma once
 #include "decode_api.cuh"
 #include "decode_table.cuh"
@@ -76,12 +77,12 @@ __device__ __forceinline__ v2h bias_odd(uint32_t u) { return as_h2(__builtin_amd
 // What the kernel needs of a format.
 // kCodes: 1 KB transfers a bank and stage (64 lanes x 16 bytes): code() the lane's source, code_at() what to add
 // for a transfer and stage. kRecs transfers for both banks' records: rec(), rec_at(). Prep: what decoding a stage needs in registers;
-// slice(): piece j (16 bytes) of operand B; with kFold also whole(), the piece without the super-block's factor fold(). kTab
+// slice(): piece j (16 bytes) of operand B; up to kFold row tiles an item also whole(), the piece without the super-block's factor fold(). kTab
 // bytes of lookup table in LDS, filled by tables(). row_factor(): a factor of a whole weight row.
 template <uint32_t FMT> struct GroupedFormat;
 
 struct GroupedWhole {                     // no factor outside the operands
-    static constexpr bool kFold = false;
+    static constexpr int kFold = 0;
     template <class P> static __device__ __forceinline__ float fold(const P &) { return 1.f; }
     template <class P> static __device__ __forceinline__ uint4 whole(P &, int) { return uint4(); }
 };
@@ -98,7 +99,7 @@ struct GroupedNibbles : GroupedHalves {   // 16 code bytes a sub-block in the ca
 };
 
 template <> struct GroupedFormat<TQMOE_IQ4_XS> : GroupedNibbles {
-    static constexpr bool kFold = true;
+    static constexpr int kFold = 2;
     static __device__ __forceinline__ const uint8_t * rec(const BankView & b0, const BankView & b1, int64_t tile0, int64_t tile1, int S, int, int lane) {
         const int l = lane & 31;   // sixteen lanes a bank; the upper half of the wave repeats the lower
         return (l < 16 ? b0.aux + tile0 * (S / 8) * 256 : b1.aux + tile1 * (S / 8) * 256) + (l & 15) * 16;
@@ -163,7 +164,7 @@ template <> struct GroupedFormat<TQMOE_Q4_K> : GroupedNibbles {
 };
 
 template <> struct GroupedFormat<TQMOE_Q6_K> : GroupedHalves {
-    static constexpr bool kFold = true;
+    static constexpr int kFold = 2;
     static constexpr int kCodes = 1, kRecs = 3;   // low nibbles; then both banks' upper bits (512 bytes each) and each bank's records
     static __device__ __forceinline__ const uint8_t * code(const BankView & b, int64_t tile, int S, int lane) { return b.codes + tile * (S / 8) * 6144 + lane * 16; }
     static __device__ __forceinline__ int code_at(int, int st) { return (st >> 2) * 6144 + (st & 3) * 1024; }
@@ -208,7 +209,7 @@ template <> struct GroupedFormat<TQMOE_Q6_K> : GroupedHalves {
 };
 
 template <> struct GroupedFormat<TQMOE_IQ3_S> : GroupedHalves {
-    static constexpr bool kFold = true;
+    static constexpr int kFold = 4;
     // Points 0..255 are the table's first 2 KB; the others follow 2 and again 4 KB behind it, so that an index's ninth bit is an
     // address bit after one shift for two of them.
     static constexpr int kCodes = 1, kRecs = 1, kTab = 6144;
@@ -394,7 +395,7 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
 
     auto body = [&](auto tag) {
         constexpr int MT = decltype(tag)::value;
-        constexpr bool FOLD = W::kFold && MT == 1;
+        constexpr bool FOLD = MT == 1 && MAX <= W::kFold;
         v16f acc[2][MT], part[2];
 #pragma unroll
         for (int b = 0; b < 2; ++b)
