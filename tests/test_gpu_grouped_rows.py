@@ -42,6 +42,13 @@ def test_layer_on_prepared_rows(tq, oracle, fmt, n, hidden, ff, shared_ff):
     assert mx < 1e-2 * (max(1.0, top) if fp8 else 1.0) and rel < (3e-3 if fp8 else 1e-3), (mx, rel)
 
 
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "Q6_K", "IQ3_S"])
+@pytest.mark.parametrize("n,hidden,ff,shared_ff", [(86, 256, 256, 0), (97, 512, 256, 0), (90, 512, 512, 256), (128, 256, 768, 0), (129, 1280, 256, 0)])
+def test_layer_on_items_of_64_rows(tq, oracle, fmt, n, hidden, ff, shared_ff):
+    """24.5 to 37 rows an expert on average: items of one and two row tiles, the last ones of 22, 33, 26, 64 and one row."""
+    test_layer_on_prepared_rows(tq, oracle, fmt, n, hidden, ff, shared_ff)
+
+
 def one_row_tile_error(tq, oracle, fmt, shared_ff, n=32):
     """Error of a layer whose products are items of n rows and fewer, against float64 on the decoded weights."""
     cfg = dict(hidden=512, ff=512, experts=7, topk=2, shared_ff=shared_ff, wtype=getattr(oracle, fmt), rtype="f32", xtype="f32")
@@ -75,6 +82,13 @@ def test_iq3_s_items_of_one_row_tile(tq, oracle, shared_ff):
 def test_items_of_one_row_tile(tq, oracle, fmt, shared_ff):
     """The same with values times integer scales past fp16's eleven bits: rounded once (2^-12 of a term at most), as the input is."""
     assert one_row_tile_error(tq, oracle, fmt, shared_ff) < 2.0 ** -11
+
+
+@pytest.mark.parametrize("shared_ff", [128, 512])
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q6_K"])
+def test_items_of_two_row_tiles(tq, oracle, fmt, shared_ff):
+    """Items of up to 64 rows keep the factor outside too: the same bound."""
+    assert one_row_tile_error(tq, oracle, fmt, shared_ff, n=100) < 2.0 ** -11
 
 
 @pytest.mark.parametrize("fmt,n,shared_ff", [("Q4_K", 2048, 128), ("Q4_K", 2047, 256), ("Q6_K", 2048, 256), ("IQ3_S", 2048, 128)])

@@ -1,0 +1,55 @@
+"""A token's result is the same bits whatever the other tokens of its batch are: they decide how many rows its experts' products
+have, and with that the size and place of its items, and nothing else."""
+import pytest
+import torch
+
+import synth
+from gpu_util import banks_on_device, dev
+
+pytestmark = pytest.mark.gpu
+
+KEPT = (0, 1, 30)    # tokens that stay
+
+
+def layer_and_rows(oracle, fmt, n, experts, act_blocks, hidden=512, ff=256):
+    import tqllm_amd as tq
+    cfg = dict(hidden=hidden, ff=ff, experts=experts, topk=4, shared_ff=256, wtype=getattr(oracle, fmt), rtype="bf16", xtype="bf16")
+    banks = banks_on_device(cfg, synth.make_banks(cfg, seed=61, distinct=5))
+    inp = synth.make_inputs(cfg, n, seed=62)
+    return tq.MoeLayer(dev(inp["router"]), dev(inp["shared_gate"]), *banks, 4, shared_ff=256, act_blocks=act_blocks), dev(inp["x"])
+
+
+def check(layer, x, crowded):
+    """The batch as it is, and with other tokens: all of them near the first kept one, so that its four experts have a row of
+    every token, then all of them its opposite, so that they have few."""
+    n, kept = x.shape[0], torch.tensor(KEPT, device="cuda")
+    others = torch.ones(n, dtype=torch.bool, device="cuda")
+    others[kept] = False
+    want, ids, _, _ = layer.forward(x, return_routing=True)
+    noise = 0.05 * torch.randn(x.shape, device="cuda", generator=torch.Generator("cuda").manual_seed(5))
+    for sign in (1, -1):
+        y = torch.where(others[:, None], (sign * x[:1].float() + noise).to(x.dtype), x)
+        out, ids2, _, _ = layer.forward(y, return_routing=True)
+        assert torch.equal(ids2[kept], ids[kept])
+        rows = [(ids2 == e).any(dim=1).sum().item() for e in ids[0].tolist()]
+        assert min(rows) > 0.6 * n if sign == 1 else max(rows) < crowded, rows
+        assert torch.equal(out[kept], want[kept]), [synth.errors(out[t].cpu().numpy(), want[t].cpu().numpy())[1] for t in KEPT]
+
+
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "Q6_K", "IQ3_S", "NVFP4G", "Q5_K", "IQ2_S"])
+@pytest.mark.parametrize("n,path", [(31, "decode"), (60, "grouped"), (250, "grouped"), (800, "grouped")])
+def test_result_does_not_depend_on_the_other_tokens(oracle, fmt, n, path):
+    """The decode products, and the grouped ones with 5, 37 and 118 rows an expert on average: items of all sizes, with one row tile
+    in one batch and several in the other."""
+    layer, x = layer_and_rows(oracle, fmt, n, 60 if n == 31 else 33, 0)
+    assert layer.path(n).startswith(path)
+    check(layer, x, 0.3 * n)
+
+
+@pytest.mark.parametrize("fmt", ["IQ4_XS", "Q4_K", "IQ3_S"])
+@pytest.mark.parametrize("n", [70, 400])
+@pytest.mark.parametrize("act_blocks", [1, 2])
+def test_int8_result_does_not_depend_on_the_other_tokens(oracle, fmt, n, act_blocks):
+    layer, x = layer_and_rows(oracle, fmt, n, 33, act_blocks)
+    assert layer.path(n) == "grouped_i8"
+    check(layer, x, 0.3 * n)

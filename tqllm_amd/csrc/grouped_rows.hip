@@ -23,13 +23,21 @@ template <uint32_t FMT> void grouped_rows_run(const GroupedArgs & k, int item_ro
 
 // Rows of an item at most. 128 spread a weight's decode over four row tiles; 64 need 168 registers in place of 256, three waves
 // a SIMD in place of two, which is what counts where most experts have a row tile or two. fp16 products, layer in us at 64 /
-// 128 rows, balanced and Zipf routing: IQ3_S, 256 experts with 16 rows 215 / 231 and 162 / 174, with 33 rows 273 / 296 and 235 / 236,
-// with 44 rows 296 / 320 and 276 / 279; IQ4_XS, 77 experts with 42 rows 189 / 197 and 201 / 203, 128 with 35 rows 166 / 168 and 164 / 162, with
-// 45 rows 187 / 185 and 187 / 178; Q4_K, 64 experts with 44 rows 98 / 102 and 109 / 126, with 60 rows 119 / 116 and 124 / 140; Q4_K / Q6_K, 128
-// experts with 45 rows 182 / 186 and 190 / 181, with 77 rows 244 / 233. Zipf routing of few tokens over many experts (IQ4_XS, 333 tokens, 7
-// rows an expert) has the other order, 124 / 116, which the averages cannot tell. (Items of 32 rows, four waves a SIMD: 238 us at IQ3_S's
-// 16 rows when 64 took 245, and slower from there.) The fp8 products' codes leave LDS for two blocks either way: 128.
+// 128 rows, balanced and Zipf routing: IQ3_S, 256 experts with 16 rows 210 / 234 and 160 / 177, with 35 rows 273 / 297 and 238 / 243,
+// with 40 rows 282 / 304 and 262 / 258; IQ4_XS, 77 experts with 40 rows 196 / 203 and 203 / 206, 128 with 35 rows 165 / 175 and 161 / 155, with
+// 40 rows 178 / 181 and 169 / 168; Q6_K, 77 with 40 rows 210 / 214 and 231 / 224; Q4_K, 64 experts with 44 rows 98 / 102 and 109 / 126, with 60
+// rows 119 / 116 and 124 / 140; Q4_K / Q6_K, 128 experts with 42 rows 177 / 183 and 182 / 177, with 84 rows 264 / 248 and 261 / 242.
+// 32, of the formats whose items of one row tile keep the super-block's factor out of the operands: all items have one then, in three
+// waves a SIMD, but an expert's weights are decoded for every 32 of its rows, which Zipf routing's popular experts feel. At 32 / 64 rows:
+// IQ4_XS, 512 experts with 3 rows 247 / 281 and 87 / 95, with 7 rows 272 / 295 and 126 / 126 (128 rows, Zipf: 116, which the averages cannot
+// tell), with 14 rows 283 / 301 and 171 / 168, with 22 rows 298 / 321 and 240 / 221, 128 experts with 22 rows 139 / 150 and 129 / 130, with 30 rows
+// 147 / 161 and 159 / 157, with 35 rows 167 / 165 and 175 / 161, 77 experts with 30 rows 181 / 177 and 179 / 174; Q6_K, 77 experts with 10 rows
+// 171 / 172 and 126 / 151, with 22 rows 195 / 188 and 171 / 181, with 30 rows 200 / 198 and 205 / 199. IQ3_S (64 rows: whole weights, three waves), 256
+// experts with 8 rows 199 / 203 and 115 / 121, with 16 rows 206 / 210 and 172 / 160, with 22 rows 231 / 231 and 218 / 188.
+// The fp8 products' codes leave LDS for two blocks either way: 128.
 int grouped_rows_per_item(uint32_t type, int64_t assignments, int experts) {
+    const int one_tile = type == TQMOE_IQ4_XS || type == TQMOE_Q6_K ? 24 : type == TQMOE_IQ3_S ? 16 : 0;
+    if (assignments <= int64_t(experts) * one_tile) return 32;
     return type != TQMOE_NVFP4G && assignments <= int64_t(experts) * 40 ? 64 : 128;
 }
 

@@ -31,7 +31,7 @@ struct RowIndex { int * tile_base, * chunk_base, * counters; int counters_n, chu
 
 bool grouped_rows_takes(uint32_t type, int rows, int cols);
 inline bool grouped_rows_aligned(const tqmoe_bank & b) { return aligned16(b.codes) && aligned16(b.aux); }   // planes that lie otherwise have the general products
-int grouped_rows_per_item(uint32_t type, int64_t assignments, int experts);   // input rows of an item at most: 64 or 128
+int grouped_rows_per_item(uint32_t type, int64_t assignments, int experts);   // input rows of an item at most: 32, 64 or 128 (type: the gate bank's)
 inline int64_t grouped_rows_items(int64_t assignments, int experts, int item_rows) { return assignments / item_rows + experts; }   // at most
 
 void enqueue_prepare_rows(const void * x, uint32_t xtype, int64_t rows, int cols, uint16_t * out, float * xs, hipStream_t s);

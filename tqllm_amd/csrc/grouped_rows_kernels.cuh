@@ -33,15 +33,17 @@
 // three fifths of that bank conflicts of the lattice's look-ups; of 139 us on another day 103 without these and their addresses,
 // 104 without signs and scales, 116 without code transfers).
 //
-// One row tile of a format with kFold (IQ3_S, IQ4_XS, Q6_K): the operands are the codes times the integer scale, and every 256
+// Items of up to kFold row tiles (IQ4_XS and Q6_K: two, IQ3_S: one): the operands are the codes times the integer scale, and every 256
 // columns the fp32 sums are multiplied by the super-block's factor instead (the weights are the second operand there, so that a
 // lane's factor is its own weight row's). IQ3_S: exact in fp16, 32 of 224 vector instructions a stage less for 16 more, and a rounding
-// fewer (512 tokens, 16 rows an expert: 222 us a layer so, 213 folded; the error against float64 5.2e-4 and 3.6e-4). IQ4_XS and
-// Q6_K: bias and scale are whole numbers that halves hold, so that one packed multiply-add, rounded once, does for a pair of weights
-// what two mixed ones and a conversion do: eight instructions fewer for eight weights, 64 a stage for the 16 (us a layer without / with, IQ4_XS
-// on 512 experts: 200 tokens 299 / 267, Zipf 103 / 98, 1023 tokens 328 / 301; Q6_K on 77, 64 tokens 174 / 165; the error 5.2e-4 / 4.6e-4).
-// Two row tiles have no registers for the second set of sums: a row's last bits say whether its item had one row tile or more. Items of
-// up to 128 rows, whose rests of one row tile are few, keep whole weights in IQ4_XS and Q6_K, and a row's bits with them.
+// fewer (the error against float64 5.2e-4 without, 3.6e-4 so). IQ4_XS and Q6_K: bias and scale are whole numbers that halves hold, so that
+// one packed multiply-add, rounded once, does for a pair of weights what two mixed ones and a conversion do: eight instructions fewer
+// for eight weights, 64 a stage for the 16 (the error 5.2e-4 / 4.6e-4). The sums of both kinds are rounded differently, by 3 to 5.5e-4 of a
+// result's norm, so that the loops of one kernel are all of one kind: a row's bits do not say how many rows its expert has from other
+// tokens. The second set of sums leaves two row tiles two waves a SIMD in place of three; four have no registers for it. Layer in us, items of
+// 64 rows, whole weights / factor outside: 77 experts with 30 rows on average IQ4_XS 181 / 177 (Zipf 178 / 174), Q6_K 203 / 198 (205 / 199), IQ3_S 179
+// / 183 (180 / 185). (Two row tiles with one weight tile after the other keep three waves and read the rows twice: level where most items have
+// one row tile, 4 to 15 % slower under Zipf.)
 #pragma once
 #include "decode_api.cuh"
 #include "decode_table.cuh"
@@ -77,7 +79,7 @@ __device__ __forceinline__ v2h bias_odd(uint32_t u) { return as_h2(__builtin_amd
 // What the kernel needs of a format.
 // kCodes: 1 KB transfers a bank and stage (64 lanes x 16 bytes): code() the lane's source, code_at() what to add
 // for a transfer and stage. kRecs transfers for both banks' records: rec(), rec_at(). Prep: what decoding a stage needs in registers;
-// slice(): piece j (16 bytes) of operand B; up to kFold row tiles an item also whole(), the piece without the super-block's factor fold(). kTab
+// slice(): piece j (16 bytes) of operand B; in items of up to kFold row tiles whole(), the piece without the super-block's factor fold(). kTab
 // bytes of lookup table in LDS, filled by tables(). row_factor(): a factor of a whole weight row.
 template <uint32_t FMT> struct GroupedFormat;
 
@@ -209,7 +211,7 @@ template <> struct GroupedFormat<TQMOE_Q6_K> : GroupedHalves {
 };
 
 template <> struct GroupedFormat<TQMOE_IQ3_S> : GroupedHalves {
-    static constexpr int kFold = 4;
+    static constexpr int kFold = 1;
     // Points 0..255 are the table's first 2 KB; the others follow 2 and again 4 KB behind it, so that an index's ninth bit is an
     // address bit after one shift for two of them.
     static constexpr int kCodes = 1, kRecs = 1, kTab = 6144;
@@ -328,9 +330,8 @@ template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
 // bytes of a wave's codes and records of one stage
 template <class W> constexpr int kStageW = 2 * W::kCodes * 1024 + W::kRecs * 1024;
 template <class W> constexpr int kStageCols = W::kFp8 ? 128 : 64;   // columns of a stage: 128 bytes of a row
-// blocks a compute unit holds (four waves each, so waves a SIMD): the accumulators of MAX row tiles set the registers, longer
-// codes the LDS
-template <class W, int MAX> constexpr int kGroupedWaves = MAX == 4 || kStageW<W> > 4096 ? 2 : 3;
+// blocks a compute unit holds (four waves each, so waves a SIMD): the accumulators of MAX row tiles set the registers
+template <class W, int MAX> constexpr int kGroupedWaves = MAX == 4 || (MAX == 2 && W::kFold == 2) ? 2 : 3;
 // Stages of input rows and of codes in LDS for MT row tiles, in the part of a compute unit's 160 KB that one of its blocks may
 // take. Codes come from HBM and may be two and more stages on their way; rows come from the L2 (an item's other blocks read
 // the same). (Q4_K at 4096 tokens: 554 us a layer with one stage of codes under way, 521 with two.) With three blocks a unit
@@ -339,14 +340,14 @@ template <class W, int MAX> constexpr int kGroupedWaves = MAX == 4 || kStageW<W>
 // to five are the same to 0.5 %.
 template <class W, int MT, int MAX> struct Rings {
     static constexpr int kLds = 163840 / kGroupedWaves<W, MAX> - W::kTab - 1280;   // what one of the unit's blocks may take
-    static constexpr int kRows = MT == 4 || MAX == 2 ? 2 : MT == 2 || kStageW<W> > 4096 ? 3 : 4;
+    static constexpr int kRows = MT == 4 || kGroupedWaves<W, MAX> == 3 ? 2 : MT == 2 || kStageW<W> > 4096 ? 3 : 4;
     static constexpr int kRoom = (kLds - kRows * MT * 4096) / (4 * kStageW<W>);
-    static constexpr int kMost = MAX == 2 ? 2 : 5, kCodes = kRoom < kMost ? kRoom : kMost;
+    static constexpr int kMost = kGroupedWaves<W, MAX> == 3 ? 2 : 5, kCodes = kRoom < kMost ? kRoom : kMost;
     static_assert(kCodes >= 2, "two stages of codes");
     static constexpr int kBytes = kRows * MT * 4096 + 4 * kCodes * kStageW<W>;
 };
 template <class W, int MAX> constexpr int grouped_lds() {
-    const int a = Rings<W, 1, MAX>::kBytes, b = Rings<W, 2, MAX>::kBytes, c = Rings<W, MAX, MAX>::kBytes;
+    const int a = Rings<W, 1, MAX>::kBytes, b = Rings<W, MAX == 4 ? 2 : MAX, MAX>::kBytes, c = Rings<W, MAX, MAX>::kBytes;
     return a > b ? (a > c ? a : c) : (b > c ? b : c);
 }
 
@@ -395,15 +396,18 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
 
     auto body = [&](auto tag) {
         constexpr int MT = decltype(tag)::value;
-        constexpr bool FOLD = MT == 1 && MAX <= W::kFold;
-        v16f acc[2][MT], part[2];
+        constexpr bool FOLD = MAX <= W::kFold;
+        v16f acc[2][MT];
+        [[maybe_unused]] v16f part[2][FOLD ? MT : 1];
 #pragma unroll
         for (int b = 0; b < 2; ++b)
 #pragma unroll
             for (int m = 0; m < MT; ++m)
 #pragma unroll
                 for (int i = 0; i < 16; ++i) acc[b][m][i] = 0.f;
-        if constexpr (FOLD) part[0] = part[1] = acc[0][0];
+        if constexpr (FOLD)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) part[0][m] = part[1][m] = acc[0][0];
         const bool any = GATEUP ? grp * 128 < row_lim : true;
         if (any) {
             using R = Rings<W, MT, MAX>;
@@ -510,13 +514,12 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                     } else {
                         if (j < 3) read_a(j + 1);
 #pragma unroll
-                        for (int b = 0; b < 2; ++b) {
-                            if constexpr (FOLD) part[b] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[j & 1][0]), __builtin_bit_cast(v8h, bw[b][j]), part[b], 0, 0, 0);
-                            else
+                        for (int b = 0; b < 2; ++b)
 #pragma unroll
-                                for (int m = 0; m < MT; ++m)
-                                    acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bw[b][j]), __builtin_bit_cast(v8h, a[j & 1][m]), acc[b][m], 0, 0, 0);
-                        }
+                            for (int m = 0; m < MT; ++m) {
+                                if constexpr (FOLD) part[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, a[j & 1][m]), __builtin_bit_cast(v8h, bw[b][j]), part[b][m], 0, 0, 0);
+                                else acc[b][m] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8h, bw[b][j]), __builtin_bit_cast(v8h, a[j & 1][m]), acc[b][m], 0, 0, 0);
+                            }
 #pragma unroll
                         for (int b = 0; b < 2; ++b) bw[b][j] = operand(pr[b], j);
                     }
@@ -526,10 +529,12 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
 #pragma unroll
                         for (int b = 0; b < 2; ++b)
 #pragma unroll
-                            for (int i = 0; i < 16; ++i) {
-                                acc[b][0][i] = fmaf(part[b][i], d[b], acc[b][0][i]);
-                                part[b][i] = 0.f;
-                            }
+                            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                                for (int i = 0; i < 16; ++i) {
+                                    acc[b][m][i] = fmaf(part[b][m][i], d[b], acc[b][m][i]);
+                                    part[b][m][i] = 0.f;
+                                }
                     }
                 }
             }
@@ -552,7 +557,7 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                     for (int i = 0; i < 16; ++i) {
                         v[i] = acc[bank][m][i];
                         if constexpr (W::kFp8) v[i] *= W::row_factor(bank ? k.b1 : k.b0, (int64_t(e) * tiles + wt[bank]) * 32 + 8 * (i >> 2) + 4 * g + (i & 3));
-                        v[i] *= FOLD ? s_scale[8 * (i >> 2) + 4 * g + (i & 3)] : scl;
+                        v[i] *= FOLD ? s_scale[m * 32 + 8 * (i >> 2) + 4 * g + (i & 3)] : scl;
                     }
                 };
                 float v[16];
@@ -606,8 +611,8 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
             }
         }
     };
-    if (cnt <= 32) body(std::integral_constant<int, 1>{});
-    else if (MAX == 2 || cnt <= 64) body(std::integral_constant<int, 2>{});
+    if (MAX == 1 || cnt <= 32) body(std::integral_constant<int, 1>{});
+    else if (MAX == 2 || cnt <= 64) body(std::integral_constant<int, MAX == 1 ? 1 : 2>{});
     else body(std::integral_constant<int, MAX>{});
 }
 
@@ -617,13 +622,17 @@ template <uint32_t FMT, int MAX> void grouped_rows_launch_max(const GroupedArgs 
         allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes);
         kernel<<<blocks, 256, bytes, s>>>(k);
     };
-    if (gateup) go(&grouped_rows_k<FMT, MAX, true, uint16_t>);
-    else if (f32_out) go(&grouped_rows_k<FMT, MAX, false, float>);
+    if (gateup) {
+        if constexpr (MAX > 1 || GroupedFormat<FMT>::kFold) go(&grouped_rows_k<FMT, MAX, true, uint16_t>);   // (grouped_rows_per_item)
+    } else if (f32_out) go(&grouped_rows_k<FMT, MAX, false, float>);
     else go(&grouped_rows_k<FMT, MAX, false, uint16_t>);
 }
 template <uint32_t FMT> void grouped_rows_launch(const GroupedArgs & k, int item_rows, bool gateup, bool f32_out, unsigned blocks, hipStream_t s) {
-    if (item_rows == 64) grouped_rows_launch_max<FMT, 2>(k, gateup, f32_out, blocks, s);
-    else grouped_rows_launch_max<FMT, 4>(k, gateup, f32_out, blocks, s);
+    if constexpr (!GroupedFormat<FMT>::kFp8) {
+        if (item_rows == 32) return grouped_rows_launch_max<FMT, 1>(k, gateup, f32_out, blocks, s);
+        if (item_rows == 64) return grouped_rows_launch_max<FMT, 2>(k, gateup, f32_out, blocks, s);
+    }
+    grouped_rows_launch_max<FMT, 4>(k, gateup, f32_out, blocks, s);
 }
 
 }  // namespace
