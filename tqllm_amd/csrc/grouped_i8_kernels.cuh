@@ -250,7 +250,7 @@ __global__ __launch_bounds__(256, MAX == 1 ? 3 : 2) void grouped_i8_k(GroupedArg
                 if constexpr (GATEUP) *reinterpret_cast<uint16_t *>(to) = live ? swiglu_half(acc[0][m][i], acc[1][m][i], scl[i], k.glu) : uint16_t(0);
                 else {
 #pragma unroll
-                    for (int b = 0; b < 2; ++b) *reinterpret_cast<uint16_t *>(to + b * 64) = scaled_half(acc[b][m][i], scl[i], k.out_bf16);
+                    for (int b = 0; b < 2; ++b) *reinterpret_cast<uint16_t *>(to + b * 64) = to_half_bits(__fmul_rn(acc[b][m][i], scl[i]));
                 }
             }
             __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
