@@ -12,10 +12,11 @@ T tokens with every input already resident in HBM. Steps rotate over several ind
 batches, over several input batches per bank) so that a step's weights stream from HBM, not from the 256 MB last-level
 cache. Per point:
   tokens_per_s  T / mean step time over exactly --steps steps, captured into one HIP graph, after --warmup untimed steps
-  roofline      the dominant kernel (gate + up + SwiGLU) over its mean duration, measured with events on the launching
-                stream around back-to-back launches of that kernel alone. Decode kernels: the bytes of the distinct
-                experts the launch must read against 8 TB/s. Grouped products: 2 operations per multiply-add of their
-                assignments against the dense matrix peak of the operand type
+  roofline      the dominant kernel (gate + up + SwiGLU) over its mean duration. Decode kernels: measured with events on the
+                launching stream around back-to-back launches of that kernel alone; the bytes of the distinct experts the
+                launch must read against 8 TB/s. Grouped products: the layer's own launches, from torch's profiler over
+                every step of the cycle; 2 operations per multiply-add of their assignments against the dense matrix peak of
+                the operand type
   layer         the whole step's algorithmic bytes and operations against the same peaks
 cpu_baseline: the CPU expert path (the scheme of the reference's tests/bench_cpu_expert_mt.cpp at this layer's shape)
 timed on this box's host cores on a bounded sample.
@@ -24,8 +25,8 @@ import argparse
 import json
 import math
 import os
+import re
 import sys
-import time
 
 ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
@@ -138,6 +139,63 @@ def time_calls(torch, fn, calls, warmup):
     return a.elapsed_time(b) / calls  # ms per call
 
 
+def decode_kernel_times(torch, tq, cfg, layers, xs, cycle, routing, rounds, args):
+    """The decode products alone: back-to-back launches over the rotating banks, inputs prepared once."""
+    k, shared_ff, prep = cfg["topk"], cfg["shared_ff"], []
+    for (b, j), ids in zip(cycle, routing):
+        l, x = layers[b], xs[b][j]
+        ext = tq.moe_extend_ids(ids, cfg["experts"]) if shared_ff else ids
+        img = tq.quant_act(x)
+        act = tq.expert_gateup(l.gate, l.up, img, ext, k, shared_ff=shared_ff)
+        prep.append((l, ext, img, act, tq.expert_down(l.down, act, ext, k, shared_ff=shared_ff)))
+
+    # (every launch writes into the rows its first run allocated: nothing but the kernel is on the stream between the events)
+    def gateup_round():
+        for l, ext, img, act, _ in prep:
+            tq.expert_gateup(l.gate, l.up, img, ext, k, shared_ff=shared_ff, act_image=act)
+
+    def down_round():
+        for l, ext, _, act, y in prep:
+            tq.expert_down(l.down, act, ext, k, shared_ff=shared_ff, y=y)
+
+    kernels, reps = {}, 4
+    for name, fn in (("gateup", gateup_round), ("down", down_round)):
+        fn()
+        torch.cuda.synchronize()
+        timed = fn
+        if not args.no_graph:   # microsecond kernels: replay a graph of them so that the host is not the bound
+            gk = torch.cuda.CUDAGraph()
+            with torch.cuda.graph(gk):
+                for _ in range(reps):
+                    fn()
+            timed = gk.replay
+        kernels[name] = time_calls(torch, timed, max(4, rounds // reps), 2) / ((reps if timed is not fn else 1) * len(cycle))
+    return kernels
+
+
+def grouped_kernel_times(torch, cfg, cycle, passes, launches):
+    """The grouped products as the layer launches them, from torch's profiler: gate / up and down in turn, `launches` of them in a
+    pass over the steps' cycle. Means over the second half of the passes (the clocks are up by then)."""
+    times = []
+    try:
+        from torch.profiler import ProfilerActivity, profile
+        cycle()
+        torch.cuda.synchronize()
+        with profile(activities=[ProfilerActivity.CUDA]) as prof:
+            for _ in range(passes):
+                cycle()
+            torch.cuda.synchronize()
+        times = sorted((e.time_range.start, e.device_time_total, e.name) for e in prof.events() if re.search("(grouped_(rows|i8)|plane_gemm|expert_gemm_f16)_k<", e.name))
+    except Exception as ex:  # noqa: BLE001
+        print("bench.py: torch's profiler: %s" % ex, file=sys.stderr)
+    if len(times) != passes * launches:
+        print("bench.py: %d product launches profiled, %d expected; their times are left out" % (len(times), passes * launches), file=sys.stderr)
+        return {"gateup": None, "down": None}
+    name = re.search(r"\w+_k<[^>]*>", times[0][2]).group(0).replace("%du" % cfg["wtype"], cfg["fmt"]).replace("unsigned short", "half")
+    us = [t for _, t, _ in times[passes // 2 * launches:]]
+    return {"name": name, "gateup": sum(us[::2]) / (len(us) // 2) / 1e3, "down": sum(us[1::2]) / (len(us) // 2) / 1e3}
+
+
 def measure_point(torch, tq, cfg, key, trios, gen, T, args, traffic):
     R = len(trios)
     h, f, k = cfg["hidden"], cfg["ff"], cfg["topk"]
@@ -212,85 +270,15 @@ def measure_point(torch, tq, cfg, key, trios, gen, T, args, traffic):
     gu_ops = T * slots * 2 * f * h * 2.0      # multiply-adds of gate and up, 2 operations each
     dn_ops = T * slots * f * h * 2.0
 
-    # ---- dominant kernels alone: back-to-back launches over the rotating banks, inputs prepared once
-    prep = []
-    fp8 = path == "grouped_fp8"
-    for (b, j), ids in zip(cycle, routing):
-        l, x = layers[b], xs[b][j]
-        ext = tq.moe_extend_ids(ids, cfg["experts"]) if shared else ids
+    kernels = {"gateup": None, "down": None}      # ms per launch
+    if not args.no_kernel_times:
         if path == "decode":
-            img = tq.quant_act(x)
-            act = tq.expert_gateup(l.gate, l.up, img, ext, k, shared_ff=cfg["shared_ff"])
-            y = tq.expert_down(l.down, act, ext, k, shared_ff=cfg["shared_ff"])
-            prep.append((l, ext, img, act, y))
+            kernels = decode_kernel_times(torch, tq, cfg, layers, xs, cycle, routing, rounds, args)
         else:
-            counts, offsets, perm, _ = tq.moe_dispatch(ext, cfg["experts"] + shared)
-            lists = (counts, offsets, perm)
-            if path == "grouped_i8" and args.act_blocks:   # a scale per 32 activations: the block scales ride along
-                xq, xsc, xbs = tq.group_rows_i8_blocks(x, lists, T * slots, slots)
-                act = tq.expert_gemm_gateup_i8_blocks(l.gate, l.up, xq, xsc, xbs, lists, T, slots, k, cfg["shared_ff"])
-                aq, asc, abs_ = tq.group_rows_i8_blocks(act, lists, T * slots, 1)
-                y = tq.expert_gemm_i8_blocks(l.down, aq, asc, abs_, lists, T, slots, k, cfg["shared_ff"])
-                prep.append((l, lists, xq, (xsc, xbs), aq, (asc, abs_), act, y))
-            elif path in ("grouped_i8", "grouped_fp8"):
-                xq, xsc = tq.group_rows_i8(x, lists, T * slots, slots, fp8=fp8)
-                act = tq.expert_gemm_gateup_i8(l.gate, l.up, xq, xsc, lists, T, slots, k, cfg["shared_ff"], fp8=fp8)
-                aq, asc = tq.group_rows_i8(act, lists, T * slots, 1, fp8=fp8)
-                y = tq.expert_gemm_i8(l.down, aq, asc, lists, T, slots, k, cfg["shared_ff"], fp8=fp8)
-                prep.append((l, lists, xq, xsc, aq, asc, act, y))
-            else:
-                act = tq.expert_gemm_gateup(l.gate, l.up, x, lists, T, slots, k, cfg["shared_ff"])
-                y = tq.expert_gemm(l.down, act, lists, T, slots, k, cfg["shared_ff"], per_expert_input=True, out_type=tq.F32)
-                prep.append((l, lists, x, act, y))
+            kernels = grouped_kernel_times(torch, cfg, lambda: run_steps(0, len(cycle)), max(16, min(rounds, 40)), 2 * len(cycle))
 
-    # (every launch writes into the rows its first run allocated: nothing but the kernel is on the stream between the events)
-    def gateup_round():
-        for item in prep:
-            if path == "decode":
-                l, ext, img, act, y = item
-                tq.expert_gateup(l.gate, l.up, img, ext, k, shared_ff=cfg["shared_ff"], act_image=act)
-            elif path in ("grouped_i8", "grouped_fp8"):
-                l, lists, xq, xsc, aq, asc, act, y = item
-                if isinstance(xsc, tuple):
-                    tq.expert_gemm_gateup_i8_blocks(l.gate, l.up, xq, xsc[0], xsc[1], lists, T, slots, k, cfg["shared_ff"], act=act)
-                else:
-                    tq.expert_gemm_gateup_i8(l.gate, l.up, xq, xsc, lists, T, slots, k, cfg["shared_ff"], fp8=fp8, act=act)
-            else:
-                l, lists, x, act, y = item
-                tq.expert_gemm_gateup(l.gate, l.up, x, lists, T, slots, k, cfg["shared_ff"], act=act)
-
-    def down_round():
-        for item in prep:
-            if path == "decode":
-                l, ext, img, act, y = item
-                tq.expert_down(l.down, act, ext, k, shared_ff=cfg["shared_ff"], y=y)
-            elif path in ("grouped_i8", "grouped_fp8"):
-                l, lists, xq, xsc, aq, asc, act, y = item
-                if isinstance(asc, tuple):
-                    tq.expert_gemm_i8_blocks(l.down, aq, asc[0], asc[1], lists, T, slots, k, cfg["shared_ff"], y=y)
-                else:
-                    tq.expert_gemm_i8(l.down, aq, asc, lists, T, slots, k, cfg["shared_ff"], fp8=fp8, y=y)
-            else:
-                l, lists, x, act, y = item
-                tq.expert_gemm(l.down, act, lists, T, slots, k, cfg["shared_ff"], per_expert_input=True, out_type=tq.F32, y=y)
-
-    kernels = {}
-    small = path == "decode"
-    reps = 4 if small else 1
-    for name, fn in (("gateup", gateup_round), ("down", down_round)):
-        fn()
-        torch.cuda.synchronize()
-        timed = fn
-        if small and not args.no_graph:   # microsecond kernels: replay a graph of them so that the host is not the bound
-            gk = torch.cuda.CUDAGraph()
-            with torch.cuda.graph(gk):
-                for _ in range(reps):
-                    fn()
-            timed = gk.replay
-        n_calls = max(4, rounds // reps) if small else max(4, min(rounds, 20))
-        kernels[name] = time_calls(torch, timed, n_calls, 2) / ((reps if timed is not fn else 1) * len(cycle))  # ms per launch
-
-    gu_s, dn_s, step_s = kernels["gateup"] * 1e-3, kernels["down"] * 1e-3, ms_step * 1e-3
+    gu_s, dn_s = (kernels[k] * 1e-3 if kernels[k] else math.nan for k in ("gateup", "down"))
+    step_s = ms_step * 1e-3
     if path == "decode":
         kname = "decode_mfma_k<%s, 2> (gate + up + SwiGLU)" % cfg["fmt"]
         roofline = {"bound": "hbm", "kernel": kname, "achieved": round(gu_bytes / gu_s / 1e9, 1), "peak": HBM_PEAK / 1e9, "unit": "GB/s",
@@ -301,10 +289,7 @@ def measure_point(torch, tq, cfg, key, trios, gen, T, args, traffic):
         dtype = "int8 x int8 -> int32 (weights exact, activations as two int8 planes), fp32 scales"
     else:
         op = {"grouped_i8": "int8", "grouped_f16": "fp16", "grouped_fp8": "fp8"}[path]
-        kname = {"grouped_i8": "plane_gemm_k<2, %s> (%sgrouped gate + up int8 MFMA product + SwiGLU%s)" % (
-                     (cfg["fmt"],) + (("the general entry's ", "; the layer runs grouped_i8_k on rows in quantiser order") if cfg["fmt"] == "IQ4_XS" else ("", ""))),
-                 "grouped_f16": "expert_gemm_f16_k<%s,2> (the general entry's grouped gate + up fp16 MFMA product + SwiGLU; the layer runs grouped_rows_k on prepared rows)" % cfg["fmt"],
-                 "grouped_fp8": "grouped_rows_k<%s> (grouped gate + up fp8 MFMA product + SwiGLU)" % cfg["fmt"]}[path]
+        kname = "%s (grouped gate + up %s MFMA product + SwiGLU, as the layer launches it)" % (kernels.get("name", "not timed"), op)
         roofline = {"bound": "mfma", "kernel": kname, "achieved": round(gu_ops / gu_s / 1e12, 2), "peak": PEAK[op] / 1e12, "unit": "TFLOP/s",
                     "frac": round(gu_ops / gu_s / PEAK[op], 4), "traffic": None,
                     "ops": "multiply-add = 2 operations; peak = dense %s %.1f POP/s" % (op, PEAK[op] / 1e15),
@@ -318,7 +303,9 @@ def measure_point(torch, tq, cfg, key, trios, gen, T, args, traffic):
                  "fp8": "E4M3 x E4M3 -> fp32 MFMA (weights and activations rounded to E4M3), fp32 scales"}[op]
     # HBM bytes per launch of the roofline kernel as the counters saw them (a committed measurement of this same point)
     roofline["traffic"] = traffic.get("config%s_tokens_%d" % (key, T), {}).get("bytes_per_launch")
-    del layers, xs, outs, prep
+    for d in (roofline, layer):           # (a figure that was not measured is null)
+        d.update({k: None for k, v in d.items() if isinstance(v, float) and math.isnan(v)})
+    del layers, xs, outs
     torch.cuda.empty_cache()
     return {"tokens": T, "tokens_per_s": round(T / step_s, 1), "ms_per_step": round(ms_step, 5), "steps": K, "warmup": W,
             "path": path, "launch": launch, "distinct_steps": len(cycle), "routing": "N(0,1) logits + Zipf(%.1f) popularity bias" % ZIPF_S if skew else "random router",
@@ -346,6 +333,7 @@ def main():
     ap.add_argument("--tokens", type=int, default=None, help="measure this one point instead of the configuration's list")
     ap.add_argument("--banks", type=int, default=8, help="independent expert banks the steps rotate over")
     ap.add_argument("--no-graph", action="store_true", help="launch every step from the host instead of replaying a HIP graph")
+    ap.add_argument("--no-kernel-times", action="store_true", help="skip the roofline kernel's own timing (runs under another profiler)")
     ap.add_argument("--no-cpu", action="store_true", help="skip the CPU baseline leg")
     ap.add_argument("--act-blocks", action="store_true", help="int8 grouped products with a scale per 32 activations in place of one per token "
                     "(the reference's TQFN_PREFILL_INT8=1); the headline numbers are measured without it")
