@@ -14,9 +14,9 @@
 //
 // Bound by vector instructions: a unit (65,536 operations) is one product (32 cycles of the matrix pipe, about 18 of the
 // vector issue) and 16 multiply-adds and 4 folds of 4 to 5 cycles each (a scale per 32 values: 32), the operand's decode (22) spread over
-// the item's row tiles. 4096 tokens of 10 of 512 experts, Zipf: gate / up 336 -> 293 us, down 226 -> 179, and the two launches that
-// gathered rows (55 us) are one that quantises them (17); 1501 tokens, a scale per 32 values, balanced: gate / up 555 -> 227 us, down
-// 326 -> 145, no launch between (a weight tile's act values are one block of 32: the gate / up product quantises them itself).
+// the item's row tiles. 4096 tokens of 10 of 512 experts, Zipf, in the kernel trace: gate / up 342 us on plane_gemm_k, 269 here (vector pipe
+// 80 % active, matrix pipe 16 %), down 231 and 161, and the two launches that gathered rows (55 us) are one that quantises them (17); with a
+// scale per 32 values gate / up 589 and 328 us (vector pipe 99 %), down 357 and 198, no launch between (a weight tile's act values are one block of 32: the gate / up product quantises them itself).
 #pragma once
 #include "decode_table.cuh"
 #include "formats.cuh"

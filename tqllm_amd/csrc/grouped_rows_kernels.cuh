@@ -25,13 +25,12 @@
 // the other's products run. Items of one and two row tiles have loops of their own with fewer products.
 //
 // What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 228 us, 0.90
-// PFLOP/s, matrix pipe 48 % busy, vector pipe 53 % (262 us, 43 and 52 % with biased codes; then 211 without the decode, 173
-// without the row reads as well, which is the rate of a large fp16 product on this card); NVFP4G, 8192 tokens, gate / up (2.1
-// TFLOP with down): 886 us, 41 % and 53 %. A product holds its SIMD's vector issue for about 18 cycles besides its own time, so
-// a stage's decode does not pass under its products for free: that sum and not a wait is what is left.
-// Items of one row tile are bound by the decode (IQ3_S, 512 tokens: gate / up 118 us, 2.9 TB/s of codes, vector pipe 64 %, LDS 52 %,
-// three fifths of that bank conflicts of the lattice's look-ups; of 139 us on another day 103 without these and their addresses,
-// 104 without signs and scales, 116 without code transfers).
+// PFLOP/s, matrix pipe 48 % busy, vector pipe 53 % (262 us with biased codes; without the decode 205, without the row reads as
+// well 178, where a large fp16 product on this card would take 170); NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 880 us,
+// 43 % and 55 %. A product holds its SIMD's vector issue for about 18 cycles besides its own time, so that a stage's decode does not
+// pass under its products for free.
+// Items of one row tile are bound by the decode (IQ3_S, 512 tokens: gate / up 117 us, 2.9 TB/s of codes, vector pipe 65 %, LDS 52 %,
+// three fifths of that bank conflicts of the lattice's look-ups).
 //
 // Items of up to kFold row tiles (IQ4_XS and Q6_K: two, IQ3_S: one): the operands are the codes times the integer scale, and every 256
 // columns the fp32 sums are multiplied by the super-block's factor instead (the weights are the second operand there, so that a
@@ -335,7 +334,7 @@ template <class W, int MAX> constexpr int kGroupedWaves = MAX == 4 || (MAX == 2 
 // Stages of input rows and of codes in LDS for MT row tiles, in the part of a compute unit's 160 KB that one of its blocks may
 // take. Codes come from HBM and may be two and more stages on their way; rows come from the L2 (an item's other blocks read
 // the same). (Q4_K at 4096 tokens: 554 us a layer with one stage of codes under way, 521 with two.) With three blocks a unit
-// their own turns hide the trip, and two stages are the faster ring (three / two, us a layer: IQ3_S, 512 tokens of 8 experts
+// their own turns hide the trip, and two stages are the faster ring (three / two, us a layer, items of 64 rows: IQ3_S, 512 tokens of 8 experts
 // of 256 215 / 211, IQ4_XS, 333 skewed tokens 127.5 / 125.6, Q4_K, 200 tokens of 64 experts 83.2 / 82.4); with two blocks two
 // to five are the same to 0.5 %.
 template <class W, int MT, int MAX> struct Rings {
