@@ -493,6 +493,7 @@ typedef struct tqmoe_layer {
     int32_t clamp_gate;
 } tqmoe_layer;
 
+/* device scratch of tqmoe_layer_forward for any batch of up to n tokens; 0: the descriptor is invalid */
 size_t  tqmoe_layer_workspace_bytes(const tqmoe_layer * layer, int32_t n);
 /* Which expert products tqmoe_layer_forward runs for n tokens of this layer (the choice depends on the batch and the
  * bank formats only, never on the data, so that a token's result does not depend on what else is routed; the reference

@@ -118,6 +118,19 @@ def test_grouped_products_refuse_more_than_4096_experts(tq, fmt):
     assert run(over, 4) == -4 and run(most, 2000) == -4
 
 
+@pytest.mark.parametrize("hidden,ff,experts,topk,shared", [(2048, 512, 512, 10, True), (1024, 768, 64, 1, False), (2048, 768, 33, 1, False), (256, 2048, 512, 4, False),
+                                                           (4096, 768, 128, 1, True), (3072, 256, 4095, 2, False)])
+def test_workspace_of_the_largest_batch_is_enough_for_every_smaller_one(tq, hidden, ff, experts, topk, shared):
+    """An engine asks for the workspace once, for its largest batch; other products and items take over at lines below it."""
+    bytes_for = tq.lib().tqmoe_layer_workspace_bytes
+    for fmt, down in (("IQ4_XS", None), ("Q4_K", "Q6_K"), ("Q6_K", None), ("IQ3_S", None), ("NVFP4G", None), ("NVFP4G", "Q6_K"), ("Q5_K", None), ("IQ2_S", None)):
+        for act_blocks in (0, 1, 2):
+            d = fake_layer(tq, hidden, ff, experts, topk, shared, getattr(tq, fmt), getattr(tq, down) if down else None)
+            d.act_blocks = act_blocks
+            sizes = [bytes_for(C.byref(d), n) for n in list(range(1, 4200)) + [8192, 50000]]
+            assert sizes[0] > 0 and sizes == sorted(sizes), (fmt, down, act_blocks)
+
+
 def test_planes_that_are_not_aligned_take_the_general_products(tq):
     """The fp8 products move 16-byte pieces to LDS: a layer whose planes start elsewhere runs on the fp16 products."""
     d = fake_layer(tq, 512, 256, 16, 4, False, tq.NVFP4G)

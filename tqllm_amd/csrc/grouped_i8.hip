@@ -9,7 +9,7 @@ bool grouped_i8_takes(uint32_t type, int rows, int cols) { return type == TQMOE_
 // place of two, which is the better where most experts have one row tile. Layer in us at 32 / 64 rows, a scale per 32 values: 512
 // experts with 22 rows on average 272 / 291, 32 rows 337 / 337, 36 rows 377 / 368 (Zipf 310 / 295), 41 rows 414 / 395, 64 rows 522 / 498;
 // 128 experts with 36 rows 151 / 158, 42 rows 170 / 169; a scale a row: 22 rows 261 / 276, 32 rows 323 / 319, 43 rows 438 / 386.
-int grouped_i8_per_item(bool blocks, int64_t assignments, int experts) { return assignments <= int64_t(experts) * (blocks ? 36 : 28) ? 32 : 64; }
+int grouped_i8_per_item(bool blocks, int64_t assignments, int experts) { return assignments <= int64_t(experts) * (blocks ? kItem32I8Blocks : kItem32I8) ? 32 : 64; }
 
 // assignments: total entries of perm (it bounds the items)
 void enqueue_grouped_i8(const tqmoe_bank & b0, const tqmoe_bank * b1, const int8_t * x, const float * xs, bool blocks, const int * perm, const int4 * plan, int64_t assignments,

@@ -36,9 +36,9 @@ template <uint32_t FMT> void grouped_rows_run(const GroupedArgs & k, int item_ro
 // experts with 8 rows 199 / 203 and 115 / 121, with 16 rows 206 / 210 and 172 / 160, with 22 rows 231 / 231 and 218 / 188.
 // The fp8 products' codes leave LDS for two blocks either way: 128.
 int grouped_rows_per_item(uint32_t type, int64_t assignments, int experts) {
-    const int one_tile = type == TQMOE_IQ4_XS || type == TQMOE_Q6_K ? 24 : type == TQMOE_IQ3_S ? 16 : 0;
+    const int one_tile = type == TQMOE_IQ4_XS || type == TQMOE_Q6_K ? kItem32 : type == TQMOE_IQ3_S ? kItem32Iq3s : 0;
     if (assignments <= int64_t(experts) * one_tile) return 32;
-    return type != TQMOE_NVFP4G && assignments <= int64_t(experts) * 40 ? 64 : 128;
+    return type != TQMOE_NVFP4G && assignments <= int64_t(experts) * kItem64 ? 64 : 128;
 }
 
 bool grouped_rows_takes(uint32_t type, int rows, int cols) {

@@ -29,6 +29,10 @@ struct GroupedArgs {
 // index of the gathered row tiles, written beside the items where tile_base is not null
 struct RowIndex { int * tile_base, * chunk_base, * counters; int counters_n, chunk_tiles; };
 
+// Rows an expert on average up to which items are of 32 rows (IQ4_XS and Q6_K; IQ3_S), of 64 (grouped_rows_per_item); int8 ones of 32, with a
+// scale a row and per 32 values (grouped_i8_per_item)
+constexpr int kItem32 = 24, kItem32Iq3s = 16, kItem64 = 40, kItem32I8 = 28, kItem32I8Blocks = 36;
+
 bool grouped_rows_takes(uint32_t type, int rows, int cols);
 inline bool grouped_rows_aligned(const tqmoe_bank & b) { return aligned16(b.codes) && aligned16(b.aux); }   // planes that lie otherwise have the general products
 int grouped_rows_per_item(uint32_t type, int64_t assignments, int experts);   // input rows of an item at most: 32, 64 or 128 (type: the gate bank's)

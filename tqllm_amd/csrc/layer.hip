@@ -233,7 +233,16 @@ using namespace tqmoe;
 
 extern "C" size_t tqmoe_layer_workspace_bytes(const tqmoe_layer * layer, int32_t n) {
     if (!layer || n <= 0 || check_layer(layer, nullptr)) return 0;
-    return plan_for(*layer, n).total + 256;   // (room to move the areas to a multiple of 16 bytes in a workspace that starts elsewhere)
+    // Enough for every smaller batch too: a caller asks once, for its largest. A plan's areas grow with the tokens, but at the lines
+    // where other products or other items take over their sum may shrink (by up to 29 %: fp16 products in place of the decode
+    // products, one expert a token, NVFP4G with a Q6_K down bank).
+    const tqmoe_layer & L = *layer;
+    const int64_t slots = L.topk + (L.has_shared ? 1 : 0), banks = L.n_expert + (L.has_shared ? 1 : 0);
+    size_t most = 0;
+    for (int64_t m : {int64_t(n), int64_t(kGroupedMin - 1), int64_t(kInt8Tokens - 1), std::min<int64_t>(kDecodeDedup, kGroupedPerBank * banks) / slots, kItem32 * banks / slots,
+                      kItem32Iq3s * banks / slots, kItem64 * banks / slots, kItem32I8 * banks / slots, kItem32I8Blocks * banks / slots})
+        if (m > 0 && m <= n) most = std::max(most, plan_for(L, int(m)).total);
+    return most + 256;   // (room to move the areas to a multiple of 16 bytes in a workspace that starts elsewhere)
 }
 
 extern "C" int32_t tqmoe_layer_path(const tqmoe_layer * layer, int32_t n) {
