@@ -180,6 +180,14 @@ def test_layer_down_bank_of_another_format(tq, oracle, gu_type, down_type, n):
     check_layer(out, ids, w, want, want_ids, want_w, clear_tokens(oracle, logits, cfg["experts"], cfg["topk"], ids, want_ids))
 
 
+@pytest.mark.parametrize("gu_type,down_type", [(21, 12), (23, 12), (12, 23), (12, 21), (14, 21)])
+@pytest.mark.parametrize("n", [40, 90])
+def test_layer_items_sized_for_the_gate_format(tq, oracle, gu_type, down_type, n):
+    """Products on prepared rows whose items (14.5 and 33 rows an expert) are as long as the gate banks' format wants them: the down
+    product takes items of 32 and 64 rows that its own format would not."""
+    test_layer_down_bank_of_another_format(tq, oracle, gu_type, down_type, n)
+
+
 @pytest.mark.parametrize("n", [1, 4, 16])
 def test_layer_config2_full_shape(tq, oracle, n):
     """Flash-Next-shaped decode layer at its real shape: 512 IQ4_XS experts + shared, top-10, bf16 router and inputs."""

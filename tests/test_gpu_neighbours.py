@@ -32,7 +32,7 @@ def check(layer, x, crowded):
         out, ids2, _, _ = layer.forward(y, return_routing=True)
         assert torch.equal(ids2[kept], ids[kept])
         rows = [(ids2 == e).any(dim=1).sum().item() for e in ids[0].tolist()]
-        assert min(rows) > 0.6 * n if sign == 1 else max(rows) < crowded, rows
+        assert min(rows) > 0.5 * n if sign == 1 else max(rows) < crowded, rows
         assert torch.equal(out[kept], want[kept]), [synth.errors(out[t].cpu().numpy(), want[t].cpu().numpy())[1] for t in kept.tolist()]
 
 

@@ -34,3 +34,9 @@ def test_neighbours_of_a_token_without_numbers(oracle, gating, n, fmt):
         ids = ids.cpu().numpy()
         assert ids.min() >= 0 and ids.max() < 33 and all(len(set(row)) == 4 for row in ids.tolist())
         assert torch.equal(out[others], want[others]) and torch.isfinite(want).all()
+
+
+@pytest.mark.parametrize("fmt,n", [("IQ4_XS", 60), ("Q6_K", 60), ("Q6_K", 250), ("IQ3_S", 60), ("IQ3_S", 250), ("IQ3_S", 800), ("NVFP4G", 60)])
+def test_neighbours_in_items_of_all_sizes(oracle, fmt, n):
+    """The token without numbers takes or leaves a row of its neighbours' experts: their items' row tiles change, their bits do not."""
+    test_neighbours_of_a_token_without_numbers(oracle, "softmax", n, fmt)
