@@ -156,3 +156,27 @@ def test_fp8_layer_excess_is_the_straddling_act_values(tq, oracle):
     assert 0 < straddle < 5e-3 * values                           # they exist and are rare (about one act value in a thousand)
     assert mx_all < MAX_ABS * max(1.0, top) and rel_all < 3e-3, (mx_all, rel_all)
     assert mx < MAX_ABS * max(1.0, top) and rel < REL_RMS, (mx, rel)
+
+
+def test_fp8_weights_of_every_scale_byte_and_code(tq, oracle):
+    """The down product on unit rows reads the weights back: all 256 scale bytes (negative ones, subnormals, the two that are not a
+    number) with all sixteen codes. A unit row is 448 in E4M3 with the scale 1 / 448: one fp32 rounding and the result's to a half
+    (2^-11, subnormals 2^-25), so that one step of a half, 2^-10, is the bound. A row of weights with a scale that is not a number is
+    none in any result."""
+    rows, cols, g = 32, 256, 0.01
+    raw = np.zeros((rows * cols // 128, 76), np.uint8)
+    raw[:, :4] = np.frombuffer(np.float32(g).tobytes(), np.uint8)
+    raw[:, 4:12] = np.arange(256, dtype=np.uint8).reshape(-1, 8)[np.arange(rows * cols // 128) % 32]
+    raw[:, 12:] = (np.arange(64) * 0x21 + 0x10 + np.arange(len(raw))[:, None] * 0x33) & 0xFF
+    raw = raw.reshape(-1)
+    want = oracle.dequantize_nvfp4_widened(raw, rows * cols).reshape(rows, cols).astype(np.float64)
+    bank = tq.ExpertBank(tq.NVFP4G, torch.from_numpy(raw).cuda(), 1, rows, cols)
+    ids = torch.zeros((cols, 1), dtype=torch.int32, device="cuda")
+    lists = tq.moe_dispatch(ids, 1)[:3]
+    xq, xs = tq.group_rows_fp8(torch.eye(cols, device="cuda"), lists, cols, 1)
+    out = tq.expert_gemm_fp8(bank, xq, xs, lists, cols, 1, 1).float().cpu().numpy().reshape(cols, rows).T.astype(np.float64)
+    none = np.zeros(rows, bool)
+    none[[7, 15, 23, 31]] = True          # bytes 0x7F and 0xFF
+    assert np.isnan(out[none]).all()
+    assert (np.abs(out[~none] - want[~none]) <= np.abs(want[~none]) * 2.0 ** -10 + 2.0 ** -25).all()
+    assert np.count_nonzero(want[~none] < 0) > 2000 and np.count_nonzero(want[~none] > 0) > 2000

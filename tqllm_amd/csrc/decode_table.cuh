@@ -26,20 +26,6 @@ constexpr Table16 table16(const int (&t)[16]) {
     auto word = [](const uint32_t * v) { return v[0] | v[1] << 8 | v[2] << 16 | v[3] << 24; };
     return Table16{word(a), word(a + 4), word(b), word(b + 4)};
 }
-// the same pools from sixteen table bytes in four dwords, at run time
-__device__ __forceinline__ uint4 table16_pools(const uint32_t (&v)[4]) {
-    auto val = [&](int i) { return (v[i >> 2] >> (8 * (i & 3))) & 0xFFu; };
-    auto neg = [](uint32_t x) { return (x & 0x80u) ? 0xFFu : 0u; };
-    uint32_t a[8], b[8];
-    a[5] = val(5) ^ 0xFFu; a[6] = val(6) ^ 0xFFu; a[7] = val(7) ^ 0xFFu; a[4] = val(4);
-    b[5] = val(13) ^ 0xFFu; b[6] = val(14) ^ 0xFFu; b[7] = val(15) ^ 0xFFu; b[4] = val(12);
-    b[3] = val(11) ^ neg(a[7]); b[2] = val(10) ^ neg(a[5]);
-    a[3] = val(3) ^ neg(b[7]); a[2] = val(2) ^ neg(b[5]); a[1] = val(1) ^ neg(b[3]);
-    b[1] = val(9) ^ neg(a[3]); b[0] = val(8) ^ neg(a[1]);
-    a[0] = val(0) ^ neg(b[1]);
-    auto word = [](const uint32_t * p) { return p[0] | p[1] << 8 | p[2] << 16 | p[3] << 24; };
-    return make_uint4(word(a), word(a + 4), word(b), word(b + 4));
-}
 __device__ __forceinline__ uint32_t pick(const Table16 & t, uint32_t c) {   // four codes, one per byte
     return __builtin_amdgcn_perm(t.a1, t.a0, c) ^ __builtin_amdgcn_perm(t.b1, t.b0, c ^ 0x08080808u);
 }

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256, MAX == 1 ? 3 : 2) void grouped_i8_k(GroupedArg
     __shared__ __attribute__((aligned(16))) uint8_t s_rows[2][MAX * 4096];      // [row][128 bytes], a row's piece p in slot p ^ (row / 2 & 7)
     __shared__ __attribute__((aligned(16))) float s_bs[BLK ? 2 : 1][BLK ? MAX * 128 : 4];   // [row tile][sub-block][32 rows]
     __shared__ __attribute__((aligned(16))) uint8_t s_out[4][32 * kPitch];
-    __shared__ int s_asg[kItemRows];
+    __shared__ int s_asg[kItemRows], s_row[kItemRows];   // assignments, their input rows
     __shared__ __attribute__((aligned(16))) float s_scale[kItemRows];
     const int xcd = int(blockIdx.x) & 7, at = int(blockIdx.x) >> 3, grp = at % k.groups;
     const int4 counts = k.plan[0];
@@ -82,8 +82,10 @@ __global__ __launch_bounds__(256, MAX == 1 ? 3 : 2) void grouped_i8_k(GroupedArg
     const int row_lim = GATEUP && is_shared ? k.shared_lim : rows;
     const int NSB = (!GATEUP && is_shared ? k.shared_lim : cols) / 256, stages = 2 * NSB;
     if (tid < kItemRows) {
-        s_asg[tid] = tid < cnt ? k.perm[item.y + tid] : -1;
-        s_scale[tid] = !BLK && tid < cnt ? k.xs[s_asg[tid] / k.xdiv] : 1.f;
+        const int asg = tid < cnt ? k.perm[item.y + tid] : -1, row = max(asg, 0) / k.xdiv;
+        s_asg[tid] = asg;
+        s_row[tid] = row;
+        s_scale[tid] = !BLK && tid < cnt ? k.xs[row] : 1.f;
     }
     __syncthreads();
     int wt[2];
@@ -113,9 +115,9 @@ __global__ __launch_bounds__(256, MAX == 1 ? 3 : 2) void grouped_i8_k(GroupedArg
             const uint8_t * x_src[MT];
             const float * s_src = nullptr;
 #pragma unroll
-            for (int m = 0; m < MT; ++m) x_src[m] = static_cast<const uint8_t *>(k.x) + int64_t(max(s_asg[m * 32 + (tid >> 3)], 0) / k.xdiv) * cols + (tid & 7) * 16;
+            for (int m = 0; m < MT; ++m) x_src[m] = static_cast<const uint8_t *>(k.x) + int64_t(s_row[m * 32 + (tid >> 3)]) * cols + (tid & 7) * 16;
             const int s_tile = MT == 2 ? tid >> 7 : 0;
-            if constexpr (BLK) s_src = k.xs + int64_t(max(s_asg[s_tile * 32 + (tid & 31)], 0) / k.xdiv) * S + ((tid >> 5) & 3);
+            if constexpr (BLK) s_src = k.xs + int64_t(s_row[s_tile * 32 + (tid & 31)]) * S + ((tid >> 5) & 3);
             const uint8_t * c_src[2], * r_src[2];
 #pragma unroll
             for (int b = 0; b < 2; ++b) {

@@ -17,7 +17,7 @@
 // pair rounds to fp16: 17 (Q4_K, whose codes are halves where they stand) to 27 (IQ4_XS) vector instructions for eight
 // weights, one rounding.
 // (Packed fp16 multiply-adds take four fewer and round twice: a quarter more error in the layer's result.)
-// NVFP4G: the sixteen products of a scale byte, rounded to E4M3, are a table in LDS (4 KB for all scales); eleven instructions
+// NVFP4G: the products of a scale byte, rounded to E4M3, are a table in LDS (2 KB for all scales); eight instructions
 // for eight weights.
 //
 // Rows per item: a weight is decoded once per item and wave, so 128 rows spread its instructions over four matrix
@@ -44,6 +44,8 @@
 // / 183 (180 / 185). (Two row tiles with one weight tile after the other keep three waves and read the rows twice: level where most items have
 // one row tile, 4 to 15 % slower under Zipf.)
 #pragma once
+#include <type_traits>
+
 #include "decode_api.cuh"
 #include "decode_table.cuh"
 #include "formats.cuh"
@@ -79,7 +81,7 @@ __device__ __forceinline__ v2h bias_odd(uint32_t u) { return as_h2(__builtin_amd
 // kCodes: 1 KB transfers a bank and stage (64 lanes x 16 bytes): code() the lane's source, code_at() what to add
 // for a transfer and stage. kRecs transfers for both banks' records: rec(), rec_at(). Prep: what decoding a stage needs in registers;
 // slice(): piece j (16 bytes) of operand B; in items of up to kFold row tiles whole(), the piece without the super-block's factor fold(). kTab
-// bytes of lookup table in LDS, filled by tables(). row_factor(): a factor of a whole weight row.
+// bytes of lookup table in LDS, filled by tables(). row_factors(): factors of whole weight rows.
 template <uint32_t FMT> struct GroupedFormat;
 
 struct GroupedWhole {                     // no factor outside the operands
@@ -91,7 +93,6 @@ struct GroupedHalves : GroupedWhole {
     static constexpr bool kFp8 = false;
     static constexpr int kTab = 16;
     static __device__ __forceinline__ void tables(uint8_t *, int) {}
-    static __device__ __forceinline__ float row_factor(const BankView &, int64_t) { return 1.f; }
 };
 struct GroupedNibbles : GroupedHalves {   // 16 code bytes a sub-block in the canonical order
     static constexpr int kCodes = 1, kRecs = 1;
@@ -273,25 +274,28 @@ template <> struct GroupedFormat<TQMOE_IQ3_S> : GroupedHalves {
 
 template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
     static constexpr bool kFp8 = true;
-    static constexpr int kCodes = 2, kRecs = 1, kTab = 256 * 16;
-    // Per scale byte the 16 products e2m1(code) * e4m3(scale) / 8, rounded to E4M3 (nearest even; an eighth keeps the largest
-    // inside the format, row_factor gives it back), as the two pools of pick().
+    static constexpr int kCodes = 2, kRecs = 1, kTab = 256 * 8;
+    // Per scale byte the products e2m1(code) * e4m3(scale) / 8 of the eight codes without a sign, rounded to E4M3 (nearest even; an
+    // eighth keeps the largest inside the format, row_factors gives it back): rounding and limit know no sign, so that a code's own is
+    // bit 7 of the result.
     static __device__ __forceinline__ void tables(uint8_t * tab, int tid) {
         const float sc = e4m3_to_float(uint32_t(tid));
-        uint32_t v[4];
+        uint32_t v[2];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 2; ++q) {
             float f[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const uint32_t twice = ((q == 0 ? kFp4T0 : q == 1 ? kFp4T1 : q == 2 ? kFp4T2 : kFp4T3) >> (8 * j)) & 0xFFu;
-                f[j] = fminf(fmaxf(float(int8_t(twice)) * 0.0625f * sc, -448.f), 448.f);
-            }
-            int w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
+            for (int j = 0; j < 4; ++j) f[j] = fminf(fmaxf(float(((q == 0 ? kFp4T0 : kFp4T1) >> (8 * j)) & 0xFFu) * 0.0625f * sc, -448.f), 448.f);
+            const int w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
             v[q] = uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w, true));
         }
-        reinterpret_cast<uint4 *>(tab)[tid] = table16_pools(v);
+        const bool none = (tid & 0x7F) == 0x7F;   // (not a number, in E4M3 too)
+        reinterpret_cast<uint2 *>(tab)[tid] = none ? make_uint2(0x7F7F7F7Fu, 0x7F7F7F7Fu) : make_uint2(v[0], v[1]);
     }
+    // The products of the low (high) nibbles of four code bytes: four instructions, where a table of sixteen takes five and six (8192
+    // tokens of 8 of 256 experts 1629 -> 1464 us a layer).
+    static __device__ __forceinline__ uint32_t low4(uint2 t, uint32_t c) { return __builtin_amdgcn_perm(t.y, t.x, c & 0x07070707u) ^ ((c << 4) & 0x80808080u); }
+    static __device__ __forceinline__ uint32_t high4(uint2 t, uint32_t c) { return __builtin_amdgcn_perm(t.y, t.x, (c >> 4) & 0x07070707u) ^ (c & 0x80808080u); }
     static __device__ __forceinline__ const uint8_t * code(const BankView & b, int64_t tile, int S, int lane) { return b.codes + tile * S * 512 + lane * 16; }
     static __device__ __forceinline__ int code_at(int i, int st) { return st * 2048 + i * 1024; }
     static __device__ __forceinline__ const uint8_t * rec(const BankView & b0, const BankView & b1, int64_t tile0, int64_t tile1, int S, int, int lane) {
@@ -299,7 +303,7 @@ template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
         return (l < 16 ? b0.aux + tile0 * (S / 4) * 256 : b1.aux + tile1 * (S / 4) * 256) + (l & 15) * 16;
     }
     static __device__ __forceinline__ int rec_at(int, int st) { return st * 256; }
-    struct Prep { uint32_t c[2][4], sc[2]; uint4 t0, t1; const uint8_t * tab; };
+    struct Prep { uint32_t c[2][4], sc[2]; uint2 t0, t1; const uint8_t * tab; };
     static __device__ __forceinline__ void prep(const uint8_t * w, int nb, int, int n, int g, const uint8_t * tab, Prep & p) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) {   // sub-blocks g and 2 + g
@@ -314,17 +318,27 @@ template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
     static __device__ __forceinline__ uint4 slice(Prep & p, int j) {
         const int i = j >> 1, h = j & 1;
         if (h == 0) {
-            p.t0 = *reinterpret_cast<const uint4 *>(p.tab + (p.sc[i] & 0xFFu) * 16);
-            p.t1 = *reinterpret_cast<const uint4 *>(p.tab + ((p.sc[i] >> 8) & 0xFFu) * 16);
+            p.t0 = *reinterpret_cast<const uint2 *>(p.tab + (p.sc[i] & 0xFFu) * 8);
+            p.t1 = *reinterpret_cast<const uint2 *>(p.tab + ((p.sc[i] >> 8) & 0xFFu) * 8);
         }
-        const Table16 lo{p.t0.x, p.t0.y, p.t0.z, p.t0.w}, hi{p.t1.x, p.t1.y, p.t1.z, p.t1.w};
-        const uint32_t a = p.c[i][2 * h], b = p.c[i][2 * h + 1], m = 0x0F0F0F0Fu;
-        return make_uint4(pick(lo, a & m), pick(hi, (a >> 4) & m), pick(lo, b & m), pick(hi, (b >> 4) & m));
+        const uint32_t a = p.c[i][2 * h], b = p.c[i][2 * h + 1];
+        return make_uint4(low4(p.t0, a), high4(p.t1, a), low4(p.t0, b), high4(p.t1, b));
     }
-    static __device__ __forceinline__ float row_factor(const BankView & b, int64_t row) {
-        return 8.f * *reinterpret_cast<const float *>(b.aux + nvfp4_global_offset(b.rows_total, b.cols) + row * 4);
+    static __device__ __forceinline__ void row_factors(const BankView & b, int64_t row, float * f) {   // of four rows
+        const float4 v = *reinterpret_cast<const float4 *>(b.aux + nvfp4_global_offset(b.rows_total, b.cols) + row * 4);
+        f[0] = 8.f * v.x; f[1] = 8.f * v.y; f[2] = 8.f * v.z; f[3] = 8.f * v.w;
     }
 };
+
+// 16-bit results: halves, or (a kernel of its own: a branch at every pair cost more than the arithmetic) bf16
+struct Bf16Row { uint16_t v; };
+template <class OT, bool PIN> __device__ __forceinline__ uint32_t pair16(float x, float y) {
+    if constexpr (std::is_same<OT, Bf16Row>::value) return float_to_bf16_bits(x) | uint32_t(float_to_bf16_bits(y)) << 16;
+    else {
+        if constexpr (PIN) asm("" : "+v"(x), "+v"(y));   // (the product is rounded before it is converted)
+        return bits_of(v2h{_Float16(x), _Float16(y)});
+    }
+}
 
 // bytes of a wave's codes and records of one stage
 template <class W> constexpr int kStageW = 2 * W::kCodes * 1024 + W::kRecs * 1024;
@@ -544,6 +558,12 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
         constexpr int kPitch = 32 * sizeof(OT) + 16, kLanes = 32 * sizeof(OT) / 16, kStep = 64 / kLanes;   // lanes a row, rows a store
         static_assert(32 * kPitch <= Rings<W, MT, MAX>::kCodes * kStageW<W>, "the tile's place");
         uint8_t * const tile_lds = lds + Rings<W, MT, MAX>::kRows * MT * 4096 + wave * Rings<W, MT, MAX>::kCodes * kStageW<W>;
+        [[maybe_unused]] float own[2][W::kFp8 ? 16 : 1];   // (read once: between an item's stores every read would wait for the memory)
+        if constexpr (W::kFp8)
+#pragma unroll
+            for (int b = 0; b < 2; ++b)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) W::row_factors(b ? k.b1 : k.b0, (int64_t(e) * tiles + min(wt[b], tiles - 1)) * 32 + 8 * c + 4 * g, &own[b][4 * c]);
         const bool clamp = k.glu.limit > 1e-6f;
 #pragma unroll
         for (int m = 0; m < MT; ++m) {
@@ -555,7 +575,7 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
 #pragma unroll
                     for (int i = 0; i < 16; ++i) {
                         v[i] = acc[bank][m][i];
-                        if constexpr (W::kFp8) v[i] *= W::row_factor(bank ? k.b1 : k.b0, (int64_t(e) * tiles + wt[bank]) * 32 + 8 * (i >> 2) + 4 * g + (i & 3));
+                        if constexpr (W::kFp8) v[i] *= own[bank][i];
                         v[i] *= FOLD ? s_scale[m * 32 + 8 * (i >> 2) + 4 * g + (i & 3)] : scl;
                     }
                 };
@@ -582,10 +602,6 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                 for (int c = 0; c < 4; ++c) {
                     const float * q = v + 4 * c;
                     uint8_t * to = tile_lds + n * kPitch;
-                    auto half2 = [&](float x, float y) {
-                        if constexpr (W::kFp8) if (k.out_bf16) return float_to_bf16_bits(x) | uint32_t(float_to_bf16_bits(y)) << 16;
-                        return bits_of(v2h{_Float16(x), _Float16(y)});
-                    };
                     if constexpr (FOLD) {
 #pragma unroll
                         for (int i = 0; i < 4; ++i) {
@@ -595,8 +611,8 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                         }
                     } else if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4 *>(to + (8 * c + 4 * g) * 4) = make_float4(q[0], q[1], q[2], q[3]);
                     else if constexpr (GATEUP && !W::kFp8)   // operand_pos: the four values stay together, 1 and 2 change places
-                        *reinterpret_cast<uint2 *>(to + operand_pos(8 * c + 4 * g) * 2) = make_uint2(half2(q[0], q[2]), half2(q[1], q[3]));
-                    else *reinterpret_cast<uint2 *>(to + (8 * c + 4 * g) * 2) = make_uint2(half2(q[0], q[1]), half2(q[2], q[3]));
+                        *reinterpret_cast<uint2 *>(to + operand_pos(8 * c + 4 * g) * 2) = make_uint2(pair16<OT, W::kFp8>(q[0], q[2]), pair16<OT, W::kFp8>(q[1], q[3]));
+                    else *reinterpret_cast<uint2 *>(to + (8 * c + 4 * g) * 2) = make_uint2(pair16<OT, W::kFp8>(q[0], q[1]), pair16<OT, W::kFp8>(q[2], q[3]));
                 }
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
@@ -621,6 +637,9 @@ template <uint32_t FMT, int MAX> void grouped_rows_launch_max(const GroupedArgs 
         allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes);
         kernel<<<blocks, 256, bytes, s>>>(k);
     };
+    if constexpr (GroupedFormat<FMT>::kFp8) {
+        if (k.out_bf16 && !f32_out) return gateup ? go(&grouped_rows_k<FMT, MAX, true, Bf16Row>) : go(&grouped_rows_k<FMT, MAX, false, Bf16Row>);
+    }
     if (gateup) {
         if constexpr (MAX > 1 || GroupedFormat<FMT>::kFold) go(&grouped_rows_k<FMT, MAX, true, uint16_t>);   // (grouped_rows_per_item)
     } else if (f32_out) go(&grouped_rows_k<FMT, MAX, false, float>);
