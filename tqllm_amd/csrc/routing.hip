@@ -136,24 +136,49 @@ template <bool F32> constexpr int kRouterGemmMin = F32 ? 56000 : 45000;
 constexpr int kRgWaves = 8, kRgRows = 64, kRgPitch = kRgRows + 4;   // floats of a token's row in the exchange space: four rows apart, other banks
 template <int TA> constexpr int kRgLds = 4 * TA * 16 * kRgPitch * int(sizeof(float));
 
-// the gate row's logits of tokens [t0, t1) (zeros without a gate row), a wave a token; and the grid's share of what is to be cleared
+// The gate row's logits of tokens [t0, t1) (zeros without a gate row), a wave a token; and the grid's share of what is to be cleared.
+// A wave has the loads of several tokens and of four passes over its columns under way at once: one after the other they were a chain
+// of trips to memory longer than the blocks beside it (2048 columns: eight tokens a wave were 32 trips).
 template <int XT>
 __device__ __forceinline__ void router_shared_column(const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x, float * __restrict__ logits, int h, int e, int n,
                                                      int t0, int t1, const RouterSide & side, int waves) {
     const int lane = threadIdx.x & 63;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < side.zero_n; i += gridDim.x * blockDim.x) side.zero[i] = 0;
-    for (int t = t0 + (threadIdx.x >> 6); t < t1; t += waves) {
-        float acc = 0.f;
+    constexpr int NT = XT == TQMOE_F32 ? 2 : 4, NP = 4, RAW = XT == TQMOE_F32 ? 2 : 1;   // tokens and passes together, 16-byte loads of eight values
+    for (int t = t0 + int(threadIdx.x >> 6); t < t1; t += NT * waves) {
+        float acc[NT] = {};
         if (shared)
-            for (int c = lane * 8; c < h; c += 512) {
-                float wv[8], xv[8];
-                load8<XT>(shared, c, wv);
-                load8<XT>(x, int64_t(t) * h + c, xv);
+            for (int c0 = lane * 8; c0 < h; c0 += NP * 512) {
+                uint4 wr[NP][RAW], xr[NT][NP][RAW];
 #pragma unroll
-                for (int j = 0; j < 8; ++j) acc = fmaf(wv[j], xv[j], acc);
+                for (int p = 0; p < NP; ++p) {
+                    const int c = c0 + p * 512;          // (past the last column: zeros on both sides)
+#pragma unroll
+                    for (int q = 0; q < RAW; ++q) {
+                        constexpr int kSize = XT == TQMOE_F32 ? 4 : 2;
+                        wr[p][q] = c < h ? *reinterpret_cast<const uint4 *>(shared + int64_t(c) * kSize + q * 16) : uint4();
+#pragma unroll
+                        for (int i = 0; i < NT; ++i)
+                            xr[i][p][q] = c < h ? *reinterpret_cast<const uint4 *>(x + (int64_t(min(t + i * waves, t1 - 1)) * h + c) * kSize + q * 16) : uint4();
+                    }
+                }
+#pragma unroll
+                for (int p = 0; p < NP; ++p) {
+                    float wv[8], xv[8];
+                    load8<XT>(wr[p], 0, wv);
+#pragma unroll
+                    for (int i = 0; i < NT; ++i) {
+                        load8<XT>(xr[i][p], 0, xv);
+#pragma unroll
+                        for (int j = 0; j < 8; ++j) acc[i] = fmaf(wv[j], xv[j], acc[i]);
+                    }
+                }
             }
-        acc = group_sum<64>(acc);
-        if (lane == 0) logits[int64_t(t) * (e + 1) + e] = acc;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+            const float sum = group_sum<64>(acc[i]);
+            if (lane == 0 && t + i * waves < t1) logits[int64_t(t + i * waves) * (e + 1) + e] = sum;
+        }
     }
 }
 
