@@ -252,7 +252,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
     constexpr bool STAGED = MODE >= 1, MULTI = MODE == 2;
     constexpr int kIn = ROUTE > 0 ? 1 : 2;   // input rows a lane half has sums of (a block that routes serves one)
     extern __shared__ __attribute__((aligned(16))) uint8_t stage[];
-    __shared__ int meta[2], s_tok[kTP];
+    __shared__ int meta[1], s_tok[kTP];
     __shared__ float s_x0[kTP];
     __shared__ __attribute__((aligned(16))) int ql[kMaxWaves * 2][32];
     __shared__ uint32_t lat[F::kLattice];
@@ -282,7 +282,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
             }
         }
     };
-    int e, wk_i, rt_l;
+    int e, wk_i, rt_l, n_tok = 1;
+    int tok[kTP] = {a, -1, -1, -1};
     if constexpr (ROUTE > 0) {
         // One wave selects, for as many rounds as its assignment needs. The token's whole routing is written down by a block of its own,
         // so that the weights' exponentials and divisions are in nobody's way (one token of the 512-expert IQ4_XS layer, launch 10.0 ->
@@ -312,12 +313,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
         __syncthreads();
         e = slot < topk ? meta[0] : route.experts;
     } else {
-        e = fetch_ids(ids, A, a, mode, reinterpret_cast<int *>(stage));
+        n_tok = chunk_rows(ids, A, a, mode, e, tok);
         rt_l = (wave >= wk) + (wave >= 2 * wk) + (wave >= 3 * wk), wk_i = wave - rt_l * wk;   // (at most four row tiles: divisions were a tenth of a short launch's instructions)
     }
     if (e < 0 || int64_t(e) * b0.rows >= b0.rows_total) return;   // skipped assignment, or an id outside the bank
-    int tok[kTP];
-    const int n_tok = ROUTE > 0 ? 1 : chunk_up(A, a, e, mode, kTP, reinterpret_cast<int *>(stage), meta, tok);   // the lists live in the dynamic space
     if (n_tok == 0) return;
     if (ROUTE == 0 && threadIdx.x < kTP) s_tok[threadIdx.x] = tok[threadIdx.x];
 
@@ -425,7 +424,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(kDecodeWave
                 for (int nb = 0; nb < NB; ++nb) { const float f = F::row_factor(nb ? b1 : b0, row); accf[nb][0] *= f; accf[nb][1] *= f; }
             }
         }
-        __syncthreads();                                       // the id list (or the previous pass's sums) is done with: the space now holds the partial sums
+        if constexpr (MULTI) __syncthreads();                  // the previous pass's sums are done with
         float (*red)[NB][kTP][32] = reinterpret_cast<float (*)[NB][kTP][32]>(stage);
 #pragma unroll
         for (int nb = 0; nb < NB; ++nb) { red[wave][nb][2 * g][n] = accf[nb][0]; red[wave][nb][2 * g + 1][n] = accf[nb][1]; }
@@ -635,10 +634,9 @@ void mfma_launch(int nb, BankView b0, BankView b1, const uint8_t * image, void *
     int tpw = waves / wk;                                                 // row tiles per block
     if (tpw > tiles) tpw = tiles;
     const unsigned threads = unsigned(wk * tpw * 64);
-    // dynamic LDS: the match list and the copy of the ids (2 * kMaxList ints), later the partial sums; behind them the input
-    // rows' planes (256 bytes per sub-block) and, for rows with a scale per sub-block, the scales
-    size_t lds = mode ? size_t(2) * kMaxList * sizeof(int) : 0;
-    if (lds < size_t(wk * tpw) * nb * kTP * 32 * sizeof(float)) lds = size_t(wk * tpw) * nb * kTP * 32 * sizeof(float);
+    // dynamic LDS: the partial sums; behind them the input rows' planes (256 bytes per sub-block) and, for rows with a scale per
+    // sub-block, the scales
+    size_t lds = size_t(wk * tpw) * nb * kTP * 32 * sizeof(float);
     // the input rows go through LDS from a dozen assignments on (the waves then overlap each other's waits, and what
     // counts is that a wave's own weight loads stay in flight under its products: 10 tokens of 8 of 128 experts, Q4_K 71.5
     // and 61.3 us a layer, NVFP4G 69.2 and 68.0, IQ3_S 67.7 and 64.7); a shorter batch is one chain of dependent steps per wave,
