@@ -76,6 +76,12 @@ __device__ __forceinline__ void quantise_block(const float (&v)[32], uint8_t * i
     reinterpret_cast<float *>(image_row + int64_t(S) * 68)[s] = float(qsum) * scale;
 }
 
+// a value and the one sixteen lanes further on or back, in the lane's row of 32: one instruction (a shuffle is a trip through LDS)
+__device__ __forceinline__ int2 both_rows(int v) {
+    const auto r = __builtin_amdgcn_permlane16_swap(uint32_t(v), uint32_t(v), false, false);
+    return make_int2(int(r[0]), int(r[1]));
+}
+
 // 32 values held one per lane by 32 consecutive lanes (lane i of the group has value i; every lane of the wave must
 // call this) -> sub-block s of an image row. q_lds: 32 ints of LDS private to the group. live: whether to store.
 __device__ __forceinline__ void quantise_block_lanes(float v, int i, bool live, int * q_lds, uint8_t * image_row, int S, int s) {
@@ -84,7 +90,8 @@ __device__ __forceinline__ void quantise_block_lanes(float v, int i, bool live, 
     amax = fmaxf(amax, dpp_f<kDppXor2>(amax));
     amax = fmaxf(amax, dpp_f<kDppHalfMirror>(amax));
     amax = fmaxf(amax, dpp_f<kDppMirror>(amax));
-    amax = fmaxf(amax, __shfl_xor(amax, 16, 64));
+    const int2 rows_max = both_rows(__float_as_int(amax));
+    amax = fmaxf(__int_as_float(rows_max.x), __int_as_float(rows_max.y));
     const float inv = amax > 0.f ? 16383.f / amax : 0.f;
     const int q = __float2int_rn(v * inv);
     q_lds[i] = q;
@@ -93,7 +100,8 @@ __device__ __forceinline__ void quantise_block_lanes(float v, int i, bool live, 
     qs += dpp_i<kDppXor2>(qs);
     qs += dpp_i<kDppHalfMirror>(qs);
     qs += dpp_i<kDppMirror>(qs);
-    qs += __shfl_xor(qs, 16, 64);
+    const int2 rows_sum = both_rows(qs);
+    qs = rows_sum.x + rows_sum.y;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // q_lds is read below by other lanes of this same wave
     __builtin_amdgcn_wave_barrier();
     if (!live) return;
