@@ -251,6 +251,18 @@ def test_dispatch_bit_exact(tq, oracle, e, n, k):
     assert counts.sum() == (ids >= 0).sum()
 
 
+@pytest.mark.parametrize("e", [3, 64, 65, 513, 1024])
+@pytest.mark.parametrize("assignments", [1025, 8 * 1024, 8 * 1024 + 1, 24 * 1024, 24 * 1024 + 1, 49 * 1024 + 7])
+def test_dispatch_chunks_are_added_up(tq, oracle, e, assignments):
+    """Chunk counts come eight or twenty-four at a time and are added by one block more than there are chunks: numbers of chunks on both
+    sides of either, experts on both sides of a wave and the most one block takes; every third expert has no assignment."""
+    rng = np.random.default_rng(assignments + e)
+    ids = (rng.integers(0, (e + 2) // 3, (assignments, 1)) * 3).astype(np.int32)
+    want_c, want_o, want_p = oracle.dispatch(ids, e)
+    counts, offsets, perm = (t.cpu().numpy() for t in tq.moe_dispatch(dev(ids), e)[:3])
+    assert np.array_equal(counts, want_c) and np.array_equal(offsets, want_o) and np.array_equal(perm, want_p)
+
+
 def test_dispatch_is_deterministic_and_truncates_groups(tq, oracle):
     rng = np.random.default_rng(9)
     ids = rng.integers(0, 32, (2000, 4)).astype(np.int32)

@@ -156,6 +156,21 @@ template <int CTRL> __device__ __forceinline__ float dpp_f(float v) {
     return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
 }
 template <int CTRL> __device__ __forceinline__ int dpp_i(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, 0xF, 0xF, true); }
+// sums of the lanes up to each one, in rows of sixteen lanes and in the whole wave (shuffles would be a trip through LDS a step)
+template <int CTRL, int ROWS> __device__ __forceinline__ int dpp_from(int v) { return __builtin_amdgcn_update_dpp(0, v, CTRL, ROWS, 0xF, false); }   // 0 where no lane is the source
+__device__ __forceinline__ int row_scan(int v) {
+    v += dpp_from<0x111, 0xF>(v);      // row_shr:1, 2, 4, 8
+    v += dpp_from<0x112, 0xF>(v);
+    v += dpp_from<0x114, 0xF>(v);
+    v += dpp_from<0x118, 0xF>(v);
+    return v;
+}
+__device__ __forceinline__ int wave_scan(int v) {
+    v = row_scan(v);
+    v += dpp_from<0x142, 0xA>(v);      // row_bcast:15 into rows 1 and 3
+    v += dpp_from<0x143, 0xC>(v);      // row_bcast:31 into rows 2 and 3
+    return v;
+}
 constexpr int kDppXor1 = 0xB1;          // quad_perm [1,0,3,2]
 constexpr int kDppXor2 = 0x4E;          // quad_perm [2,3,0,1]
 constexpr int kDppHalfMirror = 0x141;   // lane i <-> 7 - i inside 8

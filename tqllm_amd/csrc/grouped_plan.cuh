@@ -15,16 +15,16 @@ constexpr int kManyItems = 8;
 constexpr int kScans = 6;   // full runs, rests of three classes; row tiles, chunks of chunk_tiles of them
 __device__ __forceinline__ void plan_items(const int * __restrict__ counts, const int * __restrict__ offsets, int experts, int item_rows, int4 * __restrict__ plan, RowIndex index) {
     __shared__ int s_wave[kScans][16];
-    __shared__ int s_total[kScans];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int per = (experts + 1023) / 1024, lo = min(tid * per, experts), hi = min(lo + per, experts);
+    const int shift = 31 - __clz(item_rows);   // (a power of two)
     auto rest_class = [&](int c) {
-        const int full = c / item_rows, rest = c % item_rows;
+        const int full = c >> shift, rest = c & (item_rows - 1);
         return rest == 0 ? -1 : full >= 1 && full < kManyItems ? 0 : rest > 64 ? 1 : rest > 32 ? 2 : 3;
     };
     auto add = [&](int c, int (&v)[kScans]) {
         const int k = rest_class(c), t = (c + 31) / 32;
-        v[0] += c / item_rows;
+        v[0] += c >> shift;
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[i] += k == i;
         v[4] += t;
@@ -35,29 +35,30 @@ __device__ __forceinline__ void plan_items(const int * __restrict__ counts, cons
     int at[kScans];
 #pragma unroll
     for (int i = 0; i < kScans; ++i) {
-        int v = mine[i];
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) { const int u = __shfl_up(v, d, 64); if (lane >= d) v += u; }
+        const int v = wave_scan(mine[i]);
         at[i] = v - mine[i];
         if (lane == 63) s_wave[i][wave] = v;
     }
     __syncthreads();
-    if (tid < kScans) {
-        int sum = 0;
-        for (int w = 0; w < 16; ++w) { const int v = s_wave[tid][w]; s_wave[tid][w] = sum; sum += v; }
-        s_total[tid] = sum;
+    // every wave adds the sixteen waves' sums of all scans by itself: four scans in the rows of one register, two in another's
+    const int first = row_scan(s_wave[lane >> 4][lane & 15]), second = row_scan(s_wave[4 + ((lane >> 4) & 1)][lane & 15]);
+    int before[kScans], total[kScans];
+#pragma unroll
+    for (int i = 0; i < kScans; ++i) {
+        const int from = i < 4 ? first : second, row = 16 * (i & 3);
+        before[i] = wave ? __builtin_amdgcn_readlane(from, row + wave - 1) : 0;
+        total[i] = __builtin_amdgcn_readlane(from, row + 15);
     }
-    __syncthreads();
     int base = 0;
 #pragma unroll
-    for (int i = 0; i < kScans; ++i) { at[i] += s_wave[i][wave] + (i < 4 ? base : 0); if (i < 4) base += s_total[i]; }
+    for (int i = 0; i < kScans; ++i) { at[i] += before[i] + (i < 4 ? base : 0); if (i < 4) base += total[i]; }
     if (tid == 0) {
-        plan[0] = make_int4(s_total[0], s_total[1], s_total[2], s_total[3]);
-        if (index.tile_base) { index.tile_base[experts] = s_total[4]; index.chunk_base[experts] = s_total[5]; }
+        plan[0] = make_int4(total[0], total[1], total[2], total[3]);
+        if (index.tile_base) { index.tile_base[experts] = total[4]; index.chunk_base[experts] = total[5]; }
     }
     if (index.tile_base && tid < index.counters_n) index.counters[tid] = 0;
     for (int e = lo; e < hi; ++e) {
-        const int c = max(counts[e], 0), first = offsets[e], full = c / item_rows, rest = c % item_rows;
+        const int c = max(counts[e], 0), first = offsets[e], full = c >> shift, rest = c & (item_rows - 1);
         for (int f = 0; f < full; ++f) plan[1 + at[0] + f] = make_int4(e, first + f * item_rows, item_rows, at[4] + f * (item_rows / 32));
         const int k = rest_class(c);
 #pragma unroll
