@@ -82,6 +82,25 @@ def test_router_gemm_path_f32(tq, oracle, n, e, h, shared):
         assert torch.equal(part, logits[5:5 + m])
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("n,e,h", [(1000, 63, 64), (897, 64, 128), (120, 500, 192), (333, 513, 320), (512, 512, 2048), (1500, 65, 2112), (3100, 60, 1024), (30, 2000, 512)])
+def test_router_gemm_by_alignment(tq, dtype, n, e, h):
+    """Rows aligned to 16 bytes go through LDS in tiles of 16 tokens, others straight from memory: the same sums in the same order,
+    slices of the columns of an odd number of 64-byte steps and ragged last tiles among them."""
+    gen = torch.Generator().manual_seed(n + e + h)
+    w, gate, x = (torch.randn(*size, generator=gen).to(dtype).cuda() for size in ((e, h), (h,), (n, h)))
+    off = 8 // w.element_size()
+    shifted = torch.empty(n * h + off, dtype=dtype, device="cuda")[off:].view(n, h)
+    shifted.copy_(x)
+    assert x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0 and shifted.data_ptr() % 16 == 8
+    got = tq.moe_router(w, gate, x)
+    assert torch.equal(got, tq.moe_router(w, gate, shifted))
+    exact = x.cpu().double() @ torch.cat([w, gate[None]]).cpu().double().T
+    # fp32 sums of h products: the rounding of a sum's parts, each at most its size, as a random walk of 6 deviations
+    bound = 6 * 2.0 ** -24 * h ** 0.5 * float(exact.abs().max())
+    assert float((got.cpu().double() - exact).abs().max()) < bound
+
+
 def test_router_without_shared_gate_and_f16(tq, oracle):
     rng = np.random.default_rng(5)
     h, e, n = 512, 33, 7

@@ -126,7 +126,8 @@ template <int WT> int32_t launch_router_x(uint32_t xtype, const void * w, const 
 // instructions, and the eight partial tiles are added through LDS in a fixed order. No stage is waited for by the whole block:
 // a launch is one trip to memory and the bandwidth of the L2, where stages of 256 columns through LDS were a chain of eight
 // trips (512 experts, 2048 columns: 21 us for 333 tokens, 32 for 4096). TA is the largest tile that still gives every
-// compute unit a block. A token's sums do not depend on it, nor on the batch.
+// compute unit a block; one of 16 tokens goes through LDS after all, each wave's operands by themselves (router_gemm_dma_k), and is
+// left here for operands that are not aligned to 16 bytes. A token's sums do not depend on any of this, nor on the batch.
 // The last row of blocks takes the shared expert's gate row (or stores its zeros): a wave a token.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
@@ -277,6 +278,104 @@ __global__ __launch_bounds__(64 * kRgWaves) void router_gemm_k(const uint8_t * _
         if (t0 + t < n && r0 + c < e) logits[int64_t(t0 + t) * (e + 1) + r0 + c] = v;
     }
 }
+// The same tile of 16 tokens x 64 router rows with every wave's operands through a place of its own in LDS: 128 bytes of a row, a whole
+// line, in one transfer. With operands straight from memory an instruction touches sixteen rows, half a line each, and the lines of a wave's
+// loads under way are many times the first-level cache: the loads ran at 15 bytes a cycle and compute unit, the first four waves' in front of
+// the others' (333 tokens x 513 rows of 2048: waves 0 to 3 done after 11600 cycles, 4 to 7 after 21700). No wave waits for another before
+// the partial tiles are added, in the same order: same bits. Two stages of 80 rows a wave are all of a compute unit's LDS.
+// (us a launch, 2048 columns, operands from memory / so: bf16 333 tokens x 512 rows 11.8 / 7.5, with a 513th 11.7 / 7.4, 2100 x 64 11.5 / 7.5;
+// fp32 333 x 512 24.3 / 16.2, 4096 x 64 27.4 / 20.5. All of a compute unit's LDS is one block's, so the gate row's blocks wait for a free one.)
+constexpr int kRdRows = 16 + kRgRows, kRdStage = kRdRows * 128, kRdLds = kRgWaves * 2 * kRdStage;
+static_assert(kRdLds <= 163840 && kRgLds<1> <= kRdLds, "the compute unit's LDS");
+template <bool F32>
+__global__ __launch_bounds__(64 * kRgWaves) void router_gemm_dma_k(const uint8_t * __restrict__ w, const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x,
+                                                                  float * __restrict__ logits, int h, int e, int n, int gate, RouterSide side) {
+    extern __shared__ __attribute__((aligned(16))) uint8_t lds[];   // [wave][2][row][128]; then the partial tiles [4][16][kRgPitch]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
+    constexpr int kBytes = F32 ? 4 : 2, NQ = kRdRows / 8;
+    const int t0 = int(blockIdx.x) * 16, r0 = int(blockIdx.y) * kRgRows;
+    const int64_t pitch = int64_t(h) * kBytes;
+    if (blockIdx.y == gridDim.y - 1) {
+        router_shared_column<F32 ? TQMOE_F32 : TQMOE_BF16>(shared, x, logits, h, e, n, int(blockIdx.x) * gate, min(int(blockIdx.x + 1) * gate, n), side, kRgWaves);
+        return;
+    }
+    // transfer q: rows 8 q .. + 7, the tokens' in front of the router's (past the end a valid row again, not stored); a row's 16-byte piece p
+    // in slot p ^ (row / 2 & 7)
+    const uint8_t * src[NQ];
+#pragma unroll
+    for (int q = 0; q < NQ; ++q) {
+        const int row = q * 8 + (lane >> 3), piece = (lane & 7) ^ ((row >> 1) & 7);
+        src[q] = (row < 16 ? x + int64_t(min(t0 + row, n - 1)) * pitch : w + int64_t(min(r0 + row - 16, e - 1)) * pitch) + piece * 16;
+    }
+    const int steps = int(pitch / 64), s0 = wave * steps / kRgWaves, s1 = (wave + 1) * steps / kRgWaves;   // 64 bytes of every row a step, two a stage
+    uint8_t * const own = lds + wave * 2 * kRdStage;
+    const uint32_t own0 = lds_address(own);
+    auto place = [&](int st) { return int(min(int64_t(st) * 64, pitch - 128)); };   // (an odd last step is a stage's second half)
+    auto send = [&](int st, int slot) {
+        const int at = place(st);
+#pragma unroll
+        for (int q = 0; q < NQ; ++q) dma16(src[q] + at, own0 + slot * kRdStage + q * 1024);
+    };
+    v4f acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[j] = v4f{0.f, 0.f, 0.f, 0.f};
+    if (s0 < s1) {
+        send(s0, 0);
+        send(min(s0 + 2, s1 - 1), 1);
+        int slot = 0;
+        for (int st = s0; st < s1; st += 2, slot ^= 1) {
+            dma_wait<NQ, false>();             // the other slot's may be under way
+            const uint8_t * rows = own + slot * kRdStage + r * 128;
+            const int skip = (st * 64 - place(st)) / 64;
+            uint4 a[2], b[2][4];
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                const int piece = ((4 * min(q + skip, 1) + g) ^ ((r >> 1) & 7)) * 16;   // (rows 16 further on have the same low bits)
+                a[q] = *reinterpret_cast<const uint4 *>(rows + piece);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) b[q][j] = *reinterpret_cast<const uint4 *>(rows + (16 + 16 * j) * 128 + piece);
+            }
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            send(min(st + 4, s1 - 1), slot);   // (past the last stage: that one's last step again, not read)
+#pragma unroll
+            for (int q = 0; q < 2; ++q) {
+                if (st + q >= s1) break;
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    if constexpr (F32) {
+                        const v4f av = __builtin_bit_cast(v4f, a[q]), bv = __builtin_bit_cast(v4f, b[q][j]);
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[c], bv[c], acc[j], 0, 0, 0);
+                    } else acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, a[q]), __builtin_bit_cast(v8bf, b[q][j]), acc[j], 0, 0, 0);
+                }
+            }
+        }
+    }
+    dma_wait<0, true>();
+    float * const red = reinterpret_cast<float *>(lds);
+    auto at = [&](int slot, int q) { return (slot * 16 + 4 * g + q) * kRgPitch + r; };
+    if (wave >= 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) red[at(wave - 4, q) + 16 * j] = acc[j][q];
+    }
+    __syncthreads();
+    if (wave < 4) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) red[at(wave, q) + 16 * j] += acc[j][q];
+    }
+    __syncthreads();
+    for (int i = tid; i < 16 * kRgRows; i += 64 * kRgWaves) {
+        const int t = i / kRgRows, c = i % kRgRows;
+        const float * p = red + t * kRgPitch + c;
+        const float v = (p[0] + p[16 * kRgPitch]) + (p[2 * 16 * kRgPitch] + p[3 * 16 * kRgPitch]);
+        if (t0 + t < n && r0 + c < e) logits[int64_t(t0 + t) * (e + 1) + r0 + c] = v;
+    }
+}
+
 // The same for large batches of bf16 rows: 64 tokens x 128 router rows a block, operands through LDS, so that a row of x is
 // read by a quarter of the blocks. 128 bytes of every row a stage, from memory to LDS without registers, two stages under
 // way, two blocks a compute unit. The eight parts of the columns follow each other and join in the order the kernel above adds them: same bits.
@@ -398,9 +497,29 @@ template <bool F32> void launch_router_gemm(const void * w, const void * sg, con
         kernel<<<dim3(unsigned((n + 16 * ta - 1) / (16 * ta)), unsigned(rows + 1)), 64 * kRgWaves, lds, s>>>(
             static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, side);
     };
+    const bool aligned = aligned16(w) && aligned16(x), long_rows = int64_t(h) * (F32 ? 4 : 2) >= 4096;
+    auto rounds = [&](int ta) { return (blocks(ta) + 255) / 256; };
+    // (operands through LDS / straight from memory. Where straight would be tiles of 16 tokens: 1024 columns, 200 tokens x 512 rows,
+    // 5.4 / 7.2 us, 512 columns 4.7 / 7.2, 128 4.0 / 4.9; fp32 9.5 / 13.3, 6.8 / 7.8, 4.9 / 7.2. Of more blocks long rows only; bf16, us
+    // beside tiles of 32 tokens, 256 blocks of 16: 2048 columns 11.6 / 14.1, 4096 15.0 / 24.1, but 1024 9.2 / 8.6; 64 experts, 375 blocks:
+    // 1024 columns 12.8 / 9.0, 4096 26.1 / 27.0; beside the kernel of large batches, 384, 512 and 768 blocks: 2048 columns 14.1 / 19.1, 16.8 /
+    // 19.1, 24.2 / 19.6, 1024 columns 11.0 / 12.2, 14.2 / 12.3. fp32, beside 32 tokens, 512 and 768 blocks: 2048 columns 32.0 / 39.0, 46.1 / 65.0,
+    // 1024 18.8 / 22.0, 27.0 / 36.4, but 512 13.7 / 13.0; beside 64 tokens, a round of 256 blocks, one and a half, two: 2048 columns 60 / 60,
+    // 88 / 110, 120 / 115, 1024 35 / 32, 52 / 53, 70 / 59)
+    if (aligned && (F32 ? blocks(2) < 256 || (long_rows && (blocks(4) < 256 || 11 * rounds(1) < 40 * rounds(4)))
+                        : blocks(2) < 128 || (long_rows && blocks(1) <= (e > kRgRows ? 512 : 256)))) {
+        // a block of the gate row's takes 32 tokens instead of 16 where all of short rows' blocks nearly fit the chip at once (64 experts, 1024
+        // columns: 2100 tokens 5.9 us against 6.4, 3072 7.0 against 8.4; 2048 columns 8.1 against 7.4, and fp32 no better either)
+        const unsigned tiles = unsigned((n + 15) / 16);
+        const int gate = !F32 && !long_rows && blocks(1) <= 256 && blocks(1) + tiles > 256 ? 32 : 16;
+        allow_dynamic_lds(reinterpret_cast<const void *>(&router_gemm_dma_k<F32>), kRdLds);
+        router_gemm_dma_k<F32><<<dim3(tiles, unsigned(rows + 1)), 64 * kRgWaves, kRdLds, s>>>(
+            static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, gate, side);
+        return;
+    }
     if constexpr (!F32) {
         const int64_t tiles = (n + kRlTok - 1) / kRlTok, cols = (e + kRlRows - 1) / kRlRows;
-        if (tiles * cols >= kRlBlocks && e > kRgRows && h >= 512 && aligned16(w) && aligned16(x)) {
+        if (tiles * cols >= kRlBlocks && e > kRgRows && h >= 512 && aligned) {
             allow_dynamic_lds(reinterpret_cast<const void *>(&router_gemm_lds_k), kRlLds);
             router_gemm_lds_k<<<dim3(unsigned(tiles), unsigned(cols + (tiles * cols < kRlFull ? 1 : 0))), 64 * kRlWaves, kRlLds, s>>>(
                 static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, side);
