@@ -114,6 +114,26 @@ def test_quant_rows_fp8_bit_exact(tq, oracle, kind):
         assert s[r] == np.float32(ws)
 
 
+@pytest.mark.parametrize("cols", [32, 512, 544, 3040, 3072, 3104, 6176])
+@pytest.mark.parametrize("kind", ["f32", "bf16"])
+def test_quant_rows_fp8_of_every_piece(tq, oracle, kind, cols):
+    """The row's largest value in every 64th group of eight in turn, first and last, rows kept whole in registers (to 3072 values) and
+    longer ones: codes and scales of the oracle's quantiser."""
+    rng = np.random.default_rng(cols)
+    spots = sorted({min(c, cols - 1) for c in range(0, cols + 511, 512)} | {cols - 1})
+    x = rng.standard_normal((len(spots), cols)).astype(np.float32)
+    for r, c in enumerate(spots):
+        x[r, c] = -37.5 - r
+    t = torch.from_numpy(x).cuda().to({"f32": torch.float32, "bf16": torch.bfloat16}[kind])
+    xv = t.float().cpu().numpy()
+    q, s = tq.quant_rows_fp8(t)
+    q, s = natural_order(q.cpu().numpy()).view(np.uint8), s.cpu().numpy()
+    for r in range(len(spots)):
+        wq, ws = oracle.quant_act_row_e4m3(xv[r])
+        assert ((q[r] == wq) | ((q[r] & 0x7F) == 0) & ((wq & 0x7F) == 0)).all(), r      # a zero's sign is free
+        assert s[r] == np.float32(ws)
+
+
 PLANE_FORMATS = ["IQ4_XS", "IQ3_S", "Q4_K", "NVFP4G", "IQ3_XXS", "IQ2_XXS", "IQ2_XS", "IQ2_S", "IQ1_S", "IQ4_NL", "Q5_K", "Q4_0", "Q8_0"]
 
 
