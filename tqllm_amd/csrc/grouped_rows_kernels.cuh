@@ -17,8 +17,8 @@
 // pair rounds to fp16: 17 (Q4_K, whose codes are halves where they stand) to 27 (IQ4_XS) vector instructions for eight
 // weights, one rounding.
 // (Packed fp16 multiply-adds take four fewer and round twice: a quarter more error in the layer's result.)
-// NVFP4G: the products of a scale byte, rounded to E4M3, are a table in LDS (2 KB for all scales); eight instructions
-// for eight weights.
+// NVFP4G: the eight magnitudes of a scale byte, rounded to E4M3, are a table in LDS (2 KB for all scales), the code's sign is
+// put on beside the look-up; eight instructions for eight weights.
 //
 // Rows per item: a weight is decoded once per item and wave, so 128 rows spread its instructions over four matrix
 // instructions; with the two banks' eight accumulators (128 registers) two waves fit a SIMD, and one of them decodes while
@@ -26,8 +26,8 @@
 //
 // What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 228 us, 0.90
 // PFLOP/s, matrix pipe 48 % busy, vector pipe 53 % (262 us with biased codes; without the decode 205, without the row reads as
-// well 178, where a large fp16 product on this card would take 170); NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 880 us,
-// 43 % and 55 %. A product holds its SIMD's vector issue for about 18 cycles besides its own time, so that a stage's decode does not
+// well 178, where a large fp16 product on this card would take 170); NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 808 us,
+// 49 % and 52 % (880, 43 % and 55 % with the sign in the table of a scale's weights). A product holds its SIMD's vector issue for about 18 cycles besides its own time, so that a stage's decode does not
 // pass under its products for free.
 // Items of one row tile are bound by the decode (IQ3_S, 512 tokens: gate / up 117 us, 2.9 TB/s of codes, vector pipe 65 %, LDS 52 %,
 // three fifths of that bank conflicts of the lattice's look-ups).
