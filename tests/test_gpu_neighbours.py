@@ -53,3 +53,14 @@ def test_int8_result_does_not_depend_on_the_other_tokens(oracle, fmt, n, act_blo
     layer, x = layer_and_rows(oracle, fmt, n, 33, act_blocks)
     assert layer.path(n) == "grouped_i8"
     check(layer, x, 0.3 * n)
+
+
+@pytest.mark.parametrize("copies", [51, 52])
+def test_plan_of_more_chunks_than_compute_units(oracle, copies):
+    """Five assignments of each token: 255 chunks of 1024, whose items a block of its own plans, and 260, where the first chunk's does. All
+    copies of a token are the same bits, and those of a batch of one copy but for the sum's order, which the rows an expert decide: halves
+    of 2^-11 in the activations, two products behind each other."""
+    layer, x = layer_and_rows(oracle, "Q4_K", 1024, 33, 0)
+    out = layer.forward(x.repeat(copies, 1)).view(copies, 1024, -1)
+    assert torch.equal(out, out[:1].expand_as(out))
+    assert synth.errors(out[0].cpu().numpy(), layer.forward(x).cpu().numpy())[1] < 2 * 2.0 ** -11

@@ -271,10 +271,11 @@ def test_dispatch_bit_exact(tq, oracle, e, n, k):
 
 
 @pytest.mark.parametrize("e", [3, 64, 65, 513, 1024])
-@pytest.mark.parametrize("assignments", [1025, 8 * 1024, 8 * 1024 + 1, 24 * 1024, 24 * 1024 + 1, 49 * 1024 + 7])
+@pytest.mark.parametrize("assignments", [1025, 8 * 1024, 8 * 1024 + 1, 16 * 1024, 16 * 1024 + 1, 24 * 1024, 24 * 1024 + 1, 32 * 1024, 33 * 1024, 49 * 1024 + 7,
+                                         256 * 1024, 256 * 1024 + 1, 273 * 1024 - 5])
 def test_dispatch_chunks_are_added_up(tq, oracle, e, assignments):
-    """Chunk counts come eight or twenty-four at a time and are added by one block more than there are chunks: numbers of chunks on both
-    sides of either, experts on both sides of a wave and the most one block takes; every third expert has no assignment."""
+    """Chunk counts come sixteen at a time, the last ones eight or sixteen: numbers of chunks on both sides of either, and of the compute
+    units, experts on both sides of a wave and the most one block takes; every third expert has no assignment."""
     rng = np.random.default_rng(assignments + e)
     ids = (rng.integers(0, (e + 2) // 3, (assignments, 1)) * 3).astype(np.int32)
     want_c, want_o, want_p = oracle.dispatch(ids, e)

@@ -954,38 +954,49 @@ __global__ __launch_bounds__(256) void dispatch_place_k(const int * __restrict__
 // before it: where its assignments start inside each expert; all chunks: the experts' offsets); a wave finds each lane's equals
 // with a ballot per bit of the expert's number (a loop over the distinct experts of a wave's 64 assignments is 64 rounds at
 // worst), leaves its group sizes in a histogram of its own, and a prefix over the waves in index order gives every
-// assignment its place. Nothing is left to the order of atomics. One block more writes the counts and plans the products' items
-// (behind its placement the first chunk's was the launch's longest). Prefix sums go through DPP and not through LDS a step at a time. us a
-// launch, so / with the plan behind a placement and shuffles: 333 tokens of 10 of 512 experts 5.0 / 7.9, 1501 7.7 / 10.0, 4096 10.9 / 12.3; 512
-// tokens of 8 of 256 4.9 / 6.6; 4096 of 8 of 64 5.6 / 7.4.
+// assignment its place. Nothing is left to the order of atomics. One block more writes the counts and plans the products' items where it
+// finds a compute unit of its own (behind its placement the first chunk's was the launch's longest; without items, and from 256 chunks on, that
+// one does it). Prefix sums go through DPP and not through LDS a step at a time.
+// Chunk counts are loaded sixteen at a time, without a look at their end but in the last sixteen (twenty-four, past the end the last one
+// again, are half as many loads more than 16 or 32 chunks need and their addresses more scalar arithmetic than many chunks' loads take). Two
+// blocks a compute unit, or more than 256 chunks are two rounds of them: 93 scalar and 64 vector registers were one block.
+// us a launch, with the plan behind a placement, shuffles and a branch a load / a block for the plan, DPP and twenty-four / so: 333 tokens of 10
+// of 512 experts 7.4 / 5.0 / 5.3, 1501 9.0 / 6.2 / 5.4, 4096 10.9 / 9.3 / 8.2, 8192 15.4 / 15.6 / 12.4; 4096 of 10 of 1000 12.9 / 11.3 / 10.4. A
+// dispatch without items (two launches): 32768 assignments of 512 experts 10.5 / 11.5 / 10.0, 270000 24.5 / 42.5 / 22.4, of 1024 34.9 / 66 / 33.5.
 constexpr int kWideExperts = kDispatchWide, kWideWaves = kChunk / 64;
 
-__global__ __launch_bounds__(1024) void dispatch_place_wide_k(const int * __restrict__ ids, const int * __restrict__ chunk_counts, int * __restrict__ counts,
-                                                              int * __restrict__ offsets, int * __restrict__ perm, int * __restrict__ groups, int capacity,
-                                                              int A, int E, int chunks, DispatchSide side) {
+__global__ __launch_bounds__(1024) __attribute__((amdgpu_waves_per_eu(8))) void dispatch_place_wide_k(
+        const int * __restrict__ ids, const int * __restrict__ chunk_counts, int * __restrict__ counts, int * __restrict__ offsets, int * __restrict__ perm,
+        int * __restrict__ groups, int capacity, int A, int E, int chunks, DispatchSide side) {
     extern __shared__ int hist[];   // kWideWaves x E: group sizes, then each wave's first place
     __shared__ int s_start[kWideExperts], s_all[kWideExperts], s_wave[16];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), chunk = blockIdx.x;
-    const bool last = chunk == chunks;
+    const bool apart = chunk == chunks, plans = apart || (chunk == 0 && int(gridDim.x) == chunks);   // no chunk of its own; writes counts and plan
     const int a = chunk * kChunk + tid;
     int e = a < A ? ids[a] : -1;
     if (e >= E) e = -1;
     int before = 0, all = 0;
-    auto add_up = [&](auto together) {   // so many loads in flight: the loop is latency, not bandwidth
+    const int * cc = chunk_counts;
+    auto add_up = [&](auto together, auto whole, int b0) {   // so many loads in flight: the sums are latency, not bandwidth
         constexpr int N = decltype(together)::value;
-        for (int b0 = 0; b0 < chunks; b0 += N) {
-            int v[N];
+        int v[N];
+        const int * row = cc;
 #pragma unroll
-            for (int q = 0; q < N; ++q) v[q] = chunk_counts[int64_t(min(b0 + q, chunks - 1)) * E + tid];
-#pragma unroll
-            for (int q = 0; q < N; ++q) { all += b0 + q < chunks ? v[q] : 0; before += b0 + q < chunk && b0 + q < chunks ? v[q] : 0; }
+        for (int q = 0; q < N; ++q) {
+            v[q] = decltype(whole)::value || b0 + q < chunks ? row[tid] : 0;
+            row += E;                  // (q * E instead: sixteen lane addresses kept over the trips, 26 registers more)
         }
+#pragma unroll
+        for (int q = 0; q < N; ++q) { all += v[q]; before += b0 + q < chunk ? v[q] : 0; }
     };
     if (tid < E) {
-        if (chunks <= 8) add_up(std::integral_constant<int, 8>{});
-        else add_up(std::integral_constant<int, 24>{});
+        int b0 = 0;
+#pragma unroll 1
+        for (; chunks - b0 > 16; b0 += 16, cc += 16 * E) add_up(std::integral_constant<int, 16>{}, std::true_type{}, b0);
+        if (chunks - b0 <= 8) add_up(std::integral_constant<int, 8>{}, std::false_type{}, b0);
+        else add_up(std::integral_constant<int, 16>{}, std::false_type{}, b0);
     }
-    if (!last)
+    if (!apart)
         for (int j = tid; j < kWideWaves * E; j += 1024) hist[j] = 0;
     // the experts' first places: a prefix sum over the threads
     const int incl = wave_scan(all);
@@ -999,32 +1010,28 @@ __global__ __launch_bounds__(1024) void dispatch_place_wide_k(const int * __rest
     const int rank = __popcll(same & ((1ull << lane) - 1ull)), size = __popcll(same);
     __syncthreads();
     const int waves = row_scan(s_wave[lane & 15]), start = incl - all + (wave ? __builtin_amdgcn_readlane(waves, wave - 1) : 0);
-    if (last) {
-        if (tid < E) { counts[tid] = all; if (offsets) offsets[tid] = start; }
-        if (tid == E - 1 && offsets) offsets[E] = start + all;
-        if (side.item_rows) {
-            if (tid < E) { s_start[tid] = start; s_all[tid] = all; }
-            __syncthreads();
-            plan_items(s_all, s_start, E, side.item_rows, side.items, side.index);
+    if (tid < E) { s_start[tid] = start; s_all[tid] = all; }
+    if (!apart && e >= 0 && rank == size - 1) hist[wave * E + e] = size;
+    __syncthreads();
+    if (!apart) {
+        if (tid < E) {
+            int v[kWideWaves], at = start + before;
+#pragma unroll
+            for (int w = 0; w < kWideWaves; ++w) v[w] = hist[w * E + tid];
+#pragma unroll
+            for (int w = 0; w < kWideWaves; ++w) { hist[w * E + tid] = at; at += v[w]; }
         }
-        return;
+        __syncthreads();
+        if (e >= 0) {
+            const int place = hist[wave * E + e] + rank, slot = place - s_start[e];
+            if (perm) perm[place] = a;
+            if (groups && slot < capacity) groups[int64_t(e) * capacity + slot] = a;
+        }
     }
-    if (e >= 0 && rank == size - 1) hist[wave * E + e] = size;
-    if (tid < E) { s_start[tid] = start; }
-    __syncthreads();
-    if (tid < E) {
-        int v[kWideWaves], at = start + before;
-#pragma unroll
-        for (int w = 0; w < kWideWaves; ++w) v[w] = hist[w * E + tid];
-#pragma unroll
-        for (int w = 0; w < kWideWaves; ++w) { hist[w * E + tid] = at; at += v[w]; }
-    }
-    __syncthreads();
-    if (e >= 0) {
-        const int place = hist[wave * E + e] + rank, slot = place - s_start[e];
-        if (perm) perm[place] = a;
-        if (groups && slot < capacity) groups[int64_t(e) * capacity + slot] = a;
-    }
+    if (!plans) return;
+    if (tid < E) { counts[tid] = all; if (offsets) offsets[tid] = start; }
+    if (tid == E - 1 && offsets) offsets[E] = start + all;
+    if (side.item_rows) plan_items(s_all, s_start, E, side.item_rows, side.items, side.index);
 }
 
 // A <= kChunk: everything in one block
@@ -1154,7 +1161,8 @@ namespace {
 void place_wide(const int32_t * ids, const int * cc, int32_t * counts, int32_t * offsets, int32_t * perm, int32_t * groups, int32_t capacity, int32_t experts, int A,
                 int chunks, const DispatchSide & side, hipStream_t s) {
     allow_dynamic_lds(reinterpret_cast<const void *>(&dispatch_place_wide_k), int(kWideWaves * kWideExperts * sizeof(int)));
-    dispatch_place_wide_k<<<unsigned(chunks) + 1, 1024, size_t(kWideWaves) * experts * sizeof(int), s>>>(ids, cc, counts, offsets, perm, groups, capacity, A, experts, chunks, side);
+    const unsigned blocks = unsigned(chunks) + (side.item_rows && chunks < 256 ? 1 : 0);   // (one more than the compute units would open a second round)
+    dispatch_place_wide_k<<<blocks, 1024, size_t(kWideWaves) * experts * sizeof(int), s>>>(ids, cc, counts, offsets, perm, groups, capacity, A, experts, chunks, side);
 }
 // the launches of tqmoe_dispatch; cc: chunks x experts ints of scratch for more than one chunk. offsets and perm may be
 // null where the caller only wants counts and groups (spare_offsets: experts + 1 ints the scan may use instead).
