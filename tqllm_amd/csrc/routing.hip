@@ -137,38 +137,73 @@ template <bool F32> constexpr int kRouterGemmMin = F32 ? 56000 : 45000;
 constexpr int kRgWaves = 8, kRgRows = 64, kRgPitch = kRgRows + 4;   // floats of a token's row in the exchange space: four rows apart, other banks
 template <int TA> constexpr int kRgLds = 4 * TA * 16 * kRgPitch * int(sizeof(float));
 
-// The gate row's logits of tokens [t0, t1) (zeros without a gate row), a wave a token; and the grid's share of what is to be cleared.
-// A wave has the loads of several tokens and of four passes over its columns under way at once: one after the other they were a chain
-// of trips to memory longer than the blocks beside it (2048 columns: eight tokens a wave were 32 trips).
+// the gate row's logits of tokens [t0, t1) (zeros without a gate row), a wave a token; and the grid's share of what is to be cleared
 template <int XT>
 __device__ __forceinline__ void router_shared_column(const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x, float * __restrict__ logits, int h, int e, int n,
                                                      int t0, int t1, const RouterSide & side, int waves) {
     const int lane = threadIdx.x & 63;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < side.zero_n; i += gridDim.x * blockDim.x) side.zero[i] = 0;
-    constexpr int NT = XT == TQMOE_F32 ? 2 : 4, NP = 4, RAW = XT == TQMOE_F32 ? 2 : 1;   // tokens and passes together, 16-byte loads of eight values
-    for (int t = t0 + int(threadIdx.x >> 6); t < t1; t += NT * waves) {
+    for (int t = t0 + (threadIdx.x >> 6); t < t1; t += waves) {
+        float acc = 0.f;
+        if (shared)
+            for (int c = lane * 8; c < h; c += 512) {
+                float wv[8], xv[8];
+                load8<XT>(shared, c, wv);
+                load8<XT>(x, int64_t(t) * h + c, xv);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) acc = fmaf(wv[j], xv[j], acc);
+            }
+        acc = group_sum<64>(acc);
+        if (lane == 0) logits[int64_t(t) * (e + 1) + e] = acc;
+    }
+}
+
+// The same, in the same order, with the loads of several tokens and of four passes over its columns under way at once: one after the other
+// they are a chain of trips to memory, longer than the blocks beside it where those are short or wait for it (us a launch, one after the other /
+// so: 3500 tokens x 513 rows of 2048 32.3 / 21.4, 6000 x 61 of 4096 38.6 / 27.9, 8192 x 257 of 3072 38.4 / 35.6). Tokens and passes that are
+// not there are branched around: as loads of zeros and of the last token again they cost 512 columns 7 %, two tokens a wave up to 17 %.
+// The loop above stays where the gate row's blocks have time (launch_router_gemm), in the fp32 tiles straight from memory, whose main loop is
+// slower with more code beside it (512 experts, 6000 tokens of 2048 166 / 174, 8192 of 1024 114 / 118), and for shares of one pass in the
+// kernel of large batches (8192 x 513 of 512 19.9 / 20.2).
+template <int XT>
+__device__ __forceinline__ void router_shared_together(const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x, float * __restrict__ logits, int h, int e, int n,
+                                                     int t0, int t1, const RouterSide & side, int waves) {
+    const int lane = threadIdx.x & 63;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < side.zero_n; i += gridDim.x * blockDim.x) side.zero[i] = 0;
+    constexpr int NT = XT == TQMOE_F32 ? 2 : 4, NP = 4, RAW = XT == TQMOE_F32 ? 2 : 1, kSize = XT == TQMOE_F32 ? 4 : 2;   // tokens and passes together, loads of eight values
+    for (int t = t0 + __builtin_amdgcn_readfirstlane(int(threadIdx.x) >> 6); t < t1; t += NT * waves) {
         float acc[NT] = {};
         if (shared)
-            for (int c0 = lane * 8; c0 < h; c0 += NP * 512) {
+            for (int c0 = 0; c0 < h; c0 += NP * 512) {
                 uint4 wr[NP][RAW], xr[NT][NP][RAW];
 #pragma unroll
                 for (int p = 0; p < NP; ++p) {
-                    const int c = c0 + p * 512;          // (past the last column: zeros on both sides)
+                    const int c = c0 + p * 512 + lane * 8;          // (past the last column: zeros on both sides)
 #pragma unroll
                     for (int q = 0; q < RAW; ++q) {
-                        constexpr int kSize = XT == TQMOE_F32 ? 4 : 2;
-                        wr[p][q] = c < h ? *reinterpret_cast<const uint4 *>(shared + int64_t(c) * kSize + q * 16) : uint4();
+                        wr[p][q] = uint4();
+#pragma unroll
+                        for (int i = 0; i < NT; ++i) xr[i][p][q] = uint4();
+                    }
+                    if (c0 + p * 512 < h) {
+                        if (c < h)
+#pragma unroll
+                            for (int q = 0; q < RAW; ++q) wr[p][q] = *reinterpret_cast<const uint4 *>(shared + int64_t(c) * kSize + q * 16);
 #pragma unroll
                         for (int i = 0; i < NT; ++i)
-                            xr[i][p][q] = c < h ? *reinterpret_cast<const uint4 *>(x + (int64_t(min(t + i * waves, t1 - 1)) * h + c) * kSize + q * 16) : uint4();
+                            if (t + i * waves < t1 && c < h)
+#pragma unroll
+                                for (int q = 0; q < RAW; ++q) xr[i][p][q] = *reinterpret_cast<const uint4 *>(x + (int64_t(t + i * waves) * h + c) * kSize + q * 16);
                     }
                 }
 #pragma unroll
                 for (int p = 0; p < NP; ++p) {
+                    if (c0 + p * 512 >= h) break;
                     float wv[8], xv[8];
                     load8<XT>(wr[p], 0, wv);
 #pragma unroll
                     for (int i = 0; i < NT; ++i) {
+                        if (t + i * waves >= t1) break;
                         load8<XT>(xr[i][p], 0, xv);
 #pragma unroll
                         for (int j = 0; j < 8; ++j) acc[i] = fmaf(wv[j], xv[j], acc[i]);
@@ -177,13 +212,15 @@ __device__ __forceinline__ void router_shared_column(const uint8_t * __restrict_
             }
 #pragma unroll
         for (int i = 0; i < NT; ++i) {
+            if (t + i * waves >= t1) break;
             const float sum = group_sum<64>(acc[i]);
-            if (lane == 0 && t + i * waves < t1) logits[int64_t(t + i * waves) * (e + 1) + e] = sum;
+            if (lane == 0) logits[int64_t(t + i * waves) * (e + 1) + e] = sum;
         }
     }
 }
 
-template <bool F32, int TA>
+// TOGETHER: the gate row's blocks have their loads together (launch_router_gemm says when)
+template <bool F32, int TA, bool TOGETHER>
 __global__ __launch_bounds__(64 * kRgWaves) void router_gemm_k(const uint8_t * __restrict__ w, const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x,
                                                               float * __restrict__ logits, int h, int e, int n, RouterSide side) {
     extern __shared__ __attribute__((aligned(16))) float red[];   // [4][TA * 16][kRgPitch]
@@ -192,7 +229,8 @@ __global__ __launch_bounds__(64 * kRgWaves) void router_gemm_k(const uint8_t * _
     const int t0 = int(blockIdx.x) * TT, r0 = int(blockIdx.y) * kRgRows;
     const int64_t pitch = int64_t(h) * kBytes;
     if (blockIdx.y == gridDim.y - 1) {
-        router_shared_column<F32 ? TQMOE_F32 : TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + TT, n), side, kRgWaves);
+        if constexpr (TOGETHER) router_shared_together<F32 ? TQMOE_F32 : TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + TT, n), side, kRgWaves);
+        else router_shared_column<F32 ? TQMOE_F32 : TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + TT, n), side, kRgWaves);
         return;
     }
     const uint8_t * ap[TA], * bp[4];   // rows past the end repeat a valid row (not stored)
@@ -296,7 +334,7 @@ __global__ __launch_bounds__(64 * kRgWaves) void router_gemm_dma_k(const uint8_t
     const int t0 = int(blockIdx.x) * 16, r0 = int(blockIdx.y) * kRgRows;
     const int64_t pitch = int64_t(h) * kBytes;
     if (blockIdx.y == gridDim.y - 1) {
-        router_shared_column<F32 ? TQMOE_F32 : TQMOE_BF16>(shared, x, logits, h, e, n, int(blockIdx.x) * gate, min(int(blockIdx.x + 1) * gate, n), side, kRgWaves);
+        router_shared_together<F32 ? TQMOE_F32 : TQMOE_BF16>(shared, x, logits, h, e, n, int(blockIdx.x) * gate, min(int(blockIdx.x + 1) * gate, n), side, kRgWaves);
         return;
     }
     // transfer q: rows 8 q .. + 7, the tokens' in front of the router's (past the end a valid row again, not stored); a row's 16-byte piece p
@@ -397,7 +435,7 @@ __global__ __launch_bounds__(64 * kRlWaves) void router_gemm_lds_k(const uint8_t
     // The gate row's column: a last row of blocks where they find compute units free, else every block's share of its tokens.
     const int cols = (e + kRlRows - 1) / kRlRows;
     if (int(blockIdx.y) == cols) {
-        router_shared_column<TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + kRlTok, n), side, kRlWaves);
+        router_shared_together<TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + kRlTok, n), side, kRlWaves);
         return;
     }
     // transfer q of a wave is eight rows of a stage: the tokens' rows, then the router's; a row's 16-byte piece p in slot
@@ -431,7 +469,9 @@ __global__ __launch_bounds__(64 * kRlWaves) void router_gemm_lds_k(const uint8_t
     for (int i = 0; i < kRlRing - 1; ++i) send();
     if (int(gridDim.y) == cols) {   // (under the first transfers)
         const int share = (kRlTok + cols - 1) / cols, first_t = t0 + int(blockIdx.y) * share;
-        router_shared_column<TQMOE_BF16>(shared, x, logits, h, e, n, first_t, min(min(first_t + share, t0 + kRlTok), n), side, kRlWaves);
+        const int last_t = min(min(first_t + share, t0 + kRlTok), n);
+        if (h > 512) router_shared_together<TQMOE_BF16>(shared, x, logits, h, e, n, first_t, last_t, side, kRlWaves);
+        else router_shared_column<TQMOE_BF16>(shared, x, logits, h, e, n, first_t, last_t, side, kRlWaves);
     }
     const int tq = wave & 1, rq = wave >> 1;
     const uint8_t * a_row = lds + (tq * 32 + r) * 128, * b_row = lds + (kRlTok + rq * 32 + r) * 128;
@@ -492,9 +532,17 @@ __global__ __launch_bounds__(64 * kRlWaves) void router_gemm_lds_k(const uint8_t
 template <bool F32> void launch_router_gemm(const void * w, const void * sg, const void * x, float * logits, int h, int e, int n, const RouterSide & side, hipStream_t s) {
     const int64_t rows = (e + kRgRows - 1) / kRgRows;
     auto blocks = [&](int ta) { return ((n + 16 * ta - 1) / (16 * ta)) * rows; };
-    auto go = [&](auto kernel, int ta, int lds) {
-        allow_dynamic_lds(reinterpret_cast<const void *>(kernel), lds);
-        kernel<<<dim3(unsigned((n + 16 * ta - 1) / (16 * ta)), unsigned(rows + 1)), 64 * kRgWaves, lds, s>>>(
+    auto go = [&](auto tile) {
+        constexpr int TA = decltype(tile)::value;
+        const int tiles = (n + 16 * TA - 1) / (16 * TA);
+        auto kernel = &router_gemm_k<F32, TA, false>;
+        // The gate row's blocks have their loads together where they open another round of the compute units. Beside the last one they have its
+        // time, and together take from its blocks' bandwidth (bf16, us, one after the other / together: 256 blocks of 64 tokens and 128 of the
+        // gate row 19.9 / 17.0, 440 and 55 42.4 / 43.3, 128 and 128 32.8 / 34.4).
+        if constexpr (!F32)
+            if ((blocks(TA) - 1) % 256 + 1 + tiles > 256) kernel = &router_gemm_k<F32, TA, true>;
+        allow_dynamic_lds(reinterpret_cast<const void *>(kernel), kRgLds<TA>);
+        kernel<<<dim3(unsigned(tiles), unsigned(rows + 1)), 64 * kRgWaves, kRgLds<TA>, s>>>(
             static_cast<const uint8_t *>(w), static_cast<const uint8_t *>(sg), static_cast<const uint8_t *>(x), logits, h, e, n, side);
     };
     const bool aligned = aligned16(w) && aligned16(x), long_rows = int64_t(h) * (F32 ? 4 : 2) >= 4096;
@@ -528,9 +576,9 @@ template <bool F32> void launch_router_gemm(const void * w, const void * sg, con
     }
     // (2048 columns, us with 16 / 32 / 64 tokens a block: bf16, 128 blocks of 32 tokens 14.9 / 13.5 / 17.6, 128 of 64 28 / 21 / 19; fp32, 128
     // blocks of 32 tokens 27 / 43 / 71, 256 of 64 106 / 85 / 79)
-    if (blocks(4) >= (F32 ? 256 : 128)) go(&router_gemm_k<F32, 4>, 4, kRgLds<4>);
-    else if (blocks(2) >= (F32 ? 256 : 128)) go(&router_gemm_k<F32, 2>, 2, kRgLds<2>);
-    else go(&router_gemm_k<F32, 1>, 1, kRgLds<1>);
+    if (blocks(4) >= (F32 ? 256 : 128)) go(std::integral_constant<int, 4>{});
+    else if (blocks(2) >= (F32 ? 256 : 128)) go(std::integral_constant<int, 2>{});
+    else go(std::integral_constant<int, 1>{});
 }
 
 // ------------------------------------------------------------------------------------------------------ top-k
