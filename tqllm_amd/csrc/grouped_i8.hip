@@ -15,7 +15,7 @@ int grouped_i8_per_item(bool blocks, int64_t assignments, int experts) { return 
 void enqueue_grouped_i8(const tqmoe_bank & b0, const tqmoe_bank * b1, const int8_t * x, const float * xs, bool blocks, const int * perm, const int4 * plan, int64_t assignments,
                         int xdiv, void * out, float * out_scale, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows) {
     const int tiles = b0.rows / 32, per = b1 ? 4 : 8, groups = (tiles + per - 1) / per;
-    const GroupedArgs k{view(b0), b1 ? view(*b1) : view(b0), x, xs, perm, plan, xdiv, out, groups, shared_expert, shared_lim, glu, 0, 0, out_scale};
+    const GroupedArgs k{view(b0), b1 ? view(*b1) : view(b0), x, xs, perm, plan, xdiv, out, groups, shared_expert, shared_lim, glu, 0, out_scale};
     // (an XCD takes an eighth of every one of the four classes, rounded up)
     const unsigned grid = unsigned((grouped_rows_items(assignments, b0.experts, item_rows) + 28) / 8 * 8 * groups);
     if (blocks) grouped_i8_launch<TQMOE_IQ4_XS, true>(k, item_rows, b1 != nullptr, grid, s);

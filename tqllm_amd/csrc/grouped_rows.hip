@@ -60,9 +60,9 @@ void enqueue_grouped_plan(const int * counts, const int * offsets, int experts, 
 
 // assignments: total entries of perm (it bounds the items)
 void enqueue_grouped_products(const tqmoe_bank & b0, const tqmoe_bank * b1, const void * x, const float * xs, const int * perm, const int4 * plan, int64_t assignments,
-                         int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows, bool row_tiles, bool out_bf16) {
+                         int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows, bool row_tiles) {
     const int tiles = b0.rows / 32, per = b1 ? 4 : 8, groups = (tiles + per - 1) / per;
-    const GroupedArgs k{view(b0), b1 ? view(*b1) : view(b0), x, xs, perm, plan, xdiv, out, groups, shared_expert, shared_lim, glu, row_tiles, out_bf16, nullptr};
+    const GroupedArgs k{view(b0), b1 ? view(*b1) : view(b0), x, xs, perm, plan, xdiv, out, groups, shared_expert, shared_lim, glu, row_tiles, nullptr};
     // (an XCD takes an eighth of every one of the four classes, rounded up)
     const unsigned blocks = unsigned((grouped_rows_items(assignments, b0.experts, item_rows) + 28) / 8 * 8 * groups);
     switch (b0.type) {

@@ -22,7 +22,6 @@ struct GroupedArgs {
     int shared_lim;
     Glu glu;
     int row_tiles;            // NVFP4G: x is in operand-major row tiles (each expert's rows padded to whole tiles), xs by row of those
-    int out_bf16;             // NVFP4G: 16-bit results are bf16
     float * out_scale;        // int8 gate / up with a scale per 32 values: the scales of the act rows, [assignments][rows / 32]
 };
 
@@ -42,7 +41,7 @@ void enqueue_prepare_rows(const void * x, uint32_t xtype, int64_t rows, int cols
 void enqueue_grouped_plan(const int * counts, const int * offsets, int experts, int item_rows, int4 * plan, const RowIndex & index, hipStream_t s);
 // assignments: total entries of perm (it bounds the items)
 void enqueue_grouped_products(const tqmoe_bank & b0, const tqmoe_bank * b1, const void * x, const float * xs, const int * perm, const int4 * plan, int64_t assignments,
-                              int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows, bool row_tiles = false, bool out_bf16 = false);
+                              int xdiv, void * out, bool f32_out, int shared_expert, int shared_lim, Glu glu, hipStream_t s, int item_rows, bool row_tiles = false);
 
 // int8 products on rows in quantiser order (a row per token or per assignment); blocks: a scale per 32 values
 bool grouped_i8_takes(uint32_t type, int rows, int cols);

@@ -276,7 +276,7 @@ template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
     static constexpr bool kFp8 = true;
     static constexpr int kCodes = 2, kRecs = 1, kTab = 256 * 8;
     // Per scale byte the products e2m1(code) * e4m3(scale) / 8 of the eight codes without a sign, rounded to E4M3 (nearest even; an
-    // eighth keeps the largest inside the format, row_factors gives it back): rounding and limit know no sign, so that a code's own is
+    // eighth keeps the largest, 6 * 448, inside the format, row_factors gives it back): rounding knows no sign, so that a code's own is
     // bit 7 of the result.
     static __device__ __forceinline__ void tables(uint8_t * tab, int tid) {
         const float sc = e4m3_to_float(uint32_t(tid));
@@ -285,7 +285,7 @@ template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
         for (int q = 0; q < 2; ++q) {
             float f[4];
 #pragma unroll
-            for (int j = 0; j < 4; ++j) f[j] = fminf(fmaxf(float(((q == 0 ? kFp4T0 : kFp4T1) >> (8 * j)) & 0xFFu) * 0.0625f * sc, -448.f), 448.f);
+            for (int j = 0; j < 4; ++j) f[j] = float(((q == 0 ? kFp4T0 : kFp4T1) >> (8 * j)) & 0xFFu) * 0.0625f * sc;
             const int w = __builtin_amdgcn_cvt_pk_fp8_f32(f[0], f[1], 0, false);
             v[q] = uint32_t(__builtin_amdgcn_cvt_pk_fp8_f32(f[2], f[3], w, true));
         }
@@ -330,14 +330,9 @@ template <> struct GroupedFormat<TQMOE_NVFP4G> : GroupedWhole {
     }
 };
 
-// 16-bit results: halves, or (a kernel of its own: a branch at every pair cost more than the arithmetic) bf16
-struct Bf16Row { uint16_t v; };
-template <class OT, bool PIN> __device__ __forceinline__ uint32_t pair16(float x, float y) {
-    if constexpr (std::is_same<OT, Bf16Row>::value) return float_to_bf16_bits(x) | uint32_t(float_to_bf16_bits(y)) << 16;
-    else {
-        if constexpr (PIN) asm("" : "+v"(x), "+v"(y));   // (the product is rounded before it is converted)
-        return bits_of(v2h{_Float16(x), _Float16(y)});
-    }
+template <bool PIN> __device__ __forceinline__ uint32_t half_pair(float x, float y) {
+    if constexpr (PIN) asm("" : "+v"(x), "+v"(y));   // (the product is rounded before it is converted)
+    return bits_of(v2h{_Float16(x), _Float16(y)});
 }
 
 // bytes of a wave's codes and records of one stage
@@ -611,8 +606,8 @@ __global__ __launch_bounds__(256, (kGroupedWaves<GroupedFormat<FMT>, MAX>)) void
                         }
                     } else if constexpr (sizeof(OT) == 4) *reinterpret_cast<float4 *>(to + (8 * c + 4 * g) * 4) = make_float4(q[0], q[1], q[2], q[3]);
                     else if constexpr (GATEUP && !W::kFp8)   // operand_pos: the four values stay together, 1 and 2 change places
-                        *reinterpret_cast<uint2 *>(to + operand_pos(8 * c + 4 * g) * 2) = make_uint2(pair16<OT, W::kFp8>(q[0], q[2]), pair16<OT, W::kFp8>(q[1], q[3]));
-                    else *reinterpret_cast<uint2 *>(to + (8 * c + 4 * g) * 2) = make_uint2(pair16<OT, W::kFp8>(q[0], q[1]), pair16<OT, W::kFp8>(q[2], q[3]));
+                        *reinterpret_cast<uint2 *>(to + operand_pos(8 * c + 4 * g) * 2) = make_uint2(half_pair<W::kFp8>(q[0], q[2]), half_pair<W::kFp8>(q[1], q[3]));
+                    else *reinterpret_cast<uint2 *>(to + (8 * c + 4 * g) * 2) = make_uint2(half_pair<W::kFp8>(q[0], q[1]), half_pair<W::kFp8>(q[2], q[3]));
                 }
                 __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
                 __builtin_amdgcn_wave_barrier();
@@ -637,9 +632,6 @@ template <uint32_t FMT, int MAX> void grouped_rows_launch_max(const GroupedArgs 
         allow_dynamic_lds(reinterpret_cast<const void *>(kernel), bytes);
         kernel<<<blocks, 256, bytes, s>>>(k);
     };
-    if constexpr (GroupedFormat<FMT>::kFp8) {
-        if (k.out_bf16 && !f32_out) return gateup ? go(&grouped_rows_k<FMT, MAX, true, Bf16Row>) : go(&grouped_rows_k<FMT, MAX, false, Bf16Row>);
-    }
     if (gateup) {
         if constexpr (MAX > 1 || GroupedFormat<FMT>::kFold) go(&grouped_rows_k<FMT, MAX, true, uint16_t>);   // (grouped_rows_per_item)
     } else if (f32_out) go(&grouped_rows_k<FMT, MAX, false, float>);

@@ -311,7 +311,7 @@ int32_t enqueue_plane_gemm(const tqmoe_bank & b0, const tqmoe_bank * b1, const i
     if (plane_gemm_is_fp8(b0.type)) {   // on the same gathered rows, by the kernels that also take them ungathered
         const Plan plan = plan_at(plan_from ? plan_from : xs, grouped_row_tiles(assignments, experts) * 32, experts);
         enqueue_grouped_products(b0, gateup ? b1 : nullptr, xq, xs, perm, plan.items, assignments, 1, out_f16, false, shared_expert, shared_lim, glu, s,
-                                 grouped_rows_per_item(TQMOE_NVFP4G, assignments, experts), true, out_bf16 != 0);
+                                 grouped_rows_per_item(TQMOE_NVFP4G, assignments, experts), true);
         return 0;
     }
     const int nb = gateup || b0.rows % 64 == 0 ? 2 : 1;
