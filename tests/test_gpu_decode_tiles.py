@@ -38,3 +38,27 @@ def test_decode_products(oracle, fmt, rows, cols, n, experts):
         want = np.stack([dec[e] @ rows_in[a].astype(np.float64) for a, e in enumerate(ids.reshape(-1))])
         mx, rel = synth.errors(got.cpu().numpy(), want)
         assert rel < 2e-4 and mx < 1e-3, (mx, rel)
+
+
+@pytest.mark.parametrize("fmt", sorted(FORMATS))
+@pytest.mark.parametrize("assignments", [512, 513, 1024, 1025, 2048])
+def test_rows_of_a_block_are_found_past_the_first_ids(oracle, fmt, assignments):
+    """A block finds its expert's rows 512 ids at a time: an expert with four rows on both sides of id 512, one whose first row comes
+    behind it, one with many, ids that are skipped, the last id of the most one launch takes."""
+    import tqllm_amd as tq
+    wtype, rows, cols, experts = FORMATS[fmt], 64, 256, 9
+    rng = np.random.default_rng(assignments)
+    raw = oracle.quantize(wtype, (rng.standard_normal((experts * rows, cols)) * 0.02).astype(np.float32))
+    bank = tq.ExpertBank(wtype, raw, experts, rows, cols)
+    dec = oracle.dequantize(wtype, raw, experts * rows * cols).reshape(experts, rows, cols).astype(np.float64)
+    ids = rng.integers(0, 6, assignments).astype(np.int32)
+    ids[rng.random(assignments) < 0.05] = -1
+    ids[[i for i in (63, 505, 511, 512, 513, 1023, 1024) if i < assignments]] = 6       # its blocks: 63 .. 512, 513 .. 1024
+    ids[[i for i in (514, 600, 1030) if i < assignments]] = 7
+    ids[-1] = 8
+    x = rng.standard_normal((assignments, cols)).astype(np.float32)
+    image, dev_ids, live = tq.quant_act(dev(x)), dev(ids[:, None]), ids >= 0
+    want = np.stack([dec[e] @ x[a].astype(np.float64) for a, e in enumerate(ids) if e >= 0])
+    for got in (*tq.expert_matvec2(bank, bank, image, dev_ids), tq.expert_matvec(bank, image, dev_ids)):
+        mx, rel = synth.errors(got.cpu().numpy().reshape(assignments, rows)[live], want)
+        assert rel < 2e-4 and mx < 1e-3, (mx, rel)
