@@ -166,8 +166,23 @@ def test_fp8_weights_of_every_scale_byte_and_code(tq, oracle):
     rows, cols, g = 32, 256, 0.01
     raw = np.zeros((rows * cols // 128, 76), np.uint8)
     raw[:, :4] = np.frombuffer(np.float32(g).tobytes(), np.uint8)
-    raw[:, 4:12] = np.arange(256, dtype=np.uint8).reshape(-1, 8)[np.arange(rows * cols // 128) % 32]
-    raw[:, 12:] = (np.arange(64) * 0x21 + 0x10 + np.arange(len(raw))[:, None] * 0x33) & 0xFF
+    # every scale byte twice, at an even and at an odd place of its block (the bank keeps two groups' codes in the two nibbles of a byte);
+    # each time all sixteen codes, and both times together each of them in either nibble
+    j = np.arange(8, dtype=np.uint8)
+    raw[:32, 4:12] = np.arange(256, dtype=np.uint8).reshape(32, 8)
+    raw[32:, 4:12] = raw[:32, 4:12][:, j ^ 1]
+    raw[:32, 12:] = np.tile((15 - j) << 4 | j, 8)
+    raw[32:, 12:] = np.tile((7 - j) << 4 | (8 + j), 8)
+    groups = {}
+    for block in raw:
+        for at in range(8):
+            groups.setdefault(int(block[4 + at]), []).append((at & 1, block[12 + 8 * at:20 + 8 * at]))
+    assert len(groups) == 256
+    for places in groups.values():
+        assert sorted(odd for odd, _ in places) == [0, 1]
+        assert all(len({int(c) & 15 for c in b} | {int(c) >> 4 for c in b}) == 16 for _, b in places)
+        both = np.concatenate([b for _, b in places])
+        assert len(set(both & 15)) == 16 and len(set(both >> 4)) == 16
     raw = raw.reshape(-1)
     want = oracle.dequantize_nvfp4_widened(raw, rows * cols).reshape(rows, cols).astype(np.float64)
     bank = tq.ExpertBank(tq.NVFP4G, torch.from_numpy(raw).cuda(), 1, rows, cols)
