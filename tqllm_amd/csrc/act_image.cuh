@@ -76,7 +76,8 @@ __device__ __forceinline__ void quantise_block(const float (&v)[32], uint8_t * i
     reinterpret_cast<float *>(image_row + int64_t(S) * 68)[s] = float(qsum) * scale;
 }
 
-// a value and the one sixteen lanes further on or back, in the lane's row of 32: one instruction (a shuffle is a trip through LDS)
+// a value and the one sixteen lanes further on or back, in the lane's row of 32: one instruction (a shuffle is a trip through LDS; 0.1 to 0.2 %
+// of a layer of up to 32 tokens)
 __device__ __forceinline__ int2 both_rows(int v) {
     const auto r = __builtin_amdgcn_permlane16_swap(uint32_t(v), uint32_t(v), false, false);
     return make_int2(int(r[0]), int(r[1]));

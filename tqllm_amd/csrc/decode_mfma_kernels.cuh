@@ -233,7 +233,8 @@ template <> struct MfmaFormat<TQMOE_Q6_K> : MfmaBase {
 
 // NB banks (gate and up, or one). gateup != 0: out0 is the activation image that receives silu(gate) * up; else out0 /
 // out1 receive the products as rows of `ytype`. wk waves share a row's super-blocks, tpw row tiles per block.
-// Dynamic LDS: the match list and the copy of the ids while the block finds its input rows, later the partial sums.
+// Dynamic LDS: the partial sums and, behind them, the input rows' planes and scales (MODE 1, 2): nothing of the one lies in the other, so that a
+// pass's sums need no barrier in front but where another pass (MODE 2) has left its own there.
 // UNI: every sub-block of an input row has the row's one activation scale (the images tqmoe_quant_act and the top-k
 // kernel write). The 6-bit weight scales then multiply the integer results and the sums stay integers over a whole
 // super-block; otherwise (rows quantised block by block, as the fused gate / up epilogue leaves them) each sub-block's

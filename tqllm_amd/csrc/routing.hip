@@ -131,8 +131,11 @@ template <int WT> int32_t launch_router_x(uint32_t xtype, const void * w, const 
 // The last row of blocks takes the shared expert's gate row (or stores its zeros): a wave a token.
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
-// Tokens x router rows from which a router and input of one type take the GEMM (us, wave per row / GEMM, 2048 columns: bf16 32768
-// 8.4 / 10.8, 62464 14.3 / 10.7; fp32 33000 14.4 / 24.5, 62464 28.2 / 24.5; 1024 to 4096 columns cross at the same sizes).
+// Tokens x router rows from which a router and input of one type take the GEMM. Drawn for tiles straight from memory, which bf16 rows that are not
+// aligned have (us, wave per row / GEMM, 40000: 1024 columns 6.9 / 7.3, 2048 9.6 / 11.7, 4096 17.5 / 20.5). Aligned rows, whose small tiles go
+// through LDS, cross at fewer: bf16 with 4096 columns at 12300 to 16400 (7.9 / 8.6, 9.8 / 8.6), with 2048 at 20000 (6.8 / 6.5; 32800 8.7 / 6.5),
+// with 1024 at 24600 (5.5 / 5.4; 40000 6.9 / 5.5); fp32 with 4096 at 24600 (28.4 / 26.7), with 2048 at 24600 to 32800 (14.0 / 15.7, 17.5 /
+// 15.8), with 1024 at 45000 (9.9 / 9.9).
 template <bool F32> constexpr int kRouterGemmMin = F32 ? 56000 : 45000;
 constexpr int kRgWaves = 8, kRgRows = 64, kRgPitch = kRgRows + 4;   // floats of a token's row in the exchange space: four rows apart, other banks
 template <int TA> constexpr int kRgLds = 4 * TA * 16 * kRgPitch * int(sizeof(float));
