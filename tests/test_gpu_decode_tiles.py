@@ -41,10 +41,10 @@ def test_decode_products(oracle, fmt, rows, cols, n, experts):
 
 
 @pytest.mark.parametrize("fmt", sorted(FORMATS))
-@pytest.mark.parametrize("assignments", [512, 513, 1024, 1025, 2048])
+@pytest.mark.parametrize("assignments", [64, 65, 192, 193, 512, 513, 1024, 1025, 2048])
 def test_rows_of_a_block_are_found_past_the_first_ids(oracle, fmt, assignments):
-    """A block finds its expert's rows 512 ids at a time: an expert with four rows on both sides of id 512, one whose first row comes
-    behind it, one with many, ids that are skipped, the last id of the most one launch takes."""
+    """A block finds its expert's rows in 192 ids at once, or 512 at a time: an expert with four rows on both sides of id 512, one whose first row
+    comes behind it, one with many, ids that are skipped, the last id of the most one launch takes."""
     import tqllm_amd as tq
     wtype, rows, cols, experts = FORMATS[fmt], 64, 256, 9
     rng = np.random.default_rng(assignments)
