@@ -133,9 +133,11 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 // Tokens x router rows from which a router and input of one type take the GEMM. Drawn for tiles straight from memory, which bf16 rows that are not
 // aligned have (us, wave per row / GEMM, 40000: 1024 columns 6.9 / 7.3, 2048 9.6 / 11.7, 4096 17.5 / 20.5). Aligned rows, whose small tiles go
-// through LDS, cross at fewer: bf16 with 4096 columns at 12300 to 16400 (7.9 / 8.6, 9.8 / 8.6), with 2048 at 20000 (6.8 / 6.5; 32800 8.7 / 6.5),
-// with 1024 at 24600 (5.5 / 5.4; 40000 6.9 / 5.5); fp32 with 4096 at 24600 (28.4 / 26.7), with 2048 at 24600 to 32800 (14.0 / 15.7, 17.5 /
-// 15.8), with 1024 at 45000 (9.9 / 9.9).
+// through LDS, cross at fewer (31 to 1000 experts; us at 33000): bf16 with 1024 columns at 26000 (5.7 / 5.0), with 2048 at 22000 (8.0 / 6.1), with 4096
+// at 16000 (13.1 / 8.2); fp32 with 1024 at 45000, with 2048 at 33000 to 41000 (13.5 / 15.3 to 18.3 / 15.5), with 4096 at 24000 to 33000 (34 / 27).
+// The line stays for them as well: eight slices of a row on the matrix pipe are further from 64 bits than a wave's sums (root of the mean square over
+// the logits', wave per row / GEMM: bf16 2048 columns 7.5e-8 / 9.8e-8, 4096 8.4e-8 / 1.33e-7; fp32 1.23e-7 / 2.89e-7, 1.59e-7 / 4.07e-7), and no
+// batch is to get coarser logits than it had.
 template <bool F32> constexpr int kRouterGemmMin = F32 ? 56000 : 45000;
 constexpr int kRgWaves = 8, kRgRows = 64, kRgPitch = kRgRows + 4;   // floats of a token's row in the exchange space: four rows apart, other banks
 template <int TA> constexpr int kRgLds = 4 * TA * 16 * kRgPitch * int(sizeof(float));
