@@ -84,11 +84,13 @@ def test_router_gemm_path_f32(tq, oracle, n, e, h, shared):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("n,e,h", [(1000, 63, 64), (897, 64, 128), (120, 500, 192), (333, 513, 320), (512, 512, 2048), (1500, 65, 2112), (3100, 60, 1024), (30, 2000, 512),
-                                   (7000, 512, 1024), (1800, 512, 1024), (3500, 64, 576), (6000, 64, 1088)])
+                                   (7000, 512, 1024), (1800, 512, 1024), (3500, 64, 576), (6000, 64, 1088), (4096, 128, 1024), (3500, 500, 1088), (7000, 384, 1088),
+                                   (2100, 1000, 1024)])
 def test_router_gemm_by_alignment(tq, dtype, n, e, h):
     """Rows aligned to 16 bytes go through LDS in tiles of 16 tokens, others straight from memory: the same sums in the same order,
-    slices of the columns of an odd number of 64-byte steps and ragged last tiles among them. The last four: fp32 rows of four rounds of
-    64 tokens; the gate row's blocks in another round than the tiles', of 64, 16 and 32 tokens."""
+    slices of the columns of an odd number of 64-byte steps and ragged last tiles among them. The last eight: fp32 rows of four rounds of
+    64 tokens; the gate row's blocks in another round than the tiles', of 64, 16 and 32 tokens; in the bf16 kernel of large batches such blocks
+    in the tiles' round and in another, shares of the tiles' blocks with many tokens and with few."""
     gen = torch.Generator().manual_seed(n + e + h)
     w, gate, x = (torch.randn(*size, generator=gen).to(dtype).cuda() for size in ((e, h), (h,), (n, h)))
     off = 8 // w.element_size()

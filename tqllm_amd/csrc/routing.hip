@@ -168,8 +168,10 @@ __device__ __forceinline__ void router_shared_column(const uint8_t * __restrict_
 // so: 3500 tokens x 513 rows of 2048 32.3 / 21.4, 6000 x 61 of 4096 38.6 / 27.9, 8192 x 257 of 3072 38.4 / 35.6). Tokens and passes that are
 // not there are branched around: as loads of zeros and of the last token again they cost 512 columns 7 %, two tokens a wave up to 17 %.
 // The loop above stays where the gate row's blocks have time (launch_router_gemm), in the fp32 tiles straight from memory, whose main loop is
-// slower with more code beside it (512 experts, 6000 tokens of 2048 166 / 174, 8192 of 1024 114 / 118), and for shares of one pass in the
-// kernel of large batches (8192 x 513 of 512 19.9 / 20.2).
+// slower with more code beside it (512 experts, 6000 tokens of 2048 166 / 174, 8192 of 1024 114 / 118), and in the kernel of large batches for
+// blocks of the gate row's own that are all resident beside the others (8192 tokens x 129 rows of 7168 56.4 / 59.0, 5000 x 193 of 4096 35.3 / 36.3) and
+// for shares of up to four passes a wave (8192 x 513 of 512 19.9 / 20.2, 3072 x 1001 of 768 24.0 / 25.2, 7168 x 701 of 640 31.4 / 32.7; longer ones
+// gain: 8192 x 385 of 1024 29.7 / 27.8).
 template <int XT>
 __device__ __forceinline__ void router_shared_together(const uint8_t * __restrict__ shared, const uint8_t * __restrict__ x, float * __restrict__ logits, int h, int e, int n,
                                                      int t0, int t1, const RouterSide & side, int waves) {
@@ -440,7 +442,8 @@ __global__ __launch_bounds__(64 * kRlWaves) void router_gemm_lds_k(const uint8_t
     // The gate row's column: a last row of blocks where they find compute units free, else every block's share of its tokens.
     const int cols = (e + kRlRows - 1) / kRlRows;
     if (int(blockIdx.y) == cols) {
-        router_shared_together<TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + kRlTok, n), side, kRlWaves);
+        if (gridDim.x * gridDim.y > 256) router_shared_together<TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + kRlTok, n), side, kRlWaves);
+        else router_shared_column<TQMOE_BF16>(shared, x, logits, h, e, n, t0, min(t0 + kRlTok, n), side, kRlWaves);
         return;
     }
     // transfer q of a wave is eight rows of a stage: the tokens' rows, then the router's; a row's 16-byte piece p in slot
@@ -475,7 +478,7 @@ __global__ __launch_bounds__(64 * kRlWaves) void router_gemm_lds_k(const uint8_t
     if (int(gridDim.y) == cols) {   // (under the first transfers)
         const int share = (kRlTok + cols - 1) / cols, first_t = t0 + int(blockIdx.y) * share;
         const int last_t = min(min(first_t + share, t0 + kRlTok), n);
-        if (h > 512) router_shared_together<TQMOE_BF16>(shared, x, logits, h, e, n, first_t, last_t, side, kRlWaves);
+        if (h > 512 && share * ((h + 511) / 512) > 32) router_shared_together<TQMOE_BF16>(shared, x, logits, h, e, n, first_t, last_t, side, kRlWaves);
         else router_shared_column<TQMOE_BF16>(shared, x, logits, h, e, n, first_t, last_t, side, kRlWaves);
     }
     const int tq = wave & 1, rq = wave >> 1;
