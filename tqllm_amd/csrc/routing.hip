@@ -562,8 +562,9 @@ template <bool F32> void launch_router_gemm(const void * w, const void * sg, con
     // 19.1, 24.2 / 19.6, 1024 columns 11.0 / 12.2, 14.2 / 12.3. fp32, beside 32 tokens, 512 and 768 blocks: 2048 columns 32.0 / 39.0, 46.1 / 65.0,
     // 1024 18.8 / 22.0, 27.0 / 36.4, but 512 13.7 / 13.0; beside 64 tokens, a round of 256 blocks, one and a half, two: 2048 columns 60 / 60,
     // 88 / 110, 120 / 115, 1024 35 / 32, 52 / 53, 70 / 59; by rounds of 16 and of 64 tokens, 1024 columns, 7 and 2 59.7 / 59.9, 10 and 3 84.5 / 87.1,
-    // 14 and 4 119 / 109, 2048 columns 14 and 4 197 / 211)
-    if (aligned && (F32 ? blocks(2) < 256 || (long_rows && (blocks(4) < 256 || (h >= 2048 ? 11 * rounds(1) < 40 * rounds(4) : 5 * rounds(1) < 17 * rounds(4))))
+    // 14 and 4 119 / 109, 2048 columns 14 and 4 197 / 211; 10 and 3, fewer experts: 1024 columns, 8192 tokens x 320 86.9 / 81.3, 10000 x 256 88.0 / 83.2, but
+    // 1792 columns 134 / 153, 136 / 156)
+    if (aligned && (F32 ? blocks(2) < 256 || (long_rows && (blocks(4) < 256 || (h >= 2048 ? 11 * rounds(1) < 40 * rounds(4) : h > 1024 ? 5 * rounds(1) < 17 * rounds(4) : 3 * rounds(1) < 10 * rounds(4))))
                         : blocks(2) < 128 || (long_rows && blocks(1) <= (e > kRgRows ? 512 : 256)))) {
         // a block of the gate row's takes 32 tokens instead of 16 where all of short rows' blocks nearly fit the chip at once (64 experts, 1024
         // columns: 2100 tokens 5.9 us against 6.4, 3072 7.0 against 8.4; 2048 columns 8.1 against 7.4, and fp32 no better either)
