@@ -24,7 +24,7 @@
 // instructions; with the two banks' eight accumulators (128 registers) two waves fit a SIMD, and one of them decodes while
 // the other's products run. Items of one and two row tiles have loops of their own with fewer products.
 //
-// What bounds it (profiles/grouped_rows_counters.txt): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 228 us, 0.90
+// What bounds it (counters: profiles/grouped_rows_counters.txt, of a card on which these launches take 5 % longer): Q4_K, 4096 tokens of 8 experts of 64, gate / up (206 GFLOP): 228 us, 0.90
 // PFLOP/s, matrix pipe 48 % busy, vector pipe 53 % (262 us with biased codes; without the decode 205, without the row reads as
 // well 178, where a large fp16 product on this card would take 170); NVFP4G, 8192 tokens, gate / up (2.1 TFLOP with down): 808 us,
 // 49 % and 52 % (880, 43 % and 55 % with the sign in the table of a scale's weights). A product holds its SIMD's vector issue for about 18 cycles besides its own time, so that a stage's decode does not
